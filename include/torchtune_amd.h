@@ -496,6 +496,27 @@ int ttamd_dequantize_per_group_uint4(const uint8_t* q, const float* scale, const
                                      int64_t K, int group_size, void* out, void* stream);
 
 /*
+ * Forward of the converted linears at few tokens, from the integer weight itself (recipes/quantize.py:92-95 saves such
+ * models, generation and evaluation run them): y = x . dequant(q)^T (+ bias), x and y bf16, fp32 accumulation, one rounding.
+ *   ttamd_int8_group_linear_bf16:  q int8 [N,K] holding int4 values, scale / zero_point [N, K/group_size] in the dtype
+ *     `qparam_dtype` names (zero_point may be NULL = 0); x is the already fake-quantised activation.  The expanded
+ *     values are those of ttamd_dequantize_per_group_int4.
+ *   ttamd_uint4_group_linear_bf16: q uint8 [N, K/2] (even element in the high nibble), scales_and_zeros bf16
+ *     [K/group_size, N, 2]; the expanded values are those of ttamd_dequantize_per_group_uint4.
+ * x [M,K], y [M,N], bias [N] or NULL.  ttamd_int4_linear_applies says which sizes are served (at most 256 tokens,
+ * N >= 256 a multiple of 64, K a multiple of 32, group_size a power of two from 32 up that divides K); anything else returns
+ * TTAMD_EUNSUPPORTED.  workspace: ttamd_int4_linear_workspace_bytes(M, N, K) bytes (0: may be NULL).
+ */
+int ttamd_int4_linear_applies(int64_t M, int64_t N, int64_t K, int group_size);
+size_t ttamd_int4_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int ttamd_int8_group_linear_bf16(const void* x, const int8_t* q, const void* scale, const void* zero_point, int qparam_dtype,
+                                 int group_size, const void* bias, void* y, int64_t M, int64_t N, int64_t K, void* workspace,
+                                 size_t workspace_bytes, void* stream);
+int ttamd_uint4_group_linear_bf16(const void* x, const uint8_t* q, const void* scales_and_zeros, int group_size,
+                                  const void* bias, void* y, int64_t M, int64_t N, int64_t K, void* workspace,
+                                  size_t workspace_bytes, void* stream);
+
+/*
  * Conventions of the fake-quant schemes that differ between versions of the third-party package the reference takes
  * them from (torchao; the reference pins no version).  The plain entry points above use the defaults below; the `_conv`
  * variants take the same arguments plus a pointer to this struct (NULL = defaults), so a deployment that pins another

@@ -1,0 +1,74 @@
+"""Forward of the converted integer linears on the kernels that stream the integer weight (few tokens)."""
+import pytest
+import torch
+
+from torchtune_amd import ops
+from torchtune_amd.qat import Int8DynActInt4WeightLinear, WeightOnlyInt4Linear
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _layer(kind, n, k, group, bias, qp):
+    g = torch.Generator().manual_seed(n + k + group)
+    b = (torch.randn(n, generator=g) * 0.1).to(torch.bfloat16) if bias else None
+    w = (torch.randn(n, k, generator=g) * 0.05).to(torch.bfloat16).to(DEV)
+    if kind == "8da4w":
+        layer = Int8DynActInt4WeightLinear(k, n, bias, DEV, group, torch.bfloat16, qp)
+        q, scale, _ = ops.quantize_per_group_int4(w, group, qp)
+        layer.weight.copy_(q)
+        layer.scales.copy_(scale)
+        layer.zeros.copy_(torch.randint(-2, 3, layer.zeros.shape, generator=g).to(qp))  # the converter writes zeros only
+    else:
+        layer = WeightOnlyInt4Linear(k, n, bias, DEV, group, inner_k_tiles=2)
+        q, scale, zero = ops.quantize_per_group_uint4(w, group)
+        layer.weight.copy_(q)
+        layer.scales_and_zeros.copy_(torch.stack([scale.t(), zero.t()], dim=-1))
+    if bias:
+        layer.bias.data.copy_(b)
+        layer.bias.requires_grad_(False)
+    return layer
+
+
+def _operands(layer, x):
+    """What the layer multiplies, in float64."""
+    if isinstance(layer, WeightOnlyInt4Linear):
+        return x.double(), layer.dense_weight().double()
+    xq, _, _ = ops.fq_per_token_int8_asym(x, want_qparams=False, qparam_dtype=layer.scales_precision)
+    w = ops.dequantize_per_group_int4(layer.weight, layer.scales, layer.zeros, layer.groupsize, torch.bfloat16)
+    return xq.double(), w.double()
+
+
+@pytest.mark.parametrize("kind,qp", [("8da4w", torch.float32), ("8da4w", torch.bfloat16), ("4w", torch.bfloat16)])
+@pytest.mark.parametrize("n,k,group,bias", [(256, 32, 32, False), (320, 96, 32, True), (256, 4224, 64, False), (1024, 2048, 256, True), (8192, 160, 32, False)])
+@pytest.mark.parametrize("m", [1, 8, 9, 16, 17, 33, 64, 65, 96, 128, 129, 256])
+def test_few_token_forward(kind, qp, n, k, group, bias, m):
+    if kind == "4w" and k % 32:
+        pytest.skip("the weight-only layer takes multiples of 32")
+    layer = _layer(kind, n, k, group, bias, qp)
+    x = torch.randn(m, k, generator=torch.Generator().manual_seed(m)).to(torch.bfloat16).to(DEV)
+    assert ops.int4_linear_applies(m, n, k, group)
+    with torch.no_grad():
+        got = layer(x)
+    xd, w = _operands(layer, x)
+    want = xd @ w.t()
+    size = xd.abs() @ w.abs().t()
+    if bias:
+        want += layer.bias.double()
+        size += layer.bias.abs().double()
+    # one rounding to bf16 (half a unit: 2^-9 of the value, a whole one granted) and fp32 sums of k exact products
+    bound = want.abs() * 2.0 ** -8 + size * (k * 2.0 ** -23)
+    assert bool(((got.double() - want).abs() <= bound).all())
+
+
+def test_calls_the_kernels_do_not_serve_keep_the_dense_weight():
+    layer = _layer("4w", 256, 256, 64, False, torch.bfloat16)
+    for m, applies in ((256, True), (257, False)):
+        assert ops.int4_linear_applies(m, 256, 256, 64) is applies
+    x = torch.randn(5, 256, device=DEV).to(torch.bfloat16).requires_grad_()
+    y = layer(x)  # differentiable in its input
+    y.sum().backward()
+    torch.testing.assert_close(x.grad.float(), layer.dense_weight().float().sum(0).expand(5, -1), rtol=1e-2, atol=1e-2)
+    # odd widths run as before
+    narrow = _layer("8da4w", 200, 256, 32, False, torch.float32)
+    assert not ops.int4_linear_applies(5, 200, 256, 32) and narrow(x.detach()).shape == (5, 200)

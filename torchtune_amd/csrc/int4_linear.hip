@@ -1,0 +1,442 @@
+// y = x . dequant(Wq)^T (+ bias) for the converted integer linears and up to a few hundred tokens: the 8da4w layer (int4
+// values held in int8, per-group scale and zero point) and the weight-only 4w layer (two uint4 codes per byte, bf16 scale
+// and floating-point zero point).  What Int8DynActInt4WeightLinear / WeightOnlyInt4Linear.forward otherwise do in two
+// passes - write the dense bf16 weight, read it back in a library GEMM - streams the integer weight once: 1 or 0.5
+// bytes per element instead of 5 or 4.5.
+//
+// The expanded values are the bits of ttamd_dequantize_per_group_int4 / _uint4, the products are summed in fp32 and the
+// result is rounded to bf16 once: the arithmetic of the two-pass form up to the order of the fp32 sums.
+//
+// Two kernels, by the number of tokens:
+//  * int4_stream_kernel (at most 16): bound by the weight stream.  A workgroup owns 16 or 32 weight rows and the whole
+//    contraction; its waves take 128-wide chunks of K in turn (one chunk in flight per wave: neighbouring waves then read
+//    neighbouring pieces of the rows, which beats two or four chunks per wave at every size).
+//    The lane that feeds an MFMA holds 32 consecutive k of one row (whole 128-byte lines of int8 weight per row), x
+//    comes from the cache - only the lanes of tokens that exist ask for it.  Partial sums meet in LDS in wave order.
+//  * int4_tile_kernel (more): the few-token kernel would read all of x in every workgroup (at 75 tokens nine times the
+//    bytes of its weight rows).  Four waves own 64 weight rows between them and share 128-wide chunks of up to 128
+//    tokens through a double LDS buffer; a weight fragment is expanded once per 128 tokens.  Launches of few tiles cut
+//    the contraction into slices (fp32 slabs, added in slice order by int4_reduce_kernel).
+//
+// Measured against dequantise + library GEMM (us, weights from HBM, launch gaps included; int8 / uint4):
+//   14336 x 4096:  1 token 60 / 60 -> 22 / 20, 16 tokens 59 / 60 -> 28 / 21, 75 tokens 63 / 65 -> 38 / 33, 256 tokens 83 / 82 -> 67 / 69
+//   4096 x 14336:  1 token 58 / 58 -> 23 / 19, 75 tokens 79 / 78 -> 38 / 32, 256 tokens 93 / 92 -> 74 / 66
+//   1024 x 4096:   1 token 20 / 20 ->  8 /  7, 256 tokens 21 / 21 -> 17 / 16
+// A launch's fixed part is about 6 us of these; what goes beyond it streams int8 weight at 3.6 TB/s.  Above 256 tokens the
+// two m-tiles' expansion and their slabs cost what the dense copy costs, and the library's larger tiles win.
+#include "common.h"
+#include "nf4_math.h"
+
+namespace ttamd {
+namespace {
+
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ uint32_t pack_pair(float lo, float hi) {
+  bf16x2_t v;
+  v.x = (__bf16)lo;
+  v.y = (__bf16)hi;
+  return __builtin_bit_cast(uint32_t, v);
+}
+__device__ __forceinline__ float lo_of(uint32_t d) { return bits_f32(d << 16); }
+__device__ __forceinline__ float hi_of(uint32_t d) { return bits_f32(d & 0xffff0000u); }
+
+struct Int4Args {
+  const uint16_t* x;     // [M, K] bf16
+  const uint8_t* q;      // int8 [N, K] or packed uint4 [N, K/2]
+  const void* scale;     // int8 form: [N, K/g]; uint4 form: bf16 [K/g, N, 2] (scale, zero)
+  const void* zero;      // int8 form: [N, K/g] or null (= 0)
+  const uint16_t* bias;  // [N] bf16 or null
+  uint16_t* y;           // [M, N] bf16
+  float* part;           // [slices, M, N] when the contraction is cut
+  int M, N, K;
+  int log2_group;        // >= 5
+  int chunks_per_slice;
+};
+
+// How a weight is stored.
+enum Format { kInt8F32, kInt8Bf16, kUint4 };
+
+// 32 consecutive k of one weight row, as loaded.
+template <int FMT>
+struct WeightPiece;
+
+template <>
+struct WeightPiece<kUint4> {
+  u32x4_t codes;
+  uint32_t sz;
+  __device__ __forceinline__ void clear() { codes = u32x4_t{0, 0, 0, 0}; sz = 0; }
+  __device__ __forceinline__ void load(const Int4Args& a, int n, int k) {
+    codes = *reinterpret_cast<const u32x4_t*>(a.q + (((int64_t)n * a.K + k) >> 1));
+    sz = reinterpret_cast<const uint32_t*>(a.scale)[(int64_t)(k >> a.log2_group) * a.N + n];
+  }
+  // elements 8 s .. 8 s + 7 as an MFMA operand: bf16(bf16((q - 8) * scale) + zero); the first product is exact in fp32
+  __device__ __forceinline__ u32x4_t operand(int s) const {
+    const float sc = lo_of(sz), z = hi_of(sz), off = -8.0f * sc;
+    u32x4_t w;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const uint32_t byte = (codes[s] >> (8 * b)) & 0xffu;
+      const uint32_t p = pack_pair(__builtin_fmaf((float)(byte >> 4), sc, off), __builtin_fmaf((float)(byte & 15u), sc, off));
+      w[b] = pack_pair(lo_of(p) + z, hi_of(p) + z);
+    }
+    return w;
+  }
+};
+
+template <bool QP_BF16>
+struct Int8Piece {
+  u32x4_t v[2];
+  float sc, z;
+  __device__ __forceinline__ void clear() { v[0] = v[1] = u32x4_t{0, 0, 0, 0}; sc = z = 0.f; }
+  __device__ __forceinline__ void load(const Int4Args& a, int n, int k) {
+    const u32x4_t* p = reinterpret_cast<const u32x4_t*>(a.q + (int64_t)n * a.K + k);
+    v[0] = p[0];
+    v[1] = p[1];
+    const int64_t gi = (int64_t)n * (a.K >> a.log2_group) + (k >> a.log2_group);
+    if constexpr (QP_BF16) {
+      sc = bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(a.scale)[gi]);
+      z = a.zero ? bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(a.zero)[gi]) : 0.f;
+    } else {
+      sc = reinterpret_cast<const float*>(a.scale)[gi];
+      z = a.zero ? reinterpret_cast<const float*>(a.zero)[gi] : 0.f;
+    }
+  }
+  __device__ __forceinline__ u32x4_t operand(int s) const {  // bf16((q - zero) * scale)
+    u32x4_t w;
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      const uint32_t two = v[s >> 1][2 * (s & 1) + (d >> 1)] >> (16 * (d & 1));
+      w[d] = pack_pair(((float)(int8_t)(two & 0xffu) - z) * sc, ((float)(int8_t)((two >> 8) & 0xffu) - z) * sc);
+    }
+    return w;
+  }
+};
+template <>
+struct WeightPiece<kInt8F32> : Int8Piece<false> {};
+template <>
+struct WeightPiece<kInt8Bf16> : Int8Piece<true> {};
+
+constexpr int kStreamTokens = 16;
+
+// RT tiles of 16 weight rows per workgroup (they share a wave's fragments of x), at most MAXW waves.
+template <int FMT, int RT, int MAXW>
+__global__ __launch_bounds__(64 * MAXW) void int4_stream_kernel(const Int4Args a) {
+  __shared__ float red[(MAXW - 1) * RT * 256];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nw = blockDim.x >> 6;
+  const int i = lane & 15, g = lane >> 4;
+  const int n0 = (int)blockIdx.x * (16 * RT);  // N % 64 == 0: every row of the workgroup exists
+  const bool token = i < a.M;
+  const uint16_t* xrow = a.x + (int64_t)(token ? i : 0) * a.K + 32 * g;
+  const int n_chunks = (a.K + 127) >> 7;
+  f32x4_t acc[RT][4];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int s = 0; s < 4; ++s) acc[rt][s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  for (int c = wave; c < n_chunks; c += nw) {
+    WeightPiece<FMT> w[RT];
+    u32x4_t xb[4];
+    const int k = c * 128 + 32 * g;
+    const bool in = k < a.K;  // K % 32 == 0
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      if (in)
+        w[rt].load(a, n0 + 16 * rt + i, k);
+      else
+        w[rt].clear();
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      xb[s] = u32x4_t{0, 0, 0, 0};
+      if (in && token) xb[s] = *reinterpret_cast<const u32x4_t*>(xrow + c * 128 + 8 * s);
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+        acc[rt][s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w[rt].operand(s)),
+                                                             __builtin_bit_cast(bf16x8_t, xb[s]), acc[rt][s], 0, 0, 0);
+  }
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+    for (int s = 1; s < 4; ++s) acc[rt][0] += acc[rt][s];
+    if (wave > 0) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) red[((wave - 1) * RT + rt) * 256 + v * 64 + lane] = acc[rt][0][v];
+    }
+  }
+  __syncthreads();
+  if (wave != 0) return;
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    // acc[rt][0][v] = the wave's share of y[i][n0 + 16 rt + 4 g + v]
+    float o[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      o[v] = acc[rt][0][v];
+      for (int q = 0; q < nw - 1; ++q) o[v] += red[(q * RT + rt) * 256 + v * 64 + lane];
+    }
+    if (!token) continue;
+    const int nb = n0 + 16 * rt + 4 * g;
+    if (a.bias) {
+      const u32x2_t b = *reinterpret_cast<const u32x2_t*>(a.bias + nb);
+      o[0] += lo_of(b.x); o[1] += hi_of(b.x); o[2] += lo_of(b.y); o[3] += hi_of(b.y);
+    }
+    u32x2_t out;
+    out.x = pack_pair(o[0], o[1]);
+    out.y = pack_pair(o[2], o[3]);
+    *reinterpret_cast<u32x2_t*>(a.y + (int64_t)i * a.N + nb) = out;
+  }
+}
+
+// Four waves, 64 weight rows, 16 MT tokens; blockIdx = (row tile, token tile, slice of the contraction).
+template <int FMT, int MT, bool SPLIT>
+__global__ __launch_bounds__(256) void int4_tile_kernel(const Int4Args a) {
+  // 128 k of 16 MT tokens: token r's 16-byte piece p lies in slot p ^ (r % 16), so that the 16 lanes of a fragment read
+  // (16 tokens, one piece each) fall on disjoint banks
+  __shared__ u32x4_t xs[2][MT * 16 * 16];
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int i = lane & 15, g = lane >> 4;
+  const int n = (int)blockIdx.x * 64 + 16 * wave + i;  // N % 64 == 0
+  const int m0 = (int)blockIdx.y * (16 * MT);
+  const int n_chunks = (a.K + 127) >> 7;
+  const int c_first = SPLIT ? (int)blockIdx.z * a.chunks_per_slice : 0;
+  const int c_end = SPLIT ? min(c_first + a.chunks_per_slice, n_chunks) : n_chunks;
+
+  // thread t stages piece t % 16 of tokens t / 16 + 16 j
+  const int piece = t & 15, row = t >> 4;
+  const uint16_t* xsrc[MT];
+#pragma unroll
+  for (int j = 0; j < MT; ++j) {
+    int m = m0 + 16 * j + row;
+    m = m < a.M ? m : a.M - 1;  // tokens beyond M repeat the last one and are never stored
+    xsrc[j] = a.x + (int64_t)m * a.K + 8 * piece;
+  }
+  const int slot = row * 16 + (piece ^ row);
+
+  f32x4_t acc[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) acc[mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  u32x4_t xr[MT];
+  WeightPiece<FMT> w;
+  auto request = [&](int c) {
+    const int k = c * 128 + 32 * g;
+    if (k < a.K)
+      w.load(a, n, k);
+    else
+      w.clear();
+    const bool in = c * 128 + 8 * piece < a.K;
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+      xr[j] = u32x4_t{0, 0, 0, 0};
+      if (in) xr[j] = *reinterpret_cast<const u32x4_t*>(xsrc[j] + c * 128);
+    }
+  };
+  request(c_first);
+#pragma unroll
+  for (int j = 0; j < MT; ++j) xs[0][j * 256 + slot] = xr[j];
+  __syncthreads();
+  int buf = 0;
+  for (int c = c_first; c < c_end; ++c) {
+    const WeightPiece<FMT> wc = w;
+    const bool more = c + 1 < c_end;
+    if (more) request(c + 1);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const bf16x8_t wf = __builtin_bit_cast(bf16x8_t, wc.operand(s));
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+        acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            wf, __builtin_bit_cast(bf16x8_t, xs[buf][mt * 256 + i * 16 + ((4 * g + s) ^ i)]), acc[mt], 0, 0, 0);
+    }
+    buf ^= 1;
+    if (more) {
+#pragma unroll
+      for (int j = 0; j < MT; ++j) xs[buf][j * 256 + slot] = xr[j];
+    }
+    __syncthreads();
+  }
+  const int nb = (int)blockIdx.x * 64 + 16 * wave + 4 * g;
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    const int m = m0 + 16 * mt + i;
+    if (m >= a.M) continue;
+    if constexpr (SPLIT) {
+      *reinterpret_cast<f32x4_t*>(a.part + ((int64_t)blockIdx.z * a.M + m) * a.N + nb) = acc[mt];
+    } else {
+      f32x4_t o = acc[mt];
+      if (a.bias) {
+        const u32x2_t b = *reinterpret_cast<const u32x2_t*>(a.bias + nb);
+        o += f32x4_t{lo_of(b.x), hi_of(b.x), lo_of(b.y), hi_of(b.y)};
+      }
+      u32x2_t out;
+      out.x = pack_pair(o[0], o[1]);
+      out.y = pack_pair(o[2], o[3]);
+      *reinterpret_cast<u32x2_t*>(a.y + (int64_t)m * a.N + nb) = out;
+    }
+  }
+}
+
+// y = bf16(sum of the slices in order + bias), four columns per thread
+__global__ __launch_bounds__(256) void int4_reduce_kernel(const float* __restrict__ part, int slices, int64_t quads, int nq,
+                                                          const uint16_t* __restrict__ bias, uint16_t* __restrict__ y) {
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= quads) return;
+  const f32x4_t* p = reinterpret_cast<const f32x4_t*>(part) + e;
+  f32x4_t o = p[0];
+  for (int s = 1; s < slices; ++s) o += p[s * quads];
+  if (bias) {
+    const u32x2_t b = reinterpret_cast<const u32x2_t*>(bias)[e % nq];
+    o += f32x4_t{lo_of(b.x), hi_of(b.x), lo_of(b.y), hi_of(b.y)};
+  }
+  u32x2_t out;
+  out.x = pack_pair(o[0], o[1]);
+  out.y = pack_pair(o[2], o[3]);
+  reinterpret_cast<u32x2_t*>(y)[e] = out;
+}
+
+constexpr int kMaxTokens = 256;
+constexpr int kMinRows = 256;
+
+// 16-token tiles per workgroup: as few rows of padding as the instantiated sizes allow (75 tokens on 14336 x 4096 int8: five
+// tiles 38 us, eight 48 us)
+int tile_mt(int64_t M) {
+  const int64_t wg_rows = (M + 127) / 128;
+  const int mt = (int)((M + 16 * wg_rows - 1) / (16 * wg_rows));
+  return mt <= 2 ? 2 : (mt == 7 ? 8 : mt);
+}
+
+struct Slicing {
+  int slices, chunks;
+};
+Slicing slicing(int64_t M, int64_t N, int64_t K) {
+  const int64_t n_chunks = (K + 127) / 128;
+  const int64_t wgs = (N / 64) * ((M + 16 * tile_mt(M) - 1) / (16 * tile_mt(M)));
+  // two workgroups per CU and not one more: 64 tokens on 14336 x 4096 (224 row tiles, us, int8) 43 with one slice, 34 with
+  // two, 36 with three, 38 with four; on 4096 x 14336 (64 row tiles) 40 / 34 / 37 with four / eight / sixteen
+  int64_t s = wgs < 512 ? 512 / wgs : 1;
+  const int64_t most = n_chunks / 4 > 1 ? n_chunks / 4 : 1;
+  s = s < most ? s : most;
+  s = s < 16 ? s : 16;
+  const int64_t chunks = (n_chunks + s - 1) / s;
+  return {(int)((n_chunks + chunks - 1) / chunks), (int)chunks};
+}
+
+template <int FMT, bool SPLIT>
+void launch_tile(const Int4Args& a, int mt, dim3 grid, hipStream_t s) {
+  const dim3 block(256);
+  switch (mt) {
+    case 2: int4_tile_kernel<FMT, 2, SPLIT><<<grid, block, 0, s>>>(a); break;
+    case 3: int4_tile_kernel<FMT, 3, SPLIT><<<grid, block, 0, s>>>(a); break;
+    case 4: int4_tile_kernel<FMT, 4, SPLIT><<<grid, block, 0, s>>>(a); break;
+    case 5: int4_tile_kernel<FMT, 5, SPLIT><<<grid, block, 0, s>>>(a); break;
+    case 6: int4_tile_kernel<FMT, 6, SPLIT><<<grid, block, 0, s>>>(a); break;
+    default: int4_tile_kernel<FMT, 8, SPLIT><<<grid, block, 0, s>>>(a); break;
+  }
+}
+
+template <int FMT, int RT, int MAXW>
+void launch_stream(const Int4Args& a, hipStream_t s) {
+  const int n_chunks = (a.K + 127) >> 7;
+  int4_stream_kernel<FMT, RT, MAXW><<<dim3(a.N / (16 * RT)), dim3(64 * (n_chunks < MAXW ? n_chunks : MAXW)), 0, s>>>(a);
+}
+
+template <int FMT>
+int launch(Int4Args& a, void* workspace, size_t workspace_bytes, hipStream_t s) {
+  if (a.M <= kStreamTokens) {
+    // Measured (weights from HBM, us, launch gap included).  Wide layers have workgroups to spare: few waves each, and
+    // two row tiles where the reads of x weigh (int8 14336 x 4096 at 1 / 16 tokens: four waves and two tiles 21.2 / 27.8,
+    // sixteen and one 27 / 37; uint4 at 1 / 16 tokens: one tile 19.6 / 23, two 20.4 / 21.1).  Narrow ones need the waves (uint4
+    // 4096 x 14336 at 1 token: sixteen 20.0, eight 20.9; at 16 tokens 25 and 21.6).
+    const bool wide = a.N >= 8192;
+    if constexpr (FMT == kUint4) {
+      if (wide && a.M > 8) launch_stream<FMT, 2, 8>(a, s);
+      else if (wide || a.M > 8) launch_stream<FMT, 1, 8>(a, s);
+      else launch_stream<FMT, 1, 16>(a, s);
+    } else {
+      if (wide) launch_stream<FMT, 2, 4>(a, s);
+      else launch_stream<FMT, 1, 8>(a, s);
+    }
+    return check_launch("int4_linear");
+  }
+  const Slicing sl = slicing(a.M, a.N, a.K);
+  const int mt = tile_mt(a.M);
+  const dim3 grid(a.N / 64, (a.M + 16 * mt - 1) / (16 * mt), sl.slices);
+  a.chunks_per_slice = sl.chunks;
+  if (sl.slices == 1) {
+    launch_tile<FMT, false>(a, mt, grid, s);
+    return check_launch("int4_linear");
+  }
+  const size_t need = (size_t)sl.slices * a.M * a.N * sizeof(float);
+  if (!workspace || workspace_bytes < need)
+    return fail(TTAMD_EWORKSPACE, "int4_linear: workspace of %zu bytes, %zu needed", workspace_bytes, need);
+  TT_REQUIRE(aligned16(workspace), "int4_linear: the workspace must be 16-byte aligned");
+  a.part = reinterpret_cast<float*>(workspace);
+  launch_tile<FMT, true>(a, mt, grid, s);
+  if (int rc = check_launch("int4_linear")) return rc;
+  const int64_t quads = (int64_t)a.M * a.N / 4;
+  int4_reduce_kernel<<<dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s>>>(a.part, sl.slices, quads, a.N / 4, a.bias, a.y);
+  return check_launch("int4_linear: reduction");
+}
+
+int check_args(const void* x, const void* q, const void* scale, const void* y, int64_t M, int64_t N, int64_t K, int group_size) {
+  TT_REQUIRE(x && q && scale && y, "int4_linear: x, q, the scales and y must be non-null");
+  TT_REQUIRE(aligned16(x) && aligned16(q) && aligned16(scale) && aligned16(y), "int4_linear: pointers must be 16-byte aligned");
+  if (!ttamd_int4_linear_applies(M, N, K, group_size))
+    return fail(TTAMD_EUNSUPPORTED, "int4_linear: M = %lld, N = %lld, K = %lld, group_size = %d is not served", (long long)M,
+                (long long)N, (long long)K, group_size);
+  return TTAMD_OK;
+}
+
+int log2_of(int v) {
+  int l = 0;
+  while ((1 << l) < v) ++l;
+  return l;
+}
+
+}  // namespace
+}  // namespace ttamd
+
+using namespace ttamd;
+
+extern "C" int ttamd_int4_linear_applies(int64_t M, int64_t N, int64_t K, int group_size) {
+  return M > 0 && M <= kMaxTokens && N >= kMinRows && N % 64 == 0 && K > 0 && K % 32 == 0 && group_size >= 32 &&
+         is_pow2(group_size) && K % group_size == 0 && N * K < (int64_t(1) << 31);
+}
+
+extern "C" size_t ttamd_int4_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+  if (M <= kStreamTokens || M > kMaxTokens || N < 64 || K <= 0) return 0;
+  const Slicing sl = slicing(M, N, K);
+  return sl.slices > 1 ? (size_t)sl.slices * M * N * sizeof(float) : 0;
+}
+
+extern "C" int ttamd_int8_group_linear_bf16(const void* x, const int8_t* q, const void* scale, const void* zero_point,
+                                            int qparam_dtype, int group_size, const void* bias, void* y, int64_t M, int64_t N,
+                                            int64_t K, void* workspace, size_t workspace_bytes, void* stream) {
+  if (int rc = check_args(x, q, scale, y, M, N, K, group_size)) return rc;
+  TT_REQUIRE(qparam_dtype == TTAMD_BF16 || qparam_dtype == TTAMD_F32, "int8_group_linear: unknown qparam dtype code %d", qparam_dtype);
+  Int4Args a = {reinterpret_cast<const uint16_t*>(x), reinterpret_cast<const uint8_t*>(q), scale, zero_point,
+                reinterpret_cast<const uint16_t*>(bias), reinterpret_cast<uint16_t*>(y), nullptr, (int)M, (int)N, (int)K,
+                log2_of(group_size), 0};
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  return qparam_dtype == TTAMD_BF16 ? launch<kInt8Bf16>(a, workspace, workspace_bytes, s) : launch<kInt8F32>(a, workspace, workspace_bytes, s);
+}
+
+extern "C" int ttamd_uint4_group_linear_bf16(const void* x, const uint8_t* q, const void* scales_and_zeros, int group_size,
+                                             const void* bias, void* y, int64_t M, int64_t N, int64_t K, void* workspace,
+                                             size_t workspace_bytes, void* stream) {
+  if (int rc = check_args(x, q, scales_and_zeros, y, M, N, K, group_size)) return rc;
+  Int4Args a = {reinterpret_cast<const uint16_t*>(x), q, scales_and_zeros, nullptr, reinterpret_cast<const uint16_t*>(bias),
+                reinterpret_cast<uint16_t*>(y), nullptr, (int)M, (int)N, (int)K, log2_of(group_size), 0};
+  return launch<kUint4>(a, workspace, workspace_bytes, reinterpret_cast<hipStream_t>(stream));
+}

@@ -567,6 +567,17 @@ class Int8DynActInt4WeightQATLinear(FakeQuantizedLinear):
         self.enable_fake_quant(False)
 
 
+def _int4_kernels_apply(x: torch.Tensor, weight: torch.Tensor, in_features: int, groupsize: int, precision: torch.dtype,
+                        bias: Optional[torch.Tensor], qparams_ok: bool) -> bool:
+    """True when a converted linear's forward runs on the kernels that stream its integer weight (a few hundred tokens at
+    most); otherwise the dense weight is rebuilt and multiplied."""
+    if not (qparams_ok and precision == torch.bfloat16 and x.is_cuda and weight.is_cuda and x.shape[-1] == in_features and x.numel() > 0):
+        return False
+    if bias is not None and (bias.dtype != torch.bfloat16 or not bias.is_cuda or (bias.requires_grad and torch.is_grad_enabled())):
+        return False
+    return weight.is_contiguous() and ops.int4_linear_applies(x.numel() // in_features, weight.shape[0], in_features, groupsize)
+
+
 class Int8DynActInt4WeightLinear(nn.Module):
     """Result of ``convert``: int4 weight values held in int8 plus per-group scales and zeros; the input is
     quantised per token on the fly.  Forward reproduces the arithmetic the fake-quantised layer trained with."""
@@ -592,6 +603,10 @@ class Int8DynActInt4WeightLinear(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         x = x.to(self.precision)
         x_q, _, _ = ops.fq_per_token_int8_asym(x, want_qparams=False, qparam_dtype=self.scales_precision)
+        if _int4_kernels_apply(x, self.weight, self.in_features, self.groupsize, self.precision, self.bias,
+                               self.scales.dtype == self.zeros.dtype and self.scales.dtype in (torch.float32, torch.bfloat16)):
+            y = ops.int8_group_linear(x_q.reshape(-1, self.in_features), self.weight, self.scales, self.zeros, self.groupsize, self.bias)
+            return y.view(*x.shape[:-1], self.out_features)
         w = ops.dequantize_per_group_int4(self.weight, self.scales, self.zeros, self.groupsize, self.precision)
         return F.linear(x_q, w, self.bias)
 
@@ -746,7 +761,13 @@ class WeightOnlyInt4Linear(nn.Module):
         return ops.dequantize_per_group_uint4(self.weight, scale, zero, self.groupsize, self.precision)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return F.linear(x.to(self.precision), self.dense_weight(), self.bias)
+        x = x.to(self.precision)
+        # the streaming kernel has no backward: a call that will want a gradient of x multiplies with the dense weight
+        if not (torch.is_grad_enabled() and x.requires_grad) and _int4_kernels_apply(
+                x, self.weight, self.in_features, self.groupsize, self.precision, self.bias, self.scales_and_zeros.dtype == torch.bfloat16):
+            y = ops.uint4_group_linear(x.reshape(-1, self.in_features), self.weight, self.scales_and_zeros, self.groupsize, self.bias)
+            return y.view(*x.shape[:-1], self.out_features)
+        return F.linear(x, self.dense_weight(), self.bias)
 
 
 class Int4WeightOnlyQATQuantizer:
