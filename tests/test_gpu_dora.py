@@ -45,6 +45,30 @@ def test_weight_norm_and_magnitude_init(K, N, r, use_bias):
     assert (layer.magnitude.detach().cpu() == want).float().mean() > 0.9
 
 
+@pytest.mark.parametrize("K,N,r", [(64, 256, 8), (2048, 40, 24), (1216, 1024, 32), (1088, 2048, 40), (5120, 336, 16)])
+def test_weight_norm_kernel_edges(K, N, r):
+    """Half chunks, strips that end early, row tiles that are not full, ranks on both sides of one matrix step."""
+    layer, parts, A, B, _ = _layer(K, N, r, 2.0 * r, False, seed=3)
+    norm, _ = ops.nf4_dora_weight_norm(layer.weight.quantized_data, layer.weight.block_scalers(), N, K, layer.lora_a.weight.detach(),
+                                       layer.lora_b.weight.detach(), 2.0)
+    want = lora_oracle.dora_weight_norm(parts, A, B, 2.0 * r, r)
+    torch.testing.assert_close(norm.cpu().float(), want.float(), rtol=2 ** -7, atol=0)
+    assert (norm.cpu() == want).float().mean() > 0.9
+
+
+@pytest.mark.parametrize("M,N", [(1, 72), (5, 520), (1031, 1032)])
+def test_backward_prologue_edges(M, N):
+    g = torch.Generator().manual_seed(M)
+    gy, out = (torch.randn(M, N, generator=g).to(torch.bfloat16).to(DEV) for _ in range(2))
+    mns, mag = (torch.rand(N, generator=g).add(0.5).to(torch.bfloat16).to(DEV) for _ in range(2))
+    gy0, gmag = ops.dora_bwd_prologue(gy, out, mns, mag)
+    assert torch.equal(gy0, gy * mns)
+    want = (gy.double() * out.double()).sum(0) / mag.double()
+    size = (gy.double() * out.double()).abs().sum(0) / mag.double()
+    # fp32 sums of M products, one rounding to bf16
+    assert bool(((gmag.double() - want).abs() <= want.abs() * 2.0 ** -8 + size * M * 2.0 ** -23).all())
+
+
 @pytest.mark.parametrize("M,K,N,r,use_bias", [(96, 512, 512, 8, True), (300, 1024, 768, 16, False), (1024, 2048, 2048, 16, True)])
 def test_forward_backward_vs_oracle(M, K, N, r, use_bias):
     alpha = 2.0 * r
