@@ -126,7 +126,7 @@ class RMSNorm(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if _fused(x) and self.scale.dtype == torch.bfloat16 and x.shape[-1] % 8 == 0 and x.shape[-1] <= 8192:
-            return layer_ops._RMSNormFn.apply(x, self.scale, self.eps)
+            return layer_ops.rms_norm(x, self.scale, self.eps)
         xf = x.float()
         x_normed = (xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + self.eps)).type_as(x)
         return x_normed * self.scale

@@ -11,48 +11,18 @@ from __future__ import annotations
 import torch
 from torch import nn
 
-from .. import ops
+from .. import _host, ops
 
 
-class _RMSNormFn(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, x, scale, eps: float):
-        y, rstd = ops.rms_norm_fwd(x, scale, eps)
-        ctx.save_for_backward(x, scale, rstd)
-        return y.view(x.shape)
-
-    @staticmethod
-    def backward(ctx, gy):
-        x, scale, rstd = ctx.saved_tensors
-        gx, gscale = ops.rms_norm_bwd(gy, x, scale, rstd, want_gscale=ctx.needs_input_grad[1])
-        return (gx.view(x.shape) if ctx.needs_input_grad[0] else None), gscale, None
-
-
-class _AddRMSNormFn(torch.autograd.Function):
-    """(x, residual, scale) -> (h = x + residual, RMSNorm(h)).  Backward: both inputs receive
-    ``grad h + grad of the norm's input``, summed in the norm's backward pass."""
-
-    @staticmethod
-    def forward(ctx, x, residual, scale, eps: float):
-        h, y, rstd = ops.add_rms_norm_fwd(x, residual, scale, eps)
-        ctx.save_for_backward(h, scale, rstd)
-        ctx.set_materialize_grads(False)  # an output nobody used arrives as None, not as a tensor of zeros
-        return h.view(x.shape), y.view(x.shape)
-
-    @staticmethod
-    def backward(ctx, gh, gy):
-        h, scale, rstd = ctx.saved_tensors
-        if gy is None:  # the normalised output went nowhere
-            return gh, gh, None, None
-        gx, gscale = ops.rms_norm_bwd(gy, h, scale, rstd, want_gscale=ctx.needs_input_grad[2], g_add=gh)
-        gx = gx.view(h.shape)
-        return (gx if ctx.needs_input_grad[0] else None), (gx if ctx.needs_input_grad[1] else None), gscale, None
+def rms_norm(x: torch.Tensor, scale: torch.Tensor, eps: float) -> torch.Tensor:
+    """``bf16(x * rsqrt(mean(x^2) + eps)) * scale`` over the last dimension, computed in fp32."""
+    return _host.load().rms_norm(x, scale, eps)
 
 
 def add_rms_norm(x: torch.Tensor, residual: torch.Tensor, norm: "RMSNorm"):
     """``h = x + residual; return h, norm(h)``: the residual stream's addition and the norm of the next sub-block
     (``torchtune/modules/transformer.py:129-141``) as one pass forward and one backward; same bits as the separate ops."""
-    return _AddRMSNormFn.apply(x, residual, norm.scale, norm.eps)
+    return _host.load().add_rms_norm(x, residual, norm.scale, norm.eps)
 
 
 class RMSNorm(nn.Module):
@@ -70,7 +40,7 @@ class RMSNorm(nn.Module):
         self.scale = nn.Parameter(torch.ones(dim))
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return _RMSNormFn.apply(x, self.scale, self.eps)
+        return rms_norm(x, self.scale, self.eps)
 
 
 class _RopeFn(torch.autograd.Function):
@@ -90,24 +60,11 @@ def apply_rope(x: torch.Tensor, cache: torch.Tensor) -> torch.Tensor:
     return _RopeFn.apply(x, cache)
 
 
-class _QKVRopeRepeatFn(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, q, k, v, cache):
-        ctx.save_for_backward(cache)
-        ctx.n_kv = k.shape[2]
-        return ops.qkv_rope_repeat(q, k, v, cache)
-
-    @staticmethod
-    def backward(ctx, gq, gk, gv):
-        (cache,) = ctx.saved_tensors
-        return (*ops.qkv_rope_repeat_bwd(gq, gk, gv, cache, ctx.n_kv), None)
-
-
 def qkv_rope_repeat(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cache: torch.Tensor):
     """What lies between the q / k / v projections and the attention (``torchtune/modules/attention.py:255-290``) as one
     kernel per direction: ``apply_rope(q)``, ``repeat_kv(apply_rope(k), rep)``, ``repeat_kv(v, rep)`` with
     ``rep = n_h // n_kv``, bit for bit."""
-    return _QKVRopeRepeatFn.apply(q, k, v, cache)
+    return _host.load().qkv_rope_repeat(q, k, v, cache)
 
 
 class _RepeatKVFn(torch.autograd.Function):
@@ -128,22 +85,9 @@ def repeat_kv(x: torch.Tensor, rep: int) -> torch.Tensor:
     return _RepeatKVFn.apply(x, rep)
 
 
-class _SwiGLUFn(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, gate, up):
-        ctx.save_for_backward(gate, up)
-        return ops.swiglu_fwd(gate, up)
-
-    @staticmethod
-    def backward(ctx, gout):
-        gate, up = ctx.saved_tensors
-        gg, gu = ops.swiglu_bwd(gout, gate, up)
-        return gg, gu
-
-
 def swiglu(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     """``silu(gate) * up`` with the eager sequence's two bf16 roundings."""
-    return _SwiGLUFn.apply(gate, up)
+    return _host.load().swiglu(gate, up)
 
 
 class _CrossEntropySumFn(torch.autograd.Function):

@@ -15,9 +15,9 @@ from typing import List, Sequence, Tuple
 
 import torch
 
-from ... import nf4_tensor, ops
+from ... import _host, nf4_tensor, ops
 from ...nf4_tensor import _check_in_features
-from .lora import LoRALinear
+from .lora import LoRALinear, host_weight
 
 
 # The backward of ``silu(gate) * up`` inside the library call that multiplies its results with the pair's adapters (one pass
@@ -214,11 +214,28 @@ def group_applies(x: torch.Tensor, layers: Sequence[torch.nn.Module]) -> bool:
     return ops.group_shape_ok([l.out_dim for l in layers], layers[0].in_dim, [l.rank for l in layers])
 
 
+def _native_group(x: torch.Tensor, layers, gated: bool):
+    """The group call on the native host path, or None where the Python nodes above serve it."""
+    K = layers[0].in_dim
+    tokens = x.numel() // K
+    if x.shape[-1] != K or not ops.native_call(tokens):
+        return None
+    grad = torch.is_grad_enabled()
+    members = []
+    for layer in layers:
+        w = layer.weight
+        members.append((*host_weight(w, tokens, grad), layer.lora_a.weight, layer.lora_b.weight, layer.alpha / layer.rank, layer.bias))
+    return _host.load().lora_group(x, members, gated)
+
+
 def lora_swiglu_group(x: torch.Tensor, gate: torch.nn.Module, up: torch.nn.Module):
     """``silu(gate(x)) * up(x)`` (``torchtune/modules/feed_forward.py:50-53``) with the product formed in the epilogue of
     the pair's one GEMM launch where the group kernels apply; ``None`` when they do not (the caller multiplies itself)."""
     if not group_applies(x, (gate, up)) or gate.out_dim != up.out_dim:
         return None
+    out = _native_group(x, (gate, up), True)
+    if out is not None:
+        return out[0]
     flat = []
     for layer in (gate, up):
         flat += [layer.weight, layer.lora_a.weight, layer.lora_b.weight, layer.bias]
@@ -247,6 +264,9 @@ def lora_linear_group(x: torch.Tensor, layers: Sequence[torch.nn.Module]) -> Tup
     """``tuple(layer(x) for layer in layers)`` for layers that share the input ``x``."""
     if not group_applies(x, layers):
         return tuple(layer(x) for layer in layers)
+    out = _native_group(x, layers, False)
+    if out is not None:
+        return tuple(out)
     flat = []
     for layer in layers:
         flat += [layer.weight, layer.lora_a.weight, layer.lora_b.weight, layer.bias]

@@ -237,7 +237,6 @@ class NF4Tensor(torch.Tensor):
         out = ops.nf4_dequantize(*parts, self.shape, self.block_size, self.scaler_block_size)
         return out if home == dev else out.to(home)
 
-    @torch.no_grad()
     def block_scalers(self) -> torch.Tensor:
         """Dequantised per-block scalers as fp32 [n_blocks] on the GPU, cached while the scaler tensors are
         unchanged (the cache rides on the ``quantized_scalers`` tensor object and is keyed by the in-place
@@ -247,11 +246,11 @@ class NF4Tensor(torch.Tensor):
         cached = getattr(qs, "_ttamd_block_scalers", None)
         if cached is not None and cached[0] == key:
             return cached[1]
-        val = ops.nf4_block_scalers(qs, self.quantization_factor, self.scaler_mean, self.scaler_block_size)
+        with torch.no_grad():
+            val = ops.nf4_block_scalers(qs, self.quantization_factor, self.scaler_mean, self.scaler_block_size)
         qs._ttamd_block_scalers = (key, val)
         return val
 
-    @torch.no_grad()
     def backward_copy(self):
         """(codes re-packed along N, block scalers transposed) for the grad-input GEMM, or None when disabled.
 
@@ -266,7 +265,8 @@ class NF4Tensor(torch.Tensor):
         cached = getattr(qs, "_ttamd_backward_copy", None)
         if cached is not None and cached[0] == key:
             return cached[1]
-        val = ops.nf4_transpose_for_backward(self.quantized_data, self.block_scalers(), self.shape[0], self.shape[1])
+        with torch.no_grad():
+            val = ops.nf4_transpose_for_backward(self.quantized_data, self.block_scalers(), self.shape[0], self.shape[1])
         qs._ttamd_backward_copy = (key, val)
         return val
 

@@ -184,6 +184,18 @@ def set_gemm_timer(timer) -> None:
     _gemm_timer = timer
 
 
+# Calls of fewer tokens make their library calls from the native host path (``_host``): they are a handful of kernels of
+# 3 - 30 us, the Python wrappers below take 25 - 35 us per op and direction.  From here on weights may be expanded once per
+# call and handed from forward to backward, which the wrappers arrange, and the kernels are long enough to hide them.
+NATIVE_MAX_TOKENS = 1280
+
+
+def native_call(tokens: int) -> bool:
+    """True when a fused LoRA call over ``tokens`` rows runs on the native host path (never while a GEMM timer is
+    installed: it brackets the stages of the Python path)."""
+    return 0 < tokens < NATIVE_MAX_TOKENS and _gemm_timer is None
+
+
 def fused_shape_ok(N: int, K: int, rank: int) -> bool:
     """Shapes the fused bf16 GEMM accepts (NF4 block_size must also be 64)."""
     return K % 64 == 0 and N % 64 == 0 and rank % 8 == 0 and 0 <= rank <= 64
@@ -1219,63 +1231,8 @@ def dequantize_per_group_int4(q: torch.Tensor, scale: torch.Tensor, zeros: Optio
 
 
 def int4_linear_applies(M: int, N: int, K: int, group_size: int) -> bool:
-    """Sizes ``int8_group_linear`` / ``uint4_group_linear`` serve."""
+    """Sizes the kernels that stream a converted linear's integer weight serve."""
     return bool(_lib.load().ttamd_int4_linear_applies(M, N, K, group_size))
-
-
-def _int4_operands(what: str, x: torch.Tensor, q: torch.Tensor, per_byte: int, bias: Optional[torch.Tensor]):
-    x = _bf16_2d(x, what)
-    if not q.is_contiguous() or q.dim() != 2 or q.shape[1] * per_byte != x.shape[1] or q.device != x.device:
-        raise ValueError(f"{what}: the weight {tuple(q.shape)} on {q.device} does not fit the input {tuple(x.shape)} on {x.device}")
-    if bias is not None:
-        bias = _bf16_any(bias, what)
-        if bias.numel() != q.shape[0]:
-            raise ValueError(f"{what}: bias has {bias.numel()} elements, the layer {q.shape[0]} outputs")
-    return x, bias
-
-
-def int8_group_linear(x: torch.Tensor, q: torch.Tensor, scale: torch.Tensor, zeros: Optional[torch.Tensor], group_size: int,
-                      bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """``x @ ((q - zeros) * scale).T (+ bias)``: x [M, K] bf16, q int8 [N, K], scale / zeros [N, K/g] fp32 or bf16 (one dtype)."""
-    x, bias = _int4_operands("int8_group_linear", x, q, 1, bias)
-    M, K = x.shape
-    N = q.shape[0]
-    code = _code(scale.dtype, "int8_group_linear: scale")
-    scale = scale.contiguous()
-    zeros = zeros.contiguous() if zeros is not None else None
-    if q.dtype != torch.int8 or scale.numel() * group_size != N * K or (
-            zeros is not None and (zeros.numel() != scale.numel() or zeros.dtype != scale.dtype)):
-        raise ValueError("int8_group_linear: q must be int8, scale and zeros of one dtype with N * K / group_size elements")
-    lib = _lib.load()
-    y = torch.empty(M, N, dtype=torch.bfloat16, device=x.device)
-    nbytes = int(lib.ttamd_int4_linear_workspace_bytes(M, N, K))
-    ws = _workspace(nbytes, x.device) if nbytes else None
-    with _on_device(x.device):
-        rc = lib.ttamd_int8_group_linear_bf16(x.data_ptr(), q.data_ptr(), scale.data_ptr(), _ptr(zeros), code, group_size, _ptr(bias),
-                                              y.data_ptr(), M, N, K, _ptr(ws), nbytes, _stream(x))
-    _lib.check(rc, "int8_group_linear")
-    return y
-
-
-def uint4_group_linear(x: torch.Tensor, q: torch.Tensor, scales_and_zeros: torch.Tensor, group_size: int,
-                       bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """``x @ ((q - 8) * scale + zero).T (+ bias)``: x [M, K] bf16, q uint8 [N, K/2] (even element in the high nibble),
-    scales_and_zeros bf16 [K/g, N, 2]."""
-    x, bias = _int4_operands("uint4_group_linear", x, q, 2, bias)
-    M, K = x.shape
-    N = q.shape[0]
-    sz = _bf16_any(scales_and_zeros, "uint4_group_linear: scales_and_zeros")
-    if q.dtype != torch.uint8 or tuple(sz.shape) != (K // group_size, N, 2):
-        raise ValueError(f"uint4_group_linear: q must be uint8 and scales_and_zeros [{K // group_size}, {N}, 2]")
-    lib = _lib.load()
-    y = torch.empty(M, N, dtype=torch.bfloat16, device=x.device)
-    nbytes = int(lib.ttamd_int4_linear_workspace_bytes(M, N, K))
-    ws = _workspace(nbytes, x.device) if nbytes else None
-    with _on_device(x.device):
-        rc = lib.ttamd_uint4_group_linear_bf16(x.data_ptr(), q.data_ptr(), sz.data_ptr(), group_size, _ptr(bias), y.data_ptr(), M, N,
-                                               K, _ptr(ws), nbytes, _stream(x))
-    _lib.check(rc, "uint4_group_linear")
-    return y
 
 
 # ---------------------------------------------------------------------------------------------------

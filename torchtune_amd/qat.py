@@ -29,7 +29,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
-from . import ops
+from . import _host, ops
 
 
 @dataclass
@@ -602,11 +602,11 @@ class Int8DynActInt4WeightLinear(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         x = x.to(self.precision)
+        weight, scales, zeros, bias = self.weight, self.scales, self.zeros, self.bias
+        if scales.dtype == zeros.dtype == self.scales_precision and _int4_kernels_apply(
+                x, weight, self.in_features, self.groupsize, self.precision, bias, scales.is_contiguous() and zeros.is_contiguous()):
+            return _host.load().int8_dynamic_linear(x, weight, scales, zeros, self.groupsize, bias)
         x_q, _, _ = ops.fq_per_token_int8_asym(x, want_qparams=False, qparam_dtype=self.scales_precision)
-        if _int4_kernels_apply(x, self.weight, self.in_features, self.groupsize, self.precision, self.bias,
-                               self.scales.dtype == self.zeros.dtype and self.scales.dtype in (torch.float32, torch.bfloat16)):
-            y = ops.int8_group_linear(x_q.reshape(-1, self.in_features), self.weight, self.scales, self.zeros, self.groupsize, self.bias)
-            return y.view(*x.shape[:-1], self.out_features)
         w = ops.dequantize_per_group_int4(self.weight, self.scales, self.zeros, self.groupsize, self.precision)
         return F.linear(x_q, w, self.bias)
 
@@ -763,10 +763,10 @@ class WeightOnlyInt4Linear(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         x = x.to(self.precision)
         # the streaming kernel has no backward: a call that will want a gradient of x multiplies with the dense weight
+        weight, sz, bias = self.weight, self.scales_and_zeros, self.bias
         if not (torch.is_grad_enabled() and x.requires_grad) and _int4_kernels_apply(
-                x, self.weight, self.in_features, self.groupsize, self.precision, self.bias, self.scales_and_zeros.dtype == torch.bfloat16):
-            y = ops.uint4_group_linear(x.reshape(-1, self.in_features), self.weight, self.scales_and_zeros, self.groupsize, self.bias)
-            return y.view(*x.shape[:-1], self.out_features)
+                x, weight, self.in_features, self.groupsize, self.precision, bias, sz.dtype == torch.bfloat16 and sz.is_contiguous()):
+            return _host.load().uint4_group_linear(x, weight, sz, self.groupsize, bias)
         return F.linear(x, self.dense_weight(), self.bias)
 
 
