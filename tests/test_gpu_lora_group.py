@@ -461,3 +461,26 @@ def test_swiglu_backward_inside_the_adapter_backward_equals_the_two_steps_bitwis
         assert torch.equal(a0.view(torch.int16), a1.view(torch.int16))
         torch.testing.assert_close(b1.float(), b0.float(), rtol=2.0 ** -7, atol=2.0 ** -7 * float(b0.float().abs().max()))
     assert float(gh1.float().abs().max()) > 0 and float(gx1.float().abs().max()) > 0
+
+
+@pytest.mark.parametrize("M", [1, 15, 17, 333, 2048, 2049])
+@pytest.mark.parametrize("K,R", [(64, 8), (1088, 24), (2048, 48), (2112, 64), (3072, 16), (4096, 40)])
+def test_column_contractions_at_the_edges_of_their_kernels(M, K, R):
+    """h = x . A^T and gh = s . gy . B around the sizes where the kernels change: rows and ranks that do not fill a tile,
+    contractions of one chunk, the widest ones of the single-launch form and the next wider, rank tiles of their own."""
+    g = torch.Generator(device=DEV).manual_seed(M + K + R)
+    x = torch.randn(M, K, device=DEV, generator=g).to(BF)
+    a = torch.randn(R, K, device=DEV, generator=g).to(BF)
+    h = ops.lora_hidden(x, a)
+
+    def check(got, p, q, scale):
+        want = scale * (p.double() @ q.double())
+        size = scale * (p.double().abs() @ q.double().abs())
+        # fp32 sums of K exact products, the scale, one rounding to bf16
+        assert bool(((got.double() - want).abs() <= want.abs() * 2.0 ** -8 + size * (K + 1) * 2.0 ** -23).all())
+
+    check(h, x, a.t(), 1.0)
+    b = torch.randn(K, R, device=DEV, generator=g).to(BF)
+    xs = torch.randn(M, 64, device=DEV, generator=g).to(BF)
+    gh, _, _ = ops.lora_bwd(x, xs, torch.randn(M, R, device=DEV, generator=g).to(BF), b, 0.75)
+    check(gh, x, b, 0.75)

@@ -68,11 +68,12 @@ struct NtBatch {
   int M;
 };
 
+// rank_tiles (!BT): the R columns are dealt to that many workgroups, 16 RT each (blockIdx.y = split, rank tile).
 template <int RT, bool BT>
-__global__ __launch_bounds__(256) void skinny_nt_kernel(const NtBatch a) {
+__global__ __launch_bounds__(256) void skinny_nt_kernel(const NtBatch a, int rank_tiles) {
   const NtProblem& P = a.p[blockIdx.z];
-  const int split = blockIdx.y;
-  if (split >= P.splits) return;  // the batch's grid is as deep as its most sliced problem
+  const int split = (int)blockIdx.y / rank_tiles, rank0 = 16 * RT * ((int)blockIdx.y % rank_tiles);
+  if (split >= P.splits || rank0 >= P.R) return;  // the batch's grid is as deep as its most sliced problem
   const uint16_t* __restrict__ X = P.X;
   const uint16_t* __restrict__ Bm = P.bm[0];
   float* __restrict__ part = P.part;
@@ -101,7 +102,7 @@ __global__ __launch_bounds__(256) void skinny_nt_kernel(const NtBatch a) {
   bool bvalid[RT];
 #pragma unroll
   for (int t = 0; t < RT; ++t) {
-    const int r = t * 16 + i;
+    const int r = rank0 + t * 16 + i;
     bvalid[t] = r < R;
     brow[t] = Bm + 16 * g;
     if (!BT && bvalid[t]) {
@@ -233,7 +234,7 @@ __global__ __launch_bounds__(256) void skinny_nt_kernel(const NtBatch a) {
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int u = 0; u < RT; ++u) {
-        const int col = 16 * u + i;
+        const int col = rank0 + 16 * u + i;
         if (col >= R) continue;
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
@@ -247,6 +248,107 @@ __global__ __launch_bounds__(256) void skinny_nt_kernel(const NtBatch a) {
             part[((int64_t)split * M + r) * R + col] = sum;
         }
       }
+  }
+}
+
+// The same products over short rows of few tokens (NtPlan says when).  What bounds skinny_nt_kernel there is its shape: 32-row
+// tiles with four waves leave a few workgroups for the whole contraction, so it is cut over workgroups and summed by a
+// second launch, and the rank tiles of a group run one after the other.  Here a workgroup owns 16 rows and 16 ranks and its
+// sixteen waves cut the contraction inside the workgroup: one launch, no partial sums in memory.  Rows beyond M are not
+// loaded.  MFMA, lane layout and the transposing read of BT as above.
+constexpr int kNtFewWaves = 16;
+
+template <bool BT>
+__global__ __launch_bounds__(64 * kNtFewWaves) void skinny_nt_few_kernel(const NtBatch a) {
+  const NtProblem& P = a.p[blockIdx.z];
+  const int r0 = 16 * (int)blockIdx.y;
+  if (r0 >= P.R) return;  // the batch's grid is as wide as its widest problem
+  __shared__ float red[kNtFewWaves - 1][4][64];
+  constexpr int kPitchB = 32;  // 16 columns
+  __shared__ __attribute__((aligned(16))) char bstage[BT ? kNtFewWaves * 64 * kPitchB : 16];
+  const int M = a.M, Kc = P.Kc, R = P.R;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, i = lane & 15;
+  const int m0 = (int)blockIdx.x * 16, r = r0 + i;
+  const bool row_in = m0 + i < M;
+  const uint16_t* xrow = P.X + (int64_t)(row_in ? m0 + i : 0) * Kc + 16 * g;
+  const uint16_t* brow = nullptr;  // !BT: this lane's row of the stacked matrices, absent beyond R
+  if constexpr (!BT) {
+#pragma unroll
+    for (int b = 0; b < kMaxGroup; ++b)
+      if (b < P.nb && r >= P.r_off[b] && r < P.r_off[b + 1]) brow = P.bm[b] + (int64_t)(r - P.r_off[b]) * Kc + 16 * g;
+  }
+  f32x4_t acc[2];
+  acc[0] = acc[1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int chunks = Kc >> 6;
+  char* myb = bstage + (BT ? wave * 64 * kPitchB : 0);
+  const uint32_t brd = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)myb) + (16 * g + (i >> 2)) * kPitchB + 8 * (i & 3);
+  // BT: the 64 x 16 piece of a chunk is one or two 16-byte pieces of each of 64 rows (R % 8 == 0; what lies beyond R in the
+  // second is left as it is in LDS: it reaches only columns that are not stored)
+  const int ppr = R - r0 >= 16 ? 2 : 1;
+#pragma unroll 2
+  for (int c = wave; c < chunks; c += kNtFewWaves) {
+    const int k0 = c * 64;
+    u32x4_t xa[2], wb[2];
+#pragma unroll
+    for (int hh = 0; hh < 2; ++hh) {
+      xa[hh] = u32x4_t{0, 0, 0, 0};
+      if (row_in) xa[hh] = *reinterpret_cast<const u32x4_t*>(xrow + k0 + 8 * hh);
+    }
+    if constexpr (BT) {
+#if defined(__HIP_DEVICE_COMPILE__)
+      u32x4_t piece[2];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int pc = lane + 64 * q;
+        if (pc < 64 * ppr) piece[q] = *reinterpret_cast<const u32x4_t*>(P.bm[0] + (int64_t)(k0 + pc / ppr) * R + r0 + 8 * (pc % ppr));
+      }
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int pc = lane + 64 * q;
+        if (pc < 64 * ppr) *reinterpret_cast<u32x4_t*>(myb + (pc / ppr) * kPitchB + 16 * (pc % ppr)) = piece[q];
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the piece has landed (LDS operations of a wave complete in order)
+      u32x2_t lo[2], hi[2];
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh) {
+        lo[hh] = lds_read_tr16(brd, (8 * hh) * kPitchB);
+        hi[hh] = lds_read_tr16(brd, (8 * hh + 4) * kPitchB);
+      }
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh) {
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(lo[hh]), "+v"(hi[hh]));
+        wb[hh] = u32x4_t{lo[hh].x, lo[hh].y, hi[hh].x, hi[hh].y};
+      }
+#endif
+    } else {
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh) {
+        wb[hh] = u32x4_t{0, 0, 0, 0};
+        if (brow) wb[hh] = *reinterpret_cast<const u32x4_t*>(brow + k0 + 8 * hh);
+      }
+    }
+#pragma unroll
+    for (int hh = 0; hh < 2; ++hh)
+      acc[hh] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, xa[hh]), __builtin_bit_cast(bf16x8_t, wb[hh]), acc[hh], 0, 0, 0);
+  }
+  acc[0] += acc[1];
+  // acc[0][v] = the wave's share of C[m0 + 4 g + v][r]
+  if (wave > 0) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) red[wave - 1][v][lane] = acc[0][v];
+  }
+  __syncthreads();
+  if (wave > 0 || r >= R) return;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const int row = m0 + 4 * g + v;
+    if (row >= M) continue;
+    float sum = acc[0][v];
+#pragma unroll
+    for (int q = 0; q < kNtFewWaves - 1; ++q) sum += red[q][v][lane];
+    P.out[(int64_t)row * P.ldo + r] = f32_to_bf16_bits(sum * P.scale);
   }
 }
 
@@ -950,16 +1052,36 @@ __global__ __launch_bounds__(256) void sum_partials_tn_kernel(const TnSumBatch a
   P.out[r * P.stride_r + k * P.stride_k] = f32_to_bf16_bits(s * P.scale);
 }
 
-constexpr int kTargetWaves = 2048;    // row contractions (skinny_tn)
+constexpr int kTargetWaves = 2048;  // row contractions (skinny_tn)
 constexpr int kTargetWavesNt = 1024;  // column contractions (skinny_nt): few, long waves; one split needs no second pass
 
+// Which of the two kernels a column contraction takes.  skinny_nt_few_kernel streams all of a 16-row tile's x and of 16
+// ranks' lora_a through one CU, about 40 GB/s each, which pays only while that is little: measured (us, graph replay,
+// rank 16 / 48, skinny_nt_kernel + its sums -> skinny_nt_few_kernel) K = 1024: 1 token 4.5 / 6.8 -> 3.0 / 3.1, 700 tokens 6.1 / 9.2 ->
+// 4.4 / 4.6; K = 2048: 4.8 / 7.4 -> 4.0 / 4.2, 700 tokens 6.6 / 9.9 -> 6.2 / 6.3, 2048 tokens 7.1 / 10.5 -> 6.3 / 9.8, 4096 tokens
+// 8.6 / 12.9 -> 6.9 / 13.9; K = 3072: 64 tokens 6.8 / 10.0 -> 7.8 / 7.9; K = 4096: 64 tokens 5.8 / 9.0 -> 9.4 / 9.5.  The transposing
+// form (gh) gains up to 3072 columns (333 tokens, whole adapter backward 15.8 -> 15.2).  The choice depends on M and Kc
+// alone, so that a member of a group sums in the order it sums in alone.
+constexpr int kNtFewTokens = 2048, kNtFewK = 2048, kNtFewKTransposed = 3072;
+// Dealing the 16-rank tiles to workgroups of their own reads x once per tile: pays while x is small (rank 48, us: 64 x 4096 8.9 ->
+// 6.1, 333 x 4096 9.1 -> 7.4, 64 x 14336 10.6 -> 7.9; but 333 x 14336 12.4 -> 13.6).  Same sums in the same order.
+constexpr int64_t kNtRankTilesElements = int64_t(1) << 21;
+
 struct NtPlan {
+  bool few;  // skinny_nt_few_kernel
   int m_tiles, splits, chunks_per_split;
 };
-NtPlan plan_nt(int64_t M, int64_t Kc) {
+NtPlan plan_nt(int64_t M, int64_t Kc, bool bt) {
   NtPlan p;
-  p.m_tiles = (int)((M + 31) / 32);
+  p.few = M <= kNtFewTokens && Kc <= (bt ? kNtFewKTransposed : kNtFewK);
   const int total_chunks = (int)(Kc / 64);
+  if (p.few) {
+    p.m_tiles = (int)((M + 15) / 16);
+    p.splits = 1;
+    p.chunks_per_split = total_chunks;
+    return p;
+  }
+  p.m_tiles = (int)((M + 31) / 32);
   int s = kTargetWavesNt / 4 / p.m_tiles;  // workgroups of 4 waves
   s = s < 1 ? 1 : s;
   const int max_s = (total_chunks + 7) / 8;  // at least two chunks per wave
@@ -970,41 +1092,68 @@ NtPlan plan_nt(int64_t M, int64_t Kc) {
 }
 size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 // fp32 partial sums of one column contraction; 0 when a single slice writes the result directly
-size_t nt_part_bytes(int64_t M, int64_t Kc, int R) {
-  const int sp = plan_nt(M, Kc).splits;
+size_t nt_part_bytes(int64_t M, int64_t Kc, int R, bool bt) {
+  const int sp = plan_nt(M, Kc, bt).splits;
   return sp > 1 ? align256((size_t)sp * M * R * sizeof(float)) : 0;
 }
 
 // Fills in the slicing of the batch's problems (operands, Kc, R, ldo, out, scale are the caller's), hands each sliced
-// problem its piece of `ws` and launches: first pass, then the fixed-order sums of the sliced problems.
+// problem its piece of `ws` and launches: first pass (the problems of few and of many columns in a launch each where a
+// batch has both), then the fixed-order sums of the sliced problems.
 // bt: the second operand is [Kc, R] row-major (transposed inside the kernel) instead of [R, Kc].
 int run_nt_batch(NtBatch& b, int n, bool bt, float* ws, hipStream_t s) {
-  int max_splits = 1, max_r = 0;
-  int64_t max_mr = 0;
-  const int m_tiles = plan_nt(b.M, 64).m_tiles;
+  const dim3 block(256);
+  int64_t max_mr = 0, tiled_elements = 0;
   char* w = reinterpret_cast<char*>(ws);
+  NtBatch few = {}, tiled = {};
+  few.M = tiled.M = b.M;
+  int n_few = 0, n_tiled = 0, max_splits = 1, few_r = 0, tiled_r = 0, few_m_tiles = 0, m_tiles = 0;
   for (int i = 0; i < n; ++i) {
     NtProblem& P = b.p[i];
-    const NtPlan pl = plan_nt(b.M, P.Kc);
+    const NtPlan pl = plan_nt(b.M, P.Kc, bt);
     P.splits = pl.splits;
     P.chunks_per_split = pl.chunks_per_split;
     P.part = reinterpret_cast<float*>(w);
-    w += nt_part_bytes(b.M, P.Kc, P.R);
-    max_splits = pl.splits > max_splits ? pl.splits : max_splits;
-    max_r = P.R > max_r ? P.R : max_r;
+    w += nt_part_bytes(b.M, P.Kc, P.R, bt);
+    tiled_elements = !pl.few && b.M * (int64_t)P.Kc > tiled_elements ? b.M * (int64_t)P.Kc : tiled_elements;
+    if (pl.few) {
+      few.p[n_few++] = P;
+      few_r = P.R > few_r ? P.R : few_r;
+      few_m_tiles = pl.m_tiles;
+    } else {
+      tiled.p[n_tiled++] = P;
+      tiled_r = P.R > tiled_r ? P.R : tiled_r;
+      max_splits = pl.splits > max_splits ? pl.splits : max_splits;
+      m_tiles = pl.m_tiles;
+    }
     if (pl.splits > 1 && (int64_t)b.M * P.R > max_mr) max_mr = (int64_t)b.M * P.R;
   }
-  const dim3 grid((unsigned)m_tiles, (unsigned)max_splits, (unsigned)n), block(256);
-  if (bt) {
-    if (max_r <= 16) skinny_nt_kernel<1, true><<<grid, block, 0, s>>>(b);
-    else if (max_r <= 32) skinny_nt_kernel<2, true><<<grid, block, 0, s>>>(b);
-    else skinny_nt_kernel<4, true><<<grid, block, 0, s>>>(b);
-  } else {
-    if (max_r <= 16) skinny_nt_kernel<1, false><<<grid, block, 0, s>>>(b);
-    else if (max_r <= 32) skinny_nt_kernel<2, false><<<grid, block, 0, s>>>(b);
-    else skinny_nt_kernel<4, false><<<grid, block, 0, s>>>(b);
+  if (n_few > 0) {
+    const dim3 grid((unsigned)few_m_tiles, (unsigned)((few_r + 15) / 16), (unsigned)n_few), few_block(64 * kNtFewWaves);
+    if (bt)
+      skinny_nt_few_kernel<true><<<grid, few_block, 0, s>>>(few);
+    else
+      skinny_nt_few_kernel<false><<<grid, few_block, 0, s>>>(few);
   }
-  if (max_mr > 0) sum_partials_kernel<<<dim3((unsigned)((max_mr + 255) / 256), (unsigned)n), block, 0, s>>>(b);
+  if (n_tiled > 0) {
+    if (!bt && tiled_elements <= kNtRankTilesElements) {
+      const int rank_tiles = (tiled_r + 15) / 16;
+      skinny_nt_kernel<1, false><<<dim3((unsigned)m_tiles, (unsigned)(max_splits * rank_tiles), (unsigned)n_tiled), block, 0, s>>>(tiled, rank_tiles);
+    } else {
+      const dim3 grid((unsigned)m_tiles, (unsigned)max_splits, (unsigned)n_tiled);
+      if (bt) {
+        if (tiled_r <= 16) skinny_nt_kernel<1, true><<<grid, block, 0, s>>>(tiled, 1);
+        else if (tiled_r <= 32) skinny_nt_kernel<2, true><<<grid, block, 0, s>>>(tiled, 1);
+        else skinny_nt_kernel<4, true><<<grid, block, 0, s>>>(tiled, 1);
+      } else {
+        if (tiled_r <= 16) skinny_nt_kernel<1, false><<<grid, block, 0, s>>>(tiled, 1);
+        else if (tiled_r <= 32) skinny_nt_kernel<2, false><<<grid, block, 0, s>>>(tiled, 1);
+        else skinny_nt_kernel<4, false><<<grid, block, 0, s>>>(tiled, 1);
+      }
+    }
+    if (max_mr > 0)
+      sum_partials_kernel<<<dim3((unsigned)((max_mr + 255) / 256), (unsigned)n_tiled), block, 0, s>>>(tiled);
+  }
   return check_launch("skinny_nt");
 }
 
@@ -1149,7 +1298,7 @@ int check_skinny(const char* who, int64_t M, int64_t N, int64_t K, int rank) {
 
 }  // namespace
 
-size_t group_hidden_ws_bytes(int64_t M, int64_t K, int r_total) { return nt_part_bytes(M, K, r_total); }
+size_t group_hidden_ws_bytes(int64_t M, int64_t K, int r_total) { return nt_part_bytes(M, K, r_total, false); }
 
 int run_group_hidden(const uint16_t* x, const GroupSkinny& g, uint16_t* h_cat, float* ws, hipStream_t s) {
   NtBatch b = {};
@@ -1180,7 +1329,7 @@ size_t group_lora_bwd_ws_bytes(const GroupSkinny& g) {
   widths[0] = g.K;
   ranks[0] = g.r_off[g.n];
   for (int i = 0; i < g.n; ++i) {
-    nt += nt_part_bytes(g.M, g.N[i], g.rank[i]);
+    nt += nt_part_bytes(g.M, g.N[i], g.rank[i], true);
     widths[1 + i] = g.N[i];
     ranks[1 + i] = g.rank[i];
   }
@@ -1296,7 +1445,7 @@ using namespace ttamd;
 
 extern "C" size_t ttamd_lora_fwd_workspace_bytes(int64_t M, int64_t K, int rank) {
   if (M <= 0 || K <= 0 || rank <= 0 || K % 64) return 0;
-  return nt_part_bytes(M, K, rank);
+  return nt_part_bytes(M, K, rank, false);
 }
 
 extern "C" int ttamd_lora_hidden_bf16(const void* x, const void* lora_a, void* h, int64_t M, int64_t K, int rank,
@@ -1357,7 +1506,7 @@ extern "C" int ttamd_lora_hidden_static_bf16(const void* x, const void* lora_a, 
   if (int rc = check_skinny("lora_hidden_static", M, 64, K, rank)) return rc;
   TT_REQUIRE(x && lora_a && h, "lora_hidden_static: null pointer argument");
   TT_REQUIRE(aligned16(x) && aligned16(lora_a), "lora_hidden_static: pointers must be 16-byte aligned");
-  const size_t need = nt_part_bytes(M, K, rank);  // 0: one slice writes the result directly
+  const size_t need = nt_part_bytes(M, K, rank, false);  // 0: one slice writes the result directly
   if (need > kStaticScratchBytes)
     return fail(TTAMD_EWORKSPACE, "lora_hidden_static: M=%lld K=%lld rank=%d needs %zu bytes of partial sums, the built-in "
                 "scratch holds %zu; use ttamd_lora_hidden_bf16 with a workspace", (long long)M, (long long)K, rank, need,
