@@ -484,3 +484,31 @@ def test_column_contractions_at_the_edges_of_their_kernels(M, K, R):
     xs = torch.randn(M, 64, device=DEV, generator=g).to(BF)
     gh, _, _ = ops.lora_bwd(x, xs, torch.randn(M, R, device=DEV, generator=g).to(BF), b, 0.75)
     check(gh, x, b, 0.75)
+
+
+@pytest.mark.parametrize("M", [1, 4, 5, 16])
+@pytest.mark.parametrize("N,K,ranks", [(64, 64, (8, 8)), (576, 2112, (40, 24)), (8192, 1088, (16, 8)), (12288, 4160, (8, 16))])
+def test_few_token_pair_and_members(M, N, K, ranks):
+    """The gate / up pair of a handful of tokens in one launch: every output equals the member's own call and the
+    stand-alone gated product bit for bit, and a row's bits do not depend on the batch around it."""
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    members = []
+    for r in ranks:
+        rows = torch.randn(N * K, device=DEV, generator=g).mul_(0.05)
+        pad = -(N * K) % (64 * 256)  # double-quantised scalers come in blocks of 256
+        t = to_nf4(torch.cat([rows, rows.new_zeros(pad)]).to(BF).view(1, -1) if pad else rows.to(BF).view(N, K))
+        members.append(ops.GroupMember(t.quantized_data[:N * K // 2].contiguous(), t.block_scalers()[:N * K // 64].contiguous(), None,
+                                       torch.randn(r, K, device=DEV, generator=g).mul_(0.05).to(BF),
+                                       torch.randn(N, r, device=DEV, generator=g).mul_(0.05).to(BF), None, 2.0, N))
+    x = torch.randn(M, K, device=DEV, generator=g).to(BF)
+    h_cat, (gate, up, act) = ops.lora_group_fwd(x, members, swiglu=True)
+    off = 0
+    for m, y in zip(members, (gate, up)):
+        r = m.lora_a.shape[0]
+        h = ops.lora_hidden(x, m.lora_a)
+        assert torch.equal(h, h_cat[:, off:off + r])
+        assert torch.equal(y, ops.nf4_lora_linear_fwd(x, m.qdata, m.block_scalers, N, h, m.lora_b, m.scale))
+        if M > 1:
+            assert torch.equal(y[:1], ops.nf4_lora_linear_fwd(x[:1], m.qdata, m.block_scalers, N, h[:1].contiguous(), m.lora_b, m.scale))
+        off += r
+    assert torch.equal(act, ops.swiglu_fwd(gate, up))

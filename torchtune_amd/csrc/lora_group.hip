@@ -126,7 +126,12 @@ int group_fwd(const char* who, const void* x, const ttamd_lora_group_member* mem
   // slices of the contraction for a member with few output tiles, when the caller brought the memory for them
   const size_t gem = align256(fwd_gemm_ws(d));
   const bool sliced = gem > 0 && workspace != nullptr && workspace_bytes >= gem;
-  if (group_small_m(d, sliced)) return run_small_m_group(x, d.gm, h_cat, s);
+  if (group_small_m(d, sliced)) {
+    bool done = false;
+    const int rc = run_small_m_group(x, d.gm, h_cat, act, &done, s);
+    if (act_done) *act_done = done;
+    return rc;
+  }
   TT_REQUIRE(!sliced || aligned16(workspace), "%s: workspace must be 16-byte aligned", who);
   // many tokens: one launch over the members' concatenated output columns, every weight expanded once
   if (sliced && dense_group_fwd_workspace_bytes(d.gm) > 0) {

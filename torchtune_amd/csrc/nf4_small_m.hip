@@ -3,19 +3,23 @@
 // torchtune/modules/low_precision/nf4_linear.py:56-70).
 //
 // With so few rows the work is streaming the packed weight once: 0.5625 bytes per weight element against 2 for a
-// dense bf16 weight.  A workgroup owns 16 or 32 weight rows and the whole contraction; its waves (up to sixteen) take
-// groups of 128-wide chunks of K in turn, all of a group's loads in flight together, expand the codes in registers
+// dense bf16 weight.  A workgroup owns 16 or 32 weight rows and the whole contraction, expands the codes in registers
 // exactly as the large-M kernel does (byte -> fp32 pair from an LDS table, times the fp32 block scaler, one rounding to
-// bf16 - the bits of ttamd_nf4_dequantize) and feed v_mfma_f32_16x16x32_bf16 with the weight rows as the row operand
-// and up to four 16-token tiles of x as the column operand.  A lane reads 16 contiguous bytes of codes (32 elements of
+// bf16 - the bits of ttamd_nf4_dequantize) and feeds v_mfma_f32_16x16x32_bf16 with the weight rows as the row operand
+// and 16-token tiles of x as the column operand.  A lane reads 16 contiguous bytes of codes (32 elements of
 // its row: the four lane groups of a row cover one 64-byte piece) and uses one dword of them per MFMA; x is small and
-// comes from the cache.  The waves' partial sums meet in LDS in a fixed order, and wave 0 adds the adapter, the bias
-// and the column scale and stores.  What the kernel reaches is 1.4 - 2.4 TB/s of packed weight, short of the HBM
-// bound: a launch lives for a few trips to memory, and the expansion (about three vector instructions per element) is
-// not hidden behind them.
+// comes from the cache.  The waves' partial sums meet in LDS in a fixed order.
+//
+//  * nf4_few_kernel (at most 16 tokens, generation): the waves take 128-wide chunks of K in turn, one chunk each at a
+//    time.  Neighbouring waves then read neighbouring pieces of the same rows; groups of four chunks per wave, which
+//    put more bytes in flight, were slower at every size.  Only the lanes of tokens that exist ask for x.  The adapter
+//    is one more MFMA step whose operands are requested ahead of the loop, and the gate / up pair of a feed-forward
+//    shares a workgroup, so that silu(gate) * up leaves the same launch.
+//  * nf4_small_m_kernel (17 - 64 tokens): groups of U chunks per wave, two or four token tiles.
 #include "common.h"
 #include "group.h"
 #include "nf4_math.h"
+#include "swiglu_math.h"
 
 namespace ttamd {
 namespace {
@@ -135,9 +139,7 @@ __global__ __launch_bounds__(64 * MAXW) void nf4_small_m_kernel(const SmallMGrou
     if (q < grp.n - 1 && (int)blockIdx.x >= grp.wg_end[q]) which = q + 1;
   const SmallMArgs& a = grp.m[which];
   const int wg = (int)blockIdx.x - (which ? grp.wg_end[which - 1] : 0);
-  // independent MFMA chains per lane: at least four; one token tile always sums in four chains, whatever the row tiles,
-  // so that a row of up to 16 tokens gets the same bits alone and in a batch
-  constexpr int NACC = MT == 1 ? 4 : (MT * RT == 2 ? 2 : 1);
+  constexpr int NACC = MT * RT == 2 ? 2 : 1;  // independent MFMA chains per lane: at least four
   __shared__ float2 lut[256];
   extern __shared__ float red[];  // [waves - 1][MT * RT * 4][64]
   const int t = threadIdx.x, lane = t & 63;
@@ -255,22 +257,210 @@ __global__ __launch_bounds__(64 * MAXW) void nf4_small_m_kernel(const SmallMGrou
   }
 }
 
-// Shape of a launch: token tiles, row tiles per workgroup, chunks in flight per wave, most waves.  It fixes the order
-// in which a row's products are summed, so a layer gets the same bits alone and inside a group.
+constexpr int kFewTokens = 16;
+
+// RT tiles of 16 weight rows per workgroup, at most MAXW waves.  PAIR: tile 0 belongs to grp.m[0] (gate), tile 1 to grp.m[1]
+// (up projection, the same width), and act = bf16(bf16(silu(y_0)) * y_1) is written as well.
+// ONE: the launch has one member, and its arguments sit at fixed places (found through `which` they cost two dependent
+// scalar loads before the first request: 0.4 us of a launch of 6 - 8).
+template <int RT, int MAXW, bool PAIR, bool ONE>
+__global__ __launch_bounds__(64 * MAXW) void nf4_few_kernel(const SmallMGroup grp, uint16_t* __restrict__ act) {
+  static_assert(!PAIR || RT == 2, "a pair is two row tiles");
+  int which = 0;  // uniform over the workgroup
+  if constexpr (!PAIR && !ONE) {
+#pragma unroll
+    for (int q = 0; q < kGroupMax - 1; ++q)
+      if (q < grp.n - 1 && (int)blockIdx.x >= grp.wg_end[q]) which = q + 1;
+  }
+  __shared__ float2 lut[256];
+  __shared__ float red[(MAXW - 1) * RT * 256];
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int nw = blockDim.x >> 6;
+  const int i = lane & 15, g = lane >> 4;
+  const int M = grp.m[which].M, K = grp.m[which].K;
+  const int wg = (int)blockIdx.x - (!PAIR && !ONE && which ? grp.wg_end[which - 1] : 0);
+  auto member = [&](int rt) -> const SmallMArgs& { return grp.m[PAIR ? rt : which]; };
+  auto first_row = [&](int rt) { return PAIR ? 16 * wg : 16 * (RT * wg + rt); };  // N % (16 RT) == 0: every row exists
+
+  const bool token = i < M;
+  const uint16_t* xrow = grp.m[which].x + (int64_t)(token ? i : 0) * K + 32 * g;
+  const uint8_t* crow[RT];
+  const float* srow[RT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    const int64_t n = first_row(rt) + i;
+    crow[rt] = member(rt).codes + ((n * K) >> 1) + 16 * g;
+    srow[rt] = member(rt).bscal + n * (K >> 6) + (g >> 1);
+  }
+  u32x4_t cd[RT], xb[4];
+  float sc[RT];
+  auto request = [&](int c) {
+    const bool in = c * 128 + 32 * g < K;  // the last chunk of a K that is an odd multiple of 64 is half a chunk
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      cd[rt] = u32x4_t{0, 0, 0, 0};
+      sc[rt] = 0.f;
+      if (in) {
+        cd[rt] = *reinterpret_cast<const u32x4_t*>(crow[rt] + (int64_t)c * 64);
+        sc[rt] = srow[rt][2 * c];
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      xb[s] = u32x4_t{0, 0, 0, 0};
+      if (in && token) xb[s] = *reinterpret_cast<const u32x4_t*>(xrow + c * 128 + 8 * s);
+    }
+  };
+  const int n_chunks = (K + 127) >> 7;
+  // The first chunk and wave 0's adapter operands are asked for before the code table is built: a workgroup lives for
+  // little more than one trip to memory, and neither the table nor a second trip at the end must stand in its way.
+  int c = wave;
+  if (c < n_chunks) request(c);
+  auto adapter = [&](int rt, int r0, u32x4_t& hv, u32x4_t& bv) {  // ranks r0 + 8 g .. + 7 (R % 8 == 0)
+    const SmallMArgs& a = member(rt);
+    hv = bv = u32x4_t{0, 0, 0, 0};
+    if (r0 + 8 * g < a.R) {
+      bv = *reinterpret_cast<const u32x4_t*>(a.lora_b + (int64_t)(first_row(rt) + i) * a.R + r0 + 8 * g);
+      if (token) hv = *reinterpret_cast<const u32x4_t*>(a.h + (int64_t)i * a.ldh + r0 + 8 * g);
+    }
+  };
+  u32x4_t hv[RT], bv[RT];
+  if (wave == 0) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) adapter(rt, 0, hv[rt], bv[rt]);
+  }
+  for (int e = t; e < 256; e += blockDim.x)
+    lut[e] = make_float2(round_to_bf16(nf4_code_value(e >> 4)), round_to_bf16(nf4_code_value(e & 15)));
+  f32x4_t acc[RT][4];  // four chains
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int s = 0; s < 4; ++s) acc[rt][s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  __syncthreads();
+  while (c < n_chunks) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {
+        u32x4_t wf;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          const float2 p = lut[(cd[rt][s] >> (8 * b)) & 0xffu];
+          wf[b] = pack_pair(p.x * sc[rt], p.y * sc[rt]);
+        }
+        acc[rt][s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf), __builtin_bit_cast(bf16x8_t, xb[s]),
+                                                             acc[rt][s], 0, 0, 0);
+      }
+    c += nw;
+    if (c < n_chunks) request(c);
+  }
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+    for (int s = 1; s < 4; ++s) acc[rt][0] += acc[rt][s];
+    if (wave == 0) {
+      // adapter: sum_r bf16(h[m][r] * lscale) * lora_b[n][r], the operands the large-M kernel feeds its MFMA
+      const float ls = member(rt).lscale;
+      for (int r0 = 0; r0 < member(rt).R; r0 += 32) {
+        if (r0 > 0) adapter(rt, r0, hv[rt], bv[rt]);
+        u32x4_t hs;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) hs[d] = pack_pair(lo_of(hv[rt][d]) * ls, hi_of(hv[rt][d]) * ls);
+        acc[rt][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, bv[rt]), __builtin_bit_cast(bf16x8_t, hs),
+                                                             acc[rt][0], 0, 0, 0);
+      }
+    } else {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) red[((wave - 1) * RT + rt) * 256 + v * 64 + lane] = acc[rt][0][v];
+    }
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  // acc[rt][0][v] = the wave's share of y[i][first_row(rt) + 4 g + v]
+  u32x2_t out[RT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    const SmallMArgs& a = member(rt);
+    const int nb = first_row(rt) + 4 * g;
+    float o[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      o[v] = acc[rt][0][v];
+      for (int w = 0; w < nw - 1; ++w) o[v] += red[(w * RT + rt) * 256 + v * 64 + lane];
+    }
+    if (a.bias) {
+      const u32x2_t bb = *reinterpret_cast<const u32x2_t*>(a.bias + nb);
+      o[0] += lo_of(bb.x); o[1] += hi_of(bb.x); o[2] += lo_of(bb.y); o[3] += hi_of(bb.y);
+    }
+    if (a.cscale) {
+      const u32x2_t cc = *reinterpret_cast<const u32x2_t*>(a.cscale + nb);
+      o[0] *= lo_of(cc.x); o[1] *= hi_of(cc.x); o[2] *= lo_of(cc.y); o[3] *= hi_of(cc.y);
+    }
+    out[rt].x = pack_pair(o[0], o[1]);
+    out[rt].y = pack_pair(o[2], o[3]);
+    if (token) *reinterpret_cast<u32x2_t*>(a.y + (int64_t)i * a.N + nb) = out[rt];
+  }
+  if constexpr (PAIR) {
+    u32x2_t p;
+    p.x = swiglu_gate_pair(out[0].x, out[1].x);
+    p.y = swiglu_gate_pair(out[0].y, out[1].y);
+    if (token) *reinterpret_cast<u32x2_t*>(act + (int64_t)i * grp.m[0].N + 16 * wg + 4 * g) = p;
+  }
+}
+
+// Launch shape at most 16 tokens.  The waves fix the order in which a row's products are summed and depend on the
+// layer alone, so that a row gets the same bits alone, in a batch of up to 16 tokens and inside a group; row tiles do not
+// enter the sums.  Measured (us, weights from HBM, launch gap included, at 1 / 8 / 16 tokens): 14336 x 4096 four waves and one
+// row tile 14.2 / 18.6 / 23, two tiles 15.4 / 16.9 / 18.9, eight waves and one tile 14.7 / 18.2 / 23; 4096 x 14336 sixteen
+// waves 13.4 / 18.6 / 22.6, eight 15.2 / 17.8 / 21.9; 4096 x 4096 6.5 / 7.7 / 9.0 and 7.1 / 7.8 / 9.0; 8192 x 2048 eight waves
+// 6.2 / 7.5 / 9.0, four 6.8 / 7.4 / 8.5.
+struct FewConfig {
+  int rt, waves;
+  bool operator==(const FewConfig& o) const { return rt == o.rt && waves == o.waves; }
+};
+FewConfig few_config(int64_t M, int64_t N, int64_t K) {
+  if (N < 8192) return {1, 16};
+  return {M > 4 && N >= 12288 ? 2 : 1, K >= 4096 ? 4 : 8};
+}
+
+template <int RT, int MAXW, bool PAIR>
+int launch_few(SmallMGroup& g, void* act, hipStream_t s) {
+  int wgs = 0;
+  for (int i = 0; i < (PAIR ? 1 : g.n); ++i) {
+    wgs += g.m[i].N / (PAIR ? 16 : 16 * RT);
+    g.wg_end[i] = wgs;
+  }
+  const int n_chunks = (g.m[0].K + 127) >> 7;
+  const dim3 grid((unsigned)wgs), block(64 * (n_chunks < MAXW ? n_chunks : MAXW));
+  if (!PAIR && g.n == 1)
+    nf4_few_kernel<RT, MAXW, PAIR, true><<<grid, block, 0, s>>>(g, nullptr);
+  else
+    nf4_few_kernel<RT, MAXW, PAIR, false><<<grid, block, 0, s>>>(g, reinterpret_cast<uint16_t*>(act));
+  return check_launch("nf4_few");
+}
+
+int dispatch_few(SmallMGroup& g, const FewConfig& c, void* pair_act, hipStream_t s) {
+  if (pair_act) {
+    if (c.waves == 16) return launch_few<2, 16, true>(g, pair_act, s);
+    return c.waves == 8 ? launch_few<2, 8, true>(g, pair_act, s) : launch_few<2, 4, true>(g, pair_act, s);
+  }
+  if (c.waves == 16) return launch_few<1, 16, false>(g, nullptr, s);
+  if (c.waves == 8) return c.rt == 2 ? launch_few<2, 8, false>(g, nullptr, s) : launch_few<1, 8, false>(g, nullptr, s);
+  return c.rt == 2 ? launch_few<2, 4, false>(g, nullptr, s) : launch_few<1, 4, false>(g, nullptr, s);
+}
+
+// Shape of a launch of 17 - 64 tokens: token tiles, row tiles per workgroup, chunks in flight per wave, most waves.  It fixes
+// the order in which a row's products are summed, so a layer gets the same bits alone and inside a group.
 struct SmallMConfig {
   int mt, rt, u, max_waves;
   bool operator==(const SmallMConfig& o) const { return mt == o.mt && rt == o.rt && u == o.u && max_waves == o.max_waves; }
 };
-// Measured on MI355X over the projections of an 8B model (kernel time, M = 1 / 8 / 32 / 64): 4096 x 4096
-// 7 / 7 / 13 / 20 us, 14336 x 4096 15 / 17 / 26 / 43 us, 4096 x 14336 14 / 18 / 37 / 64 us.  Wide layers share an x
-// fragment between two row tiles once x is more than one token tile (x comes from L2 once per workgroup); long
-// contractions get sixteen waves, short ones four.  From 9 tokens on the wide layers take two row tiles per workgroup as
-// well: every workgroup reads all of x (16 tokens x 4096: 128 KB, 3.5 times the packed weight bytes over the 896
-// workgroups of a 14336-wide layer), and twice the rows per workgroup halve that (M = 16: 1.33 -> 1.65 TB/s of packed weight).
+// Measured on MI355X over the projections of an 8B model (kernel time, M = 32 / 64): 4096 x 4096 13 / 20 us, 14336 x 4096
+// 26 / 43 us, 4096 x 14336 37 / 64 us.  Wide layers share an x fragment between two row tiles (x comes from L2 once per
+// workgroup); long contractions of four token tiles get sixteen waves, the others four.
 SmallMConfig small_m_config(int64_t M, int64_t N, int64_t K) {
   const bool wide = N >= 8192, deep = K >= 8192;
-  if (M <= 8) return {1, 1, 4, 16};
-  if (M <= 16) return wide ? SmallMConfig{1, 2, 4, 16} : SmallMConfig{1, 1, 4, 16};
   if (M <= 32) return wide ? SmallMConfig{2, 2, 4, 4} : SmallMConfig{2, 1, 4, 4};
   return wide ? SmallMConfig{4, 2, 2, 4} : SmallMConfig{4, 1, 4, deep ? 16 : 4};
 }
@@ -297,7 +487,6 @@ int launch_small_m(SmallMGroup& g, hipStream_t s) {
 }
 
 int dispatch_small_m(SmallMGroup& g, const SmallMConfig& c, hipStream_t s) {
-  if (c.mt == 1) return c.rt == 2 ? launch_small_m<1, 2, 4, 16>(g, s) : launch_small_m<1, 1, 4, 16>(g, s);
   if (c.mt == 2) return c.rt == 2 ? launch_small_m<2, 2, 4, 4>(g, s) : launch_small_m<2, 1, 4, 4>(g, s);
   if (c.rt == 2) return launch_small_m<4, 2, 2, 4>(g, s);
   return c.max_waves > 4 ? launch_small_m<4, 1, 4, 16>(g, s) : launch_small_m<4, 1, 4, 4>(g, s);
@@ -339,34 +528,50 @@ int run_small_m(const void* x, const uint8_t* codes, const void* bscal, const vo
   a.y = reinterpret_cast<uint16_t*>(y);
   a.M = (int)M; a.N = (int)N; a.K = (int)K; a.R = R; a.ldh = ldh;
   a.lscale = lscale;
+  if (M <= kFewTokens) return dispatch_few(g, few_config(M, N, K), nullptr, s);
   return dispatch_small_m(g, small_m_config(M, N, K), s);
 }
 
 // The members of a group (same x, M, K) in as few launches as their launch shapes allow: consecutive members with
-// the same shape share one.
-int run_small_m_group(const void* x, const GroupGemm& gg, const void* h_cat, hipStream_t s) {
+// the same shape share one.  act != nullptr (two members of equal width): *act_done says whether the launch wrote
+// act = silu(y_0) * y_1 too.
+int run_small_m_group(const void* x, const GroupGemm& gg, const void* h_cat, void* act, bool* act_done, hipStream_t s) {
   TT_REQUIRE(gg.M > 0 && gg.M <= small_m_limit(), "nf4_small_m: M (%lld) out of range", (long long)gg.M);
+  SmallMArgs all[kGroupMax] = {};
+  for (int j = 0; j < gg.n; ++j) {
+    TT_REQUIRE(gg.N[j] / 16 < (int64_t(1) << 27) && gg.N[j] * gg.K < (int64_t(1) << 40), "nf4_small_m: weight too large");
+    SmallMArgs& a = all[j];
+    a.x = reinterpret_cast<const uint16_t*>(x);
+    a.codes = gg.codes[j];
+    a.bscal = gg.bscal[j];
+    a.h = reinterpret_cast<const uint16_t*>(h_cat) + gg.r_off[j];
+    a.lora_b = gg.lora_b[j];
+    a.bias = gg.bias[j];
+    a.y = gg.y[j];
+    a.M = (int)gg.M; a.N = (int)gg.N[j]; a.K = (int)gg.K; a.R = gg.rank[j]; a.ldh = gg.r_off[gg.n];
+    a.lscale = gg.scale[j];
+  }
+  const bool few = gg.M <= kFewTokens;
+  if (act && few && gg.n == 2 && gg.N[0] == gg.N[1]) {
+    SmallMGroup g = {};
+    g.m[0] = all[0];
+    g.m[1] = all[1];
+    g.n = 2;
+    *act_done = true;
+    return dispatch_few(g, few_config(gg.M, gg.N[0], gg.K), act, s);
+  }
   int i = 0;
   while (i < gg.n) {
-    const SmallMConfig c = small_m_config(gg.M, gg.N[i], gg.K);
     SmallMGroup g = {};
     int j = i;
-    for (; j < gg.n && small_m_config(gg.M, gg.N[j], gg.K) == c; ++j) {
-      TT_REQUIRE(gg.N[j] / 16 < (int64_t(1) << 27) && gg.N[j] * gg.K < (int64_t(1) << 40), "nf4_small_m: weight too large");
-      SmallMArgs& a = g.m[j - i];
-      a.x = reinterpret_cast<const uint16_t*>(x);
-      a.codes = gg.codes[j];
-      a.bscal = gg.bscal[j];
-      a.h = reinterpret_cast<const uint16_t*>(h_cat) + gg.r_off[j];
-      a.lora_b = gg.lora_b[j];
-      a.bias = gg.bias[j];
-      a.cscale = nullptr;
-      a.y = gg.y[j];
-      a.M = (int)gg.M; a.N = (int)gg.N[j]; a.K = (int)gg.K; a.R = gg.rank[j]; a.ldh = gg.r_off[gg.n];
-      a.lscale = gg.scale[j];
-    }
+    auto same = [&](int q) {
+      return few ? few_config(gg.M, gg.N[q], gg.K) == few_config(gg.M, gg.N[i], gg.K)
+                 : small_m_config(gg.M, gg.N[q], gg.K) == small_m_config(gg.M, gg.N[i], gg.K);
+    };
+    for (; j < gg.n && same(j); ++j) g.m[j - i] = all[j];
     g.n = j - i;
-    if (int rc = dispatch_small_m(g, c, s)) return rc;
+    if (int rc = few ? dispatch_few(g, few_config(gg.M, gg.N[i], gg.K), nullptr, s) : dispatch_small_m(g, small_m_config(gg.M, gg.N[i], gg.K), s))
+      return rc;
     i = j;
   }
   return TTAMD_OK;
