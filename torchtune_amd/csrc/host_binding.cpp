@@ -47,6 +47,8 @@ Tensor scratch(size_t bytes, const Tensor& like) {
   return at::empty({(int64_t)(bytes > 16 ? bytes : 16)}, like.options().dtype(at::kByte));
 }
 
+size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
+
 bool wants_grad(std::initializer_list<const Tensor*> ts) {
   if (!at::GradMode::is_enabled()) return false;
   for (const Tensor* t : ts)
@@ -287,7 +289,8 @@ struct LinearOut {
   Tensor x2, h, y;
 };
 
-LinearOut linear_forward(const Tensor& x, Member m) {
+// keep: the hidden activation is wanted for a backward; otherwise it lives at the head of the workspace
+LinearOut linear_forward(const Tensor& x, Member m, bool keep) {
   const int64_t K = x.size(-1);
   LinearOut o;
   o.x2 = bf16(x, "qlora_linear_fwd").view({-1, K});
@@ -296,11 +299,13 @@ LinearOut linear_forward(const Tensor& x, Member m) {
   const int64_t M = o.x2.size(0);
   const int rank = (int)m.a.size(0);
   o.y = at::empty(with_last(x, m.w.N), o.x2.options());
-  o.h = at::empty({M, rank}, o.x2.options());
-  const Tensor ws = scratch(ttamd_qlora_linear_fwd_workspace_bytes(M, m.w.N, K, rank), o.x2);
+  if (keep) o.h = at::empty({M, rank}, o.x2.options());
+  const size_t h_bytes = keep ? 0 : align256(M * rank * 2);
+  const Tensor ws = scratch(h_bytes + ttamd_qlora_linear_fwd_workspace_bytes(M, m.w.N, K, rank), o.x2);
+  char* w = (char*)ws.data_ptr();
   check(ttamd_qlora_linear_fwd_bf16(o.x2.data_ptr(), (const uint8_t*)m.w.q.data_ptr(), m.w.scal.data_ptr(), opt_ptr(m.w.scal_t), m.a.data_ptr(),
-                                    m.b.data_ptr(), rank, (float)m.scale, opt_ptr(m.bias), o.y.data_ptr(), o.h.data_ptr(), M, m.w.N, K,
-                                    ws.data_ptr(), ws.numel(), stream_of(x)),
+                                    m.b.data_ptr(), rank, (float)m.scale, opt_ptr(m.bias), o.y.data_ptr(), keep ? o.h.data_ptr() : w, M,
+                                    m.w.N, K, w + h_bytes, ws.numel() - h_bytes, stream_of(x)),
         "qlora_linear_fwd");
   return o;
 }
@@ -325,7 +330,7 @@ struct QLoRALinearFn : torch::autograd::Function<QLoRALinearFn> {
     m.b = b;
     if (bias) m.bias = *bias;
     m.scale = scale;
-    LinearOut o = linear_forward(x, m);
+    LinearOut o = linear_forward(x, m, true);
     ctx->save_for_backward({o.x2, o.h, a, b});
     ctx->saved_data["w"] = pack_weight(w);
     ctx->saved_data["scale"] = scale;
@@ -374,7 +379,7 @@ Tensor qlora_linear(const Tensor& x, const Tensor& q, const Tensor& scal, const 
   m.a = a;
   m.b = b;
   m.scale = scale;
-  return linear_forward(x, m).y;
+  return linear_forward(x, m, false).y;
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -400,7 +405,7 @@ void fill(ttamd_lora_group_member& e, const Member& m, const Tensor& y) {
   e.scale = (float)m.scale;
 }
 
-GroupOut group_forward(const Tensor& x, std::vector<Member>& ms, bool gated) {
+GroupOut group_forward(const Tensor& x, std::vector<Member>& ms, bool gated, bool keep) {
   const int n = (int)ms.size();
   TORCH_CHECK_VALUE(n >= 1 && n <= TTAMD_GROUP_MAX, "lora_group_fwd: a group has 1 to ", TTAMD_GROUP_MAX, " members, got ", n);
   TORCH_CHECK_VALUE(!gated || (n == 2 && ms[0].w.N == ms[1].w.N),
@@ -418,17 +423,21 @@ GroupOut group_forward(const Tensor& x, std::vector<Member>& ms, bool gated) {
     fill(arr[i], ms[i], o.ys[i]);
     r_total += ms[i].a.size(0);
   }
-  o.h_cat = at::empty({M, r_total}, o.x2.options());
+  if (keep) o.h_cat = at::empty({M, r_total}, o.x2.options());
+  const size_t h_bytes = keep ? 0 : align256(M * r_total * 2);
   const size_t hidden = ttamd_lora_group_hidden_workspace_bytes(arr, n, M, K), fwd = ttamd_lora_group_fwd_workspace_bytes(arr, n, M, K);
-  const Tensor ws = scratch(hidden > fwd ? hidden : fwd, o.x2);
+  const size_t bytes = hidden > fwd ? hidden : fwd;
+  const Tensor mem = scratch(h_bytes + bytes, o.x2);
+  void* const h_cat = keep ? o.h_cat.data_ptr() : mem.data_ptr();
+  void* const ws = (char*)mem.data_ptr() + h_bytes;
   void* s = stream_of(x);
-  check(ttamd_lora_group_hidden_bf16(o.x2.data_ptr(), arr, n, o.h_cat.data_ptr(), M, K, ws.data_ptr(), ws.numel(), s), "lora_group_hidden");
+  check(ttamd_lora_group_hidden_bf16(o.x2.data_ptr(), arr, n, h_cat, M, K, ws, bytes, s), "lora_group_hidden");
   if (gated) {
     o.act = at::empty_like(o.ys[0]);
-    check(ttamd_nf4_lora_group_swiglu_fwd_bf16(o.x2.data_ptr(), arr, n, o.h_cat.data_ptr(), o.act.data_ptr(), M, K, ws.data_ptr(), ws.numel(), s),
+    check(ttamd_nf4_lora_group_swiglu_fwd_bf16(o.x2.data_ptr(), arr, n, h_cat, o.act.data_ptr(), M, K, ws, bytes, s),
           "lora_group_fwd");
   } else {
-    check(ttamd_nf4_lora_group_fwd_bf16(o.x2.data_ptr(), arr, n, o.h_cat.data_ptr(), M, K, ws.data_ptr(), ws.numel(), s), "lora_group_fwd");
+    check(ttamd_nf4_lora_group_fwd_bf16(o.x2.data_ptr(), arr, n, h_cat, M, K, ws, bytes, s), "lora_group_fwd");
   }
   return o;
 }
@@ -441,7 +450,7 @@ struct GroupSpec {
 // Differentiable inputs: x, then per member lora_a, lora_b and, where there is one, the bias.
 struct QLoRAGroupFn : torch::autograd::Function<QLoRAGroupFn> {
   static variable_list forward(AutogradContext* ctx, const Tensor& x, at::TensorList /*adapters*/, GroupSpec& spec) {
-    GroupOut o = group_forward(x, spec.ms, spec.gated);
+    GroupOut o = group_forward(x, spec.ms, spec.gated, true);
     variable_list save = {o.x2, o.h_cat};
     std::vector<Tensor> weights;
     std::vector<int64_t> n_out, bias;
@@ -568,7 +577,7 @@ std::vector<Tensor> lora_group(const Tensor& x, const std::vector<MemberTuple>& 
     spec.ms.push_back(std::move(m));
   }
   if (grad) return QLoRAGroupFn::apply(x, at::TensorList(adapters), spec);
-  GroupOut o = group_forward(x, spec.ms, gated);
+  GroupOut o = group_forward(x, spec.ms, gated, false);
   if (gated) return {o.act};
   return o.ys;
 }

@@ -223,8 +223,8 @@ def _native_group(x: torch.Tensor, layers, gated: bool):
     grad = torch.is_grad_enabled()
     members = []
     for layer in layers:
-        w = layer.weight
-        members.append((*host_weight(w, tokens, grad), layer.lora_a.weight, layer.lora_b.weight, layer.alpha / layer.rank, layer.bias))
+        w, lora_a, lora_b, bias = layer._fused_operands()
+        members.append((*host_weight(w, tokens, grad), lora_a, lora_b, layer.alpha / layer.rank, bias))
     return _host.load().lora_group(x, members, gated)
 
 
