@@ -512,6 +512,13 @@ size_t ttamd_int4_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int ttamd_int8_group_linear_bf16(const void* x, const int8_t* q, const void* scale, const void* zero_point, int qparam_dtype,
                                  int group_size, const void* bias, void* y, int64_t M, int64_t N, int64_t K, void* workspace,
                                  size_t workspace_bytes, void* stream);
+/* The same from the activation as it is: ttamd_fq_per_token_int8_asym (qparams in `qparam_dtype`) followed by
+ * ttamd_int8_group_linear_bf16, the same bits; at a token or a few in one launch.  workspace:
+ * ttamd_int8_dynamic_linear_workspace_bytes(M, N, K) bytes (0: may be NULL). */
+size_t ttamd_int8_dynamic_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int ttamd_int8_dynamic_linear_bf16(const void* x, const int8_t* q, const void* scale, const void* zero_point, int qparam_dtype,
+                                   int group_size, const void* bias, void* y, int64_t M, int64_t N, int64_t K, void* workspace,
+                                   size_t workspace_bytes, void* stream);
 int ttamd_uint4_group_linear_bf16(const void* x, const uint8_t* q, const void* scales_and_zeros, int group_size,
                                   const void* bias, void* y, int64_t M, int64_t N, int64_t K, void* workspace,
                                   size_t workspace_bytes, void* stream);

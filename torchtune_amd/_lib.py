@@ -152,6 +152,9 @@ SIGNATURES = {
     "ttamd_int4_linear_workspace_bytes": (_size, [_i64, _i64, _i64]),
     "ttamd_int8_group_linear_bf16": (
         _int, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _int, _int, _c_void_p, _c_void_p, _i64, _i64, _i64, _c_void_p, _size, _c_void_p]),
+    "ttamd_int8_dynamic_linear_workspace_bytes": (_size, [_i64, _i64, _i64]),
+    "ttamd_int8_dynamic_linear_bf16": (
+        _int, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _int, _int, _c_void_p, _c_void_p, _i64, _i64, _i64, _c_void_p, _size, _c_void_p]),
     "ttamd_uint4_group_linear_bf16": (
         _int, [_c_void_p, _c_void_p, _c_void_p, _int, _c_void_p, _c_void_p, _i64, _i64, _i64, _c_void_p, _size, _c_void_p]),
     "ttamd_fq_per_token_int8_asym_conv": (

@@ -6,6 +6,7 @@
 // wave (or of g/8 neighbouring lanes) and min/max travel over cross-lane shuffles, so the data is read
 // from HBM exactly once.
 #include "common.h"
+#include "fq_math.h"
 #include "nf4_math.h"
 
 namespace ttamd {
@@ -14,8 +15,6 @@ namespace {
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
-
-constexpr float kF32Eps = 1.1920928955078125e-07f;  // torch.finfo(torch.float32).eps
 
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
   bf16x2_t v;
@@ -69,42 +68,6 @@ struct Chunk8<false> {
     __builtin_nontemporal_store(hi, p + 1);
   }
 };
-
-struct TokenQParams {
-  float scale, inv_scale, zp;
-};
-
-// asymmetric int8 qparams from the row extrema (already widened to include 0)
-// (the zero point is chosen with the fp32 scale; a bf16 qparam precision rounds the scale afterwards, and the rounded
-// scale is what quantises and dequantises)
-__device__ __forceinline__ TokenQParams token_qparams(float mn, float mx, bool qp_bf16, float eps) {
-  TokenQParams p;
-  float scale = (mx - mn) / 255.0f;
-  scale = scale > eps ? scale : eps;
-  const float dmin = mn / scale, dmax = mx / scale;
-  float zp = ((-128.0f + dmin) + (127.0f + dmax) > 0.0f) ? (-128.0f - dmin) : (127.0f - dmax);
-  zp = zp < -128.0f ? -128.0f : (zp > 127.0f ? 127.0f : zp);
-  p.zp = __builtin_rintf(zp);
-  if (qp_bf16) scale = round_to_bf16(scale);
-  p.scale = scale;
-  p.inv_scale = 1.0f / scale;
-  return p;
-}
-
-template <bool BF16>
-__device__ __forceinline__ float token_fq(float x, const TokenQParams& p) {
-  float q = __builtin_rintf(x * p.inv_scale) + p.zp;
-  q = q < -128.0f ? -128.0f : (q > 127.0f ? 127.0f : q);
-  return Arith<BF16>::rnd((q - p.zp) * p.scale);
-}
-
-__device__ __forceinline__ void wave_minmax(float& mn, float& mx) {
-#pragma unroll
-  for (int off = 1; off < kWave; off <<= 1) {
-    mn = fminf(mn, __shfl_xor(mn, off, kWave));
-    mx = fmaxf(mx, __shfl_xor(mx, off, kWave));
-  }
-}
 
 // One wave per token row, the whole row resident in registers: NV chunks of 8 elements per lane.
 template <bool BF16, int NV>

@@ -604,15 +604,12 @@ Tensor int8_dynamic_linear(const Tensor& x, const Tensor& q, const Tensor& scale
   const Tensor b = bias ? bf16(*bias, "int8_group_linear") : Tensor();
   TORCH_CHECK_VALUE(!b.defined() || b.numel() == N, "int8_group_linear: bias must have ", N, " elements");
   const c10::DeviceGuard guard(x.device());
-  void* s = stream_of(x);
-  const Tensor xq = at::empty_like(x2);
-  check(ttamd_fq_per_token_int8_asym(x2.data_ptr(), TTAMD_BF16, M, K, code, xq.data_ptr(), nullptr, nullptr, s), "fq_per_token_int8_asym");
   Tensor y = at::empty(with_last(x, N), x2.options());
-  const size_t bytes = ttamd_int4_linear_workspace_bytes(M, N, K);
+  const size_t bytes = ttamd_int8_dynamic_linear_workspace_bytes(M, N, K);
   const Tensor ws = bytes ? scratch(bytes, x2) : Tensor();
-  check(ttamd_int8_group_linear_bf16(xq.data_ptr(), (const int8_t*)q.data_ptr(), scale.data_ptr(), zeros.data_ptr(), code, (int)group_size,
-                                     opt_ptr(b), y.data_ptr(), M, N, K, opt_ptr(ws), bytes, s),
-        "int8_group_linear");
+  check(ttamd_int8_dynamic_linear_bf16(x2.data_ptr(), (const int8_t*)q.data_ptr(), scale.data_ptr(), zeros.data_ptr(), code, (int)group_size,
+                                       opt_ptr(b), y.data_ptr(), M, N, K, opt_ptr(ws), bytes, stream_of(x)),
+        "int8_dynamic_linear");
   return y;
 }
 

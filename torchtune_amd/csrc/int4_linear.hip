@@ -25,6 +25,7 @@
 // A launch's fixed part is about 6 us of these; what goes beyond it streams int8 weight at 3.6 TB/s.  Above 256 tokens the
 // two m-tiles' expansion and their slabs cost what the dense copy costs, and the library's larger tiles win.
 #include "common.h"
+#include "fq_math.h"
 #include "nf4_math.h"
 
 namespace ttamd {
@@ -56,6 +57,7 @@ struct Int4Args {
   int M, N, K;
   int log2_group;        // >= 5
   int chunks_per_slice;
+  int qp_bf16;           // DYN: the activation's scale is rounded to bf16
 };
 
 // How a weight is stored.
@@ -123,36 +125,130 @@ struct WeightPiece<kInt8Bf16> : Int8Piece<true> {};
 
 constexpr int kStreamTokens = 16;
 
-// RT tiles of 16 weight rows per workgroup (they share a wave's fragments of x), at most MAXW waves.
-template <int FMT, int RT, int MAXW>
+// DYN: x arrives as it is and every workgroup fake-quantises it per token into LDS while its first weights are on their way:
+// at one token that is 8 - 28 KB read from the cache per workgroup, against a launch of its own (3.8 us and a gap per
+// linear: a fifth of a generating layer's time).  A thread holds its share of x, kDynPieces pieces of 8 elements, in
+// registers between the extrema and the rounding; a wave's piece lies within one token (one token, or rows of whole pieces).
+constexpr int kDynPieces = 4;
+constexpr int kDynMaxTokens = 8;
+
+template <int T>  // threads of the workgroup
+__device__ __forceinline__ void quantise_tokens(const Int4Args& a, const u32x4_t (&raw)[kDynPieces], uint16_t* xq, float (*ext)[kDynPieces * T / 64]) {
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  constexpr int NW = T / 64;
+  const int total = a.M * (a.K >> 3);  // pieces
+  auto extrema = [&](int j, float& mn, float& mx) {  // the qparams use min(amin, 0) and max(amax, 0): zero is the neutral start
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      mn = fminf(fminf(mn, lo_of(raw[j][d])), hi_of(raw[j][d]));
+      mx = fmaxf(fmaxf(mx, lo_of(raw[j][d])), hi_of(raw[j][d]));
+    }
+  };
+  auto quantise = [&](int j, const TokenQParams& p) {
+    const int piece = j * T + t;
+    u32x4_t o;
+#pragma unroll
+    for (int d = 0; d < 4; ++d) o[d] = pack_pair(token_fq<true>(lo_of(raw[j][d]), p), token_fq<true>(hi_of(raw[j][d]), p));
+    if (piece < total) reinterpret_cast<u32x4_t*>(xq)[piece] = o;
+  };
+  if (a.M == 1) {  // one pair of extrema for the workgroup
+    float mn = 0.f, mx = 0.f;
+#pragma unroll
+    for (int j = 0; j < kDynPieces; ++j)
+      if (j * T < total) extrema(j, mn, mx);
+    wave_minmax(mn, mx);
+    if (lane == 0) {
+      ext[0][wave] = mn;
+      ext[1][wave] = mx;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      mn = fminf(mn, ext[0][w]);
+      mx = fmaxf(mx, ext[1][w]);
+    }
+    const TokenQParams p = token_qparams(mn, mx, a.qp_bf16 != 0, kF32Eps);
+#pragma unroll
+    for (int j = 0; j < kDynPieces; ++j)
+      if (j * T < total) quantise(j, p);
+  } else {
+#pragma unroll
+    for (int j = 0; j < kDynPieces; ++j) {
+      if (j * T >= total) break;
+      float mn = 0.f, mx = 0.f;
+      extrema(j, mn, mx);
+      wave_minmax(mn, mx);
+      if (lane == 0) {
+        ext[0][j * NW + wave] = mn;
+        ext[1][j * NW + wave] = mx;
+      }
+    }
+    __syncthreads();
+    const int per_token = a.K >> 9;  // wave pieces per token, at most 64
+#pragma unroll
+    for (int j = 0; j < kDynPieces; ++j) {
+      if (j * T >= total) break;
+      const int m = (j * NW + wave) / per_token;  // uniform over the wave
+      float mn = 0.f, mx = 0.f;
+      if (m < a.M && lane < per_token) {
+        mn = ext[0][m * per_token + lane];
+        mx = ext[1][m * per_token + lane];
+      }
+      wave_minmax(mn, mx);
+      quantise(j, token_qparams(mn, mx, a.qp_bf16 != 0, kF32Eps));
+    }
+  }
+  __syncthreads();
+}
+
+// RT tiles of 16 weight rows per workgroup (they share a wave's fragments of x), at most MAXW waves (DYN: exactly).
+template <int FMT, int RT, int MAXW, bool DYN>
 __global__ __launch_bounds__(64 * MAXW) void int4_stream_kernel(const Int4Args a) {
   __shared__ float red[(MAXW - 1) * RT * 256];
+  __shared__ __attribute__((aligned(16))) uint16_t xq[DYN ? kDynPieces * 8 * 64 * MAXW : 8];
+  __shared__ float ext[2][DYN ? kDynPieces * MAXW : 1];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nw = blockDim.x >> 6;
   const int i = lane & 15, g = lane >> 4;
   const int n0 = (int)blockIdx.x * (16 * RT);  // N % 64 == 0: every row of the workgroup exists
   const bool token = i < a.M;
-  const uint16_t* xrow = a.x + (int64_t)(token ? i : 0) * a.K + 32 * g;
+  const uint16_t* xrow = (DYN ? xq : a.x) + (int64_t)(token ? i : 0) * a.K + 32 * g;
   const int n_chunks = (a.K + 127) >> 7;
+  WeightPiece<FMT> w[RT];
+  auto request = [&](int c) {
+    const int k = c * 128 + 32 * g;
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      if (k < a.K)  // K % 32 == 0
+        w[rt].load(a, n0 + 16 * rt + i, k);
+      else
+        w[rt].clear();
+    }
+  };
+  int c = wave;
+  if constexpr (DYN) {
+    u32x4_t raw[kDynPieces];  // asked for ahead of the weights, which then stay in flight while it is quantised
+#pragma unroll
+    for (int j = 0; j < kDynPieces; ++j) {
+      const int piece = j * 64 * MAXW + (int)threadIdx.x;
+      raw[j] = u32x4_t{0, 0, 0, 0};
+      if (piece < a.M * (a.K >> 3)) raw[j] = reinterpret_cast<const u32x4_t*>(a.x)[piece];
+    }
+    if (c < n_chunks) request(c);
+    quantise_tokens<64 * MAXW>(a, raw, xq, ext);
+  } else {
+    if (c < n_chunks) request(c);
+  }
   f32x4_t acc[RT][4];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
     for (int s = 0; s < 4; ++s) acc[rt][s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  for (int c = wave; c < n_chunks; c += nw) {
-    WeightPiece<FMT> w[RT];
+  while (c < n_chunks) {
     u32x4_t xb[4];
-    const int k = c * 128 + 32 * g;
-    const bool in = k < a.K;  // K % 32 == 0
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-      if (in)
-        w[rt].load(a, n0 + 16 * rt + i, k);
-      else
-        w[rt].clear();
-    }
+    const bool in = c * 128 + 32 * g < a.K;
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       xb[s] = u32x4_t{0, 0, 0, 0};
@@ -164,6 +260,8 @@ __global__ __launch_bounds__(64 * MAXW) void int4_stream_kernel(const Int4Args a
       for (int rt = 0; rt < RT; ++rt)
         acc[rt][s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w[rt].operand(s)),
                                                              __builtin_bit_cast(bf16x8_t, xb[s]), acc[rt][s], 0, 0, 0);
+    c += nw;
+    if (c < n_chunks) request(c);
   }
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
@@ -346,13 +444,27 @@ void launch_tile(const Int4Args& a, int mt, dim3 grid, hipStream_t s) {
 }
 
 template <int FMT, int RT, int MAXW>
-void launch_stream(const Int4Args& a, hipStream_t s) {
+void launch_stream(const Int4Args& a, bool dyn, hipStream_t s) {
   const int n_chunks = (a.K + 127) >> 7;
-  int4_stream_kernel<FMT, RT, MAXW><<<dim3(a.N / (16 * RT)), dim3(64 * (n_chunks < MAXW ? n_chunks : MAXW)), 0, s>>>(a);
+  if constexpr (FMT != kUint4) {
+    if (dyn) {
+      int4_stream_kernel<FMT, RT, MAXW, true><<<dim3(a.N / (16 * RT)), dim3(64 * MAXW), 0, s>>>(a);
+      return;
+    }
+  }
+  int4_stream_kernel<FMT, RT, MAXW, false><<<dim3(a.N / (16 * RT)), dim3(64 * (n_chunks < MAXW ? n_chunks : MAXW)), 0, s>>>(a);
 }
 
+// Waves of the int8 launch of at most 16 tokens, and whether it can quantise these activations itself: they fit the pieces
+// its threads hold, and no wave's piece crosses a row.
+int int8_stream_waves(int64_t N) { return N >= 8192 ? 4 : 8; }
+bool quantises_in_stream(int64_t M, int64_t N, int64_t K) {
+  return M <= kDynMaxTokens && (M == 1 || K % 512 == 0) && K <= 32768 && M * K <= int8_stream_waves(N) * 64 * kDynPieces * 8;
+}
+
+// dyn: x is not quantised yet (quantises_in_stream holds)
 template <int FMT>
-int launch(Int4Args& a, void* workspace, size_t workspace_bytes, hipStream_t s) {
+int launch(Int4Args& a, bool dyn, void* workspace, size_t workspace_bytes, hipStream_t s) {
   if (a.M <= kStreamTokens) {
     // Measured (weights from HBM, us, launch gap included).  Wide layers have workgroups to spare: few waves each, and
     // two row tiles where the reads of x weigh (int8 14336 x 4096 at 1 / 16 tokens: four waves and two tiles 21.2 / 27.8,
@@ -360,12 +472,12 @@ int launch(Int4Args& a, void* workspace, size_t workspace_bytes, hipStream_t s) 
     // 4096 x 14336 at 1 token: sixteen 20.0, eight 20.9; at 16 tokens 25 and 21.6).
     const bool wide = a.N >= 8192;
     if constexpr (FMT == kUint4) {
-      if (wide && a.M > 8) launch_stream<FMT, 2, 8>(a, s);
-      else if (wide || a.M > 8) launch_stream<FMT, 1, 8>(a, s);
-      else launch_stream<FMT, 1, 16>(a, s);
+      if (wide && a.M > 8) launch_stream<FMT, 2, 8>(a, dyn, s);
+      else if (wide || a.M > 8) launch_stream<FMT, 1, 8>(a, dyn, s);
+      else launch_stream<FMT, 1, 16>(a, dyn, s);
     } else {
-      if (wide) launch_stream<FMT, 2, 4>(a, s);
-      else launch_stream<FMT, 1, 8>(a, s);
+      if (wide) launch_stream<FMT, 2, 4>(a, dyn, s);
+      else launch_stream<FMT, 1, 8>(a, dyn, s);
     }
     return check_launch("int4_linear");
   }
@@ -427,9 +539,42 @@ extern "C" int ttamd_int8_group_linear_bf16(const void* x, const int8_t* q, cons
   TT_REQUIRE(qparam_dtype == TTAMD_BF16 || qparam_dtype == TTAMD_F32, "int8_group_linear: unknown qparam dtype code %d", qparam_dtype);
   Int4Args a = {reinterpret_cast<const uint16_t*>(x), reinterpret_cast<const uint8_t*>(q), scale, zero_point,
                 reinterpret_cast<const uint16_t*>(bias), reinterpret_cast<uint16_t*>(y), nullptr, (int)M, (int)N, (int)K,
-                log2_of(group_size), 0};
+                log2_of(group_size), 0, 0};
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  return qparam_dtype == TTAMD_BF16 ? launch<kInt8Bf16>(a, workspace, workspace_bytes, s) : launch<kInt8F32>(a, workspace, workspace_bytes, s);
+  return qparam_dtype == TTAMD_BF16 ? launch<kInt8Bf16>(a, false, workspace, workspace_bytes, s)
+                                    : launch<kInt8F32>(a, false, workspace, workspace_bytes, s);
+}
+
+namespace {
+size_t quantised_bytes(int64_t M, int64_t N, int64_t K) {
+  return quantises_in_stream(M, N, K) ? 0 : ((size_t)M * K * 2 + 255) / 256 * 256;
+}
+}  // namespace
+
+extern "C" size_t ttamd_int8_dynamic_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+  if (M <= 0 || M > kMaxTokens || N < 64 || K <= 0) return 0;
+  return quantised_bytes(M, N, K) + ttamd_int4_linear_workspace_bytes(M, N, K);
+}
+
+extern "C" int ttamd_int8_dynamic_linear_bf16(const void* x, const int8_t* q, const void* scale, const void* zero_point,
+                                              int qparam_dtype, int group_size, const void* bias, void* y, int64_t M, int64_t N,
+                                              int64_t K, void* workspace, size_t workspace_bytes, void* stream) {
+  if (int rc = check_args(x, q, scale, y, M, N, K, group_size)) return rc;
+  TT_REQUIRE(qparam_dtype == TTAMD_BF16 || qparam_dtype == TTAMD_F32, "int8_dynamic_linear: unknown qparam dtype code %d", qparam_dtype);
+  const size_t head = quantised_bytes(M, N, K), need = ttamd_int8_dynamic_linear_workspace_bytes(M, N, K);
+  if (need > 0 && (!workspace || workspace_bytes < need))
+    return fail(TTAMD_EWORKSPACE, "int8_dynamic_linear: workspace of %zu bytes, %zu needed", workspace_bytes, need);
+  TT_REQUIRE(need == 0 || aligned16(workspace), "int8_dynamic_linear: the workspace must be 16-byte aligned");
+  if (head > 0) {
+    if (int rc = ttamd_fq_per_token_int8_asym(x, TTAMD_BF16, M, K, qparam_dtype, workspace, nullptr, nullptr, stream)) return rc;
+    return ttamd_int8_group_linear_bf16(workspace, q, scale, zero_point, qparam_dtype, group_size, bias, y, M, N, K,
+                                        reinterpret_cast<char*>(workspace) + head, workspace_bytes - head, stream);
+  }
+  Int4Args a = {reinterpret_cast<const uint16_t*>(x), reinterpret_cast<const uint8_t*>(q), scale, zero_point,
+                reinterpret_cast<const uint16_t*>(bias), reinterpret_cast<uint16_t*>(y), nullptr, (int)M, (int)N, (int)K,
+                log2_of(group_size), 0, qparam_dtype == TTAMD_BF16 ? 1 : 0};
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  return qparam_dtype == TTAMD_BF16 ? launch<kInt8Bf16>(a, true, nullptr, 0, s) : launch<kInt8F32>(a, true, nullptr, 0, s);
 }
 
 extern "C" int ttamd_uint4_group_linear_bf16(const void* x, const uint8_t* q, const void* scales_and_zeros, int group_size,
@@ -437,6 +582,6 @@ extern "C" int ttamd_uint4_group_linear_bf16(const void* x, const uint8_t* q, co
                                              size_t workspace_bytes, void* stream) {
   if (int rc = check_args(x, q, scales_and_zeros, y, M, N, K, group_size)) return rc;
   Int4Args a = {reinterpret_cast<const uint16_t*>(x), q, scales_and_zeros, nullptr, reinterpret_cast<const uint16_t*>(bias),
-                reinterpret_cast<uint16_t*>(y), nullptr, (int)M, (int)N, (int)K, log2_of(group_size), 0};
-  return launch<kUint4>(a, workspace, workspace_bytes, reinterpret_cast<hipStream_t>(stream));
+                reinterpret_cast<uint16_t*>(y), nullptr, (int)M, (int)N, (int)K, log2_of(group_size), 0, 0};
+  return launch<kUint4>(a, false, workspace, workspace_bytes, reinterpret_cast<hipStream_t>(stream));
 }
