@@ -403,6 +403,17 @@ int ttamd_nf4_group_bwd_dx_ws_bf16(const ttamd_lora_group_member* members, int n
                                    int64_t K, void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * Plain bf16 products (fp32 accumulation, one rounding) of a few dozen to about two thousand rows: the matmuls of a
+ * fake-quantised linear at short sequences (F.linear and its autograd on torchao's FakeQuantizedLinear; the recipes reach
+ * it from recipes/qat_single_device.py).  kind 0: c[M,N] = a[M,K] . b[N,K]^T (+ bias [N] or NULL); 1: c[M,N] = a[M,K] . b[K,N];
+ * 2: c[M,N] = a[K,M]^T . b[K,N].  N % 64 == 0; kinds 0 and 1: K % 64 == 0; kind 2: M % 64 == 0, any K.  workspace:
+ * ttamd_gemm_mid_workspace_bytes(M, N, K) bytes (0: may be NULL).
+ */
+size_t ttamd_gemm_mid_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int ttamd_gemm_mid_bf16(int kind, const void* a, const void* b, const void* bias, void* c, int64_t M, int64_t N, int64_t K,
+                        void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * One expansion for both directions of a group.  ttamd_nf4_group_fwd_leaves_tiles says what the group's forward call
  * (ttamd_nf4_lora_group_fwd_bf16; swiglu != 0: ttamd_nf4_lora_group_swiglu_fwd_bf16) leaves at the start of a workspace
  * of the size its query asks for: 0 nothing reusable, 1 the members' weights expanded to bf16 and stacked by rows in

@@ -1,0 +1,57 @@
+"""Fake-quantised linears below the sizes of the 256 x 256-tile kernels: the three products of ``ttamd_gemm_mid_bf16`` through
+``FakeQuantizedLinear``, against fp32 matmuls of the same fake-quantised operands."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from torchtune_amd import ops
+from torchtune_amd.qat import FakeQuantizeConfig, FakeQuantizedLinear
+
+pytestmark = pytest.mark.gpu
+
+
+def _close(got, want, length):
+    # fp32 sums of exact products in some order (length * 2^-24 of the sum of magnitudes; random signs: its root), one bf16 rounding
+    slack = 2.0 ** -8 * want.abs() + length ** 0.5 * 2.0 ** -23 * want.abs().max()
+    assert bool(((got.double() - want).abs() <= slack).all())
+
+
+# one k step and fewer (tokens are the contraction of the weight gradient), tile edges, widths of half a tile, split contractions
+@pytest.mark.parametrize("M,N,K,bias", [(1, 256, 64, True), (31, 320, 128, False), (33, 256, 320, True), (128, 256, 256, False),
+                                        (129, 448, 4096, True), (257, 4096, 192, False), (1000, 512, 2048, False), (700, 2048, 1088, True)])
+def test_linear_and_gradients(M, N, K, bias):
+    torch.manual_seed(M + N + K)
+    layer = FakeQuantizedLinear(K, N, bias, FakeQuantizeConfig(torch.int8, "per_token", is_symmetric=False),
+                                FakeQuantizeConfig(torch.int4, group_size=32), device="cuda", dtype=torch.bfloat16)
+    x = torch.randn(1, M, K, device="cuda").bfloat16().requires_grad_()
+    gy = torch.randn(1, M, N, device="cuda").bfloat16()
+    assert layer._mid_ok(x)
+    y = layer(x)
+    y.backward(gy)
+    xq = ops.fq_per_token_int8_asym(x.detach())[0].double().view(M, K)
+    wq, scale = ops.fq_per_group_int4_sym(layer.weight.detach(), 32)
+    assert torch.equal(layer.weight_fake_quantizer.scale, scale)
+    wq, g2 = wq.double(), gy.double().view(M, N)
+    _close(y.view(M, N), xq @ wq.t() + (layer.bias.double() if bias else 0), K)
+    _close(x.grad.view(M, K), g2 @ wq, N)
+    _close(layer.weight.grad, g2.t() @ xq, M)
+    if bias:
+        assert torch.equal(layer.bias.grad, gy.view(M, N).sum(0))
+    with torch.no_grad():
+        assert torch.equal(layer(x), y)
+
+
+def test_second_derivative():
+    torch.manual_seed(0)
+    layer = FakeQuantizedLinear(128, 256, False, None, FakeQuantizeConfig(torch.int4, group_size=32), device="cuda", dtype=torch.bfloat16)
+    x = torch.randn(16, 128, device="cuda").bfloat16().requires_grad_()
+    assert layer._mid_ok(x)
+    gx, = torch.autograd.grad(layer(x).square().sum(), x, create_graph=True)
+    gx.float().square().sum().backward()
+    wq = ops.fq_per_group_int4_sym(layer.weight.detach(), 32)[0].float().requires_grad_()
+    xr = x.detach().float().requires_grad_()
+    gr, = torch.autograd.grad(F.linear(xr, wq).square().sum(), xr, create_graph=True)
+    gr.square().sum().backward()
+    # bf16 intermediates: a few roundings of 2^-8 each
+    for got, want in ((x.grad, xr.grad), (layer.weight.grad, wq.grad)):
+        assert float((got.float() - want).norm() / want.norm()) < 4 * 2.0 ** -8

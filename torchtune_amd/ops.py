@@ -11,7 +11,7 @@ from typing import List, Optional, Sequence, Tuple
 
 import torch
 
-from . import _lib
+from . import _host, _lib
 
 _DTYPE_CODE = {torch.bfloat16: _lib.TTAMD_BF16, torch.float32: _lib.TTAMD_F32}
 
@@ -769,6 +769,9 @@ def fq_per_token_int8_asym(x: torch.Tensor, want_qparams: bool = True, qparam_dt
     ``qparam_dtype=torch.bfloat16`` rounds the scale to bf16 before it quantises and dequantises.
     ``eps``: lower bound of the scale (None = ``finfo(float32).eps``, the convention the oracle documents)."""
     _need_gpu(x, "fq_per_token_int8_asym")
+    if _fq_timer is None:
+        _code(qparam_dtype, "fq_per_token_int8_asym (qparams)")
+        return _host.load().fq_per_token(x, want_qparams, qparam_dtype == torch.bfloat16, eps)
     code = _code(x.dtype, "fq_per_token_int8_asym")
     qcode = _code(qparam_dtype, "fq_per_token_int8_asym (qparams)")
     xc = x.contiguous()
@@ -796,6 +799,9 @@ def fq_per_group_int4_sym(w: torch.Tensor, group_size: int, want_scale: bool = T
     ``qparam_dtype=torch.bfloat16`` rounds the scales to bf16 before they quantise and dequantise.
     ``eps``: lower bound of the scale (None = ``finfo(float32).eps``)."""
     _need_gpu(w, "fq_per_group_int4_sym")
+    if _fq_timer is None:
+        _code(qparam_dtype, "fq_per_group_int4_sym (qparams)")
+        return _host.load().fq_per_group(w, group_size, want_scale, qparam_dtype == torch.bfloat16, eps)
     code = _code(w.dtype, "fq_per_group_int4_sym")
     qcode = _code(qparam_dtype, "fq_per_group_int4_sym (qparams)")
     wc = w.contiguous()

@@ -139,19 +139,6 @@ class FakeQuantizeConfig:
         )
 
 
-class _StraightThrough(torch.autograd.Function):
-    """y = fake_quantise(x); dy/dx = 1.  The reference masks the gradient with (qmin <= q <= qmax) evaluated on the
-    already clamped q, which is identically true."""
-
-    @staticmethod
-    def forward(ctx, x, fq):
-        return fq
-
-    @staticmethod
-    def backward(ctx, g):
-        return g, None
-
-
 class FakeQuantizer(nn.Module):
     """Fake-quantise the input according to ``config``.  ``enabled = False`` makes it the identity."""
 
@@ -218,27 +205,29 @@ class FakeQuantizer(nn.Module):
         if hit is not None and hit[0] is _ref:
             FakeQuantizer._last.entry = None
 
+    def values(self, x: torch.Tensor) -> torch.Tensor:
+        """The fake-quantised values of ``x``, outside autograd; records the quantisation parameters."""
+        c = self.config
+        if isinstance(c.granularity, PerToken):
+            fq, scale, zp = self._per_token(x)
+        else:
+            gs = c.group_size
+            if x.shape[-1] % gs != 0:
+                raise ValueError(f"last dimension ({x.shape[-1]}) must be divisible by group_size ({gs})")
+            if self._weight_only_int4(c):
+                fq, scale, zp = ops.fq_per_group_uint4_asym(x.detach(), gs, c.scale_precision, min_scale=c.eps)
+            else:
+                (fq, scale), zp = ops.fq_per_group_int4_sym(x.detach(), gs, qparam_dtype=c.scale_precision, eps=c.eps), None
+        self.scale = scale.to(c.scale_precision)
+        self.zero_point = None if zp is None else zp.to(c.zero_point_precision)
+        return fq
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        """``fq(x)`` with the gradient of ``x``: the reference masks it with (qmin <= q <= qmax) evaluated on the already
+        clamped q, which is identically true."""
         if not self.enabled:
             return x
-        with torch.no_grad():
-            if isinstance(self.config.granularity, PerToken):
-                fq, scale, zp = self._per_token(x)
-                self.scale = scale.to(self.config.scale_precision)
-                self.zero_point = zp.to(self.config.zero_point_precision)
-            else:
-                gs = self.config.group_size
-                if x.shape[-1] % gs != 0:
-                    raise ValueError(f"last dimension ({x.shape[-1]}) must be divisible by group_size ({gs})")
-                if self._weight_only_int4(self.config):
-                    fq, scale, zp = ops.fq_per_group_uint4_asym(x.detach(), gs, self.config.scale_precision, min_scale=self.config.eps)
-                    self.scale = scale.to(self.config.scale_precision)
-                    self.zero_point = zp.to(self.config.zero_point_precision)
-                else:
-                    fq, scale = ops.fq_per_group_int4_sym(x.detach(), gs, qparam_dtype=self.config.scale_precision, eps=self.config.eps)
-                    self.scale = scale.to(self.config.scale_precision)
-                    self.zero_point = None
-        return _StraightThrough.apply(x, fq.view(x.shape))
+        return _host.load().straight_through(x, self.values(x))
 
     def __repr__(self) -> str:
         return f"FakeQuantizer({self.config})"
@@ -254,6 +243,11 @@ TILED_GEMM = True
 TILED_GEMM_MIN_ROWS = 2048
 TILED_GEMM_MIN_TILES = 256
 TN_GEMM_MIN_TILES = 192
+# Most products (rows * N * K) of a linear whose matmuls run on ``ttamd_gemm_mid_bf16``.  Up to here the two libraries are
+# level on the GPU (three products at 200 tokens of 14336 x 4096: 164 us, vendor library 199; 500 tokens of 8192 x 2048: 85
+# and 96; 1000 tokens: 142 and 132), while a vendor call takes 31 us of host time, of ours 5; above it the vendor's larger
+# tiles win (500 tokens of 4096 x 14336: 287 and 255; 1000: 481 and 384).
+MID_GEMM_MAX = 1 << 34
 # the weight gradients of a group's members (they share fq(x)) as one launch; False: one launch per member (A/B timing)
 TN_GROUP_GEMM = True
 
@@ -497,11 +491,25 @@ class FakeQuantizedLinear(nn.Linear):
         return (x.shape[-1] == self.in_features and rows >= TILED_GEMM_MIN_ROWS and full_round
                 and ops.tiled_weight_shape_ok(self.out_features, self.in_features, c.group_size))
 
+    def _mid_ok(self, x: torch.Tensor) -> bool:
+        """The products run on the library's 128 x 128-tile kernels (``ttamd_gemm_mid_bf16``) instead of the vendor library:
+        the sizes below ``_tiled_ok``'s where they take about as long on the GPU and the vendor calls' host time counts."""
+        q, w, b = self.weight_fake_quantizer, self.weight, self.bias
+        if not TILED_GEMM or q is None or not q.enabled or not x.is_cuda or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not w.is_cuda:
+            return False
+        if type(x) is not torch.Tensor or type(w) is not nn.Parameter or (b is not None and (type(b) is not nn.Parameter or b.dtype != torch.bfloat16)):
+            return False
+        N, K = w.shape
+        return (0 < x.numel() * N <= MID_GEMM_MAX and N >= 256 and N % 64 == 0 and K % 64 == 0 and x.shape[-1] == K
+                and not torch.is_autocast_enabled("cuda"))
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self.activation_fake_quantizer is not None:
             x = self.activation_fake_quantizer(x)
         if self._tiled_ok(x):
             return _TiledFakeQuantLinearFn.apply(x, self.weight, self.bias, self.weight_fake_quantizer)
+        if self._mid_ok(x):
+            return _host.load().straight_through_linear(x, self.weight, self.weight_fake_quantizer.values(self.weight), self.bias)
         w = self.weight if self.weight_fake_quantizer is None else self.weight_fake_quantizer(self.weight)
         return F.linear(x, w, self.bias)
 
