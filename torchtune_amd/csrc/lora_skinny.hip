@@ -253,15 +253,16 @@ __global__ __launch_bounds__(256) void skinny_nt_kernel(const NtBatch a, int ran
 
 // The same products over short rows of few tokens (NtPlan says when).  What bounds skinny_nt_kernel there is its shape: 32-row
 // tiles with four waves leave a few workgroups for the whole contraction, so it is cut over workgroups and summed by a
-// second launch, and the rank tiles of a group run one after the other.  Here a workgroup owns 16 rows and 16 ranks and its
-// sixteen waves cut the contraction inside the workgroup: one launch, no partial sums in memory.  Rows beyond M are not
+// second launch, and the rank tiles of a group run one after the other.  Here a workgroup owns 16 rows and up to 16 ranks (the
+// MFMAs of fewer cost the same, but only the workgroup's own are loaded) and its sixteen waves cut the contraction inside
+// the workgroup: one launch, no partial sums in memory.  Rows beyond M are not
 // loaded.  MFMA, lane layout and the transposing read of BT as above.
 constexpr int kNtFewWaves = 16;
 
 template <bool BT>
-__global__ __launch_bounds__(64 * kNtFewWaves) void skinny_nt_few_kernel(const NtBatch a) {
+__global__ __launch_bounds__(64 * kNtFewWaves) void skinny_nt_few_kernel(const NtBatch a, int ranks) {
   const NtProblem& P = a.p[blockIdx.z];
-  const int r0 = 16 * (int)blockIdx.y;
+  const int r0 = ranks * (int)blockIdx.y;
   if (r0 >= P.R) return;  // the batch's grid is as wide as its widest problem
   __shared__ float red[kNtFewWaves - 1][4][64];
   constexpr int kPitchB = 32;  // 16 columns
@@ -271,13 +272,13 @@ __global__ __launch_bounds__(64 * kNtFewWaves) void skinny_nt_few_kernel(const N
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, i = lane & 15;
   const int m0 = (int)blockIdx.x * 16, r = r0 + i;
-  const bool row_in = m0 + i < M;
+  const bool row_in = m0 + i < M, rank_in = i < ranks && r < R;
   const uint16_t* xrow = P.X + (int64_t)(row_in ? m0 + i : 0) * Kc + 16 * g;
   const uint16_t* brow = nullptr;  // !BT: this lane's row of the stacked matrices, absent beyond R
   if constexpr (!BT) {
 #pragma unroll
     for (int b = 0; b < kMaxGroup; ++b)
-      if (b < P.nb && r >= P.r_off[b] && r < P.r_off[b + 1]) brow = P.bm[b] + (int64_t)(r - P.r_off[b]) * Kc + 16 * g;
+      if (rank_in && b < P.nb && r >= P.r_off[b] && r < P.r_off[b + 1]) brow = P.bm[b] + (int64_t)(r - P.r_off[b]) * Kc + 16 * g;
   }
   f32x4_t acc[2];
   acc[0] = acc[1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -340,7 +341,7 @@ __global__ __launch_bounds__(64 * kNtFewWaves) void skinny_nt_few_kernel(const N
     for (int v = 0; v < 4; ++v) red[wave - 1][v][lane] = acc[0][v];
   }
   __syncthreads();
-  if (wave > 0 || r >= R) return;
+  if (wave > 0 || !rank_in) return;
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
     const int row = m0 + 4 * g + v;
@@ -1063,6 +1064,10 @@ constexpr int kTargetWavesNt = 1024;  // column contractions (skinny_nt): few, l
 // form (gh) gains up to 3072 columns (333 tokens, whole adapter backward 15.8 -> 15.2).  The choice depends on M and Kc
 // alone, so that a member of a group sums in the order it sums in alone.
 constexpr int kNtFewTokens = 2048, kNtFewK = 2048, kNtFewKTransposed = 3072;
+// Few workgroups share the ranks more finely, each then streams less of lora_a: halved while the launch stays within this
+// many (K = 2048, us, 16 ranks -> the rule's: 1 token 4.1 -> 3.2, 16 tokens rank 48 6.0 -> 5.0, 700 tokens rank 16 6.0 -> 5.5; beyond
+// a workgroup per CU x costs more than that: 700 tokens rank 48 6.3 -> 8.4).  Same sums in the same order.
+constexpr int kNtFewWorkgroups = 192;
 // Dealing the 16-rank tiles to workgroups of their own reads x once per tile: pays while x is small (rank 48, us: 64 x 4096 8.9 ->
 // 6.1, 333 x 4096 9.1 -> 7.4, 64 x 14336 10.6 -> 7.9; but 333 x 14336 12.4 -> 13.6).  Same sums in the same order.
 constexpr int64_t kNtRankTilesElements = int64_t(1) << 21;
@@ -1129,11 +1134,13 @@ int run_nt_batch(NtBatch& b, int n, bool bt, float* ws, hipStream_t s) {
     if (pl.splits > 1 && (int64_t)b.M * P.R > max_mr) max_mr = (int64_t)b.M * P.R;
   }
   if (n_few > 0) {
-    const dim3 grid((unsigned)few_m_tiles, (unsigned)((few_r + 15) / 16), (unsigned)n_few), few_block(64 * kNtFewWaves);
+    int ranks = 16;  // of a workgroup
+    while (!bt && ranks > 1 && few_m_tiles * ((few_r + ranks / 2 - 1) / (ranks / 2)) * n_few <= kNtFewWorkgroups) ranks /= 2;
+    const dim3 grid((unsigned)few_m_tiles, (unsigned)((few_r + ranks - 1) / ranks), (unsigned)n_few), few_block(64 * kNtFewWaves);
     if (bt)
-      skinny_nt_few_kernel<true><<<grid, few_block, 0, s>>>(few);
+      skinny_nt_few_kernel<true><<<grid, few_block, 0, s>>>(few, ranks);
     else
-      skinny_nt_few_kernel<false><<<grid, few_block, 0, s>>>(few);
+      skinny_nt_few_kernel<false><<<grid, few_block, 0, s>>>(few, ranks);
   }
   if (n_tiled > 0) {
     if (!bt && tiled_elements <= kNtRankTilesElements) {
