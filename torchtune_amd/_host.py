@@ -7,6 +7,8 @@ import importlib.util
 import threading
 from pathlib import Path
 
+import torch
+
 from . import _lib
 
 MODULE_NAME = "torchtune_amd_host"
@@ -30,3 +32,34 @@ def load():
                 spec.loader.exec_module(module)
                 _module = module
     return _module
+
+
+class _TracedCall(torch.autograd.Function):
+    """A host call as one node of a ``torch.jit.trace``, which records Python nodes but not native ones.  Backward: the call
+    again, differentiated."""
+
+    @staticmethod
+    def forward(ctx, name: str, *args):
+        ctx.name, ctx.rest = name, [None if isinstance(a, torch.Tensor) else (a,) for a in args]
+        ctx.save_for_backward(*(a for a in args if isinstance(a, torch.Tensor)))
+        return getattr(load(), name)(*args)
+
+    @staticmethod
+    def backward(ctx, *grads):
+        saved = iter(ctx.saved_tensors)
+        with torch.enable_grad():
+            args = [next(saved).detach().requires_grad_(need) if a is None else a[0]
+                    for a, need in zip(ctx.rest, ctx.needs_input_grad[1:])]
+            outs = getattr(load(), ctx.name)(*args)
+            need = [a for a, n in zip(args, ctx.needs_input_grad[1:]) if n]
+            got = iter(torch.autograd.grad(outs, need, grads if isinstance(outs, tuple) else grads[0], allow_unused=True))
+        return (None, *(next(got) if n else None for n in ctx.needs_input_grad[1:]))
+
+
+def tracing() -> bool:
+    return torch._C._get_tracing_state() is not None
+
+
+def call(name: str, *args):
+    """The host function ``name``; under ``torch.jit.trace`` as a node the trace can hold."""
+    return _TracedCall.apply(name, *args) if tracing() else getattr(load(), name)(*args)

@@ -49,11 +49,30 @@ Tensor scratch(size_t bytes, const Tensor& like) {
 
 size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
 
+// True when the call has to be a node: something is differentiated backward, or carries a forward-mode tangent (the node
+// then raises: none of them has a forward-mode rule, and a plain call would drop the tangent).
 bool wants_grad(std::initializer_list<const Tensor*> ts) {
-  if (!at::GradMode::is_enabled()) return false;
+  const bool grad = at::GradMode::is_enabled();
   for (const Tensor* t : ts)
-    if (t->defined() && t->requires_grad()) return true;
+    if (t->defined() && ((grad && t->requires_grad()) || t->_fw_grad(0).defined())) return true;
   return false;
+}
+
+// A tensor the kernels may read in place of torch's own ops: no forward-mode tangent, no function transform's wrapper, no
+// subclass with a dispatch of its own.
+bool ordinary(const Tensor& t) {
+  constexpr c10::DispatchKeySet wrapped({c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                         c10::DispatchKey::Functionalize, c10::DispatchKey::Python});
+  return !t.key_set().has_any(wrapped) && !t._fw_grad(0).defined();
+}
+
+// The kernels that took over from torch's matmul read 16 bytes at a time; a contiguous view may begin anywhere.
+Tensor aligned(const Tensor& t) { return !t.defined() || (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15u) == 0 ? t : t.clone(); }
+
+int64_t last_dim(const Tensor& t, const char* what) {
+  const int64_t n = t.size(-1);
+  TORCH_CHECK_VALUE(n > 0, what, ": the last dimension is empty");
+  return n;
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -66,7 +85,7 @@ struct NormOut {
 NormOut norm_forward(const Tensor& x, const Tensor* residual, const Tensor& scale, double eps) {
   const Tensor xc = bf16(x, "rms_norm_fwd: x"), sc = bf16(scale, "rms_norm_fwd: scale");
   const c10::DeviceGuard guard(xc.device());
-  const int64_t D = xc.size(-1), rows = xc.numel() / D;
+  const int64_t D = last_dim(xc, "rms_norm_fwd"), rows = xc.numel() / D;
   TORCH_CHECK_VALUE(sc.numel() == D, "rms_norm_fwd: scale has ", sc.numel(), " elements, the rows ", D);
   NormOut o;
   o.y = at::empty_like(xc);
@@ -90,7 +109,7 @@ std::pair<Tensor, Tensor> norm_backward(const Tensor& gy, const Tensor& x, const
                                         const Tensor& g_add) {
   const Tensor gc = bf16(gy, "rms_norm_bwd: gy"), xc = bf16(x, "rms_norm_bwd: x"), sc = bf16(scale, "rms_norm_bwd: scale");
   const c10::DeviceGuard guard(xc.device());
-  const int64_t D = xc.size(-1), rows = xc.numel() / D;
+  const int64_t D = last_dim(xc, "rms_norm_bwd"), rows = xc.numel() / D;
   const Tensor ga = g_add.defined() ? bf16(g_add, "rms_norm_bwd: g_add") : Tensor();
   TORCH_CHECK_VALUE(gc.numel() == xc.numel() && (!ga.defined() || ga.numel() == xc.numel()), "rms_norm_bwd: gradients and x differ in size");
   Tensor gx = at::empty_like(xc), gscale, ws;
@@ -238,11 +257,11 @@ Tensor swiglu(const Tensor& gate, const Tensor& up) {
 // ---------------------------------------------------------------------------------------------------
 // LoRA linears over NF4 weights, fewer tokens than the expand-once path takes
 // ---------------------------------------------------------------------------------------------------
-// The frozen weight's tensors: codes, block scalers and, where a call may need them, the transposed copies.  They are
-// kept by the node as plain references (no saved variables: nothing to pack, nothing to check for writes, they are the
-// layer's own).
+// The frozen weight's tensors: codes, block scalers and, where a call may need them, the transposed copies, which the node
+// keeps as plain references.  The weight they belong to is a saved variable beside them, so that a write to it between
+// forward and backward is an error (the copies would no longer be its).
 struct Weight {
-  Tensor q, scal, q_t, scal_t;
+  Tensor whole, q, scal, q_t, scal_t;
   int64_t N = 0;
 };
 
@@ -331,7 +350,7 @@ struct QLoRALinearFn : torch::autograd::Function<QLoRALinearFn> {
     if (bias) m.bias = *bias;
     m.scale = scale;
     LinearOut o = linear_forward(x, m, true);
-    ctx->save_for_backward({o.x2, o.h, a, b});
+    ctx->save_for_backward({o.x2, o.h, a, b, w.whole});
     ctx->saved_data["w"] = pack_weight(w);
     ctx->saved_data["scale"] = scale;
     ctx->saved_data["shape"] = x.sizes().vec();
@@ -366,9 +385,10 @@ struct QLoRALinearFn : torch::autograd::Function<QLoRALinearFn> {
   }
 };
 
-Tensor qlora_linear(const Tensor& x, const Tensor& q, const Tensor& scal, const std::optional<Tensor>& q_t, const std::optional<Tensor>& scal_t,
+Tensor qlora_linear(const Tensor& x, const Tensor& weight, const Tensor& q, const Tensor& scal, const std::optional<Tensor>& q_t, const std::optional<Tensor>& scal_t,
                     int64_t N, const Tensor& a, const Tensor& b, double scale, const std::optional<Tensor>& bias) {
   Member m;
+  m.w.whole = weight;
   m.w.q = q;
   m.w.scal = scal;
   if (q_t) m.w.q_t = *q_t;
@@ -467,6 +487,7 @@ struct QLoRAGroupFn : torch::autograd::Function<QLoRAGroupFn> {
       save.push_back(o.ys[0]);
       save.push_back(o.ys[1]);
     }
+    for (const Member& m : spec.ms) save.push_back(m.w.whole);
     ctx->save_for_backward(std::move(save));
     ctx->saved_data["w"] = weights;
     ctx->saved_data["N"] = n_out;
@@ -551,8 +572,8 @@ struct QLoRAGroupFn : torch::autograd::Function<QLoRAGroupFn> {
   }
 };
 
-// members: (q, scal, q_t | None, scal_t | None, N, lora_a, lora_b, scale, bias | None) each
-using MemberTuple = std::tuple<Tensor, Tensor, std::optional<Tensor>, std::optional<Tensor>, int64_t, Tensor, Tensor, double, std::optional<Tensor>>;
+// members: (weight, q, scal, q_t | None, scal_t | None, N, lora_a, lora_b, scale, bias | None) each
+using MemberTuple = std::tuple<Tensor, Tensor, Tensor, std::optional<Tensor>, std::optional<Tensor>, int64_t, Tensor, Tensor, double, std::optional<Tensor>>;
 
 std::vector<Tensor> lora_group(const Tensor& x, const std::vector<MemberTuple>& members, bool gated) {
   GroupSpec spec;
@@ -561,15 +582,16 @@ std::vector<Tensor> lora_group(const Tensor& x, const std::vector<MemberTuple>& 
   bool grad = wants_grad({&x});
   for (const auto& t : members) {
     Member m;
-    m.w.q = std::get<0>(t);
-    m.w.scal = std::get<1>(t);
-    if (std::get<2>(t)) m.w.q_t = *std::get<2>(t);
-    if (std::get<3>(t)) m.w.scal_t = *std::get<3>(t);
-    m.w.N = std::get<4>(t);
-    m.a = std::get<5>(t);
-    m.b = std::get<6>(t);
-    m.scale = std::get<7>(t);
-    if (std::get<8>(t)) m.bias = *std::get<8>(t);
+    m.w.whole = std::get<0>(t);
+    m.w.q = std::get<1>(t);
+    m.w.scal = std::get<2>(t);
+    if (std::get<3>(t)) m.w.q_t = *std::get<3>(t);
+    if (std::get<4>(t)) m.w.scal_t = *std::get<4>(t);
+    m.w.N = std::get<5>(t);
+    m.a = std::get<6>(t);
+    m.b = std::get<7>(t);
+    m.scale = std::get<8>(t);
+    if (std::get<9>(t)) m.bias = *std::get<9>(t);
     grad = grad || wants_grad({&m.a, &m.b, &m.bias});
     adapters.push_back(m.a);
     adapters.push_back(m.b);
@@ -594,20 +616,21 @@ int dtype_code(at::ScalarType t, const char* what) {
 Tensor int8_dynamic_linear(const Tensor& x, const Tensor& q, const Tensor& scale, const Tensor& zeros, int64_t group_size,
                            const std::optional<Tensor>& bias) {
   const int64_t N = q.size(0), K = q.size(1);
-  const Tensor x2 = bf16(x, "int8_group_linear").view({-1, K});
+  const Tensor x2 = aligned(bf16(x, "int8_group_linear").view({-1, K}));
   const int64_t M = x2.size(0);
   const int code = dtype_code(scale.scalar_type(), "int8_group_linear: scale");
   TORCH_CHECK_VALUE(q.scalar_type() == at::kChar && q.is_contiguous() && q.device() == x.device() && scale.is_contiguous() &&
-                        zeros.is_contiguous() && scale.numel() * group_size == N * K && zeros.numel() == scale.numel() &&
+                        scale.device() == x.device() && zeros.device() == x.device() && zeros.is_contiguous() && scale.numel() * group_size == N * K && zeros.numel() == scale.numel() &&
                         zeros.scalar_type() == scale.scalar_type(),
-                    "int8_group_linear: q must be int8 on x's device, scale and zeros of one dtype with N * K / group_size elements");
-  const Tensor b = bias ? bf16(*bias, "int8_group_linear") : Tensor();
-  TORCH_CHECK_VALUE(!b.defined() || b.numel() == N, "int8_group_linear: bias must have ", N, " elements");
+                    "int8_group_linear: q must be int8, scale and zeros of one dtype, all on x's device, with N * K / group_size elements");
+  const Tensor b = bias ? aligned(bf16(*bias, "int8_group_linear")) : Tensor();
+  TORCH_CHECK_VALUE(!b.defined() || (b.numel() == N && b.device() == x.device()), "int8_group_linear: bias must have ", N, " elements on x's device");
+  const Tensor qa = aligned(q), sa = aligned(scale), za = aligned(zeros);
   const c10::DeviceGuard guard(x.device());
   Tensor y = at::empty(with_last(x, N), x2.options());
   const size_t bytes = ttamd_int8_dynamic_linear_workspace_bytes(M, N, K);
   const Tensor ws = bytes ? scratch(bytes, x2) : Tensor();
-  check(ttamd_int8_dynamic_linear_bf16(x2.data_ptr(), (const int8_t*)q.data_ptr(), scale.data_ptr(), zeros.data_ptr(), code, (int)group_size,
+  check(ttamd_int8_dynamic_linear_bf16(x2.data_ptr(), (const int8_t*)qa.data_ptr(), sa.data_ptr(), za.data_ptr(), code, (int)group_size,
                                        opt_ptr(b), y.data_ptr(), M, N, K, opt_ptr(ws), bytes, stream_of(x)),
         "int8_dynamic_linear");
   return y;
@@ -615,18 +638,19 @@ Tensor int8_dynamic_linear(const Tensor& x, const Tensor& q, const Tensor& scale
 
 Tensor uint4_group_linear(const Tensor& x, const Tensor& q, const Tensor& sz, int64_t group_size, const std::optional<Tensor>& bias) {
   const int64_t N = q.size(0), K = q.size(1) * 2;
-  const Tensor x2 = bf16(x, "uint4_group_linear").view({-1, K});
+  const Tensor x2 = aligned(bf16(x, "uint4_group_linear").view({-1, K}));
   const int64_t M = x2.size(0);
   TORCH_CHECK_VALUE(q.scalar_type() == at::kByte && q.is_contiguous() && q.device() == x.device() && sz.scalar_type() == at::kBFloat16 &&
-                        sz.is_contiguous() && sz.dim() == 3 && sz.size(0) * group_size == K && sz.size(1) == N && sz.size(2) == 2,
-                    "uint4_group_linear: q must be uint8 on x's device and scales_and_zeros [K / group_size, N, 2] bf16");
-  const Tensor b = bias ? bf16(*bias, "uint4_group_linear") : Tensor();
-  TORCH_CHECK_VALUE(!b.defined() || b.numel() == N, "uint4_group_linear: bias must have ", N, " elements");
+                        sz.is_contiguous() && sz.device() == x.device() && sz.dim() == 3 && sz.size(0) * group_size == K && sz.size(1) == N && sz.size(2) == 2,
+                    "uint4_group_linear: q must be uint8 and scales_and_zeros [K / group_size, N, 2] bf16, both on x's device");
+  const Tensor b = bias ? aligned(bf16(*bias, "uint4_group_linear")) : Tensor();
+  TORCH_CHECK_VALUE(!b.defined() || (b.numel() == N && b.device() == x.device()), "uint4_group_linear: bias must have ", N, " elements on x's device");
+  const Tensor qa = aligned(q), sa = aligned(sz);
   const c10::DeviceGuard guard(x.device());
   Tensor y = at::empty(with_last(x, N), x2.options());
   const size_t bytes = ttamd_int4_linear_workspace_bytes(M, N, K);
   const Tensor ws = bytes ? scratch(bytes, x2) : Tensor();
-  check(ttamd_uint4_group_linear_bf16(x2.data_ptr(), (const uint8_t*)q.data_ptr(), sz.data_ptr(), (int)group_size, opt_ptr(b), y.data_ptr(),
+  check(ttamd_uint4_group_linear_bf16(x2.data_ptr(), (const uint8_t*)qa.data_ptr(), sa.data_ptr(), (int)group_size, opt_ptr(b), y.data_ptr(),
                                       M, N, K, opt_ptr(ws), bytes, stream_of(x)),
         "uint4_group_linear");
   return y;
@@ -646,7 +670,7 @@ std::tuple<Tensor, MaybeTensor, MaybeTensor> fq_per_token(const Tensor& x, bool 
   need_gpu(x, "fq_per_token_int8_asym");
   const int code = dtype_code(x.scalar_type(), "fq_per_token_int8_asym");
   const Tensor xc = x.detach().contiguous();
-  const int64_t K = xc.size(-1), rows = xc.numel() / K;
+  const int64_t K = last_dim(xc, "fq_per_token_int8_asym"), rows = xc.numel() / K;
   const c10::DeviceGuard guard(x.device());
   Tensor out = at::empty_like(xc);
   MaybeTensor scale, zp;
@@ -666,7 +690,7 @@ std::pair<Tensor, MaybeTensor> fq_per_group(const Tensor& w, int64_t group_size,
   need_gpu(w, "fq_per_group_int4_sym");
   const int code = dtype_code(w.scalar_type(), "fq_per_group_int4_sym");
   const Tensor wc = w.detach().contiguous();
-  const int64_t K = wc.size(-1), rows = wc.numel() / K;
+  const int64_t K = last_dim(wc, "fq_per_group_int4_sym"), rows = wc.numel() / K;
   const c10::DeviceGuard guard(w.device());
   Tensor out = at::empty_like(wc);
   MaybeTensor scale;
@@ -690,7 +714,8 @@ Tensor straight_through(const Tensor& x, const Tensor& value) {
 }
 
 // c = a . b^T (+ bias), a . b or a^T . b (kinds 0, 1, 2 of ttamd_gemm_mid_bf16) of contiguous matrices
-Tensor gemm_mid(int kind, const Tensor& a, const Tensor& b, const Tensor& bias) {
+Tensor gemm_mid(int kind, const Tensor& a_in, const Tensor& b_in, const Tensor& bias_in) {
+  const Tensor a = aligned(a_in), b = aligned(b_in), bias = aligned(bias_in);
   const int64_t M = kind == 2 ? a.size(1) : a.size(0), K = kind == 2 ? a.size(0) : a.size(1), N = kind == 0 ? b.size(0) : b.size(1);
   TORCH_CHECK_VALUE((kind == 0 ? b.size(1) : b.size(0)) == K, "gemm_mid: ", a.sizes(), " and ", b.sizes(), " do not fit");
   const c10::DeviceGuard guard(a.device());
@@ -704,33 +729,41 @@ Tensor gemm_mid(int kind, const Tensor& a, const Tensor& b, const Tensor& bias) 
 Tensor ste_linear_forward(const Tensor& x, const Tensor& wq, const MaybeTensor& bias) {
   const Tensor x2 = bf16(x, "straight_through_linear").view({-1, x.size(-1)});
   const Tensor b = bias ? bf16(*bias, "straight_through_linear") : Tensor();
-  TORCH_CHECK_VALUE(!b.defined() || b.numel() == wq.size(0), "straight_through_linear: bias must have ", wq.size(0), " elements");
+  TORCH_CHECK_VALUE(!b.defined() || (b.numel() == wq.size(0) && b.device() == x.device()), "straight_through_linear: bias must have ", wq.size(0),
+                    " elements on x's device");
   return gemm_mid(0, x2, wq, b).view(with_last(x, wq.size(0)));
 }
 
 // F.linear(x, wq, bias) with the gradient of wq handed to weight
 struct StraightThroughLinearFn : torch::autograd::Function<StraightThroughLinearFn> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight, const Tensor& wq, const MaybeTensor& bias) {
-    ctx->save_for_backward({x, weight, wq});
+    // as F.linear does: each operand for the other's gradient only.  The weight itself (a leaf) is no operand: it may be
+    // stepped before the backward, and serves a second differentiation alone.
+    ctx->save_for_backward({weight.requires_grad() ? x : Tensor(), x.requires_grad() ? wq : Tensor()});
+    ctx->saved_data["weight"] = weight;
+    ctx->saved_data["shape"] = x.sizes().vec();
     ctx->saved_data["bias"] = bias.has_value();
     return ste_linear_forward(x, wq, bias);
   }
   static variable_list backward(AutogradContext* ctx, variable_list g) {
     const auto saved = ctx->get_saved_variables();
-    const Tensor &x = saved[0], &weight = saved[1];
+    const Tensor& x = saved[0];
+    const std::vector<int64_t> shape = ctx->saved_data["shape"].toIntVector();
     const bool need_b = ctx->saved_data["bias"].toBool() && ctx->needs_input_grad(3);
-    Tensor wq = saved[2], gx, gw, gb;
+    Tensor wq = saved[1], gx, gw, gb;
     if (at::GradMode::is_enabled()) {  // a second differentiation: products that autograd can follow
-      wq = wq + (weight - weight.detach());
       const Tensor gy = g[0].reshape({-1, g[0].size(-1)});
-      if (ctx->needs_input_grad(0)) gx = gy.matmul(wq).view(x.sizes());
-      if (ctx->needs_input_grad(1)) gw = gy.t().matmul(x.reshape({-1, x.size(-1)}));
+      if (ctx->needs_input_grad(0)) {
+        const Tensor weight = ctx->saved_data["weight"].toTensor();
+        gx = gy.matmul(wq + (weight - weight.detach())).view(shape);
+      }
+      if (ctx->needs_input_grad(1)) gw = gy.t().matmul(x.reshape({-1, shape.back()}));
       if (need_b) gb = gy.sum(0);
       return {gx, gw, Tensor(), gb};
     }
     const Tensor gy = bf16(g[0], "straight_through_linear_bwd").view({-1, g[0].size(-1)});
-    if (ctx->needs_input_grad(0)) gx = gemm_mid(1, gy, wq, Tensor()).view(x.sizes());
-    if (ctx->needs_input_grad(1)) gw = gemm_mid(2, gy, x.contiguous().view({-1, x.size(-1)}), Tensor());
+    if (ctx->needs_input_grad(0)) gx = gemm_mid(1, gy, wq, Tensor()).view(shape);
+    if (ctx->needs_input_grad(1)) gw = gemm_mid(2, gy, x.contiguous().view({-1, shape.back()}), Tensor());
     if (need_b) gb = gy.sum(0);
     return {gx, gw, Tensor(), gb};
   }
@@ -748,6 +781,7 @@ Tensor straight_through_linear(const Tensor& x, const Tensor& weight, const Tens
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("ordinary", &ordinary);
   m.def("rms_norm", &rms_norm);
   m.def("add_rms_norm", &add_rms_norm);
   m.def("qkv_rope_repeat", &qkv_rope_repeat);

@@ -16,13 +16,13 @@ from .. import _host, ops
 
 def rms_norm(x: torch.Tensor, scale: torch.Tensor, eps: float) -> torch.Tensor:
     """``bf16(x * rsqrt(mean(x^2) + eps)) * scale`` over the last dimension, computed in fp32."""
-    return _host.load().rms_norm(x, scale, eps)
+    return _host.call("rms_norm", x, scale, eps)
 
 
 def add_rms_norm(x: torch.Tensor, residual: torch.Tensor, norm: "RMSNorm"):
     """``h = x + residual; return h, norm(h)``: the residual stream's addition and the norm of the next sub-block
     (``torchtune/modules/transformer.py:129-141``) as one pass forward and one backward; same bits as the separate ops."""
-    return _host.load().add_rms_norm(x, residual, norm.scale, norm.eps)
+    return _host.call("add_rms_norm", x, residual, norm.scale, norm.eps)
 
 
 class RMSNorm(nn.Module):
@@ -64,7 +64,7 @@ def qkv_rope_repeat(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cache: to
     """What lies between the q / k / v projections and the attention (``torchtune/modules/attention.py:255-290``) as one
     kernel per direction: ``apply_rope(q)``, ``repeat_kv(apply_rope(k), rep)``, ``repeat_kv(v, rep)`` with
     ``rep = n_h // n_kv``, bit for bit."""
-    return _host.load().qkv_rope_repeat(q, k, v, cache)
+    return _host.call("qkv_rope_repeat", q, k, v, cache)
 
 
 class _RepeatKVFn(torch.autograd.Function):
@@ -87,7 +87,7 @@ def repeat_kv(x: torch.Tensor, rep: int) -> torch.Tensor:
 
 def swiglu(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     """``silu(gate) * up`` with the eager sequence's two bf16 roundings."""
-    return _host.load().swiglu(gate, up)
+    return _host.call("swiglu", gate, up)
 
 
 class _CrossEntropySumFn(torch.autograd.Function):

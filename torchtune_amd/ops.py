@@ -192,8 +192,8 @@ NATIVE_MAX_TOKENS = 1280
 
 def native_call(tokens: int) -> bool:
     """True when a fused LoRA call over ``tokens`` rows runs on the native host path (never while a GEMM timer is
-    installed: it brackets the stages of the Python path)."""
-    return 0 < tokens < NATIVE_MAX_TOKENS and _gemm_timer is None
+    installed: it brackets the stages of the Python path, nor under ``torch.jit.trace``, which records Python nodes only)."""
+    return not _host.tracing() and 0 < tokens < NATIVE_MAX_TOKENS and _gemm_timer is None
 
 
 def fused_shape_ok(N: int, K: int, rank: int) -> bool:

@@ -497,11 +497,12 @@ class FakeQuantizedLinear(nn.Linear):
         q, w, b = self.weight_fake_quantizer, self.weight, self.bias
         if not TILED_GEMM or q is None or not q.enabled or not x.is_cuda or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not w.is_cuda:
             return False
+        if torch.is_autocast_enabled("cuda") or not _host.load().ordinary(x):
+            return False
         if type(x) is not torch.Tensor or type(w) is not nn.Parameter or (b is not None and (type(b) is not nn.Parameter or b.dtype != torch.bfloat16)):
             return False
         N, K = w.shape
-        return (0 < x.numel() * N <= MID_GEMM_MAX and N >= 256 and N % 64 == 0 and K % 64 == 0 and x.shape[-1] == K
-                and not torch.is_autocast_enabled("cuda"))
+        return (0 < x.numel() * N <= MID_GEMM_MAX and N * K < 1 << 30 and N >= 256 and N % 64 == 0 and K % 64 == 0 and x.shape[-1] == K)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self.activation_fake_quantizer is not None:
@@ -579,7 +580,11 @@ def _int4_kernels_apply(x: torch.Tensor, weight: torch.Tensor, in_features: int,
                         bias: Optional[torch.Tensor], qparams_ok: bool) -> bool:
     """True when a converted linear's forward runs on the kernels that stream its integer weight (a few hundred tokens at
     most); otherwise the dense weight is rebuilt and multiplied."""
-    if not (qparams_ok and precision == torch.bfloat16 and x.is_cuda and weight.is_cuda and x.shape[-1] == in_features and x.numel() > 0):
+    if not (qparams_ok and precision == torch.bfloat16 and x.is_cuda and weight.is_cuda):
+        return False
+    if torch.is_autocast_enabled("cuda") or not _host.load().ordinary(x):
+        return False
+    if x.shape[-1] != in_features or x.numel() == 0:
         return False
     if bias is not None and (bias.dtype != torch.bfloat16 or not bias.is_cuda or (bias.requires_grad and torch.is_grad_enabled())):
         return False
