@@ -512,3 +512,35 @@ def test_few_token_pair_and_members(M, N, K, ranks):
             assert torch.equal(y[:1], ops.nf4_lora_linear_fwd(x[:1], m.qdata, m.block_scalers, N, h[:1].contiguous(), m.lora_b, m.scale))
         off += r
     assert torch.equal(act, ops.swiglu_fwd(gate, up))
+
+
+@pytest.mark.parametrize("M", [65, 128, 129, 300])
+@pytest.mark.parametrize("steps", [1, 2, 3, 5, 7])
+def test_eight_wave_tiles_at_short_and_odd_contractions(M, steps):
+    """128-row tiles whose contraction is halved between two wave groups: one group without a k-step, one more step in the
+    first, segments that end inside a half; rows and columns that do not fill a tile.  Too short to be sliced.  bf16 results
+    of fp32 sums: one rounding, 2^-9 of the value, beside the sums' order (1e-5 of the largest)."""
+    kc, width, rank = 64 * steps, 768, 8
+    g = torch.Generator(device=DEV).manual_seed(M + steps)
+
+    def close(got, want):
+        torch.testing.assert_close(got.float(), want, rtol=2 ** -8, atol=2e-5 * want.abs().max().item())
+
+    ((m, t, *_),) = _members(kc, (width,), (rank,), seed=steps)
+    x, h = (torch.randn(M, n, device=DEV, generator=g).to(BF) for n in (kc, rank))
+    y = ops.nf4_lora_linear_fwd(x, m.qdata, m.block_scalers, width, h, m.lora_b, 1.0, block_scalers_t=m.transposed[1])
+    close(y, x.float() @ t.get_original_weight().float().t() + h.float() @ m.lora_b.float().t())
+    ((m, t, *_),) = _members(width, (kc,), (rank,), seed=steps)
+    gx = ops.nf4_linear_bwd_dx(x, m.qdata, m.block_scalers, width, h, m.lora_a, transposed=m.transposed)
+    close(gx, x.float() @ t.get_original_weight().float() + h.float() @ m.lora_a.float())
+    mem = _members(width, (kc, 128, 64), (rank, 8, 16), seed=steps)
+    gys = [torch.randn(M, n, device=DEV, generator=g).to(BF) for n in (kc, 128, 64)]
+    xs = torch.randn(M, width, device=DEV, generator=g).to(BF)
+    h_cat = torch.randn(M, 32, device=DEV, generator=g).to(BF)
+    gx, _, gh = ops.lora_group_bwd(xs, h_cat, [e[0] for e in mem], gys)
+    want, off = 0, 0
+    for (m, t, *_), gy in zip(mem, gys):
+        r = m.lora_a.shape[0]
+        want = want + gy.float() @ t.get_original_weight().float() + gh[:, off:off + r].float() @ m.lora_a.float()
+        off += r
+    close(gx, want)

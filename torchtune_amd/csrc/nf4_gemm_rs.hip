@@ -8,10 +8,10 @@
 //   backward : Wv = W^T [K, N]  (a transposed copy of the codes), one scaler per contraction element per
 //              64 output columns (NF4 blocks run along K, i.e. along the output columns of this view)
 //
-// Work split.  256 threads = 4 waves; the workgroup owns a BM x 256 tile of C, wave w the 64 output columns
-// [64w, 64w+64) for ALL BM rows.  A lane of the MFMA weight operand needs 8 consecutive contraction elements
-// of one output column: exactly one dword of codes.  Each lane expands its own code dwords in registers
-// (byte -> pair of fp32 code points from a 256-entry LDS table, multiply by the scaler in fp32, round to bf16:
+// Work split.  4 waves, or two groups of 4 that halve the contraction between them; the workgroup owns a BM x 256 tile of
+// C, wave w of a group the 64 output columns [64w, 64w+64) for ALL BM rows.  A lane of the MFMA weight operand needs 8
+// consecutive contraction elements of one output column: exactly one dword of codes.  Each lane expands its own code dwords
+// in registers (byte -> pair of fp32 code points from a 256-entry LDS table, multiply by the scaler in fp32, round to bf16:
 // bit-identical to the stand-alone dequantise kernel) one k-substep ahead of the MFMA that consumes them.
 //
 // Every global read of the main loop is a direct-to-LDS load (global_load_lds_*): the activation tile with an
@@ -83,16 +83,18 @@ struct RsSegs {
 constexpr int kBN = 256;
 constexpr int kLutBytes = 256 * 8;  // 256 byte values x (fp32 nf4[hi nibble], fp32 nf4[lo nibble])
 
-// LDS: a ring of 4 activation tiles (shared by the waves), a ring of 3 wave-private {code bytes, scalers} slots, the table
-template <int BM>
+// LDS, per wave group: a ring of activation tiles (shared by the group's waves), a ring of 3 wave-private {code bytes, scalers}
+// slots; the table once
+template <int BM, bool SPLIT>
 struct RsLayout {
+  static constexpr int kGroups = BM == 128 && !SPLIT ? 2 : 1;  // wave groups, each with its own share of the contraction
   static constexpr int kStageA = BM * 128;   // activation tile: BM rows x 64 bf16
-  static constexpr int kAStages = 4;
+  static constexpr int kAStages = kGroups == 2 ? 3 : 4;
   static constexpr int kWOff = kAStages * kStageA;
   static constexpr int kStageW = 8192 + 2048;  // code bytes [wave][tile j][lane] x 16 B, then scalers [wave] x 512 B
   static constexpr int kWStages = 3;
-  static constexpr int kLutOff = kWOff + kWStages * kStageW;
-  static constexpr int kTotal = kLutOff;  // dynamic part; the table is a static LDS object of kLutBytes
+  static constexpr int kGroupBytes = kWOff + kWStages * kStageW;
+  static constexpr int kTotal = kGroups * kGroupBytes;  // dynamic part; the table is a static LDS object of kLutBytes
 };
 
 // MODE 0: one scaler per (output column, 64-wide k-step), scaler tensor laid out like the weight's blocks
@@ -102,14 +104,25 @@ struct RsLayout {
 // workgroup then leaves its tile as fp32 in g.part (slice 0 includes the adapter) and bias, column scale and the
 // rounding to bf16 happen in nf4_gemm_rs_reduce_kernel, which adds the slices in a fixed order.
 // SEG: segmented contraction (see RsSegs); only with MODE 1 and without SPLIT.
+// BM 128 without SPLIT: eight waves.  A wave's k-step is 300 instructions beside 1024 cycles of MFMA, and with one wave per
+// SIMD nothing covers the waits between them: a k-step took 2200 cycles, whatever the tile's rows (96: the same).  Two
+// waves per SIMD cover each other; a tile of 256 rows has no registers for that, one of 128 rows has.  The second four
+// waves take the second half of the workgroup's k-steps on rings of their own (three activation stages do when batch t + 2 is
+// issued after the barrier of step t), and the two halves of the sum meet in LDS, each group finishing half of the rows.
+// Measured (us, four waves -> eight): 4096 x 14336 at 2048 tokens 239 -> 209, at 1500 199 -> 180; 4096 x 4096 at 2048 75 -> 67;
+// 14336 x 4096 at 333 63 -> 53; 8192 x 2048 at 700 35.5 -> 33.  What bounds it then is LDS: the 128 table reads of a k-step
+// beside the operand reads.  A slice of a SPLIT launch is 13 - 45 k-steps long and the second ring's start and the
+// exchange cost what the loop gains (4096 x 4096 at 333 tokens in five slices 23 -> 24, 2048 x 2048 at 700 16.5 -> 19.4):
+// those keep four waves.  (32 copies of the table, one bank pair per lane, changed nothing with four waves, and
+// beside two sets of rings there is no room for them.)
 template <int BM, int MODE, bool SPLIT, bool SEG = false>
-__global__ __launch_bounds__(256) void nf4_gemm_rs_kernel(const RsArgs g, const RsSegs sg) {
+__global__ __launch_bounds__((256 * RsLayout<BM, SPLIT>::kGroups)) void nf4_gemm_rs_kernel(const RsArgs g, const RsSegs sg) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the body uses LDS address-space casts and gfx950 builtins the host pass cannot parse
   static_assert(BM == 256 || BM == 128, "BM");
   static_assert(!SEG || (MODE == 1 && !SPLIT), "segments: grad-input kernels only");
   constexpr bool PER_ELEM = MODE == 1;
   constexpr bool SCAL_T = MODE == 2;
-  using L = RsLayout<BM>;
+  using L = RsLayout<BM, SPLIT>;
   constexpr int MT = BM / 32;       // activation tiles (MFMA columns) per wave
   constexpr int NT = 2;             // weight tiles (MFMA rows) per wave
   constexpr int kALoads = BM / 32;  // direct-to-LDS instructions per wave per k-step for the activation tile (8 rows each)
@@ -118,7 +131,10 @@ __global__ __launch_bounds__(256) void nf4_gemm_rs_kernel(const RsArgs g, const 
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  constexpr int G = L::kGroups;
+  const int wv = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);
+  const int kg = G == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
+  char* const rings = smem + kg * L::kGroupBytes;  // this group's
   const int l31 = lane & 31, h = lane >> 5;
 
   int tile_m, tile_n;
@@ -148,10 +164,19 @@ __global__ __launch_bounds__(256) void nf4_gemm_rs_kernel(const RsArgs g, const 
     nk = nkf - kb < g.ksteps ? nkf - kb : g.ksteps;
   }
 
+  // a group's k-steps, and the k-steps of the operands from its first one on: batches issued past the group's end stay inside
+  int steps = nk, nvalid = nk;
+  if constexpr (G == 2) {
+    const int half = (nk + 1) >> 1;
+    steps = kg ? nk - half : half;
+    kb += kg ? (steps ? half : 0) : 0;
+    nvalid = nkf - kb;
+  }
+
   // ---- table: entry(byte) = (nf4[byte >> 4], nf4[byte & 15]) as two fp32 (each exactly a bf16 value)
   //      It is a separate LDS object so that the compiler can tell table reads from the direct-to-LDS destinations.
   __shared__ float2 lut_s[256];
-  lut_s[tid] = make_float2(round_to_bf16(kNF4Rs[tid >> 4]), round_to_bf16(kNF4Rs[tid & 15]));
+  if (G == 1 || kg == 0) lut_s[tid] = make_float2(round_to_bf16(kNF4Rs[tid >> 4]), round_to_bf16(kNF4Rs[tid & 15]));
   const char* lut = reinterpret_cast<const char*>(lut_s);
 
   // ---- activation tile.  A row is eight 16-byte chunks; chunk c of row r is stored in slot c ^ ((r >> 1) & 7), which
@@ -207,7 +232,7 @@ __global__ __launch_bounds__(256) void nf4_gemm_rs_kernel(const RsArgs g, const 
     asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
                  ::"v"(voff), "s"(base), "s"(lds), "n"(imm) : "memory", "m0", "scc");
   };
-  const uint32_t lds0 = (uint32_t)(uintptr_t)TT_LDS_PTR(smem);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)TT_LDS_PTR(rings);
   // A batch (k-step t) is kBatch loads: the activation tile -> A stage, this wave's code bytes and scalers -> W stage.
   // They are issued one at a time between MFMAs (slot d of the batch), never back to back: the address unit takes
   // tens of cycles per 64-lane load and a wave that finds its queue full cannot issue anything else meanwhile.
@@ -229,7 +254,7 @@ __global__ __launch_bounds__(256) void nf4_gemm_rs_kernel(const RsArgs g, const 
     return b;
   };
   auto batch_addr = [&](int t, int sa, int sw) -> BatchAddr {
-    const int tk = kb + (t < nk ? t : nk - 1);
+    const int tk = kb + (t < nvalid ? t : nvalid - 1);
     return batch_addr_at(reinterpret_cast<const char*>(g.X) + ((int64_t)tk << 7),      // + k0 * 2 bytes
                          reinterpret_cast<const char*>(g.codes) + ((int64_t)tk << 5),  // + k0 / 2 bytes
                          reinterpret_cast<const char*>(g.scal) + tk * s_stride, sa, sw);
@@ -279,13 +304,13 @@ __global__ __launch_bounds__(256) void nf4_gemm_rs_kernel(const RsArgs g, const 
   };
   auto load_s8 = [&](float (&s8)[8], int sw, int ks) {
     if constexpr (PER_ELEM) {
-      const f32x4_t* sp = reinterpret_cast<const f32x4_t*>(smem + L::kWOff + sw * L::kStageW + 8192 + wv * 512 + (32 * h + 8 * ks) * 4);
+      const f32x4_t* sp = reinterpret_cast<const f32x4_t*>(rings + L::kWOff + sw * L::kStageW + 8192 + wv * 512 + (32 * h + 8 * ks) * 4);
       const f32x4_t a = sp[0], b = sp[1];
       s8[0] = a.x; s8[1] = a.y; s8[2] = a.z; s8[3] = a.w; s8[4] = b.x; s8[5] = b.y; s8[6] = b.z; s8[7] = b.w;
     }
   };
   auto load_codes = [&](int sw, float (&s_out)[NT]) {
-    const char* wbase = smem + L::kWOff + sw * L::kStageW;
+    const char* wbase = rings + L::kWOff + sw * L::kStageW;
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
       const u32x4_t v = *reinterpret_cast<const u32x4_t*>(wbase + (wv * NT + j) * 1024 + lane * 16);
@@ -319,7 +344,7 @@ __global__ __launch_bounds__(256) void nf4_gemm_rs_kernel(const RsArgs g, const 
                    int d_first, int d_per_quarter_even, int d_per_quarter_odd) {
     float s8[8];
     load_s8(s8, sw_fin, ks_fin);
-    const char* sA = smem + st_next * L::kStageA;
+    const char* sA = rings + st_next * L::kStageA;
     int d = d_first;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -358,6 +383,8 @@ __global__ __launch_bounds__(256) void nf4_gemm_rs_kernel(const RsArgs g, const 
   // That one barrier per step also orders stage reuse: a wave issuing batch t+2 into the A stage of tile t-2 has
   // passed barrier t-1, which every wave reaches only after finishing step t-2.  W stages are wave-private.
   // Weights are expanded just in time: substep ks is fetched two phases and finished one phase before its MFMAs.
+  // (Two groups: batch t+2 is issued in phases 2, 3, behind the barrier that says every wave is done with tile t-1, whose
+  // stage it takes, and the wait before that barrier is for batch t+1, the only one in flight.)
   // Global bases of the next batch to issue, carried through the main loop and bumped by a constant per k-step.
   const char *pxb, *pcb, *psb;
   auto seg_base = [&](int q, int step) {
@@ -365,7 +392,36 @@ __global__ __launch_bounds__(256) void nf4_gemm_rs_kernel(const RsArgs g, const 
     pcb = reinterpret_cast<const char*>(sg.codes[q]) + ((int64_t)step << 5);
     psb = reinterpret_cast<const char*>(sg.scal[q]) + (int64_t)step * 256;
   };
-  if constexpr (SEG) {  // segment 0 has at least two k-steps (the host puts the widest first): batches 0 and 1 are its
+  // two groups, SEG: the next batch's segment and its k-steps left, that batch included
+  int sq = 0, sleft = 0;
+  auto seg_advance = [&]() {
+    if (--sleft > 0) {
+      pxb += 128;
+      pcb += 32;
+      psb += 256;
+    } else if (sq + 1 < sg.n) {
+      ++sq;
+      sleft = sg.Kc[sq] >> 6;
+      set_offsets(sg.Kc[sq]);
+      seg_base(sq, 0);
+    } else {
+      sleft = 1;  // past the end of the contraction the last tile is reloaded, never consumed
+    }
+  };
+  if constexpr (SEG && G == 2) {
+    int at = kg ? kb : 0;  // the group's first k-step (nk >= 2: both have one)
+    while (at >= (sg.Kc[sq] >> 6)) at -= sg.Kc[sq++] >> 6;
+    sleft = (sg.Kc[sq] >> 6) - at;
+    set_offsets(sg.Kc[sq]);
+    seg_base(sq, at);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const BatchAddr bt = batch_addr_at(pxb, pcb, psb, t, t);
+#pragma unroll
+      for (int d = 0; d < kBatch; ++d) issue_one(bt, d);
+      seg_advance();
+    }
+  } else if constexpr (SEG) {  // segment 0 has at least two k-steps (the host puts the widest first): batches 0 and 1 are its
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       seg_base(0, t);
@@ -377,7 +433,7 @@ __global__ __launch_bounds__(256) void nf4_gemm_rs_kernel(const RsArgs g, const 
     issue(0, 0, 0);
     issue(1, 1, 1);
   }
-  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(kBatch) : "memory");  // batch 0 landed everywhere, table written
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kBatch) : "memory");  // batch 0 landed everywhere, table written
   load_codes(0, sc);
   {
     float s8[8];
@@ -392,7 +448,7 @@ __global__ __launch_bounds__(256) void nf4_gemm_rs_kernel(const RsArgs g, const 
       }
   }
 #pragma unroll
-  for (int i = 0; i < MT; ++i) xfa[i] = *reinterpret_cast<const bf16x8_t*>(smem + i * 4096 + x_off[0]);
+  for (int i = 0; i < MT; ++i) xfa[i] = *reinterpret_cast<const bf16x8_t*>(rings + i * 4096 + x_off[0]);
 
   constexpr int kDEven = (kBatch + 7) / 8 > 1 ? 2 : 1;  // loads per even quarter over the 8 quarters of phases 0 and 1
   constexpr int kDOdd = (kBatch - 4 * kDEven + 3) / 4;  // and per odd quarter
@@ -418,7 +474,38 @@ __global__ __launch_bounds__(256) void nf4_gemm_rs_kernel(const RsArgs g, const 
     a0 = a1;
     w0 = w1;
   };
-  if constexpr (!SEG) {
+  // The same with two groups; the batch issued is that of the carried bases, which the caller moves on.
+  auto k_step2 = [&]() {
+    const int a1 = a0 == 2 ? 0 : a0 + 1, a2 = a1 == 2 ? 0 : a1 + 1;  // the rings are equally long: W slots likewise
+    const BatchAddr b = batch_addr_at(pxb, pcb, psb, a2, a2);
+    phase(xfa, wfa, xfb, a0, 1, wfb, sc, a0, 1, 2, b, kBatch, 0, 0);
+    phase(xfb, wfb, xfa, a0, 2, wfa, sc, a0, 2, 3, b, kBatch, 0, 0);
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    load_codes(a1, sc_next);
+    phase(xfa, wfa, xfb, a0, 3, wfb, sc, a0, 3, 0, b, 0, kDEven, kDOdd);
+    phase(xfb, wfb, xfa, a1, 0, wfa, sc_next, a1, 0, 1, b, 2 * (kDEven + kDOdd), kDEven, kDOdd);
+#pragma unroll
+    for (int j = 0; j < NT; ++j) sc[j] = sc_next[j];
+    a0 = a1;
+  };
+  if constexpr (G == 2) {
+    if constexpr (!SEG) {
+      const BatchAddr b2 = batch_addr(2, 0, 0);
+      pxb = b2.xb; pcb = b2.cb; psb = b2.sb;
+    }
+    for (int kt = 0; kt < steps; ++kt) {
+      k_step2();
+      if constexpr (SEG) {
+        seg_advance();
+      } else {
+        const int64_t adv = kt + 3 < nvalid ? 1 : 0;
+        pxb += adv << 7;
+        pcb += adv << 5;
+        psb += adv * s_stride;
+      }
+    }
+    if (steps < ((nk + 1) >> 1)) asm volatile("s_barrier" ::: "memory");  // the other group's last step
+  } else if constexpr (!SEG) {
     const BatchAddr b2 = batch_addr(2, 0, 0);  // global bases of k-step 2
     pxb = b2.xb; pcb = b2.cb; psb = b2.sb;
     for (int kt = 0; kt < nk; ++kt) k_step(kt + 3 < nk ? 1 : 0);
@@ -445,6 +532,45 @@ __global__ __launch_bounds__(256) void nf4_gemm_rs_kernel(const RsArgs g, const 
   }
 
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the clamped batches issued by the last two steps
+  // ---- the two groups' sums: each gives the other half of its rows away through LDS (lane-private 16-byte pieces) and keeps
+  //      the first (group 0) or second half, row tiles [kg MT / 2, + MT / 2)
+  constexpr int MR = MT / G;
+  const int mr0 = m0 + kg * 32 * MR;  // the wave's rows of C
+  constexpr int kGive = NT * MR * 16 * 64 * (int)sizeof(float);
+  static_assert(G == 1 || 8 * kGive <= L::kTotal, "the exchange fits the rings");
+  char* const mine = smem + (G == 2 ? (4 * (1 - kg) + wv) * kGive : wv * (BM * 128));  // only this wave reads it: the band later
+  f32x16_t res[NT][MR];
+  if constexpr (G == 2) {
+    __syncthreads();  // every wave is done with the rings
+    char* const out = smem + (4 * kg + wv) * kGive + lane * 16;
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int i = 0; i < MR; ++i) {
+        res[j][i] = kg ? acc[j][i + MR] : acc[j][i];
+        const f32x16_t other = kg ? acc[j][i] : acc[j][i + MR];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *reinterpret_cast<f32x4_t*>(out + ((j * MR + i) * 4 + q) * 1024) = f32x4_t{other[4 * q], other[4 * q + 1], other[4 * q + 2], other[4 * q + 3]};
+      }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int i = 0; i < MR; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const f32x4_t o = *reinterpret_cast<const f32x4_t*>(mine + lane * 16 + ((j * MR + i) * 4 + q) * 1024);
+#pragma unroll
+          for (int v = 0; v < 4; ++v) res[j][i][4 * q + v] += o[v];
+        }
+  } else {
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int i = 0; i < MR; ++i) res[j][i] = acc[j][i];
+  }
+
   // ---- adapter: R extra contraction steps, operands straight from global memory
   //      (a SEG kernel has one adapter per segment)
   const int n_adapters = SEG ? sg.n : 1;
@@ -456,13 +582,13 @@ __global__ __launch_bounds__(256) void nf4_gemm_rs_kernel(const RsArgs g, const 
     for (int rc = 0; rc < R; rc += 16) {
       const int r0 = rc + 8 * h;
       const bool in = r0 < R;  // R % 8 == 0: a lane's 8 indices are all in or all out
-      bf16x8_t wfr[NT], xfr[MT];
+      bf16x8_t wfr[NT], xfr[MR];
       // every request of the step first, then their uses: one trip to memory per step (with the scaling between two
       // loads the compiler waited for each of them in turn)
-      u32x4_t xraw[MT];
+      u32x4_t xraw[MR];
 #pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        int row = m0 + 32 * i + l31;
+      for (int i = 0; i < MR; ++i) {
+        int row = mr0 + 32 * i + l31;
         row = row < g.M ? row : g.M - 1;
         xraw[i] = u32x4_t{0, 0, 0, 0};
         if (in) xraw[i] = *reinterpret_cast<const u32x4_t*>(lX + (int64_t)row * g.ldlx + r0);
@@ -487,7 +613,7 @@ __global__ __launch_bounds__(256) void nf4_gemm_rs_kernel(const RsArgs g, const 
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 0; i < MT; ++i) {
+      for (int i = 0; i < MR; ++i) {
         u32x4_t raw = xraw[i];
         if (g.lscale != 1.0f) {
 #pragma unroll
@@ -499,12 +625,12 @@ __global__ __launch_bounds__(256) void nf4_gemm_rs_kernel(const RsArgs g, const 
 #pragma unroll
       for (int j = 0; j < NT; ++j)
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
-          acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wfr[j], xfr[i], acc[j][i], 0, 0, 0);
+        for (int i = 0; i < MR; ++i)
+          res[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wfr[j], xfr[i], res[j][i], 0, 0, 0);
     }
   }
 
-  // ---- epilogue.  acc[j][i][v] = C[m][n] with m = m0 + 32 i + l31 and n = n0 + 64 wv + 32 j + 8 (v/4) + 4 h + v%4.
+  // ---- epilogue.  res[j][i][v] = C[m][n] with m = mr0 + 32 i + l31 and n = n0 + 64 wv + 32 j + 8 (v/4) + 4 h + v%4.
   //      Stored straight from these registers a wave would write 16-byte pieces of 32 different rows per instruction,
   //      which the memory system turns into partial-line read-modify-writes.  Instead each wave transposes its
   //      BM x 64 band through LDS (the activation ring is free now: BM x 128 bytes per wave) and writes whole
@@ -515,22 +641,22 @@ __global__ __launch_bounds__(256) void nf4_gemm_rs_kernel(const RsArgs g, const 
     if (n0 + wv * 64 >= g.Nout) return;
     float* P = g.part + (int64_t)blockIdx.y * g.M * g.Nout + n0 + wv * 64 + 4 * h;
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      const int row = m0 + 32 * i + l31;
+    for (int i = 0; i < MR; ++i) {
+      const int row = mr0 + 32 * i + l31;
       if (row >= g.M) continue;
 #pragma unroll
       for (int j = 0; j < NT; ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
           *reinterpret_cast<f32x4_t*>(P + (int64_t)row * g.Nout + 32 * j + 8 * q) =
-              f32x4_t{acc[j][i][4 * q], acc[j][i][4 * q + 1], acc[j][i][4 * q + 2], acc[j][i][4 * q + 3]};
+              f32x4_t{res[j][i][4 * q], res[j][i][4 * q + 1], res[j][i][4 * q + 2], res[j][i][4 * q + 3]};
     }
     return;
   }
-  __syncthreads();                      // every wave is done reading the activation ring
+  if constexpr (G == 1) __syncthreads();  // every wave is done reading the activation ring
   if (n0 + wv * 64 >= g.Nout) return;  // the whole 64-column band of this wave lies outside (no barrier follows)
   {
-    char* band = smem + wv * (BM * 128);
+    char* band = mine;
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
@@ -548,11 +674,11 @@ __global__ __launch_bounds__(256) void nf4_gemm_rs_kernel(const RsArgs g, const 
           c4[2] = bits_f32(cc.y << 16); c4[3] = bits_f32(cc.y & 0xffff0000u);
         }
 #pragma unroll
-        for (int i = 0; i < MT; ++i) {
+        for (int i = 0; i < MR; ++i) {
           const int r = 32 * i + l31;
           u32x2_t o;
-          o.x = pack_bf16x2((acc[j][i][4 * q + 0] + b4[0]) * c4[0], (acc[j][i][4 * q + 1] + b4[1]) * c4[1]);
-          o.y = pack_bf16x2((acc[j][i][4 * q + 2] + b4[2]) * c4[2], (acc[j][i][4 * q + 3] + b4[3]) * c4[3]);
+          o.x = pack_bf16x2((res[j][i][4 * q + 0] + b4[0]) * c4[0], (res[j][i][4 * q + 1] + b4[1]) * c4[1]);
+          o.y = pack_bf16x2((res[j][i][4 * q + 2] + b4[2]) * c4[2], (res[j][i][4 * q + 3] + b4[3]) * c4[3]);
           *reinterpret_cast<u32x2_t*>(band + r * 128 + (((4 * j + q) ^ (r & 7)) << 4) + 8 * h) = o;
         }
       }
@@ -562,10 +688,10 @@ __global__ __launch_bounds__(256) void nf4_gemm_rs_kernel(const RsArgs g, const 
     const int c = lane & 7;
     uint16_t* crow = g.C + n0 + wv * 64 + 8 * c;
 #pragma unroll 8
-    for (int t = 0; t < BM / 8; ++t) {
+    for (int t = 0; t < 4 * MR; ++t) {
       const int r = 8 * t + (lane >> 3);
       const u32x4_t v = *reinterpret_cast<const u32x4_t*>(band + r * 128 + ((c ^ (r & 7)) << 4));
-      if (m0 + r < g.M) *reinterpret_cast<u32x4_t*>(crow + (int64_t)(m0 + r) * g.Nout) = v;
+      if (mr0 + r < g.M) *reinterpret_cast<u32x4_t*>(crow + (int64_t)(mr0 + r) * g.Nout) = v;
     }
   }
 #endif
@@ -590,7 +716,7 @@ __global__ __launch_bounds__(256) void nf4_gemm_rs16_kernel(const RsArgs g, cons
   static_assert(!SEG || (MODE == 1 && !SPLIT), "segments: grad-input kernels only");
   constexpr bool PER_ELEM = MODE == 1;
   constexpr bool SCAL_T = MODE == 2;
-  using L = RsLayout<BM>;
+  using L = RsLayout<BM, SPLIT>;
   constexpr int MT = BM / 16;       // 16-row activation tiles (MFMA columns) per wave
   constexpr int MH = MT / 2;        // of which a phase takes half
   constexpr int NT = 4;             // 16-column weight tiles (MFMA rows) per wave
@@ -1094,7 +1220,7 @@ __global__ __launch_bounds__(256) void nf4_gemm_rs_reduce_kernel(const float* __
 
 template <int BM, int MODE, bool SPLIT, bool SEG = false>
 int launch_rs(RsArgs& g, int splits, hipStream_t s, const RsSegs* segs = nullptr) {
-  using L = RsLayout<BM>;
+  using L = RsLayout<BM, SPLIT>;
   g.tiles_m = (g.M + BM - 1) / BM;
   g.tiles_n = (g.Nout + kBN - 1) / kBN;
   // Full tiles of a single layer run the 16 x 16 x 32 form of the loop: 1 - 5 % faster there (the part clocks 15 % higher
@@ -1117,7 +1243,7 @@ int launch_rs(RsArgs& g, int splits, hipStream_t s, const RsSegs* segs = nullptr
     if (dev >= 0) attr_set[dev] = true;
   }
   static const RsSegs no_segs = {};
-  const dim3 grid((unsigned)(g.tiles_m * g.tiles_n), (unsigned)splits), block(256);
+  const dim3 grid((unsigned)(g.tiles_m * g.tiles_n), (unsigned)splits), block(256 * (kMfma16 ? 1 : L::kGroups));
   if constexpr (kMfma16)
     nf4_gemm_rs16_kernel<BM, MODE, SPLIT, SEG><<<grid, block, L::kTotal, s>>>(g, segs ? *segs : no_segs);
   else
