@@ -544,3 +544,26 @@ def test_eight_wave_tiles_at_short_and_odd_contractions(M, steps):
         want = want + gy.float() @ t.get_original_weight().float() + gh[:, off:off + r].float() @ m.lora_a.float()
         off += r
     close(gx, want)
+
+
+@pytest.mark.parametrize("M,K,Ns", [(65, 1024, (512, 256, 256)), (129, 1088, (256, 768)), (300, 4096, (1024, 256, 512, 256)), (130, 256, (8192, 8192)),
+                                    (200, 1024, (576, 192, 64)), (70, 1024, (64, 1024, 128, 192))])
+@pytest.mark.parametrize("bias", [False, True])
+def test_grouped_launches_of_few_tiles(M, K, Ns, bias):
+    """Forward members in one launch (sliced; one round of tiles unsliced; widths that keep them apart) and the grad-input's
+    concatenated contraction in slices that begin and end inside a member.  bf16 results of fp32 sums, as above."""
+    ranks = (8, 16, 8, 24)[:len(Ns)]
+    mem = _members(K, Ns, ranks, seed=M + K, bias=bias)
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x = torch.randn(M, K, device=DEV, generator=g).to(BF)
+    gys = [torch.randn(M, n, device=DEV, generator=g).to(BF) for n in Ns]
+    h_cat, ys = ops.lora_group_fwd(x, [e[0] for e in mem])
+    gx, _, gh = ops.lora_group_bwd(x, h_cat, [e[0] for e in mem], gys)
+    dx, off = 0, 0
+    for (m, t, *_), y, gy, r in zip(mem, ys, gys, ranks):
+        w, h = t.get_original_weight().float(), (h_cat[:, off:off + r].float() * m.scale).to(BF).float()
+        want = x.float() @ w.t() + h @ m.lora_b.float().t() + (m.bias.float() if bias else 0.0)
+        torch.testing.assert_close(y.float(), want, rtol=2 ** -8, atol=2e-5 * want.abs().max().item())
+        dx = dx + gy.float() @ w + gh[:, off:off + r].float() @ m.lora_a.float()
+        off += r
+    torch.testing.assert_close(gx.float(), dx, rtol=2 ** -8, atol=2e-5 * dx.abs().max().item())

@@ -56,7 +56,11 @@ int run_gemm_rs(const void* X, const uint8_t* codes, const void* scal, int mode,
                 bool lw_row_major, int R, float lscale, const void* bias, const void* cscale, void* C, int64_t M, int64_t Nout,
                 int64_t Kc, void* workspace, size_t workspace_bytes, hipStream_t s);
 size_t gemm_rs_workspace_bytes(int64_t M, int64_t Nout, int64_t Kc);
-int run_gemm_rs_group_dx(const GroupDx& d, const void* gh_cat, void* gx, hipStream_t s);
+// memory for the slices of a grouped launch of few tiles (0: it is not sliced)
+size_t group_dx_slices_bytes(const GroupDx& d);
+size_t group_fwd_slices_bytes(const GroupGemm& d);
+int run_gemm_rs_group_dx(const GroupDx& d, const void* gh_cat, void* gx, hipStream_t s, void* workspace = nullptr, size_t workspace_bytes = 0);
+int run_gemm_rs_group_fwd(const void* x, const GroupGemm& d, const void* h_cat, void* workspace, size_t workspace_bytes, bool* done, hipStream_t s);
 
 // nf4_gemm_dense.hip: expand the weight once into scratch memory, then a plain bf16 GEMM (many tokens)
 bool dense_path_applies(int64_t M, int64_t Nout, int64_t Kc);

@@ -63,7 +63,6 @@ int decode(const char* who, const ttamd_lora_group_member* m, int n, int64_t M, 
   return TTAMD_OK;
 }
 
-// slices of the largest sliced member GEMM, or the expanded weight(s) of the many-token path
 // the few-token launch serves the group when it would serve the member with the largest weight
 bool group_small_m(const Decoded& d, bool sliced_ok) {
   int64_t n_max = 0;
@@ -71,6 +70,7 @@ bool group_small_m(const Decoded& d, bool sliced_ok) {
   return small_m_applies(d.gm.M, n_max, d.gm.K, sliced_ok);
 }
 
+// slices of the grouped launch or of the largest sliced member GEMM, or the expanded weight(s) of the many-token path
 size_t fwd_gemm_ws(const Decoded& d) {
   const bool tiled = !group_small_m(d, true);
   size_t w = tiled ? dense_group_fwd_workspace_bytes(d.gm) : 0;
@@ -79,6 +79,10 @@ size_t fwd_gemm_ws(const Decoded& d) {
       const size_t b = gemm_rs_workspace_bytes(d.gm.M, d.gm.N[i], d.gm.K);
       w = b > w ? b : w;
     }
+  if (tiled) {
+    const size_t b = group_fwd_slices_bytes(d.gm);
+    w = b > w ? b : w;
+  }
   return w;
 }
 
@@ -139,6 +143,10 @@ int group_fwd(const char* who, const void* x, const ttamd_lora_group_member* mem
     if (act_done) *act_done = gated;
     return run_gemm_dense_group_fwd(x, d.gm, h_cat, workspace, s, gated ? act : nullptr);
   }
+  // fewer tokens: one launch over the members' tiles where they make at most one round of them
+  bool one_launch = false;
+  if (int rc = run_gemm_rs_group_fwd(x, d.gm, h_cat, sliced ? workspace : nullptr, sliced ? workspace_bytes : 0, &one_launch, s)) return rc;
+  if (one_launch) return TTAMD_OK;
   const int ldh = d.gm.r_off[d.gm.n];
   for (int i = 0; i < d.gm.n; ++i) {
     const void* sc = d.gm.bscal_t[i] ? d.gm.bscal_t[i] : d.gm.bscal[i];
@@ -222,7 +230,8 @@ extern "C" int ttamd_nf4_group_bwd_dx_bf16(const ttamd_lora_group_member* member
 extern "C" size_t ttamd_nf4_group_bwd_dx_workspace_bytes(const ttamd_lora_group_member* members, int n_members, int64_t M, int64_t K) {
   Decoded d;
   if (decode("nf4_group_bwd_dx_workspace_bytes", members, n_members, M, K, false, d) != TTAMD_OK) return 0;
-  return dense_group_dx_workspace_bytes(d.dx);
+  const size_t expanded = dense_group_dx_workspace_bytes(d.dx);
+  return expanded > 0 ? expanded : group_dx_slices_bytes(d.dx);
 }
 
 extern "C" int ttamd_nf4_group_bwd_dx_ws_bf16(const ttamd_lora_group_member* members, int n_members, const void* gh_cat, void* gx,
@@ -230,6 +239,12 @@ extern "C" int ttamd_nf4_group_bwd_dx_ws_bf16(const ttamd_lora_group_member* mem
   Decoded d;
   if (int rc = decode("nf4_group_bwd_dx", members, n_members, M, K, false, d)) return rc;
   const size_t need = dense_group_dx_workspace_bytes(d.dx);
+  const size_t slices = need == 0 ? group_dx_slices_bytes(d.dx) : 0;
+  if (slices > 0 && workspace != nullptr && workspace_bytes >= slices) {
+    TT_REQUIRE(gh_cat && gx && aligned16(gh_cat) && aligned16(gx), "nf4_group_bwd_dx: gh_cat and gx must be non-null and 16-byte aligned");
+    for (int i = 0; i < n_members; ++i) TT_REQUIRE(aligned16(d.dx.codes_t[i]), "nf4_group_bwd_dx: member %d: the transposed copies must be 16-byte aligned", i);
+    return run_gemm_rs_group_dx(d.dx, gh_cat, gx, reinterpret_cast<hipStream_t>(stream), workspace, workspace_bytes);
+  }
   if (need == 0 || workspace == nullptr || workspace_bytes < need)
     return ttamd_nf4_group_bwd_dx_bf16(members, n_members, gh_cat, gx, M, K, stream);
   TT_REQUIRE(gh_cat && gx && aligned16(gh_cat) && aligned16(gx), "nf4_group_bwd_dx: gh_cat and gx must be non-null and 16-byte aligned");

@@ -27,6 +27,8 @@
 #include "group.h"
 #include "nf4_math.h"
 
+#include <type_traits>
+
 namespace ttamd {
 namespace {
 
@@ -80,6 +82,23 @@ struct RsSegs {
   int n;
 };
 
+// MEM kernels: the forwards of layers with a common input X as one launch.  Member q has the workgroups [wg_end[q - 1],
+// wg_end[q]): its tiles, or (SPLIT) those of its first slice, of its second, ..., with the slices a launch of its own has (the
+// same bits), and its partial products [slices, M, Nout[q]] at part_at[q].  g.codes / scal / lX / lW / R / lscale / bias /
+// C / Nout / ksteps are then unused, MODE is 2.
+struct RsMembers {
+  const uint8_t* codes[kGroupMax];
+  const float* scal[kGroupMax];
+  const uint16_t* lX[kGroupMax];
+  const uint16_t* lW[kGroupMax];
+  const uint16_t* bias[kGroupMax];
+  uint16_t* C[kGroupMax];
+  int64_t part_at[kGroupMax];
+  int Nout[kGroupMax], R[kGroupMax], wg_end[kGroupMax], ksteps[kGroupMax];
+  float lscale[kGroupMax];
+  int n;
+};
+
 constexpr int kBN = 256;
 constexpr int kLutBytes = 256 * 8;  // 256 byte values x (fp32 nf4[hi nibble], fp32 nf4[lo nibble])
 
@@ -103,7 +122,7 @@ struct RsLayout {
 // SPLIT: the contraction is cut into gridDim.y slices so that a launch with few output tiles still fills the chip; a
 // workgroup then leaves its tile as fp32 in g.part (slice 0 includes the adapter) and bias, column scale and the
 // rounding to bf16 happen in nf4_gemm_rs_reduce_kernel, which adds the slices in a fixed order.
-// SEG: segmented contraction (see RsSegs); only with MODE 1 and without SPLIT.
+// SEG: segmented contraction (see RsSegs), only with MODE 1.  MEM: several layers (see RsMembers), only with MODE 2.
 // BM 128 without SPLIT: eight waves.  A wave's k-step is 300 instructions beside 1024 cycles of MFMA, and with one wave per
 // SIMD nothing covers the waits between them: a k-step took 2200 cycles, whatever the tile's rows (96: the same).  Two
 // waves per SIMD cover each other; a tile of 256 rows has no registers for that, one of 128 rows has.  The second four
@@ -115,11 +134,14 @@ struct RsLayout {
 // exchange cost what the loop gains (4096 x 4096 at 333 tokens in five slices 23 -> 24, 2048 x 2048 at 700 16.5 -> 19.4):
 // those keep four waves.  (32 copies of the table, one bank pair per lane, changed nothing with four waves, and
 // beside two sets of rings there is no room for them.)
-template <int BM, int MODE, bool SPLIT, bool SEG = false>
-__global__ __launch_bounds__((256 * RsLayout<BM, SPLIT>::kGroups)) void nf4_gemm_rs_kernel(const RsArgs g, const RsSegs sg) {
+template <int BM, int MODE, bool SPLIT, bool SEG = false, bool MEM = false>
+__global__ __launch_bounds__((256 * RsLayout<BM, SPLIT>::kGroups)) void nf4_gemm_rs_kernel(
+    const RsArgs ga, const std::conditional_t<MEM, RsMembers, RsSegs> sg) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the body uses LDS address-space casts and gfx950 builtins the host pass cannot parse
   static_assert(BM == 256 || BM == 128, "BM");
-  static_assert(!SEG || (MODE == 1 && !SPLIT), "segments: grad-input kernels only");
+  static_assert(!SEG || MODE == 1, "segments: grad-input kernels only");
+  static_assert(!MEM || (MODE == 2 && !SEG), "members: forward kernels only");
+  RsArgs g = ga;
   constexpr bool PER_ELEM = MODE == 1;
   constexpr bool SCAL_T = MODE == 2;
   using L = RsLayout<BM, SPLIT>;
@@ -137,8 +159,30 @@ __global__ __launch_bounds__((256 * RsLayout<BM, SPLIT>::kGroups)) void nf4_gemm
   char* const rings = smem + kg * L::kGroupBytes;  // this group's
   const int l31 = lane & 31, h = lane >> 5;
 
-  int tile_m, tile_n;
-  {
+  int tile_m, tile_n, slice = blockIdx.y;
+  if constexpr (MEM) {
+    int q = 0;
+    while ((int)blockIdx.x >= sg.wg_end[q]) ++q;  // uniform; the grid ends at wg_end[n - 1]
+    g.codes = sg.codes[q];
+    g.scal = sg.scal[q];
+    g.lX = sg.lX[q];
+    g.lW = sg.lW[q];
+    g.bias = sg.bias[q];
+    g.C = sg.C[q];
+    g.Nout = sg.Nout[q];
+    g.R = sg.R[q];
+    g.lscale = sg.lscale[q];
+    const int at = (int)blockIdx.x - (q ? sg.wg_end[q - 1] : 0);
+    const int tn = (g.Nout + kBN - 1) / kBN;
+    if constexpr (SPLIT) {
+      g.part += sg.part_at[q];
+      g.ksteps = sg.ksteps[q];
+      slice = at / (g.tiles_m * tn);
+    }
+    const int tile = at - slice * g.tiles_m * tn;
+    tile_m = tile / tn;
+    tile_n = tile % tn;
+  } else {
     // workgroup ids are dealt round-robin to the 8 XCDs (one L2 each): give every XCD a band of m-tiles and walk it
     // column by column, so the workgroups resident on an XCD share each weight tile through its L2 (the weight is
     // then fetched once per XCD instead of once per m-tile)
@@ -153,15 +197,17 @@ __global__ __launch_bounds__((256 * RsLayout<BM, SPLIT>::kGroups)) void nf4_gemm
     }
   }
   const int m0 = tile_m * BM, n0 = tile_n * kBN;
-  const int Kc = SEG ? sg.Kc[0] : g.Kc;
+  int Kc = g.Kc;
+  if constexpr (SEG) Kc = sg.Kc[0];
   const int nkf = Kc >> 6;  // k-steps of the whole contraction: the row stride of the MODE 0 scalers
   int kb = 0, nk = nkf;     // this workgroup's k-steps are [kb, kb + nk)
   if constexpr (SEG) {
     for (int q = 1; q < sg.n; ++q) nk += sg.Kc[q] >> 6;
   }
   if constexpr (SPLIT) {
-    kb = blockIdx.y * g.ksteps;
-    nk = nkf - kb < g.ksteps ? nkf - kb : g.ksteps;
+    kb = slice * g.ksteps;
+    const int left = (SEG ? nk : nkf) - kb;
+    nk = left < g.ksteps ? left : g.ksteps;
   }
 
   // a group's k-steps, and the k-steps of the operands from its first one on: batches issued past the group's end stay inside
@@ -388,14 +434,18 @@ __global__ __launch_bounds__((256 * RsLayout<BM, SPLIT>::kGroups)) void nf4_gemm
   // Global bases of the next batch to issue, carried through the main loop and bumped by a constant per k-step.
   const char *pxb, *pcb, *psb;
   auto seg_base = [&](int q, int step) {
+    if constexpr (SEG) {
     pxb = reinterpret_cast<const char*>(sg.X[q]) + ((int64_t)step << 7);
     pcb = reinterpret_cast<const char*>(sg.codes[q]) + ((int64_t)step << 5);
     psb = reinterpret_cast<const char*>(sg.scal[q]) + (int64_t)step * 256;
+    }
   };
-  // two groups, SEG: the next batch's segment and its k-steps left, that batch included
+  // SEG in two groups or slices: the next batch's segment and its k-steps left, that batch included
+  constexpr bool WALK = SEG && (G == 2 || SPLIT);
   int sq = 0, sleft = 0;
   auto seg_advance = [&]() {
-    if (--sleft > 0) {
+    if constexpr (!WALK) {
+    } else if (--sleft > 0) {
       pxb += 128;
       pcb += 32;
       psb += 256;
@@ -408,8 +458,8 @@ __global__ __launch_bounds__((256 * RsLayout<BM, SPLIT>::kGroups)) void nf4_gemm
       sleft = 1;  // past the end of the contraction the last tile is reloaded, never consumed
     }
   };
-  if constexpr (SEG && G == 2) {
-    int at = kg ? kb : 0;  // the group's first k-step (nk >= 2: both have one)
+  if constexpr (WALK) {
+    int at = kb;  // the group's or slice's first k-step (two groups: nk >= 2, both have one)
     while (at >= (sg.Kc[sq] >> 6)) at -= sg.Kc[sq++] >> 6;
     sleft = (sg.Kc[sq] >> 6) - at;
     set_offsets(sg.Kc[sq]);
@@ -505,6 +555,11 @@ __global__ __launch_bounds__((256 * RsLayout<BM, SPLIT>::kGroups)) void nf4_gemm
       }
     }
     if (steps < ((nk + 1) >> 1)) asm volatile("s_barrier" ::: "memory");  // the other group's last step
+  } else if constexpr (WALK) {
+    for (int kt = 0; kt < nk; ++kt) {
+      k_step(0);
+      seg_advance();
+    }
   } else if constexpr (!SEG) {
     const BatchAddr b2 = batch_addr(2, 0, 0);  // global bases of k-step 2
     pxb = b2.xb; pcb = b2.cb; psb = b2.sb;
@@ -578,7 +633,7 @@ __global__ __launch_bounds__((256 * RsLayout<BM, SPLIT>::kGroups)) void nf4_gemm
     const uint16_t* __restrict__ lX = SEG ? sg.lX[ad] : g.lX;
     const uint16_t* __restrict__ lW = SEG ? sg.lW[ad] : g.lW;
     const int R = SEG ? sg.R[ad] : g.R;
-    if (!(R > 0 && lX != nullptr && (!SPLIT || blockIdx.y == 0))) continue;
+    if (!(R > 0 && lX != nullptr && (!SPLIT || slice == 0))) continue;
     for (int rc = 0; rc < R; rc += 16) {
       const int r0 = rc + 8 * h;
       const bool in = r0 < R;  // R % 8 == 0: a lane's 8 indices are all in or all out
@@ -639,7 +694,7 @@ __global__ __launch_bounds__((256 * RsLayout<BM, SPLIT>::kGroups)) void nf4_gemm
     // fp32 partial tile, straight from the registers: a lane holds four consecutive columns of a row (16 bytes), the
     // two halves of a wave make 32 bytes and the four q of a weight tile complete the row's 128-byte line
     if (n0 + wv * 64 >= g.Nout) return;
-    float* P = g.part + (int64_t)blockIdx.y * g.M * g.Nout + n0 + wv * 64 + 4 * h;
+    float* P = g.part + (int64_t)slice * g.M * g.Nout + n0 + wv * 64 + 4 * h;
 #pragma unroll
     for (int i = 0; i < MR; ++i) {
       const int row = mr0 + 32 * i + l31;
@@ -1179,12 +1234,39 @@ __global__ __launch_bounds__(256) void nf4_gemm_rs16_kernel(const RsArgs g, cons
 #endif
 }
 
+// What the slices of a launch add up to.  Output q is elements [end[q - 1], end[q]) of the launch; its partial products lie
+// at part[q], one slice of `mn` elements after the other.
+struct RsReduce {
+  const float* part[kGroupMax];
+  const uint16_t* bias[kGroupMax];
+  const uint16_t* cscale[kGroupMax];
+  uint16_t* C[kGroupMax];
+  int64_t end[kGroupMax];
+  int Nout[kGroupMax], splits[kGroupMax];
+};
+
 // C[m][n] = bf16((sum over slices of part[s][m][n] + bias[n]) * cscale[n]); a thread takes 8 consecutive columns.
-__global__ __launch_bounds__(256) void nf4_gemm_rs_reduce_kernel(const float* __restrict__ part, int splits, int64_t mn,
-                                                                 int Nout, const uint16_t* __restrict__ bias,
-                                                                 const uint16_t* __restrict__ cscale, uint16_t* __restrict__ C) {
-  const int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
-  if (e >= mn) return;
+__global__ __launch_bounds__(256) void nf4_gemm_rs_reduce_kernel(const RsReduce r) {
+  int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
+  if (e >= r.end[kGroupMax - 1]) return;
+  int Nout = r.Nout[0], splits = r.splits[0];
+  int64_t at = 0, mn = r.end[0];
+  const float* part = r.part[0];
+  const uint16_t *bias = r.bias[0], *cscale = r.cscale[0];
+  uint16_t* C = r.C[0];
+#pragma unroll
+  for (int q = 1; q < kGroupMax; ++q)
+    if (e >= r.end[q - 1]) {
+      Nout = r.Nout[q];
+      splits = r.splits[q];
+      at = r.end[q - 1];
+      mn = r.end[q] - at;
+      part = r.part[q];
+      bias = r.bias[q];
+      cscale = r.cscale[q];
+      C = r.C[q];
+    }
+  e -= at;
   float v[8];
   {
     const f32x4_t a = *reinterpret_cast<const f32x4_t*>(part + e), b = *reinterpret_cast<const f32x4_t*>(part + e + 4);
@@ -1218,20 +1300,38 @@ __global__ __launch_bounds__(256) void nf4_gemm_rs_reduce_kernel(const float* __
   *reinterpret_cast<u32x4_t*>(C + e) = o;
 }
 
-template <int BM, int MODE, bool SPLIT, bool SEG = false>
-int launch_rs(RsArgs& g, int splits, hipStream_t s, const RsSegs* segs = nullptr) {
+int launch_reduce(const RsReduce& r, hipStream_t s) {
+  nf4_gemm_rs_reduce_kernel<<<dim3((unsigned)((r.end[kGroupMax - 1] / 8 + 255) / 256)), dim3(256), 0, s>>>(r);
+  return check_launch("nf4_gemm_rs_reduce");
+}
+
+// The sum over `splits` slices into one output
+int launch_reduce(const RsArgs& g, int splits, hipStream_t s) {
+  RsReduce r = {};
+  r.part[0] = g.part;
+  r.splits[0] = splits;
+  r.bias[0] = g.bias;
+  r.cscale[0] = g.cscale;
+  r.C[0] = g.C;
+  r.Nout[0] = g.Nout;
+  for (int64_t& end : r.end) end = (int64_t)g.M * g.Nout;
+  return launch_reduce(r, s);
+}
+
+template <int BM, int MODE, bool SPLIT, bool SEG = false, bool MEM = false>
+int launch_rs(RsArgs& g, int splits, hipStream_t s, const std::conditional_t<MEM, RsMembers, RsSegs>* segs = nullptr) {
   using L = RsLayout<BM, SPLIT>;
   g.tiles_m = (g.M + BM - 1) / BM;
   g.tiles_n = (g.Nout + kBN - 1) / kBN;
   // Full tiles of a single layer run the 16 x 16 x 32 form of the loop: 1 - 5 % faster there (the part clocks 15 % higher
   // on that MFMA shape, and the loop needs 15 % more cycles for the 64 extra MFMA issues of a k-step); with 128-row tiles
   // it is 1 - 5 % slower and with segments it spills, so those keep the 32 x 32 x 16 form.
-  constexpr bool kMfma16 = BM == 256 && !SPLIT && !SEG;
+  constexpr bool kMfma16 = BM == 256 && !SPLIT && !SEG && !MEM;
   const void* fn;
   if constexpr (kMfma16)
     fn = reinterpret_cast<const void*>(&nf4_gemm_rs16_kernel<BM, MODE, SPLIT, SEG>);
   else
-    fn = reinterpret_cast<const void*>(&nf4_gemm_rs_kernel<BM, MODE, SPLIT, SEG>);
+    fn = reinterpret_cast<const void*>(&nf4_gemm_rs_kernel<BM, MODE, SPLIT, SEG, MEM>);
   // the LDS limit is a per-device attribute of the function: set it for the current device once (a race only repeats the call)
   static bool attr_set[64] = {};
   int dev = 0;
@@ -1242,12 +1342,14 @@ int launch_rs(RsArgs& g, int splits, hipStream_t s, const RsSegs* segs = nullptr
       return fail(TTAMD_ELAUNCH, "nf4_gemm_rs: cannot reserve %d bytes of LDS: %s", L::kTotal, hipGetErrorString(e));
     if (dev >= 0) attr_set[dev] = true;
   }
-  static const RsSegs no_segs = {};
-  const dim3 grid((unsigned)(g.tiles_m * g.tiles_n), (unsigned)splits), block(256 * (kMfma16 ? 1 : L::kGroups));
+  static const std::conditional_t<MEM, RsMembers, RsSegs> no_segs = {};
+  unsigned wgs = (unsigned)(g.tiles_m * g.tiles_n);
+  if constexpr (MEM) wgs = (unsigned)segs->wg_end[segs->n - 1];
+  const dim3 grid(wgs, (unsigned)splits), block(256 * (kMfma16 ? 1 : L::kGroups));
   if constexpr (kMfma16)
     nf4_gemm_rs16_kernel<BM, MODE, SPLIT, SEG><<<grid, block, L::kTotal, s>>>(g, segs ? *segs : no_segs);
   else
-    nf4_gemm_rs_kernel<BM, MODE, SPLIT, SEG><<<grid, block, L::kTotal, s>>>(g, segs ? *segs : no_segs);
+    nf4_gemm_rs_kernel<BM, MODE, SPLIT, SEG, MEM><<<grid, block, L::kTotal, s>>>(g, segs ? *segs : no_segs);
   return check_launch("nf4_gemm_rs");
 }
 
@@ -1262,6 +1364,11 @@ int choose_splits(int64_t M, int64_t Nout, int64_t Kc) {
   sp = sp < by_k ? sp : by_k;
   sp = sp < 16 ? sp : 16;
   return sp < 2 ? 1 : (int)sp;
+}
+// k-steps per slice, and the slices that then hold at least one
+void slice_steps(int64_t Kc, int splits, int& ksteps, int& used) {
+  ksteps = (int)(((Kc >> 6) + splits - 1) / splits);
+  used = (int)(((Kc >> 6) + ksteps - 1) / ksteps);
 }
 
 }  // namespace
@@ -1297,7 +1404,7 @@ int run_gemm_rs(const void* X, const uint8_t* codes, const void* scal, int mode,
   // many tokens and room for the expanded weight: expand once, then the plain bf16 GEMM
   if (workspace != nullptr && dense_path_applies(M, Nout, Kc) && workspace_bytes >= dense_workspace_bytes(M, Nout, Kc))
     return run_gemm_dense(X, codes, scal, mode, lX, ldlx, lW, lw_row_major, R, lscale, bias, cscale, C, M, Nout, Kc, workspace, s);
-  RsArgs g;
+  RsArgs g = {};
   g.X = reinterpret_cast<const uint16_t*>(X);
   g.codes = codes;
   g.scal = reinterpret_cast<const float*>(scal);
@@ -1310,22 +1417,16 @@ int run_gemm_rs(const void* X, const uint8_t* codes, const void* scal, int mode,
   g.lw_row_major = lw_row_major ? 1 : 0;
   g.ldlx = ldlx;
   g.lscale = lscale;
-  g.part = nullptr;
-  g.ksteps = 0;
   const int splits = choose_splits(M, Nout, Kc);
   if (splits > 1 && workspace != nullptr && workspace_bytes >= gemm_rs_workspace_bytes(M, Nout, Kc)) {
     TT_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 15u) == 0, "nf4_gemm: workspace must be 16-byte aligned");
     g.part = reinterpret_cast<float*>(workspace);
-    g.ksteps = (int)(((Kc >> 6) + splits - 1) / splits);
-    const int used = (int)(((Kc >> 6) + g.ksteps - 1) / g.ksteps);  // slices that hold at least one k-step
+    int used;
+    slice_steps(Kc, splits, g.ksteps, used);
     int rc = mode == 1 ? launch_rs<128, 1, true>(g, used, s)
              : mode == 2 ? launch_rs<128, 2, true>(g, used, s)
                          : launch_rs<128, 0, true>(g, used, s);
-    if (rc != TTAMD_OK) return rc;
-    const int64_t mn = M * Nout;
-    nf4_gemm_rs_reduce_kernel<<<dim3((unsigned)((mn / 8 + 255) / 256)), dim3(256), 0, s>>>(g.part, used, mn, (int)Nout, g.bias,
-                                                                                          g.cscale, g.C);
-    return check_launch("nf4_gemm_rs_reduce");
+    return rc != TTAMD_OK ? rc : launch_reduce(g, used, s);
   }
   const int64_t tiles256 = ((M + 255) / 256) * ((Nout + kBN - 1) / kBN);
   const bool big = tiles256 >= 256;
@@ -1335,11 +1436,98 @@ int run_gemm_rs(const void* X, const uint8_t* codes, const void* scal, int mode,
 }
 
 
+size_t group_dx_slices_bytes(const GroupDx& d) {
+  int64_t n_total = 0;
+  for (int i = 0; i < d.n; ++i) {
+    if (!d.codes_t[i] || !d.scal_t[i]) return 0;
+    n_total += d.N[i];
+  }
+  const int sp = choose_splits(d.M, d.K, n_total);
+  return sp > 1 ? (size_t)sp * (size_t)d.M * (size_t)d.K * sizeof(float) : 0;
+}
+
+namespace {
+// How the members' forwards make one launch: 0 they do not, 1 unsliced, 2 every member in the slices of a launch of its own.
+// Sliced launches leave CUs idle and end in a sum each: 4096 + 1024 + 1024 rows of 4096 at 333 tokens 75 us in three launches
+// and three sums, 54 in one and one.
+// Unsliced members share a launch where their tiles make at most one round on the 256 CUs; with more, the last round of
+// one launch and the first of the next overlap anyway.
+int group_form(const GroupGemm& d) {
+  int64_t tiles = 0;
+  int sliced = 0;
+  for (int i = 0; i < d.n; ++i) {
+    if (!d.bscal_t[i] || d.N[i] * d.K / 2 >= (int64_t(1) << 32)) return 0;
+    tiles += ((d.M + 127) / 128) * ((d.N[i] + kBN - 1) / kBN);
+    sliced += choose_splits(d.M, d.N[i], d.K) > 1;
+  }
+  if (d.n < 2 || d.M * d.K * 2 >= (int64_t(1) << 32) || d.K * 2 * 256 >= (int64_t(1) << 32)) return 0;
+  if (sliced == d.n) return 2;
+  return sliced == 0 && tiles <= 256 ? 1 : 0;
+}
+}  // namespace
+
+size_t group_fwd_slices_bytes(const GroupGemm& d) {
+  if (group_form(d) != 2) return 0;
+  size_t bytes = 0;
+  for (int i = 0; i < d.n; ++i) bytes += (size_t)choose_splits(d.M, d.N[i], d.K) * (size_t)d.M * (size_t)d.N[i] * sizeof(float);
+  return bytes;
+}
+
+// The members' forwards as one launch (and, sliced, one sum); *done = false where the rule above refuses it or the memory for
+// the slices is missing.
+int run_gemm_rs_group_fwd(const void* x, const GroupGemm& d, const void* h_cat, void* workspace, size_t workspace_bytes, bool* done, hipStream_t s) {
+  const int form = group_form(d);
+  *done = form == 1 || (form == 2 && workspace != nullptr && workspace_bytes >= group_fwd_slices_bytes(d));
+  if (!*done) return TTAMD_OK;
+  RsMembers m = {};
+  RsReduce r = {};
+  RsArgs g = {};
+  g.X = reinterpret_cast<const uint16_t*>(x);
+  g.M = (int)d.M;
+  g.Kc = (int)d.K;
+  g.lw_row_major = 1;
+  g.ldlx = d.r_off[d.n];
+  g.part = reinterpret_cast<float*>(workspace);
+  m.n = d.n;
+  int64_t out = 0, part = 0;
+  int wgs = 0;
+  for (int i = 0; i < kGroupMax; ++i) {
+    if (i < d.n) {
+      const int64_t mn = d.M * d.N[i];
+      m.codes[i] = d.codes[i];
+      m.scal[i] = d.bscal_t[i];
+      m.lX[i] = reinterpret_cast<const uint16_t*>(h_cat) + d.r_off[i];
+      m.lW[i] = d.lora_b[i];
+      m.bias[i] = r.bias[i] = d.bias[i];
+      m.C[i] = r.C[i] = d.y[i];
+      m.Nout[i] = r.Nout[i] = (int)d.N[i];
+      m.R[i] = d.rank[i];
+      m.lscale[i] = d.scale[i];
+      slice_steps(d.K, form == 2 ? choose_splits(d.M, d.N[i], d.K) : 1, m.ksteps[i], r.splits[i]);
+      wgs += (int)(((d.M + 127) / 128) * ((d.N[i] + kBN - 1) / kBN)) * r.splits[i];
+      m.part_at[i] = part;
+      r.part[i] = g.part + (form == 2 ? part : 0);
+      part += mn * r.splits[i];
+      out += mn;
+    }
+    m.wg_end[i] = wgs;
+    r.end[i] = out;
+  }
+  if (form == 1) return launch_rs<128, 2, false, false, true>(g, 1, s, &m);
+  TT_REQUIRE(aligned16(workspace), "nf4_lora_group_fwd: workspace must be 16-byte aligned");
+  if (int rc = launch_rs<128, 2, true, false, true>(g, 1, s, &m)) return rc;
+  return launch_reduce(r, s);
+}
+
 // Grad-input of a group of layers with a common input, as one GEMM over the concatenated contraction:
 //   gx[M, K] = sum_i gy_i[M, N_i] . D(W_i)[N_i, K] + gh_i[M, R_i] . A_i[R_i, K]
 // with the members' transposed copies (codes [K, N_i / 2], per-element scalers [K / 64, N_i]); gh_i = columns
 // [r_off[i], r_off[i + 1]) of gh_cat.  The sum over members is taken in fp32, before the one rounding to bf16.
-int run_gemm_rs_group_dx(const GroupDx& d, const void* gh_cat, void* gx, hipStream_t s) {
+// A launch of few tiles is sliced like a single layer's when the caller brought group_dx_slices_bytes(d) of memory: unsliced it
+// takes its 256 - 448 k-steps however few workgroups there are.  Unsliced -> sliced, us: 14336 + 14336 rows of 4096 at 100
+// tokens 287 -> 49, at 333 293 -> 111, at 1000 302 -> 246; 4096 + 1024 + 1024 at 333 67 -> 38, at 1000 75 -> 70; 8192 + 8192
+// rows of 2048 at 333 164 -> 45.
+int run_gemm_rs_group_dx(const GroupDx& d, const void* gh_cat, void* gx, hipStream_t s, void* workspace, size_t workspace_bytes) {
   TT_REQUIRE(d.n >= 1 && d.n <= kGroupMax, "nf4_group_dx: %d members", d.n);
   RsSegs sg = {};
   sg.n = d.n;
@@ -1374,6 +1562,17 @@ int run_gemm_rs_group_dx(const GroupDx& d, const void* gh_cat, void* gx, hipStre
   g.lw_row_major = 0;
   g.ldlx = d.r_off[d.n];
   g.lscale = 1.0f;
+  const size_t need = group_dx_slices_bytes(d);
+  if (need > 0 && workspace != nullptr && workspace_bytes >= need) {
+    TT_REQUIRE(aligned16(workspace), "nf4_group_dx: workspace must be 16-byte aligned");
+    g.part = reinterpret_cast<float*>(workspace);
+    int64_t n_total = 0;
+    for (int i = 0; i < d.n; ++i) n_total += d.N[i];
+    int used;
+    slice_steps(n_total, choose_splits(d.M, d.K, n_total), g.ksteps, used);
+    const int rc = launch_rs<128, 1, true, true>(g, used, s, &sg);
+    return rc != TTAMD_OK ? rc : launch_reduce(g, used, s);
+  }
   const int64_t tiles256 = ((d.M + 255) / 256) * ((d.K + kBN - 1) / kBN);
   return tiles256 >= 256 ? launch_rs<256, 1, false, true>(g, 1, s, &sg) : launch_rs<128, 1, false, true>(g, 1, s, &sg);
 }
