@@ -111,6 +111,26 @@ def test_every_bf16_scaled_value_and_divisor_range():
     assert torch.equal(to_nf4(w.to(DEV), 64, 256).quantized_data.cpu(), nf4_oracle.nf4_quantize(w, 64, 256).quantized_data)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("bs", [8, 32, 64, 256, 512])
+def test_codes_at_the_ends_of_the_fast_range_and_of_a_workgroup(dtype, bs):
+    """Absmaxes to both sides of where the shared reciprocal is given up (2^-119 / 2^126 in bf16, 2^-64 / 2^64 in fp32),
+    infinite, NaN and zero ones between ordinary blocks; block counts that leave a workgroup's 8192 elements ragged, down
+    to a single block.  Codes only: the mean of such absmaxes means nothing."""
+    g = torch.Generator().manual_seed(bs)
+    low, high = (-119, 126) if dtype == torch.bfloat16 else (-64, 64)
+    one_below = 1 - 2.0 ** (-8 if dtype == torch.bfloat16 else -24)
+    amax = [2.0 ** low, 2.0 ** low * one_below, 2.0 ** high, 2.0 ** high * one_below, 0.0, float("inf"), float("nan"), 0.02]
+    for n_blocks in (1, 8192 // bs - 1, 8192 // bs + 1, 3 * 8192 // bs + 5):
+        w = torch.rand(n_blocks, bs, generator=g) * 2 - 1
+        a = torch.tensor([amax[(i * 3) % len(amax)] if i % 2 else 0.05 for i in range(n_blocks)])
+        finite = torch.where(a.isfinite(), a, torch.ones(()))
+        w = (w * finite[:, None]).to(dtype)
+        w[:, bs // 2] = (-a).to(dtype)
+        got = ops.nf4_quantize(w.to(DEV), bs, 1)[0].cpu()
+        assert torch.equal(got, nf4_oracle.nf4_quantize(w, bs, 1).quantized_data), n_blocks
+
+
 def test_degenerate_inputs():
     z = to_nf4(torch.zeros(512, 512, dtype=torch.bfloat16, device=DEV))
     assert torch.all(z.quantized_data == 0) and torch.all(z.quantized_scalers == 0)

@@ -99,6 +99,40 @@ def host_math(tmp_path_factory):
         'extern "C" void codes_bf16(const float* s, int n, int* out) { for (int i = 0; i < n; ++i) out[i] = code_bf16(s[i]); }\n'
         'extern "C" void codes_f32(const float* s, int n, int* out) { for (int i = 0; i < n; ++i) out[i] = code_f32(s[i]); }\n'
         % os.path.join(ROOT, "torchtune_amd", "csrc", "nf4_math.h")
+        + """
+using namespace ttamd;
+// every pair of significands, |x| from absmax down to 2^-16 of it, the reciprocal exact and one unit to either side
+extern "C" long binned_bf16_mismatches() {
+  Nf4BinTable<true> t;
+  if (!nf4_fill_bins<true>(t)) return -1;
+  long bad = 0;
+  for (uint32_t mm = 0x3f80; mm < 0x4000; ++mm)
+    for (uint32_t xm = mm - 0x0800; xm <= mm; ++xm) {
+      const float m = bf16_bits_to_f32((uint16_t)mm);
+      for (int neg = 0; neg < 2; ++neg) {
+        const float x = bf16_bits_to_f32((uint16_t)(xm | (neg ? 0x8000u : 0u)));
+        const uint32_t want = (uint32_t)nf4_nearest_code<true>(round_to_bf16(x / m));
+        for (int d = -1; d <= 1; ++d) {
+          const float s = x * bits_f32(f32_bits(1.0f / m) + (uint32_t)d);
+          const uint32_t e = t.words[nf4_bin_offset(s) >> 2];
+          bad += nf4_code_below(e) + (nf4_above_edge_bf16(s, e) ? 1u : 0u) != want;
+        }
+      }
+    }
+  return bad;
+}
+extern "C" long binned_f32_mismatches(const float* x, const float* m, long n) {
+  Nf4BinTable<false> t;
+  if (!nf4_fill_bins<false>(t)) return -1;
+  long bad = 0;
+  for (long i = 0; i < n; ++i) {
+    const float q = nf4_shared_quotient(x[i], m[i], 1.0f / m[i]);
+    const uint32_t at = nf4_bin_offset(q) >> 2;
+    bad += t.words[kNf4Bins + at] + (q >= bits_f32(t.words[at]) ? 1u : 0u) != (uint32_t)nf4_nearest_code<false>(x[i] / m[i]);
+  }
+  return bad;
+}
+"""
     )
     so = d / "host_math.so"
     subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-ffp-contract=off", str(src), "-o", str(so)], check=True)
@@ -132,6 +166,24 @@ def test_kernel_code_search_matches_oracle_fp32(host_math):
     got = torch.empty(s.numel(), dtype=torch.int32)
     host_math.codes_f32(ctypes.c_void_p(s.data_ptr()), s.numel(), ctypes.c_void_p(got.data_ptr()))
     assert torch.equal(got, want)
+
+
+def test_binned_code_search_equals_the_search_of_all_codes(host_math):
+    """The quantise kernels find a code by one table entry and one comparison.  bf16: every operand pair.  fp32: random
+    operands over the absmaxes the rule accepts, and elements within a few units of every edge."""
+    host_math.binned_bf16_mismatches.restype = ctypes.c_long
+    assert host_math.binned_bf16_mismatches() == 0
+    g = torch.Generator().manual_seed(0)
+    table = torch.tensor(nf4_oracle.NF4_TABLE)
+    n = 400000
+    m = torch.exp2(torch.rand(n, generator=g) * 127.9 - 63.95)
+    mids = ((table[1:] + table[:-1]) / 2)[torch.randint(15, (n,), generator=g)]
+    near = (mids * m).view(torch.int32) + torch.randint(-4, 5, (n,), generator=g, dtype=torch.int32)
+    x = torch.cat([(torch.rand(n, generator=g) * 2 - 1) * m, near.view(torch.float32), m, -m, m * 0, m * 1e-30])
+    m = m.repeat(6)
+    host_math.binned_f32_mismatches.restype = ctypes.c_long
+    bad = host_math.binned_f32_mismatches(ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(m.data_ptr()), ctypes.c_long(x.numel()))
+    assert bad == 0
 
 
 def test_kernel_block_scaler_matches_oracle(host_math):

@@ -9,6 +9,8 @@
 //   quantized_scalers i8 [numel/bs]       one per block of `bs` consecutive elements
 //   quantization_factor T [numel/bs/SB]   one per `SB` consecutive blocks
 //   scaler_mean      T   [1]
+#include <type_traits>
+
 #include "common.h"
 #include "nf4_math.h"
 
@@ -32,24 +34,6 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
 __device__ __forceinline__ float nanmax(float a, float b) { return (a != a) ? a : ((b != b) ? b : (a > b ? a : b)); }
 
 template <bool BF16>
-__device__ __forceinline__ void load8(const void* base, int64_t chunk, float v[8]) {
-  if constexpr (BF16) {
-    uint4 r = reinterpret_cast<const uint4*>(base)[chunk];
-    uint32_t d[4] = {r.x, r.y, r.z, r.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      v[2 * i] = bits_f32(d[i] << 16);
-      v[2 * i + 1] = bits_f32(d[i] & 0xffff0000u);
-    }
-  } else {
-    const float4* p = reinterpret_cast<const float4*>(base) + 2 * chunk;
-    float4 a = p[0], b = p[1];
-    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
-    v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-  }
-}
-
-template <bool BF16>
 __device__ __forceinline__ float load1(const void* base, int64_t i) {
   if constexpr (BF16)
     return bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(base)[i]);
@@ -66,149 +50,140 @@ __device__ __forceinline__ void store1(void* base, int64_t i, float v) {
 }
 
 // ---------------------------------------------------------------------------------------------------
-// quantise, pass 1: per-block absmax and the 4-bit codes.  One lane owns 8 consecutive elements (one
-// 128-bit load for bf16); a block of `bs` elements is spread over bs/8 neighbouring lanes of one wave.
-// ---------------------------------------------------------------------------------------------------
-template <bool BF16>
-__global__ __launch_bounds__(256) void nf4_quantize_blocks_kernel(const void* __restrict__ w, int64_t n_chunks,
-                                                                  int lanes_per_block, int log2_lpb,
-                                                                  uint32_t* __restrict__ qdata, float* __restrict__ absmax) {
-  const int64_t chunk = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const bool live = chunk < n_chunks;
-  float v[8];
-  if (live) {
-    load8<BF16>(w, chunk, v);
-  } else {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = 0.f;
-  }
-  float m = __builtin_fabsf(v[0]);
-#pragma unroll
-  for (int i = 1; i < 8; ++i) m = nanmax(m, __builtin_fabsf(v[i]));
-  for (int off = 1; off < lanes_per_block; off <<= 1) m = nanmax(m, __shfl_xor(m, off, kWave));
-  if (!live) return;
-  if ((threadIdx.x & (lanes_per_block - 1)) == 0) absmax[chunk >> log2_lpb] = m;
-  uint32_t packed = 0;
-#pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    int hi = nf4_nearest_code<BF16>(Arith<BF16>::rnd(v[2 * b] / m));
-    int lo = nf4_nearest_code<BF16>(Arith<BF16>::rnd(v[2 * b + 1] / m));
-    packed |= (uint32_t)((hi << 4) | lo) << (8 * b);
-  }
-  qdata[chunk] = packed;
-}
-
-// ---------------------------------------------------------------------------------------------------
-// quantise, pass 1 for bfloat16, the fast form of the kernel above (identical results).
+// quantise, pass 1: per-block absmax and the 4-bit codes.  One lane owns 8 consecutive elements (128 bits of bf16, twice
+// that of float); a block of `bs` elements is spread over bs/8 neighbouring lanes of one wave.
 //
-// (a) The scaled value bf16(x / absmax) is one of 65536 bit patterns, so "nearest code under the reference's rule"
-//     is a table lookup.  Every pattern with |value| < 2^-5 maps to code 7 (the zero code: its neighbours' midpoints
-//     are -0.0455 and +0.0398) and |value| <= 1 always, so the table only spans magnitudes 0x3D00 (2^-5) .. 0x3F80
-//     (1.0) for each sign: 2 x 641 bytes.  The host fills it once with nf4_nearest_code<true>, checks the two
-//     claims above over all patterns, and passes it by value; NaN (0/0 of an all-zero block) yields code 0.
-// (b) x / absmax for 64 elements shares the divisor: y = 1 / absmax is divided once (correctly rounded) and each
-//     quotient is q0 = x * y, r = fma(-q0, absmax, x), q = fma(r, y, q0).  For bf16 operands with absmax >= 2^-119
-//     and |x| <= absmax this rounds to the same bf16 as the correctly rounded quotient for EVERY operand pair
-//     (checked exhaustively on a CPU, 5.3e8 pairs); smaller or non-finite divisors take the plain division.
+// Vector-ALU bound when every element took a division and a search, so the work per element is what counts:
+// * the maximum is one of bit patterns without signs (a NaN is above every number, as torch.max has it), for bf16 two
+//   elements at a time, and for blocks of 64 travels between lanes as DPP operands instead of through the LDS;
+// * the block's elements share one reciprocal, and a code is one read of a 64-word table, whose entries lie in banks of
+//   their own, and one comparison (nf4_math.h says why that is exact);
+// * a thread's four chunks are all requested before the first is used.
+// 9 vector-ALU instructions per bf16 element (about 15 and a byte read from a 1.3 KB table before): 14336 x 4096 in bf16
+// takes 25 us = 6.0 TB/s, what a streaming copy reaches; quantising and dequantising it 101 -> 82 us.
+// An absmax outside the range where the shared reciprocal is exact (zero, denormal, huge, infinite, NaN) takes the
+// division and the search of the 16 codes.
 // ---------------------------------------------------------------------------------------------------
-constexpr int kCodeTabBase = 0x3D00;
-constexpr int kCodeTabLast = 0x3F80;
-constexpr int kCodeTabN = kCodeTabLast - kCodeTabBase + 1;  // 641
-constexpr int kCodeTabStride = 644;                          // per sign, padded to a multiple of 4
-struct Nf4CodeTable {
-  uint32_t words[2 * kCodeTabStride / 4];
-};
 constexpr int kQuantChunksPerThread = 4;
 
-__global__ __launch_bounds__(256) void nf4_quantize_blocks_bf16_kernel(const void* __restrict__ w, int64_t n_chunks,
-                                                                       int lanes_per_block, int log2_lpb,
-                                                                       uint32_t* __restrict__ qdata, float* __restrict__ absmax,
-                                                                       const Nf4CodeTable table) {
-  __shared__ uint32_t tab_words[2 * kCodeTabStride / 4];
-  for (int i = threadIdx.x; i < 2 * kCodeTabStride / 4; i += 256) tab_words[i] = table.words[i];
-  __syncthreads();
-  const uint8_t* tab = reinterpret_cast<const uint8_t*>(tab_words);
+typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
+
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_max(uint32_t m) {
+  const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, CTRL, 0xf, 0xf, true);
+  return m > o ? m : o;
+}
+
+// LPB: lanes per block, 0 = the argument (any power of two up to 64)
+template <bool BF16, int LPB>
+__global__ __launch_bounds__(256) void nf4_quantize_blocks_kernel(const u32x4_t* __restrict__ w, int64_t n_chunks, int lpb_arg,
+                                                                  int log2_lpb, uint32_t fast_low, uint32_t fast_high,
+                                                                  uint32_t* __restrict__ qdata, float* __restrict__ absmax,
+                                                                  const Nf4BinTable<BF16> table) {
+  constexpr int U = kQuantChunksPerThread;
+  constexpr int V = BF16 ? 1 : 2;  // 128-bit words per chunk
+  __shared__ uint32_t tab[Nf4BinTable<BF16>::kWords];
+  const int64_t chunk0 = (int64_t)blockIdx.x * (U * 256) + threadIdx.x;
+  u32x4_t raw[U][V];
 #pragma unroll
-  for (int u = 0; u < kQuantChunksPerThread; ++u) {
-    const int64_t chunk = ((int64_t)blockIdx.x * kQuantChunksPerThread + u) * 256 + threadIdx.x;
-    const bool live = chunk < n_chunks;  // uniform per block of lanes: n_chunks is a multiple of lanes_per_block
+  for (int u = 0; u < U; ++u) {
+    const int64_t chunk = chunk0 + u * 256;
+    const int64_t at = chunk < n_chunks ? chunk : n_chunks - 1;  // past the end: any valid chunk, not stored
+#pragma unroll
+    for (int h = 0; h < V; ++h) raw[u][h] = w[V * at + h];
+  }
+  if (threadIdx.x < Nf4BinTable<BF16>::kWords) tab[threadIdx.x] = table.words[threadIdx.x];
+  __syncthreads();
+  const int lpb = LPB ? LPB : lpb_arg;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int64_t chunk = chunk0 + u * 256;
+    uint32_t m_bits;
+    if constexpr (BF16) {
+      u16x2_t mm = __builtin_bit_cast(u16x2_t, raw[u][0][0] & 0x7fff7fffu);
+#pragma unroll
+      for (int i = 1; i < 4; ++i) mm = __builtin_elementwise_max(mm, __builtin_bit_cast(u16x2_t, raw[u][0][i] & 0x7fff7fffu));
+      const uint32_t lo = mm[0], hi = mm[1];
+      m_bits = (lo > hi ? lo : hi) << 16;
+    } else {
+      m_bits = 0;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const uint32_t a = raw[u][(i >> 2) * (V - 1)][i & 3] & 0x7fffffffu;
+        m_bits = m_bits > a ? m_bits : a;
+      }
+    }
+    if constexpr (LPB == 8) {
+      m_bits = dpp_max<0xb1>(m_bits);   // quad_perm [1, 0, 3, 2]
+      m_bits = dpp_max<0x4e>(m_bits);   // quad_perm [2, 3, 0, 1]
+      m_bits = dpp_max<0x141>(m_bits);  // row_half_mirror: the other four lanes
+    } else {
+      for (int off = 1; off < lpb; off <<= 1) {
+        const uint32_t o = (uint32_t)__shfl_xor((int)m_bits, off, kWave);
+        m_bits = m_bits > o ? m_bits : o;
+      }
+    }
+    if (chunk >= n_chunks) continue;  // a whole block of lanes: n_chunks is a multiple of lpb
+    const float m = bits_f32(m_bits);
+    if ((threadIdx.x & (lpb - 1)) == 0) absmax[chunk >> log2_lpb] = m;
     float v[8];
-    if (live) {
-      load8<true>(w, chunk, v);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if constexpr (BF16)
+        v[i] = bits_f32((i & 1) ? raw[u][0][i >> 1] & 0xffff0000u : raw[u][0][i >> 1] << 16);
+      else
+        v[i] = bits_f32(raw[u][(i >> 2) * (V - 1)][i & 3]);
+    }
+    uint32_t packed = 0;
+    if (m_bits >= fast_low && m_bits < fast_high) {
+      const float y = BF16 ? __builtin_amdgcn_rcpf(m) : 1.0f / m;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float t = BF16 ? v[i] * y : nf4_shared_quotient(v[i], m, y);
+        const uint32_t* entry = reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(tab) + nf4_bin_offset(t));
+        uint32_t code;
+        if constexpr (BF16)
+          code = nf4_code_below(entry[0]) + (nf4_above_edge_bf16(t, entry[0]) ? 1u : 0u);
+        else
+          code = entry[kNf4Bins] + (t >= bits_f32(entry[0]) ? 1u : 0u);
+        packed |= code << (8 * (i >> 1) + ((i & 1) ? 0 : 4));
+      }
     } else {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = 0.f;
-    }
-    float m = __builtin_fabsf(v[0]);
-#pragma unroll
-    for (int i = 1; i < 8; ++i) m = nanmax(m, __builtin_fabsf(v[i]));
-    for (int off = 1; off < lanes_per_block; off <<= 1) m = nanmax(m, __shfl_xor(m, off, kWave));
-    if (!live) continue;
-    if ((threadIdx.x & (lanes_per_block - 1)) == 0) absmax[chunk >> log2_lpb] = m;
-    const bool fast = m >= 0x1p-119f && m < __builtin_inff();  // false for NaN too
-    const float y = 1.0f / m;
-    uint32_t packed = 0;
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      float qf[2];
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const float x = v[2 * b + e];
-        if (fast) {
-          const float q0 = x * y;
-          const float r = __builtin_fmaf(-q0, m, x);
-          qf[e] = __builtin_fmaf(r, y, q0);
-        } else {
-          qf[e] = x / m;
-        }
-      }
-      const uint32_t pr = pack_bf16x2(qf[0], qf[1]);  // low half: element 2b (high nibble), high half: element 2b+1
-      uint32_t code[2];
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const uint32_t bits = e ? (pr >> 16) : (pr & 0xffffu);
-        const uint32_t mag = bits & 0x7fffu;
-        uint32_t idx = mag > (uint32_t)kCodeTabBase ? mag - kCodeTabBase : 0u;
-        idx = idx < (uint32_t)(kCodeTabN - 1) ? idx : (uint32_t)(kCodeTabN - 1);
-        idx += (bits >> 15) * kCodeTabStride;
-        const uint32_t c = tab[idx];
-        code[e] = mag > 0x7f80u ? 0u : c;
-      }
-      packed |= ((code[0] << 4) | code[1]) << (8 * b);
+      for (int i = 0; i < 8; ++i)
+        packed |= (uint32_t)nf4_nearest_code<BF16>(Arith<BF16>::rnd(v[i] / m)) << (8 * (i >> 1) + ((i & 1) ? 0 : 4));
     }
     qdata[chunk] = packed;
   }
 }
 
-// Host side of (a): the table, filled and verified once per process.
-struct Nf4CodeTableHost {
-  Nf4CodeTable table;
+// The table, filled and verified once per process.
+template <bool BF16>
+struct Nf4BinTableHost {
+  Nf4BinTable<BF16> table;
   bool ok;
-  Nf4CodeTableHost() : ok(true) {
-    uint8_t* bytes = reinterpret_cast<uint8_t*>(table.words);
-    memset(table.words, 0, sizeof(table.words));
-    for (int sign = 0; sign < 2; ++sign) {
-      for (int mag = 0; mag <= kCodeTabLast; ++mag) {
-        const uint16_t bits = (uint16_t)((sign << 15) | mag);
-        const int c = nf4_nearest_code<true>(bf16_bits_to_f32(bits));
-        if (mag < kCodeTabBase) {
-          if (c != 7) ok = false;  // claim: everything below 2^-5 is the zero code
-        } else {
-          bytes[sign * kCodeTabStride + (mag - kCodeTabBase)] = (uint8_t)c;
-        }
-      }
-    }
-    if (nf4_nearest_code<true>(bf16_bits_to_f32(0x7fc0)) != 0) ok = false;  // NaN -> code 0
-  }
+  Nf4BinTableHost() { ok = nf4_fill_bins<BF16>(table); }
 };
-const Nf4CodeTableHost& code_table() {
-  static const Nf4CodeTableHost t;
-  return t;
+
+template <bool BF16>
+void launch_quantize_blocks(const void* w, int64_t n_chunks, int lpb, int log2_lpb, uint8_t* qdata, float* absmax, hipStream_t s) {
+  static const Nf4BinTableHost<BF16> host;
+  const uint32_t low = host.ok ? Nf4FastRange<BF16>::low : 0u, high = host.ok ? Nf4FastRange<BF16>::high : 0u;
+  const int64_t per_wg = 256 * kQuantChunksPerThread;
+  const dim3 grid((unsigned)((n_chunks + per_wg - 1) / per_wg));
+  auto launch = [&](auto kernel) {
+    kernel<<<grid, dim3(256), 0, s>>>(reinterpret_cast<const u32x4_t*>(w), n_chunks, lpb, log2_lpb, low, high,
+                                      reinterpret_cast<uint32_t*>(qdata), absmax, host.table);
+  };
+  if (lpb == 8)
+    launch(nf4_quantize_blocks_kernel<BF16, 8>);
+  else
+    launch(nf4_quantize_blocks_kernel<BF16, 0>);
 }
 
 // ---------------------------------------------------------------------------------------------------
 // quantise, pass 2: mean of the block absmaxes.  Summed in fp64 in a fixed order (256 partial sums, each
-// a fixed strided walk followed by a fixed LDS tree) so the result does not depend on scheduling; for
+// a fixed strided walk followed by a fixed LDS tree, added by pass 3) so the result does not depend on scheduling; for
 // realistic dynamic ranges the fp64 sum is exact.  mean = dtype(float(sum / n)).
 // ---------------------------------------------------------------------------------------------------
 constexpr int kMeanPartials = 256;
@@ -233,29 +208,21 @@ __global__ __launch_bounds__(256) void nf4_absmax_partial_sum_kernel(const float
   if (threadIdx.x == 0) partial[blockIdx.x] = s;
 }
 
-template <bool BF16>
-__global__ __launch_bounds__(256) void nf4_absmax_mean_kernel(const double* __restrict__ partial, int64_t n_blocks,
-                                                              void* __restrict__ scaler_mean, float* __restrict__ mean_f32) {
-  __shared__ double sh[256];
-  double s = block_sum_256(partial[threadIdx.x], sh);
-  if (threadIdx.x == 0) {
-    float mean = Arith<BF16>::rnd((float)(s / (double)n_blocks));
-    store1<BF16>(scaler_mean, 0, mean);
-    *mean_f32 = mean;
-  }
-}
-
 // ---------------------------------------------------------------------------------------------------
-// quantise, pass 3: double quantisation of the block scalers.  One wave per scaler block of SB blocks.
+// quantise, pass 3: double quantisation of the block scalers.  One wave per scaler block of SB blocks.  Every workgroup
+// finishes the mean for itself (256 partial sums in the same order: the same bits), which saves a launch of one workgroup.
 // ---------------------------------------------------------------------------------------------------
 template <bool BF16>
 __global__ __launch_bounds__(256) void nf4_quantize_scalers_kernel(const float* __restrict__ absmax,
-                                                                   const float* __restrict__ mean_f32, int64_t n_sb, int SB,
-                                                                   int8_t* __restrict__ qscalers, void* __restrict__ qfactor) {
+                                                                   const double* __restrict__ partial, int64_t n_blocks,
+                                                                   int64_t n_sb, int SB, int8_t* __restrict__ qscalers,
+                                                                   void* __restrict__ qfactor, void* __restrict__ scaler_mean) {
+  __shared__ double sh[256];
+  const float mean = Arith<BF16>::rnd((float)(block_sum_256(partial[threadIdx.x], sh) / (double)n_blocks));
+  if (blockIdx.x == 0 && threadIdx.x == 0) store1<BF16>(scaler_mean, 0, mean);
   const int64_t sb = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (sb >= n_sb) return;  // whole wave leaves together
   const int lane = threadIdx.x & 63;
-  const float mean = *mean_f32;
   const float* a = absmax + sb * SB;
   float m = 0.f;
   for (int i = lane; i < SB; i += kWave) m = nanmax(m, __builtin_fabsf(Arith<BF16>::rnd(a[i] - mean)));
@@ -353,7 +320,6 @@ int log2_exact(int64_t v) {
 struct QuantWorkspace {
   float* absmax;    // [n_blocks]
   double* partial;  // [kMeanPartials]
-  float* mean;      // [1]
 };
 
 size_t quant_ws_bytes(int64_t n_blocks) {
@@ -402,7 +368,6 @@ extern "C" int ttamd_nf4_quantize(const void* w, int dtype, int64_t numel, int b
   ws.absmax = reinterpret_cast<float*>(workspace);
   size_t absmax_bytes = ((size_t)n_blocks * sizeof(float) + 255) & ~size_t(255);
   ws.partial = reinterpret_cast<double*>(reinterpret_cast<char*>(workspace) + absmax_bytes);
-  ws.mean = reinterpret_cast<float*>(ws.partial + kMeanPartials);
 
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const int64_t n_chunks = numel / 8;
@@ -410,28 +375,17 @@ extern "C" int ttamd_nf4_quantize(const void* w, int dtype, int64_t numel, int b
   const int64_t grid1 = (n_chunks + 255) / 256;
   TT_REQUIRE(grid1 < (int64_t(1) << 31), "nf4_quantize: tensor too large for one launch");
   const int64_t grid3 = (n_sb + 3) / 4;
-  if (dtype == TTAMD_BF16) {
-    const Nf4CodeTableHost& ct = code_table();
-    if (ct.ok) {
-      const int64_t per_wg = 256 * kQuantChunksPerThread;
-      nf4_quantize_blocks_bf16_kernel<<<dim3((unsigned)((n_chunks + per_wg - 1) / per_wg)), dim3(256), 0, s>>>(
-          w, n_chunks, lpb, log2_exact(lpb), reinterpret_cast<uint32_t*>(quantized_data), ws.absmax, ct.table);
-    } else {  // the table's premises failed their check: search the 16 codes directly
-      nf4_quantize_blocks_kernel<true><<<dim3((unsigned)grid1), dim3(256), 0, s>>>(
-          w, n_chunks, lpb, log2_exact(lpb), reinterpret_cast<uint32_t*>(quantized_data), ws.absmax);
-    }
+  auto run = [&](auto bf16) {
+    constexpr bool BF16 = decltype(bf16)::value;
+    launch_quantize_blocks<BF16>(w, n_chunks, lpb, log2_exact(lpb), quantized_data, ws.absmax, s);
     nf4_absmax_partial_sum_kernel<<<dim3(kMeanPartials), dim3(256), 0, s>>>(ws.absmax, n_blocks, ws.partial);
-    nf4_absmax_mean_kernel<true><<<dim3(1), dim3(256), 0, s>>>(ws.partial, n_blocks, scaler_mean, ws.mean);
-    nf4_quantize_scalers_kernel<true><<<dim3((unsigned)grid3), dim3(256), 0, s>>>(
-        ws.absmax, ws.mean, n_sb, scaler_block_size, quantized_scalers, quantization_factor);
-  } else {
-    nf4_quantize_blocks_kernel<false><<<dim3((unsigned)grid1), dim3(256), 0, s>>>(
-        w, n_chunks, lpb, log2_exact(lpb), reinterpret_cast<uint32_t*>(quantized_data), ws.absmax);
-    nf4_absmax_partial_sum_kernel<<<dim3(kMeanPartials), dim3(256), 0, s>>>(ws.absmax, n_blocks, ws.partial);
-    nf4_absmax_mean_kernel<false><<<dim3(1), dim3(256), 0, s>>>(ws.partial, n_blocks, scaler_mean, ws.mean);
-    nf4_quantize_scalers_kernel<false><<<dim3((unsigned)grid3), dim3(256), 0, s>>>(
-        ws.absmax, ws.mean, n_sb, scaler_block_size, quantized_scalers, quantization_factor);
-  }
+    nf4_quantize_scalers_kernel<BF16><<<dim3((unsigned)grid3), dim3(256), 0, s>>>(
+        ws.absmax, ws.partial, n_blocks, n_sb, scaler_block_size, quantized_scalers, quantization_factor, scaler_mean);
+  };
+  if (dtype == TTAMD_BF16)
+    run(std::true_type{});
+  else
+    run(std::false_type{});
   return check_launch("nf4_quantize");
 }
 
