@@ -17,7 +17,7 @@ import pytest
 import torch
 
 from oracle import lora_oracle, nf4_oracle
-from torchtune_amd import ops
+from torchtune_amd import _lib, ops
 from torchtune_amd.modules import layer_ops
 from torchtune_amd.modules.peft import LoRALinear, group_applies, lora_feed_forward, lora_linear_group, lora_swiglu_group
 from torchtune_amd.nf4_tensor import to_nf4
@@ -567,3 +567,41 @@ def test_grouped_launches_of_few_tiles(M, K, Ns, bias):
         dx = dx + gy.float() @ w + gh[:, off:off + r].float() @ m.lora_a.float()
         off += r
     torch.testing.assert_close(gx.float(), dx, rtol=2 ** -8, atol=2e-5 * dx.abs().max().item())
+
+
+@pytest.mark.parametrize("M,widths,expands", [(1281, (14336, 14336), True), (1500, (14336, 14336), True), (1536, (14336, 14336), True),
+                                              (2047, (14336, 14336), True), (1301, (8192, 8192, 1024), True), (1601, (8192, 1024, 1024), False), (1500, (14336,), False),
+                                              (1793, (14336,), True), (1000, (14336,), False), (600, (14336,), False)])
+def test_tiles_below_2048_tokens_are_chosen_by_their_rounds(M, widths, expands):
+    """Groups and single layers of a full round of output tiles and more: the expanded weight from 1280 tokens where its rounds cost
+    less, else 256- or 128-row tiles of the fused kernel; forward, gated product and grad-input.  bf16 results of fp32
+    sums, as above; the gated product rounds silu(gate) to bf16 once more."""
+    K, n = 256, len(widths)
+    mem = _members(K, widths, (8,) * n, seed=M)
+    members = [e[0] for e in mem]
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x = torch.randn(M, K, device=DEV, generator=g).to(BF)
+    if n > 1:
+        pair = n == 2
+        h_cat, ys = ops.lora_group_fwd(x, members, swiglu=pair, return_tiles=True)[:2]
+        lib = _lib.load()
+        need = lib.ttamd_lora_group_fwd_workspace_bytes(ops._group_array("t", members, K, list(ys[:n]), M)[0], n, M, K)
+        assert (need == 2 * K * sum(widths)) == expands
+        if pair:
+            want = torch.nn.functional.silu(ys[0].float()).to(BF).float() * ys[1].float()
+            torch.testing.assert_close(ys[2].float(), want, rtol=2 ** -7, atol=1e-6 * want.abs().max().item())
+    else:
+        m = members[0]
+        h_cat = ops.lora_hidden(x, m.lora_a)
+        ys = [ops.nf4_lora_linear_fwd(x, m.qdata, m.block_scalers, m.N, h_cat, m.lora_b, m.scale)]
+        assert bool(_lib.load().ttamd_nf4_gemm_expands_weight(M, m.N, K)) == expands
+    for i, (m, t, *_) in enumerate(mem):
+        h = (h_cat[:, 8 * i:8 * i + 8].float() * m.scale).to(BF).float()
+        want = x.float() @ t.get_original_weight().float().t() + h @ m.lora_b.float().t()
+        torch.testing.assert_close(ys[i].float(), want, rtol=2 ** -8, atol=2e-5 * want.abs().max().item())
+    if n == 1:  # the grad-input of a layer that is as wide on its other side
+        ((m, t, *_),) = _members(14336, (K,), (8,), seed=M)
+        gh = torch.randn(M, 8, device=DEV, generator=g).to(BF)
+        gx = ops.nf4_linear_bwd_dx(x, m.qdata, m.block_scalers, 14336, gh, m.lora_a, transposed=m.transposed)
+        want = x.float() @ t.get_original_weight().float() + gh.float() @ m.lora_a.float()
+        torch.testing.assert_close(gx.float(), want, rtol=2 ** -8, atol=2e-5 * want.abs().max().item())

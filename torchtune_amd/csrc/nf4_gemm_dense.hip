@@ -1194,8 +1194,9 @@ int launch_dense(DenseArgs& g, hipStream_t s) {
 
 // When the expand-once path is taken, from its 256 x 256 output tiles against the 256 CUs (measured against the fused
 // kernel, whose tiles have 128 rows, on 8B / 70B shapes):
-//   * at least a full round of tiles and 2048 tokens: always (below 2048 tokens the expansion, which costs as much as
-//     the GEMM of ~360 tokens, and the second round eat the gain);
+//   * at least a full round of tiles and 2048 tokens: always;
+//   * at least a full round and 1280 - 2047 tokens: where its rounds and the expansion cost less than the rounds of the
+//     fused kernel (part_filled_rounds_pay; a group's members are fused launches of their own);
 //   * between half a round and a full one, from 1280 tokens: the fused kernel needs a second round of its tiles there
 //     (+ 60 %), one partly filled round of this kernel is 15 - 30 % faster;
 //   * up to half a round the fused kernel fills the chip in one round of its own and wins.
@@ -1205,11 +1206,39 @@ bool dense_tiles_apply(int64_t M, int64_t tiles) {
   return (M >= kDenseMinRows && tiles >= 256) || (M >= kDenseMinRowsPartRound && tiles > 128 && tiles < 256);
 }
 
-bool dense_path_applies(int64_t M, int64_t Nout, int64_t Kc) {
+int64_t rounds_of(int64_t M, int64_t rows, int64_t Nout) { return (((M + rows - 1) / rows) * ((Nout + 255) / 256) + 255) / 256; }
+
+// 1280 - 2047 tokens and a full round or more.  Costs in us of a round of tiles on the 256 CUs at 4096 contraction steps (all
+// of them, the expansion too, grow with the contraction): 88 here and 0.47 per 256 expanded rows, 64 for the fused
+// kernel's 128-row tiles (up to half a round is cut into slices that fill one, and a sum), 105 for its 256-row ones.
+// The gate / up pair of 14336 x 4096 at 1500 tokens takes 3 rounds here and 2 x 3 of the smaller tiles (its layer forward +
+// backward 1743 -> 1668 us); alone at that size 2 rounds and the expansion are no faster than 3 small ones, from 1665
+// tokens (4 small ones or 2 full) they are: 1900 tokens 217 -> 196 us.
+bool part_filled_rounds_pay(int64_t M, const int64_t* N, int n) {
+  if (M < kDenseMinRowsPartRound || M >= kDenseMinRows) return false;
+  int64_t n_total = 0;
+  double fused = 0;
+  for (int i = 0; i < n; ++i) {
+    n_total += N[i];
+    const int64_t tiles = ((M + 127) / 128) * ((N[i] + 255) / 256);
+    const double small = tiles <= 128 ? 0.25 * (double)tiles + 8.0 : 64.0 * (double)rounds_of(M, 128, N[i]);
+    const double full = 105.0 * (double)rounds_of(M, 256, N[i]);
+    fused += small < full ? small : full;
+  }
+  if (((M + 255) / 256) * ((n_total + 255) / 256) < 256) return false;
+  const double dense = 88.0 * (double)rounds_of(M, 256, n_total) + 0.47 * (double)((n_total + 255) / 256);
+  return dense * 1.03 < fused;
+}
+
+bool dense_shape_served(int64_t M, int64_t Nout, int64_t Kc) {
   if (Nout % 64 != 0 || Kc % 64 != 0) return false;
-  if (!dense_tiles_apply(M, ((M + 255) / 256) * ((Nout + 255) / 256))) return false;
   // per-lane byte offsets inside the kernel are 32-bit
   return M * Kc * 2 < (int64_t(1) << 32) && Kc * 2 * 256 < (int64_t(1) << 32);
+}
+
+bool dense_path_applies(int64_t M, int64_t Nout, int64_t Kc) {
+  if (!dense_tiles_apply(M, ((M + 255) / 256) * ((Nout + 255) / 256)) && !part_filled_rounds_pay(M, &Nout, 1)) return false;
+  return dense_shape_served(M, Nout, Kc);
 }
 
 size_t dense_workspace_bytes(int64_t M, int64_t Nout, int64_t Kc) {
@@ -1263,7 +1292,8 @@ size_t dense_group_fwd_workspace_bytes(const GroupGemm& d) {
     if (d.N[i] % 256 != 0) return 0;  // a tile belongs to one member
     n_total += d.N[i];
   }
-  return d.n >= 2 && dense_path_applies(d.M, n_total, d.K) ? (size_t)n_total * (size_t)d.K * 2 : 0;
+  const bool pays = dense_tiles_apply(d.M, ((d.M + 255) / 256) * (n_total / 256)) || part_filled_rounds_pay(d.M, d.N, d.n);
+  return d.n >= 2 && pays && dense_shape_served(d.M, n_total, d.K) ? (size_t)n_total * (size_t)d.K * 2 : 0;
 }
 
 bool dense_group_gated_applies(const GroupGemm& d) {

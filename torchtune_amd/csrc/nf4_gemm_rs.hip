@@ -1365,6 +1365,14 @@ int choose_splits(int64_t M, int64_t Nout, int64_t Kc) {
   sp = sp < 16 ? sp : 16;
   return sp < 2 ? 1 : (int)sp;
 }
+// Whether a single layer's unsliced launch takes 256-row tiles: a round of them on the 256 CUs costs 1.8 rounds of 128-row
+// ones (4096 contraction steps: 105 us against 56 - 64).  256-row -> 128-row tiles: 14336 x 4096 at 1200 tokens 200 -> 183 us,
+// at 1500 202 -> 191, grad-input of 4096 x 14336 at 1400 237 -> 211; 128-row -> 256-row: 14336 x 4096 at 1000 136 -> 112.
+bool full_tiles_pay(int64_t M, int64_t Nout) {
+  const int64_t tiles_n = (Nout + kBN - 1) / kBN;
+  const int64_t rounds256 = (((M + 255) / 256) * tiles_n + 255) / 256, rounds128 = (((M + 127) / 128) * tiles_n + 255) / 256;
+  return rounds256 * 9 < rounds128 * 5;
+}
 // k-steps per slice, and the slices that then hold at least one
 void slice_steps(int64_t Kc, int splits, int& ksteps, int& used) {
   ksteps = (int)(((Kc >> 6) + splits - 1) / splits);
@@ -1428,8 +1436,7 @@ int run_gemm_rs(const void* X, const uint8_t* codes, const void* scal, int mode,
                          : launch_rs<128, 0, true>(g, used, s);
     return rc != TTAMD_OK ? rc : launch_reduce(g, used, s);
   }
-  const int64_t tiles256 = ((M + 255) / 256) * ((Nout + kBN - 1) / kBN);
-  const bool big = tiles256 >= 256;
+  const bool big = full_tiles_pay(M, Nout);
   if (mode == 1) return big ? launch_rs<256, 1, false>(g, 1, s) : launch_rs<128, 1, false>(g, 1, s);
   if (mode == 2) return big ? launch_rs<256, 2, false>(g, 1, s) : launch_rs<128, 2, false>(g, 1, s);
   return big ? launch_rs<256, 0, false>(g, 1, s) : launch_rs<128, 0, false>(g, 1, s);
