@@ -605,3 +605,33 @@ def test_tiles_below_2048_tokens_are_chosen_by_their_rounds(M, widths, expands):
         gx = ops.nf4_linear_bwd_dx(x, m.qdata, m.block_scalers, 14336, gh, m.lora_a, transposed=m.transposed)
         want = x.float() @ t.get_original_weight().float() + gh.float() @ m.lora_a.float()
         torch.testing.assert_close(gx.float(), want, rtol=2 ** -8, atol=2e-5 * want.abs().max().item())
+
+
+@pytest.mark.parametrize("M,n_out,widths", [(1100, 4096, (14336,)), (1153, 4096, (12288, 4096)), (1153, 4096, (14336, 14336)), (600, 8064, (20480,))])
+def test_slices_of_part_filled_rounds(M, n_out, widths):
+    """129 - 255 tiles of a long contraction, cut into slices whose workgroups fill their rounds: the grad-input of a group and
+    of a single layer, and its forward.  bf16 results of fp32 sums, as above (longer ones: 1e-4 of the largest)."""
+    n, kc = len(widths), sum(widths)
+    lib = _lib.load()
+    slices = lib.ttamd_nf4_gemm_workspace_bytes(M, n_out, kc) // (M * n_out * 4)
+    assert 2 <= slices <= 8 and not lib.ttamd_nf4_gemm_expands_weight(M, n_out, kc)
+    mem = _members(n_out, widths, (8,) * n, seed=M)
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x, h_cat = (torch.randn(M, w, device=DEV, generator=g).to(BF) for w in (n_out, 8 * n))
+    gys = [torch.randn(M, w, device=DEV, generator=g).to(BF) for w in widths]
+
+    def close(got, want):
+        torch.testing.assert_close(got.float(), want, rtol=2 ** -8, atol=1e-4 * want.abs().max().item())
+
+    want = 0
+    if n > 1:
+        gx, _, gh = ops.lora_group_bwd(x, h_cat, [e[0] for e in mem], gys)
+    else:
+        m, gh = mem[0][0], h_cat
+        gx = ops.nf4_linear_bwd_dx(gys[0], m.qdata, m.block_scalers, n_out, gh, m.lora_a, transposed=m.transposed)
+        ((f, t, *_),) = _members(kc, (n_out,), (8,), seed=M)
+        y = ops.nf4_lora_linear_fwd(gys[0], f.qdata, f.block_scalers, n_out, gh, f.lora_b, 1.0, block_scalers_t=f.transposed[1])
+        close(y, gys[0].float() @ t.get_original_weight().float().t() + gh.float() @ f.lora_b.float().t())
+    for i, ((m, t, *_), gy) in enumerate(zip(mem, gys)):
+        want = want + gy.float() @ t.get_original_weight().float() + gh[:, 8 * i:8 * i + 8].float() @ m.lora_a.float()
+    close(gx, want)

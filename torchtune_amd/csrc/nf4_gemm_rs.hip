@@ -1353,11 +1353,30 @@ int launch_rs(RsArgs& g, int splits, hipStream_t s, const std::conditional_t<MEM
   return check_launch("nf4_gemm_rs");
 }
 
+// Slices for a launch that fills half a round to a whole one: `sp` of them make sp * tiles workgroups of a sp-th of the
+// contraction, whose rounds may be fuller.  Costs in us: a round 64 at 4096 steps, the slabs' way out and back at 4 TB/s, the
+// sum's launch 6; a fuller chip clocks lower, so a sixth has to be gained.  144 tiles (the grad-input of an 8B layer's gate / up
+// pair and its down projection at 1100 tokens): 5 and 3 slices, the layer's forward + backward 1537 -> 1466 us; 192 tiles in 4
+// slices (13 % less by these costs) measured the same.
+int slices_of_a_part_filled_round(int64_t tiles, int64_t M, int64_t Nout, int64_t Kc) {
+  const double whole = 64.0 * (double)Kc / 4096.0;
+  double best = whole / 1.2;
+  int best_sp = 1;
+  for (int sp = 2; sp <= 8 && Kc / sp >= 1024; ++sp) {
+    const double cost = whole * (double)((tiles * sp + 255) / 256) / sp + 6.0 + (double)sp * (double)(M * Nout) * 8.0 / 4e6;
+    if (cost < best) {
+      best = cost;
+      best_sp = sp;
+    }
+  }
+  return best_sp;
+}
+
 // Slices of the contraction for a launch that would leave half of the chip or more idle: enough to reach about one
 // workgroup per CU, at least four k-steps (256 elements) each, at most 16.  1 = do not split.
 int choose_splits(int64_t M, int64_t Nout, int64_t Kc) {
   const int64_t tiles = ((M + 127) / 128) * ((Nout + kBN - 1) / kBN);  // small launches use 128-row tiles
-  if (tiles > 128) return 1;
+  if (tiles > 128) return tiles < 256 && !dense_path_applies(M, Nout, Kc) ? slices_of_a_part_filled_round(tiles, M, Nout, Kc) : 1;
   if (tiles > 64 && Kc < 4096) return 1;  // two slices of a short contraction: the reduction costs what the slicing gains
   int64_t sp = 256 / tiles;
   const int64_t by_k = (Kc / 64) / 4;
