@@ -5,7 +5,7 @@ import torch
 import torch.nn.functional as F
 
 from torchtune_amd import ops
-from torchtune_amd.qat import FakeQuantizeConfig, FakeQuantizedLinear
+from torchtune_amd.qat import FakeQuantizeConfig, FakeQuantizedLinear, FakeQuantizer
 
 pytestmark = pytest.mark.gpu
 
@@ -55,3 +55,42 @@ def test_second_derivative():
     # bf16 intermediates: a few roundings of 2^-8 each
     for got, want in ((x.grad, xr.grad), (layer.weight.grad, wq.grad)):
         assert float((got.float() - want).norm() / want.norm()) < 4 * 2.0 ** -8
+
+
+@pytest.mark.parametrize("how", ["hook", "pre_hook", "subclass", "replacement", "patched", "global"])
+def test_a_weight_quantizer_that_does_more_is_called(how):
+    layer = FakeQuantizedLinear(128, 256, False, None, FakeQuantizeConfig(torch.int4, group_size=32), device="cuda", dtype=torch.bfloat16)
+    x = torch.randn(16, 128, device="cuda").bfloat16()
+    assert layer._mid_ok(x)
+    want = F.linear(x, 2 * layer.weight_fake_quantizer(layer.weight))
+    q, handle = layer.weight_fake_quantizer, None
+
+    class Doubled(FakeQuantizer):
+        def forward(self, w):
+            return 2 * super().forward(w)
+
+    class Other(torch.nn.Module):
+        enabled, config = True, q.config
+
+        def forward(self, w):
+            return 2 * q(w)
+
+    if how == "hook":
+        q.register_forward_hook(lambda mod, args, out: 2 * out)
+    elif how == "pre_hook":
+        q.register_forward_pre_hook(lambda mod, args: (2 * args[0],))
+    elif how == "subclass":
+        layer.weight_fake_quantizer = Doubled(q.config)
+    elif how == "replacement":
+        layer.weight_fake_quantizer = Other()
+    elif how == "patched":
+        plain = q.forward
+        q.forward = lambda w: 2 * plain(w)
+    else:
+        handle = torch.nn.modules.module.register_module_forward_hook(lambda mod, args, out: 2 * out if mod is q else None)
+    try:
+        # doubling is exact: in the weight, or in the quantised weight
+        assert torch.equal(layer(x), want)
+    finally:
+        if handle is not None:
+            handle.remove()

@@ -450,6 +450,13 @@ def _group_tiled_ok(x: torch.Tensor, layers) -> bool:
             and ops.tiled_weight_shape_ok(n_total, K, first.weight_fake_quantizer.config.group_size))
 
 
+def _runs_as_written(q: nn.Module) -> bool:
+    """Calling the module ``q`` is ``FakeQuantizer.forward`` and nothing else: no other class, no hooks, no patched method."""
+    return (type(q) is FakeQuantizer and "forward" not in q.__dict__
+            and not (q._forward_hooks or q._forward_pre_hooks or q._backward_hooks or q._backward_pre_hooks)
+            and not nn.modules.module._has_any_global_hook())
+
+
 class FakeQuantizedLinear(nn.Linear):
     """``nn.Linear`` that fake-quantises its input and/or weight before the matmul."""
 
@@ -493,9 +500,12 @@ class FakeQuantizedLinear(nn.Linear):
 
     def _mid_ok(self, x: torch.Tensor) -> bool:
         """The products run on the library's 128 x 128-tile kernels (``ttamd_gemm_mid_bf16``) instead of the vendor library:
-        the sizes below ``_tiled_ok``'s where they take about as long on the GPU and the vendor calls' host time counts."""
+        the sizes below ``_tiled_ok``'s where they take about as long on the GPU and the vendor calls' host time counts.
+        The weight's fake quantizer is then read, not called, so one that does more when called keeps the dense product."""
         q, w, b = self.weight_fake_quantizer, self.weight, self.bias
-        if not TILED_GEMM or q is None or not q.enabled or not x.is_cuda or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not w.is_cuda:
+        if q is None or not _runs_as_written(q):
+            return False
+        if not TILED_GEMM or not q.enabled or not x.is_cuda or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not w.is_cuda:
             return False
         if torch.is_autocast_enabled("cuda") or not _host.load().ordinary(x):
             return False
