@@ -2,8 +2,9 @@
 import pytest
 import torch
 import torch.autograd.forward_ad as fwAD
+from torch.utils.flop_counter import FlopCounterMode
 
-from torchtune_amd import Int4WeightOnlyQATQuantizer, _host, ops
+from torchtune_amd import Int4WeightOnlyQATQuantizer, Int8DynActInt4WeightQATQuantizer, _host, ops
 from torchtune_amd.modules.peft import LoRALinear, lora_linear_group, lora_swiglu_group
 
 pytestmark = pytest.mark.gpu
@@ -140,6 +141,20 @@ def test_products_that_replace_torchs_keep_its_views_and_transforms(converted):
     torch.testing.assert_close(tangent.float(), want, **near)
     if converted:
         torch.testing.assert_close(torch.func.vmap(model)(x.view(2, 3, 256)).float(), want.view(2, 3, 512), **near)
+
+
+@pytest.mark.parametrize("form", ["qat", "8da4w", "4w"])
+def test_products_that_replace_torchs_are_seen_by_a_dispatch_mode(form):
+    quantizer = (Int4WeightOnlyQATQuantizer(groupsize=32) if form == "4w" else Int8DynActInt4WeightQATQuantizer(groupsize=32, precision=BF))
+    model = quantizer.prepare(torch.nn.Sequential(torch.nn.Linear(256, 512, bias=False, device=DEV, dtype=BF)))
+    if form != "qat":
+        model = quantizer.convert(model)
+    x = torch.randn(5, 256, device=DEV).to(BF)
+    want = model(x)
+    with FlopCounterMode(display=False) as counter:
+        got = model(x)
+    assert counter.get_total_flops() == 2 * 5 * 256 * 512
+    torch.testing.assert_close(got.float(), want.float(), rtol=2 ** -7, atol=2 ** -7)  # as above: another order of the sums
 
 
 def test_an_empty_last_dimension_is_an_error():

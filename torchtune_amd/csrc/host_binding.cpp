@@ -11,6 +11,7 @@
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <pybind11/stl.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/utils/pybind.h>
@@ -59,8 +60,10 @@ bool wants_grad(std::initializer_list<const Tensor*> ts) {
 }
 
 // A tensor the kernels may read in place of torch's own ops: no forward-mode tangent, no function transform's wrapper, no
-// subclass with a dispatch of its own.
+// subclass with a dispatch of its own, and no dispatch mode that would have seen those ops (a FLOP counter, a selective
+// checkpoint's list of what to save).
 bool ordinary(const Tensor& t) {
+  if (c10::impl::TorchDispatchModeTLS::any_modes_set()) return false;
   constexpr c10::DispatchKeySet wrapped({c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
                                          c10::DispatchKey::Functionalize, c10::DispatchKey::Python});
   return !t.key_set().has_any(wrapped) && !t._fw_grad(0).defined();
