@@ -5,7 +5,7 @@ import torch.autograd.forward_ad as fwAD
 from torch.utils.flop_counter import FlopCounterMode
 
 from torchtune_amd import Int4WeightOnlyQATQuantizer, Int8DynActInt4WeightQATQuantizer, _host, ops
-from torchtune_amd.modules.peft import LoRALinear, lora_linear_group, lora_swiglu_group
+from torchtune_amd.modules.peft import LoRALinear, group, lora_linear_group, lora_swiglu_group
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -58,6 +58,30 @@ def test_native_path_equals_the_python_nodes_bitwise(tokens, kind, bias, x_grad,
     for a, b in zip(got, want):
         assert a.shape == b.shape and torch.equal(a.view(torch.int16), b.view(torch.int16))
     for a, b in zip(plain if isinstance(plain, tuple) else [plain], want):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+@pytest.mark.parametrize("bias", [False, True])
+def test_the_gated_pairs_backward_follows_its_switch(bias, monkeypatch):
+    """Fused or in two steps, as ``group.FUSED_SWIGLU_BWD`` says; the same bits."""
+    layers = _layers([512, 512], 256, bias)
+    g = torch.Generator(device=DEV).manual_seed(1)
+    x = torch.randn(1, 33, 256, device=DEV, generator=g).to(BF)
+    gys = [torch.randn(1, 33, 512, device=DEV, generator=g).to(BF)]
+    native, asked, runs = _host.load(), [], []
+
+    class Recorder:
+        @staticmethod
+        def lora_group(*args):
+            asked.append(args[-1])
+            return native.lora_group(*args)
+
+    monkeypatch.setattr(group._host, "load", lambda: Recorder)
+    for fused in (True, False):
+        monkeypatch.setattr(group, "FUSED_SWIGLU_BWD", fused)
+        runs.append(_run(lambda t: lora_swiglu_group(t, *layers), layers, x, gys, True))
+    assert asked == [True, False]
+    for a, b in zip(*runs):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16))
 
 

@@ -468,6 +468,7 @@ GroupOut group_forward(const Tensor& x, std::vector<Member>& ms, bool gated, boo
 struct GroupSpec {
   std::vector<Member> ms;
   bool gated = false;
+  bool fused_swiglu_bwd = true;  // gated: the gradients of gate and up come out of the adapters' backward, not of a launch before it
 };
 
 // Differentiable inputs: x, then per member lora_a, lora_b and, where there is one, the bias.
@@ -497,6 +498,7 @@ struct QLoRAGroupFn : torch::autograd::Function<QLoRAGroupFn> {
     ctx->saved_data["bias"] = bias;
     ctx->saved_data["scales"] = scales;
     ctx->saved_data["gated"] = spec.gated;
+    ctx->saved_data["fused_swiglu_bwd"] = spec.fused_swiglu_bwd;
     ctx->saved_data["shape"] = x.sizes().vec();
     if (spec.gated) return {o.act};
     return o.ys;
@@ -518,7 +520,7 @@ struct QLoRAGroupFn : torch::autograd::Function<QLoRAGroupFn> {
     ttamd_lora_group_member arr[TTAMD_GROUP_MAX];
     bool any_bias = false;
     for (int i = 0; i < n; ++i) any_bias = any_bias || bias[i];
-    const bool fused_swiglu = gated && !any_bias;  // the gradients of gate and up come out of the adapters' backward
+    const bool fused_swiglu = gated && !any_bias && ctx->saved_data["fused_swiglu_bwd"].toBool();
     if (gated && !fused_swiglu) {
       auto [gg, gu] = swiglu_backward(g[0], saved[2 + 2 * n], saved[3 + 2 * n]);
       gys = {gg, gu};
@@ -578,9 +580,10 @@ struct QLoRAGroupFn : torch::autograd::Function<QLoRAGroupFn> {
 // members: (weight, q, scal, q_t | None, scal_t | None, N, lora_a, lora_b, scale, bias | None) each
 using MemberTuple = std::tuple<Tensor, Tensor, Tensor, std::optional<Tensor>, std::optional<Tensor>, int64_t, Tensor, Tensor, double, std::optional<Tensor>>;
 
-std::vector<Tensor> lora_group(const Tensor& x, const std::vector<MemberTuple>& members, bool gated) {
+std::vector<Tensor> lora_group(const Tensor& x, const std::vector<MemberTuple>& members, bool gated, bool fused_swiglu_bwd) {
   GroupSpec spec;
   spec.gated = gated;
+  spec.fused_swiglu_bwd = fused_swiglu_bwd;
   std::vector<Tensor> adapters;
   bool grad = wants_grad({&x});
   for (const auto& t : members) {

@@ -225,7 +225,7 @@ def _native_group(x: torch.Tensor, layers, gated: bool):
     for layer in layers:
         w, lora_a, lora_b, bias = layer._fused_operands()
         members.append((*host_weight(w, tokens, grad), lora_a, lora_b, layer.alpha / layer.rank, bias))
-    return _host.load().lora_group(x, members, gated)
+    return _host.load().lora_group(x, members, gated, FUSED_SWIGLU_BWD)
 
 
 def lora_swiglu_group(x: torch.Tensor, gate: torch.nn.Module, up: torch.nn.Module):
