@@ -398,6 +398,23 @@ def test_feed_forward_node_matches_gated_pair_then_down(M, K, width):
     assert lora_feed_forward(x, pair[0], pair[1], narrow) is None
 
 
+def test_the_grouped_grad_input_keeps_its_slices_without_the_expanded_path(monkeypatch):
+    """``ops.EXPANDED_WEIGHT_PATH`` decides about weights expanded per call, not about the slices of a launch of few tiles:
+    where nothing is expanded it changes no bit."""
+    layers, _ = _layers(512, (1024, 1024), (16, 16), 32.0, False, seed=3)
+    g = torch.Generator().manual_seed(8)
+    x = torch.randn(1300, 512, generator=g).to(BF).to(DEV)
+    gys = [torch.randn(1300, 1024, generator=g).to(BF).to(DEV) for _ in range(2)]
+    assert not ops.native_call(1300) and not ops.group_dx_expands(1300, 512, [1024, 1024])
+    grads = []
+    for expanded in (True, False):
+        monkeypatch.setattr(ops, "EXPANDED_WEIGHT_PATH", expanded)
+        xg = x.clone().requires_grad_()
+        torch.autograd.backward(lora_linear_group(xg, layers), gys)
+        grads.append(xg.grad)
+    assert torch.equal(grads[0].view(torch.int16), grads[1].view(torch.int16))
+
+
 def test_group_falls_back_when_it_does_not_apply():
     layers, _ = _layers(512, (256, 128), (16, 16), 32.0, False, seed=1)
     x = torch.randn(4, 512, device=DEV, dtype=BF)

@@ -719,7 +719,10 @@ def lora_group_bwd(x: torch.Tensor, h_cat: torch.Tensor, members: Sequence[Group
                 rc = lib.ttamd_nf4_group_bwd_dx_tiles_bf16(arr, n, gh_cat.data_ptr(), gx.data_ptr(), M, K, tiles.data_ptr(),
                                                            1 if paired else 0, _stream(x))
             else:
-                dx_bytes = int(lib.ttamd_nf4_group_bwd_dx_workspace_bytes(arr, n, M, K)) if EXPANDED_WEIGHT_PATH else 0
+                # the expanded weights or, where the library does not expand them, the slices of a launch of few tiles
+                dx_bytes = int(lib.ttamd_nf4_group_bwd_dx_workspace_bytes(arr, n, M, K))
+                if not EXPANDED_WEIGHT_PATH and lib.ttamd_nf4_gemm_expands_weight(M, K, sum(m.N for m in members)):
+                    dx_bytes = 0  # less than the library asks for: it keeps the fused kernel
                 dx_ws = torch.empty(dx_bytes // 4, dtype=torch.float32, device=dev) if dx_bytes else None
                 if events:
                     events[0].record()
