@@ -415,6 +415,20 @@ def test_the_grouped_grad_input_keeps_its_slices_without_the_expanded_path(monke
     assert torch.equal(grads[0].view(torch.int16), grads[1].view(torch.int16))
 
 
+def test_a_group_that_alone_expands_follows_the_switch(monkeypatch):
+    """1500 tokens of a 14336-wide pair: worth expanding together, not one by one."""
+    members = [m[0] for m in _members(256, (14336, 14336), (8, 8), seed=4)]
+    x = torch.randn(1500, 256, generator=torch.Generator().manual_seed(9)).to(BF).to(DEV)
+    assert not ops.gemm_expands_weight(1500, 14336, 256)
+    with_tiles = ops.lora_group_fwd(x, members, return_tiles=True)
+    assert with_tiles[2] is not None
+    monkeypatch.setattr(ops, "EXPANDED_WEIGHT_PATH", False)
+    without = ops.lora_group_fwd(x, members, return_tiles=True)
+    assert without[2] is None
+    for a, b in zip(with_tiles[1], without[1]):
+        torch.testing.assert_close(a.float(), b.float(), rtol=1e-2, atol=2e-3)  # as for a single layer: another order of the sums
+
+
 def test_group_falls_back_when_it_does_not_apply():
     layers, _ = _layers(512, (256, 128), (16, 16), 32.0, False, seed=1)
     x = torch.randn(4, 512, device=DEV, dtype=BF)

@@ -626,7 +626,9 @@ def lora_group_fwd(x: torch.Tensor, members: Sequence[GroupMember], swiglu: bool
     h_cat = torch.empty(M, r_total, dtype=torch.bfloat16, device=dev)
     lib = _lib.load()
     fwd_bytes = lib.ttamd_lora_group_fwd_workspace_bytes(arr, n, M, K)
-    if not EXPANDED_WEIGHT_PATH and any(lib.ttamd_nf4_gemm_expands_weight(M, m.N, K) for m in members):
+    # a group may be worth expanding where none of its members alone is
+    if not EXPANDED_WEIGHT_PATH and (lib.ttamd_nf4_group_fwd_leaves_tiles(arr, n, M, K, 1 if swiglu else 0)
+                                     or any(lib.ttamd_nf4_gemm_expands_weight(M, m.N, K) for m in members)):
         fwd_bytes = 0  # less than the library asks for: it keeps the fused kernel
     on_tiles = (tiles is not None and fwd_bytes > 0
                 and int(lib.ttamd_nf4_group_fwd_leaves_tiles(arr, n, M, K, 1 if swiglu else 0)) == (2 if paired else 1))
