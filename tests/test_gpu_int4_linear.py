@@ -61,6 +61,23 @@ def test_few_token_forward(kind, qp, n, k, group, bias, m):
     assert bool(((got.double() - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("m", [5, 20])  # the streaming and the tiled kernel
+def test_scales_at_the_top_of_the_range_expand_to_the_dense_weights_bits(m):
+    """One-hot rows read single weights: (q - 8) * scale is finite for every code but 0, while 8 * scale is not."""
+    layer = _layer("4w", 256, 64, 32, False, torch.bfloat16)
+    g = torch.Generator().manual_seed(0)
+    layer.weight.copy_(torch.randint(1, 16, (256, 32), generator=g) * 16 + torch.randint(1, 16, (256, 32), generator=g))
+    layer.scales_and_zeros[..., 0] = 4.5e37
+    layer.scales_and_zeros[..., 1] = torch.randn(2, 256, generator=g).to(torch.bfloat16)
+    dense = layer.dense_weight()
+    assert bool(dense.isfinite().all())
+    for first in range(0, 64, m):
+        k = torch.arange(first, first + m) % 64
+        x = torch.nn.functional.one_hot(k, 64).to(torch.bfloat16).to(DEV)
+        with torch.no_grad():
+            assert torch.equal(layer(x), dense[:, k.to(DEV)].t())
+
+
 def test_calls_the_kernels_do_not_serve_keep_the_dense_weight():
     layer = _layer("4w", 256, 256, 64, False, torch.bfloat16)
     for m, applies in ((256, True), (257, False)):

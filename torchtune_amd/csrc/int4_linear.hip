@@ -76,14 +76,16 @@ struct WeightPiece<kUint4> {
     codes = *reinterpret_cast<const u32x4_t*>(a.q + (((int64_t)n * a.K + k) >> 1));
     sz = reinterpret_cast<const uint32_t*>(a.scale)[(int64_t)(k >> a.log2_group) * a.N + n];
   }
-  // elements 8 s .. 8 s + 7 as an MFMA operand: bf16(bf16((q - 8) * scale) + zero); the first product is exact in fp32
+  // elements 8 s .. 8 s + 7 as an MFMA operand: bf16(bf16((q - 8) * scale) + zero).  The first product is that of 16 (q - 8), a
+  // byte with the nibble on top, and scale / 16, both exact (8 * scale, which a fused multiply-add would subtract, overflows
+  // for scales above 2^125 whose small multiples do not).
   __device__ __forceinline__ u32x4_t operand(int s) const {
-    const float sc = lo_of(sz), z = hi_of(sz), off = -8.0f * sc;
+    const float sc = lo_of(sz) * 0.0625f, z = hi_of(sz);
+    const uint32_t c = codes[s] ^ 0x88888888u, high = c & 0xf0f0f0f0u, low = (c << 4) & 0xf0f0f0f0u;
     u32x4_t w;
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
-      const uint32_t byte = (codes[s] >> (8 * b)) & 0xffu;
-      const uint32_t p = pack_pair(__builtin_fmaf((float)(byte >> 4), sc, off), __builtin_fmaf((float)(byte & 15u), sc, off));
+      const uint32_t p = pack_pair((float)(int8_t)(high >> (8 * b)) * sc, (float)(int8_t)(low >> (8 * b)) * sc);
       w[b] = pack_pair(lo_of(p) + z, hi_of(p) + z);
     }
     return w;
