@@ -633,3 +633,17 @@ def test_grad_input_swiglu_entry_point_validates_its_arguments_on_the_host():
     assert f(p, p, p, None, None, None, None, 0, p, p + 2, p, p, 8, 64, 64, None, 0, None) == -1 and b"aligned" in lib.ttamd_last_error()
     assert f(p, p, p, None, None, None, None, 0, p, p, p, p, 8, 64, 96, None, 0, None) == -1      # K not a multiple of 64
     assert f(p, p, p, p, None, None, None, 0, p, p, p, p, 8, 64, 64, None, 0, None) == -1 and b"together" in lib.ttamd_last_error()
+
+
+def test_small_bf16_products_of_few_tiles_are_sliced_within_one_workgroup_per_cu():
+    """``ttamd_gemm_mid_workspace_bytes`` needs no GPU: one fp32 slab per slice, none where the contraction stays whole.
+    Up to 128 tiles of 128 x 128, more workgroups than the 256 CUs measured slower than the split that fills them."""
+    lib = _lib.load()
+    for M, N, K, slices in ((1000, 2048, 8192, 2), (200, 4096, 14336, 4), (3950, 512, 6912, 2), (1000, 8192, 2048, 0), (64, 2048, 8192, 8)):
+        assert lib.ttamd_gemm_mid_workspace_bytes(M, N, K) == 4 * M * N * slices, (M, N, K)
+    for M in (1, 60, 127, 200, 500, 1000, 2047, 4000):
+        for N in (256, 512, 1024, 2048, 4096, 8192):
+            tiles = -(-M // 128) * -(-N // 128)
+            for K in (64, 1024, 4096, 14336):
+                slices = lib.ttamd_gemm_mid_workspace_bytes(M, N, K) // (4 * M * N)
+                assert slices == 0 or tiles > 128 or tiles * slices <= 256, (M, N, K)

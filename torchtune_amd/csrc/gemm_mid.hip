@@ -12,10 +12,10 @@
 // contraction is read from LDS as 16-byte pieces, one that lies across it through the transposing read
 // (ds_read_b64_tr_b16); the 16-byte chunks of a stage are permuted on the global-address side of the loads so that the
 // lanes served together fall on disjoint banks.  The 64 x 64 wave tile needs 128 bytes of LDS reads per cycle at the full
-// matrix rate, so the kernel tops out near 900 TFLOP/s (1000 x 8192 x 2048, second kind: 36.4 us).
-// Against the vendor library (its kernel alone; choosing it costs 31 us of host time): 1000 x 2048 x 2048 forward 20.6 and
-// 16.6 us, grad-input 21.0 and 20.6, weight gradient 16.7 and 22.8; 1000 x 2048 x 8192 forward 44.7 and 46.3.  A training
-// pass of a 1B-shaped layer over 1000 tokens with its 21 products: 1380 -> 827 us.
+// matrix rate, so the kernel tops out near 850 TFLOP/s (1000 x 8192 x 2048, second kind: 40 us).
+// Against the vendor library (its kernel alone, behind a queue of other products; choosing it costs 31 us of host time):
+// 1000 x 2048 x 2048 forward 22.0 and 16.8 us, grad-input 22.4 and 21.1, weight gradient 17.8 and 23.3; 1000 x 2048 x 8192
+// forward 51 and 51.  A training pass of a 1B-shaped layer over 1000 tokens with its 21 products: 1380 -> 830 us.
 // Launches of few tiles cut the contraction into slices (fp32 slabs, added in slice order by gemm_mid_reduce_kernel).
 #include "common.h"
 #include "nf4_math.h"
@@ -262,8 +262,10 @@ struct MidPlan {
 };
 // Slices of the contraction: the split with the least of (steps of one workgroup) + (slabs written and read, one more
 // launch), with the times measured on this kernel: 0.3 us a step when a CU has one workgroup (load latency), 0.22 us for
-// each of two (LDS bandwidth), slabs at about 4 TB/s, 4 us for the reduction's launch.  1000 rows, 2048 x 8192: 64 us
-// whole, 45 in two slices, 51 in four; 2048 x 2048: 20.6, 20.9 and 26.2.
+// each of two (LDS bandwidth), slabs at about 4 TB/s, 4 us for the reduction's launch.  Up to 128 tiles the slices stay within
+// one workgroup per CU: past that the model says level and the extra slabs lose (1000 rows of 2048 x 8192, 128 tiles: 74 us
+// whole, 52 in two slices, 60 in four; 200 x 4096 x 14336, 64 tiles: 46 in four, 51 in eight).  Over 222 products of 53 - 8192
+// rows and 256 - 14336 columns the split picked is 0.7 % slower than the fastest of 1 - 8 on average.
 MidPlan plan_mid(int64_t M, int64_t N, int64_t K) {
   MidPlan p;
   p.tiles_m = (M + kMidTile - 1) / kMidTile;
@@ -274,6 +276,7 @@ MidPlan plan_mid(int64_t M, int64_t N, int64_t K) {
   p.slices = 1;
   for (int64_t s = 1; s <= 8 && s <= nk; ++s) {
     const int64_t steps = (nk + s - 1) / s, slices = (nk + steps - 1) / steps, per_cu = (p.tiles * slices + 255) / 256;
+    if (slices > 1 && p.tiles <= 128 && p.tiles * slices > 256) break;
     const double t = (double)steps * (per_cu == 1 ? 0.3 : 0.22 * (double)per_cu) +
                      (slices > 1 ? 4.0 + 8e-6 / 4 * (double)slices * (double)M * (double)N : 0.0);
     if (s == 1 || t < best) {
