@@ -404,7 +404,7 @@ int ttamd_nf4_group_bwd_dx_ws_bf16(const ttamd_lora_group_member* members, int n
                                    int64_t K, void* workspace, size_t workspace_bytes, void* stream);
 
 /*
- * Plain bf16 products (fp32 accumulation, one rounding) of a few dozen to about two thousand rows: the matmuls of a
+ * Plain bf16 products (fp32 accumulation, one rounding) of a few dozen to some thousand rows: the matmuls of a
  * fake-quantised linear at short sequences (F.linear and its autograd on torchao's FakeQuantizedLinear; the recipes reach
  * it from recipes/qat_single_device.py).  kind 0: c[M,N] = a[M,K] . b[N,K]^T (+ bias [N] or NULL); 1: c[M,N] = a[M,K] . b[K,N];
  * 2: c[M,N] = a[K,M]^T . b[K,N].  N % 64 == 0; kinds 0 and 1: K % 64 == 0; kind 2: M % 64 == 0, any K.  workspace:

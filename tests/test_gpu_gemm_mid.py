@@ -41,6 +41,13 @@ def test_linear_and_gradients(M, N, K, bias):
         assert torch.equal(layer(x), y)
 
 
+@pytest.mark.parametrize("M,N,K,mid", [(2047, 2048, 4096, True), (4096, 2048, 2048, False), (3584, 2048, 2048, True), (16384, 1024, 1024, True),
+                                       (16385, 1024, 1024, False)])
+def test_rows_and_products_the_kernels_serve(M, N, K, mid):
+    layer = FakeQuantizedLinear(K, N, False, None, FakeQuantizeConfig(torch.int4, group_size=32), device="cuda", dtype=torch.bfloat16)
+    assert layer._mid_ok(torch.empty(M, K, device="cuda", dtype=torch.bfloat16)) is mid
+
+
 def test_second_derivative():
     torch.manual_seed(0)
     layer = FakeQuantizedLinear(128, 256, False, None, FakeQuantizeConfig(torch.int4, group_size=32), device="cuda", dtype=torch.bfloat16)

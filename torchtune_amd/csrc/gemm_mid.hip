@@ -1,4 +1,4 @@
-// Plain bf16 products of a few dozen to 2047 rows: the three matmuls of a fake-quantised linear below the sizes of the
+// Plain bf16 products of a few dozen to some thousand rows: the three matmuls of a fake-quantised linear below the sizes of the
 // 256 x 256-tile kernels (torchtune/modules: F.linear(fq(x), fq(W)) and what autograd derives from it).
 //
 //   kind 0   C[M, N] = A[M, K] . B[N, K]^T (+ bias)     forward

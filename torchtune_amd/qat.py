@@ -248,6 +248,14 @@ TN_GEMM_MIN_TILES = 192
 # and 96; 1000 tokens: 142 and 132), while a vendor call takes 31 us of host time, of ours 5; above it the vendor's larger
 # tiles win (500 tokens of 4096 x 14336: 287 and 255; 1000: 481 and 384).
 MID_GEMM_MAX = 1 << 34
+# The same bound from 2048 rows on.  The kernels are not built for tall products (four 64 x 64 wave tiles, LDS bound): the
+# vendor's larger tiles win on the GPU from about 8 * 2^30 on, by 5 % at first and 10 - 25 % from 13 * 2^30 (three products, us,
+# these kernels and the vendor's: 2600 tokens of 2048 x 2048 103 and 108, 3300 122 and 117, 4096 142 and 118; 5200 of
+# 2816 x 1024 160 and 127).  Whole layers gain from the vendor only where they are not host bound with it: layer of dim 2048 at 4096
+# tokens 1768 -> 1718 us forward + backward, of dim 1024 at 5200 932 -> 955.  Narrow weights (N * K up to 2^20) keep the bound
+# above: their weight gradient, few tiles over a long contraction, is where the vendor loses (16384 tokens of 1024 x 1024
+# 158 and 171, 65536 of 256 x 1024 221 and 335).
+MID_GEMM_MAX_TALL = 14 << 30
 # the weight gradients of a group's members (they share fq(x)) as one launch; False: one launch per member (A/B timing)
 TN_GROUP_GEMM = True
 
@@ -512,7 +520,8 @@ class FakeQuantizedLinear(nn.Linear):
         if type(x) is not torch.Tensor or type(w) is not nn.Parameter or (b is not None and (type(b) is not nn.Parameter or b.dtype != torch.bfloat16)):
             return False
         N, K = w.shape
-        return (0 < x.numel() * N <= MID_GEMM_MAX and N * K < 1 << 30 and N >= 256 and N % 64 == 0 and K % 64 == 0 and x.shape[-1] == K)
+        most = MID_GEMM_MAX_TALL if x.numel() >= 2048 * K and N * K > 1 << 20 else MID_GEMM_MAX
+        return (0 < x.numel() * N <= most and N * K < 1 << 30 and N >= 256 and N % 64 == 0 and K % 64 == 0 and x.shape[-1] == K)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self.activation_fake_quantizer is not None:
