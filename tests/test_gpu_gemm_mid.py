@@ -4,7 +4,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from torchtune_amd import ops
+from torchtune_amd import _lib, ops
 from torchtune_amd.qat import FakeQuantizeConfig, FakeQuantizedLinear, FakeQuantizer
 
 pytestmark = pytest.mark.gpu
@@ -16,10 +16,17 @@ def _close(got, want, length):
     assert bool(((got.double() - want).abs() <= slack).all())
 
 
+# the weight gradient in slices of the tokens, which end in a part-filled step or not (tokens % 32)
+SLICED_TOKENS = [(1000, 256, 1024, False), (1001, 256, 64, True), (1024, 320, 256, False), (2015, 256, 1536, False), (4097, 256, 128, True)]
+
+
 # one k step and fewer (tokens are the contraction of the weight gradient), tile edges, widths of half a tile, split contractions
 @pytest.mark.parametrize("M,N,K,bias", [(1, 256, 64, True), (31, 320, 128, False), (33, 256, 320, True), (128, 256, 256, False),
-                                        (129, 448, 4096, True), (257, 4096, 192, False), (1000, 512, 2048, False), (700, 2048, 1088, True)])
+                                        (129, 448, 4096, True), (257, 4096, 192, False), (1000, 512, 2048, False), (700, 2048, 1088, True),
+                                        (3000, 1024, 512, False)] + SLICED_TOKENS)
 def test_linear_and_gradients(M, N, K, bias):
+    if (M, N, K, bias) in SLICED_TOKENS:
+        assert _lib.load().ttamd_gemm_mid_workspace_bytes(N, K, M) > 0
     torch.manual_seed(M + N + K)
     layer = FakeQuantizedLinear(K, N, bias, FakeQuantizeConfig(torch.int8, "per_token", is_symmetric=False),
                                 FakeQuantizeConfig(torch.int4, group_size=32), device="cuda", dtype=torch.bfloat16)
