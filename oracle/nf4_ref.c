@@ -277,11 +277,11 @@ void ref_fq_per_group_uint4_asym(const void* w, int is_bf16, int qp_bf16, int64_
 }
 
 /* ---------------------------------------------------------------------------------------------------
- * Checkers for two shortcuts of the bf16 quantise kernel (they restate nothing of the reference; they
- * prove, by enumeration, that the shortcuts cannot change a result).
+ * Checkers by enumeration (they restate nothing of the reference): a shortcut of the weight-only uint4
+ * fake-quantise kernel that cannot change a result, and the codes of all bf16 values.
  * ------------------------------------------------------------------------------------------------- */
 
-/* Shortcut 1: with y = 1/a divided once per block, q = fma(fma(-x*y, a, x), y, x*y) must round to the same
+/* With y = 1/a divided once per block, q = fma(fma(-x*y, a, x), y, x*y) must round to the same
  * bf16 as the correctly rounded x / a.  Enumerates every bf16 divisor a with bit pattern in [a_lo, a_hi) and
  * every bf16 numerator 0 <= x <= a (signs are symmetric); returns the number of pairs that differ.  The `_upto`
  * form takes numerators up to max_quotient * a (the weight-only uint4 kernel divides a group's offsets, up to 15 steps
@@ -314,8 +314,7 @@ int64_t ref_check_shared_reciprocal_division(int a_lo, int a_hi) {
   return ref_check_shared_reciprocal_division_upto(a_lo, a_hi, 1.0f);
 }
 
-/* Shortcut 2: the code of a scaled bf16 value is looked up in a table that only spans magnitudes 2^-5 .. 1.
- * Returns the number of bf16 patterns below 2^-5 (either sign) whose code is not 7, plus 1 if NaN is not code 0;
+/* Returns the number of bf16 patterns below 2^-5 (either sign) whose code is not 7, plus 1 if NaN is not code 0;
  * table_out, if not NULL, receives the codes of magnitudes 0x3D00..0x3F80 for sign 0 then sign 1 (2 x 641 bytes). */
 int ref_check_code_table(uint8_t* table_out) {
   int bad = 0;

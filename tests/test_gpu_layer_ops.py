@@ -114,8 +114,18 @@ def test_rms_norm_leading_dimensions_and_validation():
     lib = _lib.load()
     assert lib.ttamd_rms_norm_fwd_bf16(x.data_ptr(), w.data_ptr(), 1e-6, y.data_ptr(), None, 6, 100, None) == -1
     assert b"multiple of 8" in lib.ttamd_last_error()
-    with pytest.raises(RuntimeError, match="HIP kernels"):
-        ops.rms_norm_fwd(x.cpu(), w.cpu(), 1e-6)
+    for norm in (ops.rms_norm_fwd, layer_ops.rms_norm):  # the mirror of the C ABI, and what the layers call
+        with pytest.raises(RuntimeError, match="HIP kernels"):
+            norm(x.cpu(), w.cpu(), 1e-6)
+    with pytest.raises(TypeError, match="bfloat16"):
+        layer_ops.rms_norm(x.float(), w, 1e-6)
+    with pytest.raises(ValueError, match="scale"):
+        layer_ops.rms_norm(x, w[:128], 1e-6)
+    m = layer_ops.RMSNorm(256).to(DEV, BF)
+    with pytest.raises(ValueError, match="residual"):
+        layer_ops.add_rms_norm(x, x[:1], m)
+    with pytest.raises(ValueError, match="shapes differ"):
+        layer_ops.swiglu(x, x[:1])
 
 
 @pytest.mark.parametrize("b,s,nh,hd", [(1, 5, 1, 8), (2, 37, 4, 64), (2, 128, 8, 128)])
@@ -274,5 +284,11 @@ def test_qkv_rope_repeat_refuses_heads_that_do_not_divide():
     q = torch.zeros(1, 4, 6, 16, dtype=BF, device=DEV)
     k = torch.zeros(1, 4, 4, 16, dtype=BF, device=DEV)
     cache = torch.zeros(4, 8, 2, device=DEV)
-    with pytest.raises(ValueError, match="heads"):
-        ops.qkv_rope_repeat(q, k, k, cache)
+    for f in (ops.qkv_rope_repeat, layer_ops.qkv_rope_repeat):
+        with pytest.raises(ValueError, match="heads"):
+            f(q, k, k, cache)
+    q = q[:, :, :4].contiguous()
+    with pytest.raises(ValueError, match="cache"):
+        layer_ops.qkv_rope_repeat(q, k, k, cache[:3])
+    with pytest.raises(ValueError, match="n_kv"):
+        layer_ops.qkv_rope_repeat(q, k, k[:, :3], cache)

@@ -215,10 +215,9 @@ def test_linear_nf4_is_linear_on_dequantised_weight():
 
 
 def test_shared_reciprocal_division_is_exact_for_bf16(c_oracle):
-    """The bf16 quantise kernel divides 1/absmax once per block and forms each quotient with two fused
-    multiply-adds.  Enumerate EVERY pair of bf16 operands 0 <= x <= a with a >= 2^-119 (the kernel's guard): the
-    bf16-rounded quotient must equal that of the correctly rounded division.  Below the guard the shortcut does
-    fail, which is why the guard exists."""
+    """Division by one correctly rounded reciprocal and two fused multiply-adds, the way the per-group uint4 fake quantiser divides.
+    Enumerate EVERY pair of bf16 operands 0 <= x <= a with a >= 2^-119: the bf16-rounded quotient must equal that of the
+    correctly rounded division.  Below that the shortcut does fail."""
     from concurrent.futures import ThreadPoolExecutor
 
     lo, hi = 0x0400, 0x7F80  # 2^-119 .. the largest finite bf16
@@ -246,9 +245,9 @@ def test_shared_reciprocal_division_is_exact_for_uint4_group_offsets(c_oracle):
     assert sum(bad) == 0
 
 
-def test_code_table_premises_and_monotone_codes(c_oracle):
-    """Every bf16 scaled value below 2^-5 is the zero code and NaN is code 0 (what lets the kernel's table span only
-    2^-5..1); inside the table the code never decreases with the value."""
+def test_codes_of_every_bf16_scaled_value(c_oracle):
+    """The C oracle's code of every bf16 value from -1 to 1: below 2^-5 in magnitude it is the zero code, NaN is code 0, from
+    there on it never decreases with the value, and the eager oracle says the same."""
     import ctypes
 
     buf = (ctypes.c_uint8 * (2 * 641))()

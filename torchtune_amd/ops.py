@@ -1271,53 +1271,6 @@ def rms_norm_fwd(x: torch.Tensor, scale: torch.Tensor, eps: float):
     return y, rstd
 
 
-def add_rms_norm_fwd(x: torch.Tensor, residual: torch.Tensor, scale: torch.Tensor, eps: float):
-    """-> (h = x + residual, y = RMSNorm(h), rstd): the addition of the residual stream and the norm that follows it in
-    one pass; the bits of ``x + residual`` followed by ``rms_norm_fwd``."""
-    xc = _bf16_any(x, "add_rms_norm_fwd: x")
-    rc_ = _bf16_any(residual, "add_rms_norm_fwd: residual")
-    sc = _bf16_any(scale, "add_rms_norm_fwd: scale")
-    if xc.shape != rc_.shape:
-        raise ValueError(f"add_rms_norm_fwd: x {tuple(xc.shape)} and residual {tuple(rc_.shape)} differ in shape")
-    D = xc.shape[-1]
-    rows = xc.numel() // D
-    h = torch.empty_like(xc)
-    y = torch.empty_like(xc)
-    rstd = torch.empty(rows, dtype=torch.float32, device=x.device)
-    lib = _lib.load()
-    with torch.cuda.device(x.device):
-        rc = lib.ttamd_add_rms_norm_fwd_bf16(xc.data_ptr(), rc_.data_ptr(), sc.data_ptr(), float(eps), h.data_ptr(), y.data_ptr(),
-                                             rstd.data_ptr(), rows, D, _stream(x))
-    _lib.check(rc, "add_rms_norm_fwd")
-    return h, y, rstd
-
-
-def rms_norm_bwd(gy: torch.Tensor, x: torch.Tensor, scale: torch.Tensor, rstd: torch.Tensor, want_gscale: bool,
-                 g_add: Optional[torch.Tensor] = None):
-    """-> (gx like x, gscale [D] bf16 | None); ``g_add`` (like x): a gradient that reaches x on another way, added to gx in
-    the same pass (``bf16(bf16(gx) + g_add)``)."""
-    gc = _bf16_any(gy, "rms_norm_bwd: gy")
-    xc = _bf16_any(x, "rms_norm_bwd: x")
-    sc = _bf16_any(scale, "rms_norm_bwd: scale")
-    D = xc.shape[-1]
-    rows = xc.numel() // D
-    gx = torch.empty_like(xc)
-    lib = _lib.load()
-    gscale = torch.empty(D, dtype=torch.bfloat16, device=x.device) if want_gscale else None
-    nbytes = lib.ttamd_rms_norm_bwd_workspace_bytes(D) if want_gscale else 0
-    ws = _workspace(nbytes, x.device) if want_gscale else None
-    ga = None
-    if g_add is not None:
-        ga = _bf16_any(g_add, "rms_norm_bwd: g_add")
-        if ga.shape != xc.shape:
-            raise ValueError(f"rms_norm_bwd: g_add {tuple(ga.shape)} and x {tuple(xc.shape)} differ in shape")
-    with torch.cuda.device(x.device):
-        rc = lib.ttamd_rms_norm_bwd_add_bf16(gc.data_ptr(), xc.data_ptr(), sc.data_ptr(), rstd.data_ptr(), _ptr(ga), gx.data_ptr(),
-                                             _ptr(gscale), rows, D, _ptr(ws), nbytes, _stream(x))
-    _lib.check(rc, "rms_norm_bwd")
-    return gx, gscale
-
-
 def rope(x: torch.Tensor, cache: torch.Tensor, inverse: bool = False) -> torch.Tensor:
     """x [b, s, n_h, h_d] bf16, cache [s, h_d/2, 2] fp32 -> rotated x (inverse: by the negative angle)"""
     xc = _bf16_any(x, "rope: x")
@@ -1371,12 +1324,12 @@ def _rope_cache_arg(cache: torch.Tensor, s: int, hd: int, who: str) -> torch.Ten
     return cache.contiguous()
 
 
-def _qkv_shapes(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, n_kv: Optional[int], who: str):
+def _qkv_shapes(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, who: str):
     if q.dim() != 4 or k.dim() != 4 or v.shape != k.shape or q.shape[:2] != k.shape[:2] or q.shape[3] != k.shape[3]:
         raise ValueError(f"{who}: expected [b, s, n_h, h_d] and two [b, s, n_kv, h_d], got {tuple(q.shape)}, {tuple(k.shape)}, {tuple(v.shape)}")
     b, s, nh, hd = q.shape
-    nkv = k.shape[2] if n_kv is None else n_kv
-    if nkv < 1 or nh % nkv or (n_kv is not None and k.shape[2] != nh):
+    nkv = k.shape[2]
+    if nkv < 1 or nh % nkv:
         raise ValueError(f"{who}: {nh} query heads against {nkv} key / value heads (tensors {tuple(q.shape)}, {tuple(k.shape)})")
     return b, s, nh, nkv, hd
 
@@ -1385,7 +1338,7 @@ def qkv_rope_repeat(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cache: to
     """``rope(q)``, ``repeat_kv(rope(k), n_h // n_kv)``, ``repeat_kv(v, n_h // n_kv)`` from one launch; q ``[b, s, n_h, h_d]``,
     k and v ``[b, s, n_kv, h_d]`` bf16, cache ``[s, h_d/2, 2]`` fp32.  The bits of :func:`rope` and :func:`repeat_kv`."""
     qc, kc, vc = _bf16_any(q, "qkv_rope_repeat: q"), _bf16_any(k, "qkv_rope_repeat: k"), _bf16_any(v, "qkv_rope_repeat: v")
-    b, s, nh, nkv, hd = _qkv_shapes(qc, kc, vc, None, "qkv_rope_repeat")
+    b, s, nh, nkv, hd = _qkv_shapes(qc, kc, vc, "qkv_rope_repeat")
     cc = _rope_cache_arg(cache, s, hd, "qkv_rope_repeat")
     qo, ko, vo = torch.empty_like(qc), torch.empty_like(qc), torch.empty_like(qc)
     lib = _lib.load()
@@ -1394,23 +1347,6 @@ def qkv_rope_repeat(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cache: to
                                             ko.data_ptr(), vo.data_ptr(), b, s, nh, nkv, hd, _stream(q))
     _lib.check(rc, "qkv_rope_repeat")
     return qo, ko, vo
-
-
-def qkv_rope_repeat_bwd(gq_out: torch.Tensor, gk_out: torch.Tensor, gv_out: torch.Tensor, cache: torch.Tensor, n_kv: int):
-    """The gradients of q, k, v of :func:`qkv_rope_repeat` from those of its three outputs (each ``[b, s, n_h, h_d]``)."""
-    a, bb, c = (_bf16_any(gq_out, "qkv_rope_repeat_bwd: gq"), _bf16_any(gk_out, "qkv_rope_repeat_bwd: gk"),
-                _bf16_any(gv_out, "qkv_rope_repeat_bwd: gv"))
-    b, s, nh, nkv, hd = _qkv_shapes(a, bb, c, n_kv, "qkv_rope_repeat_bwd")
-    cc = _rope_cache_arg(cache, s, hd, "qkv_rope_repeat_bwd")
-    gq = torch.empty_like(a)
-    gk = torch.empty(b, s, nkv, hd, dtype=torch.bfloat16, device=a.device)
-    gv = torch.empty_like(gk)
-    lib = _lib.load()
-    with torch.cuda.device(a.device):
-        rc = lib.ttamd_qkv_rope_repeat_bwd_bf16(a.data_ptr(), bb.data_ptr(), c.data_ptr(), cc.data_ptr(), gq.data_ptr(),
-                                                gk.data_ptr(), gv.data_ptr(), b, s, nh, nkv, hd, _stream(a))
-    _lib.check(rc, "qkv_rope_repeat_bwd")
-    return gq, gk, gv
 
 
 def swiglu_fwd(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
