@@ -518,7 +518,8 @@ def test_column_contractions_at_the_edges_of_their_kernels(M, K, R):
 
 
 @pytest.mark.parametrize("M", [1, 4, 5, 16])
-@pytest.mark.parametrize("N,K,ranks", [(64, 64, (8, 8)), (576, 2112, (40, 24)), (8192, 1088, (16, 8)), (12288, 4160, (8, 16))])
+@pytest.mark.parametrize("N,K,ranks", [(64, 64, (8, 8)), (576, 2112, (40, 24)), (8192, 1088, (16, 8)), (12288, 4160, (8, 16)), (4160, 1088, (8, 8)),
+                                       (4160, 4160, (8, 8)), (8192, 2560, (8, 8)), (12352, 3328, (8, 16)), (12352, 8192, (8, 8))])
 def test_few_token_pair_and_members(M, N, K, ranks):
     """The gate / up pair of a handful of tokens in one launch: every output equals the member's own call and the
     stand-alone gated product bit for bit, and a row's bits do not depend on the batch around it."""

@@ -411,17 +411,25 @@ __global__ __launch_bounds__(64 * MAXW) void nf4_few_kernel(const SmallMGroup gr
 
 // Launch shape at most 16 tokens.  The waves fix the order in which a row's products are summed and depend on the
 // layer alone, so that a row gets the same bits alone, in a batch of up to 16 tokens and inside a group; row tiles do not
-// enter the sums.  Measured (us, weights from HBM, launch gap included, at 1 / 8 / 16 tokens): 14336 x 4096 four waves and one
-// row tile 14.2 / 18.6 / 23, two tiles 15.4 / 16.9 / 18.9, eight waves and one tile 14.7 / 18.2 / 23; 4096 x 14336 sixteen
-// waves 13.4 / 18.6 / 22.6, eight 15.2 / 17.8 / 21.9; 4096 x 4096 6.5 / 7.7 / 9.0 and 7.1 / 7.8 / 9.0; 8192 x 2048 eight waves
-// 6.2 / 7.5 / 9.0, four 6.8 / 7.4 / 8.5.
+// enter the sums.  Measured over 48 layers of 256 - 28672 rows and 1024 - 28672 columns (us, weights from HBM, launch gap included):
+//  * up to 4096 rows a CU has one workgroup, which wants all the waves: one token, sixteen and eight waves: 4096 x 4096 7.5 and 7.9,
+//    4096 x 14336 15.8 and 18.9.  Layers below 8192 rows that are no wider than their input keep sixteen, too: a query projection
+//    then shares a launch with its key / value members.
+//  * up to 12288 rows eight: one token, sixteen / eight / four: 6912 x 2560 9.4 / 7.7 / 8.7, 8192 x 8192 18.9 / 17.1 / 22.0, 12288 x 2048
+//    11.3 / 7.9 / 8.5.  With two row tiles, which halve the reads of x, where those weigh and the layer is no wider than 8192 (16
+//    tokens, one and two tiles: 8192 x 28672 83.8 and 58.8, 8192 x 4096 14.8 and 13.4, but 8192 x 2048 9.1 and 9.9; 12 tokens, 12288 x 4096
+//    18.4 and 19.5).
+//  * beyond, three workgroups of eight waves per CU do not hold the layer any more: four (one token, eight and four: 14336 x 4096
+//    17.0 and 15.6, 16384 x 1024 7.9 and 6.9), unless the contraction is long (28672 x 8192 46.8 and 49.3); two tiles from 5 tokens on
+//    where x is large enough (14336 x 4096 at 8 tokens 21.2 and 18.4, 16384 x 1024 7.7 and 8.7).
 struct FewConfig {
   int rt, waves;
   bool operator==(const FewConfig& o) const { return rt == o.rt && waves == o.waves; }
 };
 FewConfig few_config(int64_t M, int64_t N, int64_t K) {
-  if (N < 8192) return {1, 16};
-  return {M > 4 && N >= 12288 ? 2 : 1, K >= 4096 ? 4 : 8};
+  if (N <= 4096 || (N < 8192 && N <= K)) return {1, 16};
+  if (N <= 12288) return {N <= 8192 && M * K >= 40960 ? 2 : 1, 8};
+  return {M > 4 && M * K >= 16384 ? 2 : 1, K < 8192 ? 4 : 8};
 }
 
 template <int RT, int MAXW, bool PAIR>
