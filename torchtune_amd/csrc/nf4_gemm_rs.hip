@@ -1234,39 +1234,10 @@ __global__ __launch_bounds__(256) void nf4_gemm_rs16_kernel(const RsArgs g, cons
 #endif
 }
 
-// What the slices of a launch add up to.  Output q is elements [end[q - 1], end[q]) of the launch; its partial products lie
-// at part[q], one slice of `mn` elements after the other.
-struct RsReduce {
-  const float* part[kGroupMax];
-  const uint16_t* bias[kGroupMax];
-  const uint16_t* cscale[kGroupMax];
-  uint16_t* C[kGroupMax];
-  int64_t end[kGroupMax];
-  int Nout[kGroupMax], splits[kGroupMax];
-};
-
-// C[m][n] = bf16((sum over slices of part[s][m][n] + bias[n]) * cscale[n]); a thread takes 8 consecutive columns.
-__global__ __launch_bounds__(256) void nf4_gemm_rs_reduce_kernel(const RsReduce r) {
-  int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
-  if (e >= r.end[kGroupMax - 1]) return;
-  int Nout = r.Nout[0], splits = r.splits[0];
-  int64_t at = 0, mn = r.end[0];
-  const float* part = r.part[0];
-  const uint16_t *bias = r.bias[0], *cscale = r.cscale[0];
-  uint16_t* C = r.C[0];
-#pragma unroll
-  for (int q = 1; q < kGroupMax; ++q)
-    if (e >= r.end[q - 1]) {
-      Nout = r.Nout[q];
-      splits = r.splits[q];
-      at = r.end[q - 1];
-      mn = r.end[q] - at;
-      part = r.part[q];
-      bias = r.bias[q];
-      cscale = r.cscale[q];
-      C = r.C[q];
-    }
-  e -= at;
+// C[m][n] = bf16((sum over slices of part[s][m][n] + bias[n]) * cscale[n]); a thread takes 8 consecutive columns, those from
+// element e on; mn = M * Nout elements per slice.
+__device__ __forceinline__ void sum_slices(int64_t e, const float* __restrict__ part, int splits, int64_t mn, int Nout,
+                                           const uint16_t* __restrict__ bias, const uint16_t* __restrict__ cscale, uint16_t* __restrict__ C) {
   float v[8];
   {
     const f32x4_t a = *reinterpret_cast<const f32x4_t*>(part + e), b = *reinterpret_cast<const f32x4_t*>(part + e + 4);
@@ -1300,22 +1271,40 @@ __global__ __launch_bounds__(256) void nf4_gemm_rs_reduce_kernel(const RsReduce 
   *reinterpret_cast<u32x4_t*>(C + e) = o;
 }
 
-int launch_reduce(const RsReduce& r, hipStream_t s) {
-  nf4_gemm_rs_reduce_kernel<<<dim3((unsigned)((r.end[kGroupMax - 1] / 8 + 255) / 256)), dim3(256), 0, s>>>(r);
-  return check_launch("nf4_gemm_rs_reduce");
+constexpr int kReduceElements = 256 * 8;  // of a workgroup
+
+// A launch of 5 - 6 us, half of it the way to the first load, which a choice among outputs lengthens (33 x 1024 in sixteen slices
+// 6.7 us when every thread looked its output up, 6.1 as it is): one output's sum takes its arguments as they are ...
+__global__ __launch_bounds__(256) void nf4_gemm_rs_reduce_kernel(const float* __restrict__ part, int splits, int64_t mn, int Nout,
+                                                                 const uint16_t* __restrict__ bias, const uint16_t* __restrict__ cscale,
+                                                                 uint16_t* __restrict__ C) {
+  const int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
+  if (e < mn) sum_slices(e, part, splits, mn, Nout, bias, cscale, C);
 }
+
+// ... and those of a group find theirs once per workgroup: output q is the business of the workgroups [wg_end[q - 1], wg_end[q]).
+struct RsReduce {
+  const float* part[kGroupMax];
+  const uint16_t* bias[kGroupMax];
+  uint16_t* C[kGroupMax];
+  int64_t mn[kGroupMax];
+  int Nout[kGroupMax], splits[kGroupMax], wg_end[kGroupMax];
+};
+__global__ __launch_bounds__(256) void nf4_gemm_rs_group_reduce_kernel(const RsReduce r) {
+  int q = 0;
+  while ((int)blockIdx.x >= r.wg_end[q]) ++q;  // uniform; the grid ends at wg_end[kGroupMax - 1]
+  const int wg = (int)blockIdx.x - (q ? r.wg_end[q - 1] : 0);
+  const int64_t e = ((int64_t)wg * 256 + threadIdx.x) * 8;
+  if (e < r.mn[q]) sum_slices(e, r.part[q], r.splits[q], r.mn[q], r.Nout[q], r.bias[q], nullptr, r.C[q]);
+}
+
+int reduce_workgroups(int64_t elements) { return (int)((elements + kReduceElements - 1) / kReduceElements); }
 
 // The sum over `splits` slices into one output
 int launch_reduce(const RsArgs& g, int splits, hipStream_t s) {
-  RsReduce r = {};
-  r.part[0] = g.part;
-  r.splits[0] = splits;
-  r.bias[0] = g.bias;
-  r.cscale[0] = g.cscale;
-  r.C[0] = g.C;
-  r.Nout[0] = g.Nout;
-  for (int64_t& end : r.end) end = (int64_t)g.M * g.Nout;
-  return launch_reduce(r, s);
+  const int64_t mn = (int64_t)g.M * g.Nout;
+  nf4_gemm_rs_reduce_kernel<<<dim3((unsigned)reduce_workgroups(mn)), dim3(256), 0, s>>>(g.part, splits, mn, g.Nout, g.bias, g.cscale, g.C);
+  return check_launch("nf4_gemm_rs_reduce");
 }
 
 template <int BM, int MODE, bool SPLIT, bool SEG = false, bool MEM = false>
@@ -1515,8 +1504,8 @@ int run_gemm_rs_group_fwd(const void* x, const GroupGemm& d, const void* h_cat, 
   g.ldlx = d.r_off[d.n];
   g.part = reinterpret_cast<float*>(workspace);
   m.n = d.n;
-  int64_t out = 0, part = 0;
-  int wgs = 0;
+  int64_t part = 0;
+  int wgs = 0, sum_wgs = 0;
   for (int i = 0; i < kGroupMax; ++i) {
     if (i < d.n) {
       const int64_t mn = d.M * d.N[i];
@@ -1524,25 +1513,32 @@ int run_gemm_rs_group_fwd(const void* x, const GroupGemm& d, const void* h_cat, 
       m.scal[i] = d.bscal_t[i];
       m.lX[i] = reinterpret_cast<const uint16_t*>(h_cat) + d.r_off[i];
       m.lW[i] = d.lora_b[i];
-      m.bias[i] = r.bias[i] = d.bias[i];
-      m.C[i] = r.C[i] = d.y[i];
-      m.Nout[i] = r.Nout[i] = (int)d.N[i];
+      m.bias[i] = d.bias[i];
+      m.C[i] = d.y[i];
+      m.Nout[i] = (int)d.N[i];
       m.R[i] = d.rank[i];
       m.lscale[i] = d.scale[i];
-      slice_steps(d.K, form == 2 ? choose_splits(d.M, d.N[i], d.K) : 1, m.ksteps[i], r.splits[i]);
-      wgs += (int)(((d.M + 127) / 128) * ((d.N[i] + kBN - 1) / kBN)) * r.splits[i];
+      int slices;
+      slice_steps(d.K, form == 2 ? choose_splits(d.M, d.N[i], d.K) : 1, m.ksteps[i], slices);
+      wgs += (int)(((d.M + 127) / 128) * ((d.N[i] + kBN - 1) / kBN)) * slices;
       m.part_at[i] = part;
       r.part[i] = g.part + (form == 2 ? part : 0);
-      part += mn * r.splits[i];
-      out += mn;
+      r.bias[i] = d.bias[i];
+      r.C[i] = d.y[i];
+      r.mn[i] = mn;
+      r.Nout[i] = (int)d.N[i];
+      r.splits[i] = slices;
+      part += mn * slices;
+      sum_wgs += reduce_workgroups(mn);
     }
     m.wg_end[i] = wgs;
-    r.end[i] = out;
+    r.wg_end[i] = sum_wgs;
   }
   if (form == 1) return launch_rs<128, 2, false, false, true>(g, 1, s, &m);
   TT_REQUIRE(aligned16(workspace), "nf4_lora_group_fwd: workspace must be 16-byte aligned");
   if (int rc = launch_rs<128, 2, true, false, true>(g, 1, s, &m)) return rc;
-  return launch_reduce(r, s);
+  nf4_gemm_rs_group_reduce_kernel<<<dim3((unsigned)sum_wgs), dim3(256), 0, s>>>(r);
+  return check_launch("nf4_gemm_rs_reduce");
 }
 
 // Grad-input of a group of layers with a common input, as one GEMM over the concatenated contraction:
