@@ -78,6 +78,21 @@ def test_scales_at_the_top_of_the_range_expand_to_the_dense_weights_bits(m):
             assert torch.equal(layer(x), dense[:, k.to(DEV)].t())
 
 
+@pytest.mark.parametrize("kind,qp,name", [("8da4w", torch.float32, "dequantize_per_group_int4"), ("4w", torch.bfloat16, "dequantize_per_group_uint4")])
+@pytest.mark.parametrize("m,n,streams", [(192, 16448, True), (193, 16448, False), (256, 16384, True)])
+def test_wide_layers_of_many_tokens_multiply_with_the_dense_weight(kind, qp, name, m, n, streams, monkeypatch):
+    layer = _layer(kind, n, 128, 64, False, qp)
+    x = torch.randn(m, 128, generator=torch.Generator().manual_seed(m)).to(torch.bfloat16).to(DEV)
+    dense, dequantize = [], getattr(ops, name)
+    with torch.no_grad(), monkeypatch.context() as patch:
+        patch.setattr(ops, name, lambda *a: dense.append(1) or dequantize(*a))
+        got = layer(x)
+    assert bool(dense) is not streams
+    xd, w = _operands(layer, x)
+    want = xd @ w.t()
+    assert bool(((got.double() - want).abs() <= want.abs() * 2.0 ** -8 + (xd.abs() @ w.abs().t()) * (128 * 2.0 ** -23)).all())
+
+
 def test_calls_the_kernels_do_not_serve_keep_the_dense_weight():
     layer = _layer("4w", 256, 256, 64, False, torch.bfloat16)
     for m, applies in ((256, True), (257, False)):

@@ -607,7 +607,14 @@ def _int4_kernels_apply(x: torch.Tensor, weight: torch.Tensor, in_features: int,
         return False
     if bias is not None and (bias.dtype != torch.bfloat16 or not bias.is_cuda or (bias.requires_grad and torch.is_grad_enabled())):
         return False
-    return weight.is_contiguous() and ops.int4_linear_applies(x.numel() // in_features, weight.shape[0], in_features, groupsize)
+    rows, N = x.numel() // in_features, weight.shape[0]
+    # More than 192 tokens are two tiles of rows, and a layer of more than 16384 outputs then has more than two workgroups per CU,
+    # which expand its weight twice: the dense copy and the library's larger tiles win (us at 200 tokens, these kernels and the
+    # two passes, int8 / uint4: 28672 x 8192 278 / 280 and 255 / 281, 20480 x 5120 161 / 145 and 130 / 136; at 192 tokens 117 / 104 and
+    # 132 / 136; 16384 x 4096 at 200 75 / 77 and 83 / 87).
+    if rows > 192 and N > 16384:
+        return False
+    return weight.is_contiguous() and ops.int4_linear_applies(rows, N, in_features, groupsize)
 
 
 class Int8DynActInt4WeightLinear(nn.Module):
