@@ -131,6 +131,30 @@ def test_native_nodes_under_checkpointing_and_saved_tensor_hooks(how):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16))
 
 
+@pytest.mark.parametrize("max_tokens", [0, 1280])  # the Python nodes, the native ones
+@pytest.mark.parametrize("kind", ["single", "group", "gated"])
+def test_a_weight_that_asks_for_a_gradient_gets_none_but_a_graph(max_tokens, kind, monkeypatch):
+    """An NF4 weight is made with ``requires_grad``: where nothing else asks, the output belongs to the graph all the same."""
+    monkeypatch.setattr(ops, "NATIVE_MAX_TOKENS", max_tokens)
+    layers = _layers([256, 256], 256, True)
+    x = torch.randn(5, 256, device=DEV).to(BF)
+    fn = {"single": lambda: layers[0](x), "group": lambda: lora_linear_group(x, layers)[1], "gated": lambda: lora_swiglu_group(x, *layers)}[kind]
+    plain = fn()
+    for layer in layers:
+        for p in layer.parameters():
+            p.requires_grad_(False)
+    assert not fn().requires_grad
+    for layer in layers:
+        layer.weight.requires_grad_(True)
+    out = fn()
+    assert out.requires_grad and torch.equal(out, plain)
+    out.sum().backward()
+    assert all(layer.weight.grad is None for layer in layers)
+    layers[0].lora_a.weight.requires_grad_(True)
+    fn().sum().backward()
+    assert all(layer.weight.grad is None for layer in layers) and (layers[0].lora_a.weight.grad is not None or kind == "group")
+
+
 def _weight_only_qat(k, n):
     layer = torch.nn.Sequential(torch.nn.Linear(k, n, bias=False, device=DEV, dtype=BF))
     quantizer = Int4WeightOnlyQATQuantizer(groupsize=32)

@@ -343,9 +343,10 @@ Weight unpack_weight(const c10::List<Tensor>& l, int64_t at, int64_t N) {
   return w;
 }
 
+// asking: the weight where it asks for a gradient.  It gets none, but the output then belongs to the graph.
 struct QLoRALinearFn : torch::autograd::Function<QLoRALinearFn> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& a, const Tensor& b, const std::optional<Tensor>& bias,
-                        const Weight& w, double scale) {
+                        const std::optional<Tensor>& /*asking*/, const Weight& w, double scale) {
     Member m;
     m.w = w;
     m.a = a;
@@ -384,9 +385,11 @@ struct QLoRALinearFn : torch::autograd::Function<QLoRALinearFn> {
             "qlora_linear_bwd");
     }
     if (has_bias && ctx->needs_input_grad(3)) gbias = gy.sum(0);
-    return {gx, ga, gb, gbias, Tensor(), Tensor()};
+    return {gx, ga, gb, gbias, Tensor(), Tensor(), Tensor()};
   }
 };
+
+bool asks_for_gradient(const Tensor& weight) { return at::GradMode::is_enabled() && weight.requires_grad(); }
 
 Tensor qlora_linear(const Tensor& x, const Tensor& weight, const Tensor& q, const Tensor& scal, const std::optional<Tensor>& q_t, const std::optional<Tensor>& scal_t,
                     int64_t N, const Tensor& a, const Tensor& b, double scale, const std::optional<Tensor>& bias) {
@@ -398,7 +401,8 @@ Tensor qlora_linear(const Tensor& x, const Tensor& weight, const Tensor& q, cons
   if (scal_t) m.w.scal_t = *scal_t;
   m.w.N = N;
   if (bias) m.bias = *bias;
-  if (wants_grad({&x, &a, &b, &m.bias})) return QLoRALinearFn::apply(x, a, b, bias, m.w, scale);
+  const std::optional<Tensor> asking = asks_for_gradient(weight) ? std::optional<Tensor>(weight) : std::nullopt;
+  if (asking || wants_grad({&x, &a, &b, &m.bias})) return QLoRALinearFn::apply(x, a, b, bias, asking, m.w, scale);
   m.a = a;
   m.b = b;
   m.scale = scale;
@@ -471,9 +475,11 @@ struct GroupSpec {
   bool fused_swiglu_bwd = true;  // gated: the gradients of gate and up come out of the adapters' backward, not of a launch before it
 };
 
-// Differentiable inputs: x, then per member lora_a, lora_b and, where there is one, the bias.
+// Differentiable inputs: x, then per member lora_a, lora_b and, where there is one, the bias; behind them the weights that ask
+// for a gradient (as for a single layer).
 struct QLoRAGroupFn : torch::autograd::Function<QLoRAGroupFn> {
-  static variable_list forward(AutogradContext* ctx, const Tensor& x, at::TensorList /*adapters*/, GroupSpec& spec) {
+  static variable_list forward(AutogradContext* ctx, const Tensor& x, at::TensorList inputs, GroupSpec& spec) {
+    ctx->saved_data["inputs"] = (int64_t)inputs.size();
     GroupOut o = group_forward(x, spec.ms, spec.gated, true);
     variable_list save = {o.x2, o.h_cat};
     std::vector<Tensor> weights;
@@ -572,7 +578,8 @@ struct QLoRAGroupFn : torch::autograd::Function<QLoRAGroupFn> {
         ++at_input;
       }
     }
-    out.emplace_back();  // the specification
+    out.resize(1 + ctx->saved_data["inputs"].toInt());  // the weights that ask
+    out.emplace_back();                                 // the specification
     return out;
   }
 };
@@ -584,7 +591,7 @@ std::vector<Tensor> lora_group(const Tensor& x, const std::vector<MemberTuple>& 
   GroupSpec spec;
   spec.gated = gated;
   spec.fused_swiglu_bwd = fused_swiglu_bwd;
-  std::vector<Tensor> adapters;
+  std::vector<Tensor> inputs;
   bool grad = wants_grad({&x});
   for (const auto& t : members) {
     Member m;
@@ -598,13 +605,15 @@ std::vector<Tensor> lora_group(const Tensor& x, const std::vector<MemberTuple>& 
     m.b = std::get<7>(t);
     m.scale = std::get<8>(t);
     if (std::get<9>(t)) m.bias = *std::get<9>(t);
-    grad = grad || wants_grad({&m.a, &m.b, &m.bias});
-    adapters.push_back(m.a);
-    adapters.push_back(m.b);
-    if (m.bias.defined()) adapters.push_back(m.bias);
+    grad = grad || asks_for_gradient(m.w.whole) || wants_grad({&m.a, &m.b, &m.bias});
+    inputs.push_back(m.a);
+    inputs.push_back(m.b);
+    if (m.bias.defined()) inputs.push_back(m.bias);
     spec.ms.push_back(std::move(m));
   }
-  if (grad) return QLoRAGroupFn::apply(x, at::TensorList(adapters), spec);
+  for (const Member& m : spec.ms)
+    if (asks_for_gradient(m.w.whole)) inputs.push_back(m.w.whole);
+  if (grad) return QLoRAGroupFn::apply(x, at::TensorList(inputs), spec);
   GroupOut o = group_forward(x, spec.ms, gated, false);
   if (gated) return {o.act};
   return o.ys;
