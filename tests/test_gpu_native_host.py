@@ -1,4 +1,8 @@
 """Layer calls on the native host path (few tokens) against the Python autograd nodes: the same library calls, the same bits."""
+import sys
+import threading
+import time
+
 import pytest
 import torch
 import torch.autograd.forward_ad as fwAD
@@ -153,6 +157,42 @@ def test_a_weight_that_asks_for_a_gradient_gets_none_but_a_graph(max_tokens, kin
     layers[0].lora_a.weight.requires_grad_(True)
     fn().sum().backward()
     assert all(layer.weight.grad is None for layer in layers) and (layers[0].lora_a.weight.grad is not None or kind == "group")
+
+
+@pytest.mark.parametrize("call", ["norm", "linear", "fake_quant"])
+def test_native_calls_let_other_threads_run(call):
+    """With a switch interval no call outlasts, a thread gets its turn only where the interpreter's lock is given up."""
+    (layer,) = _layers([256], 256, False)
+    x = torch.randn(5, 256, device=DEV).to(BF)
+    w, scal, q = x[0].clone(), layer.weight.block_scalers(), layer.weight.quantized_data
+    host = _host.load()
+    f = {"norm": lambda: host.rms_norm(x, w, 1e-6), "fake_quant": lambda: host.fq_per_token(x, True, False, None),
+         "linear": lambda: host.qlora_linear(x, layer.weight, q, scal, None, None, 256, layer.lora_a.weight, layer.lora_b.weight, 2.0, None)}[call]
+    f()
+    turns, stop, started = [0], threading.Event(), threading.Event()
+
+    def other():
+        started.set()
+        while not stop.is_set():
+            turns[0] += 1
+            time.sleep(0)
+
+    interval = sys.getswitchinterval()
+    thread = threading.Thread(target=other)
+    thread.start()
+    started.wait()
+    try:
+        sys.setswitchinterval(100.0)
+        before = turns[0]
+        for _ in range(300):
+            f()
+        got = turns[0] - before
+    finally:
+        sys.setswitchinterval(interval)
+        stop.set()
+        thread.join()
+    torch.cuda.synchronize()
+    assert got > 2  # one turn may have been under way
 
 
 def _weight_only_qat(k, n):

@@ -796,17 +796,19 @@ Tensor straight_through_linear(const Tensor& x, const Tensor& weight, const Tens
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  // like torch's own ops the calls run without the interpreter's lock: a launch waits where the queue is full
+  const py::call_guard<py::gil_scoped_release> unlocked;
   m.def("ordinary", &ordinary);
-  m.def("rms_norm", &rms_norm);
-  m.def("add_rms_norm", &add_rms_norm);
-  m.def("qkv_rope_repeat", &qkv_rope_repeat);
-  m.def("swiglu", &swiglu);
-  m.def("qlora_linear", &qlora_linear);
-  m.def("lora_group", &lora_group);
-  m.def("int8_dynamic_linear", &int8_dynamic_linear);
-  m.def("uint4_group_linear", &uint4_group_linear);
-  m.def("fq_per_token", &fq_per_token);
-  m.def("fq_per_group", &fq_per_group);
-  m.def("straight_through", &straight_through);
-  m.def("straight_through_linear", &straight_through_linear);
+  m.def("rms_norm", &rms_norm, unlocked);
+  m.def("add_rms_norm", &add_rms_norm, unlocked);
+  m.def("qkv_rope_repeat", &qkv_rope_repeat, unlocked);
+  m.def("swiglu", &swiglu, unlocked);
+  m.def("qlora_linear", &qlora_linear, unlocked);
+  m.def("lora_group", &lora_group, unlocked);
+  m.def("int8_dynamic_linear", &int8_dynamic_linear, unlocked);
+  m.def("uint4_group_linear", &uint4_group_linear, unlocked);
+  m.def("fq_per_token", &fq_per_token, unlocked);
+  m.def("fq_per_group", &fq_per_group, unlocked);
+  m.def("straight_through", &straight_through, unlocked);
+  m.def("straight_through_linear", &straight_through_linear, unlocked);
 }
