@@ -380,6 +380,14 @@ int ttamd_nf4_lora_group_fwd_bf16(const void* x, const ttamd_lora_group_member* 
  * formed in the epilogue of the one GEMM launch (the two outputs are not read back); otherwise in a pass of its own. */
 int ttamd_nf4_lora_group_swiglu_fwd_bf16(const void* x, const ttamd_lora_group_member* members, int n_members, const void* h_cat,
                                          void* act, int64_t M, int64_t K, void* workspace, size_t workspace_bytes, void* stream);
+/* A handful of tokens (at most 16): every member's h and y (and act, the gated product of a gate / up pair, where it is not
+ * NULL) in as few launches as there are launch shapes, usually one; h_cat receives the hidden activations or is NULL where no
+ * backward wants them.  Ranks of at most 32.  ttamd_lora_few_fwd_applies says whether this is the better way for a shape
+ * (the call returns TTAMD_EUNSUPPORTED where it does not).  Same roundings as the calls above (h and y once each to bf16);
+ * the fp32 sums of h run in another order. */
+int ttamd_lora_few_fwd_applies(const ttamd_lora_group_member* members, int n_members, int64_t M, int64_t K, int swiglu);
+int ttamd_lora_few_fwd_bf16(const void* x, const ttamd_lora_group_member* members, int n_members, void* h_cat, void* act, int64_t M,
+                            int64_t K, void* stream);
 /* gh_cat out, bf16 [M, sum of ranks]; every member's grad_lora_a and grad_lora_b; members[i].y = gy_i */
 size_t ttamd_lora_group_bwd_workspace_bytes(const ttamd_lora_group_member* members, int n_members, int64_t M, int64_t K);
 int ttamd_lora_group_bwd_bf16(const void* x, const void* h_cat, const ttamd_lora_group_member* members, int n_members,

@@ -667,3 +667,60 @@ def test_slices_of_part_filled_rounds(M, n_out, widths):
     for i, ((m, t, *_), gy) in enumerate(zip(mem, gys)):
         want = want + gy.float() @ t.get_original_weight().float() + gh[:, 8 * i:8 * i + 8].float() @ m.lora_a.float()
     close(gx, want)
+
+
+@pytest.mark.parametrize("M", [1, 4, 5, 16])
+@pytest.mark.parametrize("Ns,K,ranks", [((64,), 64, (8,)), ((576,), 2112, (24,)), ((4032, 64), 1088, (8, 32)), ((8192,), 1088, (16,)), ((16384,), 192, (8,)),
+                                        ((64,), 16448, (16,)), ((128,), 33088, (32,)), ((320, 64, 64, 128), 576, (8, 16, 8, 16)), ((64, 64), 64, (8, 16)),
+                                        ((8192,), 8256, (16,)), ((2816, 2816), 1088, (16, 8)),
+                                        ((12352, 12352), 4160, (8, 16))])
+@pytest.mark.parametrize("bias", [False, True])
+def test_few_tokens_with_the_hidden_product_inside(M, Ns, K, ranks, bias):
+    """Half chunks at the end of the contraction, several segments of it, ragged ranks, one and two row tiles.  h against
+    float64 within its bf16 rounding; y bit for bit what the forward gives for the h the launch left; the same bits without
+    h_cat, and for the first row alone."""
+    from torchtune_amd import _lib
+
+    lib = _lib.load()
+    g = torch.Generator(device=DEV).manual_seed(M + K + sum(Ns))
+    x = torch.randn(M, K, device=DEV, generator=g).to(BF)
+    members, gated = [], len(Ns) == 2 and Ns[0] == Ns[1]
+    for n, r in zip(Ns, ranks):
+        q = torch.randint(0, 256, (n * K // 2,), device=DEV, generator=g, dtype=torch.uint8)
+        s = torch.rand(n * K // 64, device=DEV, generator=g).mul_(0.1)
+        members.append(ops.GroupMember(q, s, None, torch.randn(r, K, device=DEV, generator=g).mul_(K ** -0.5).to(BF),
+                                       torch.randn(n, r, device=DEV, generator=g).mul_(0.05).to(BF),
+                                       torch.randn(n, device=DEV, generator=g).to(BF) if bias else None, 2.0, n))
+
+    if gated and Ns[0] > 12288 and M > 4:  # two rank tiles beside four row tiles leave no room for more tokens
+        ys = [torch.empty(M, n, device=DEV, dtype=BF) for n in Ns]
+        arr, keep = ops._group_array("test", members, K, ys, M)
+        assert lib.ttamd_lora_few_fwd_applies(arr, 2, M, K, 1) == 0
+        assert lib.ttamd_lora_few_fwd_bf16(x.data_ptr(), arr, 2, None, ys[0].data_ptr(), M, K, 0) == -2
+        return
+
+    def run(rows, want_h):
+        ys = [torch.full((rows, n), float("nan"), device=DEV, dtype=BF) for n in Ns]
+        act = torch.full((rows, Ns[0]), float("nan"), device=DEV, dtype=BF) if gated else None
+        h = torch.full((rows, sum(ranks)), float("nan"), device=DEV, dtype=BF) if want_h else None
+        arr, keep = ops._group_array("test", members, K, ys, rows)
+        _lib.check(lib.ttamd_lora_few_fwd_bf16(x.data_ptr(), arr, len(Ns), h.data_ptr() if want_h else None, act.data_ptr() if gated else None,
+                                               rows, K, torch.cuda.current_stream().cuda_stream), "lora_few_fwd")
+        return h, ys, act
+
+    h, ys, act = run(M, True)
+    _, again, _ = run(M, False)
+    _, first, _ = run(1, True)
+    off = 0
+    for m, y, y2, y1 in zip(members, ys, again, first):
+        r = m.lora_a.shape[0]
+        got = h[:, off:off + r].double()
+        want = x.double() @ m.lora_a.double().t()
+        # one rounding to bf16, and fp32 sums: K products of about |x| |a| each rounded at 2^-24 of a partial sum
+        bound = want.abs() * 2 ** -8 + (x.double().abs() @ m.lora_a.double().abs().t()) * 2 ** -20
+        assert bool(((got - want).abs() <= bound).all())
+        direct = ops.nf4_lora_linear_fwd(x, m.qdata, m.block_scalers, m.N, h[:, off:off + r].contiguous(), m.lora_b, m.scale, m.bias)
+        assert torch.equal(y, direct) and torch.equal(y, y2) and torch.equal(y[:1], y1)
+        off += r
+    if gated:
+        assert torch.equal(act, ops.swiglu_fwd(*ys))

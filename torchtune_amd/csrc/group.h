@@ -89,6 +89,10 @@ int small_m_limit();
 // the forward of M tokens on an [N, K] weight runs the few-token kernel (sliced_ok: a slicing workspace is at hand)
 bool small_m_applies(int64_t M, int64_t N, int64_t K, bool sliced_ok);
 int run_small_m_group(const void* x, const GroupGemm& g, const void* h_cat, void* act, bool* act_done, hipStream_t s);
+// the same with h_i = x . lora_a[i]^T formed inside the launches (gated: two members of equal width, act is written too), where
+// that is the better way; h_cat receives it, or is null
+bool few_forms_hidden(const GroupGemm& g, bool gated);
+int run_few_with_hidden(const void* x, const GroupGemm& g, const uint16_t* const* lora_a, void* h_cat, void* act, hipStream_t s);
 
 // lora_skinny.hip
 size_t group_hidden_ws_bytes(int64_t M, int64_t K, int r_total);

@@ -307,6 +307,21 @@ void check_member(Member& m, int64_t K, const char* what) {
   }
 }
 
+void fill(ttamd_lora_group_member& e, const Member& m, const Tensor& y) {
+  e = {};
+  e.quantized_data = (const uint8_t*)m.w.q.data_ptr();
+  e.block_scalers = m.w.scal.data_ptr();
+  e.block_scalers_t = opt_ptr(m.w.scal_t);
+  e.quantized_data_t = (const uint8_t*)opt_ptr(m.w.q_t);
+  e.lora_a = m.a.data_ptr();
+  e.lora_b = m.b.data_ptr();
+  e.bias = opt_ptr(m.bias);
+  e.y = y.data_ptr();
+  e.N = m.w.N;
+  e.rank = (int)m.a.size(0);
+  e.scale = (float)m.scale;
+}
+
 struct LinearOut {
   Tensor x2, h, y;
 };
@@ -322,6 +337,12 @@ LinearOut linear_forward(const Tensor& x, Member m, bool keep) {
   const int rank = (int)m.a.size(0);
   o.y = at::empty(with_last(x, m.w.N), o.x2.options());
   if (keep) o.h = at::empty({M, rank}, o.x2.options());
+  ttamd_lora_group_member one;
+  fill(one, m, o.y);
+  if (ttamd_lora_few_fwd_applies(&one, 1, M, K, 0)) {
+    check(ttamd_lora_few_fwd_bf16(o.x2.data_ptr(), &one, 1, opt_ptr(o.h), nullptr, M, K, stream_of(x)), "lora_few_fwd");
+    return o;
+  }
   const size_t h_bytes = keep ? 0 : align256(M * rank * 2);
   const Tensor ws = scratch(h_bytes + ttamd_qlora_linear_fwd_workspace_bytes(M, m.w.N, K, rank), o.x2);
   char* w = (char*)ws.data_ptr();
@@ -417,21 +438,6 @@ struct GroupOut {
   std::vector<Tensor> ys;
 };
 
-void fill(ttamd_lora_group_member& e, const Member& m, const Tensor& y) {
-  e = {};
-  e.quantized_data = (const uint8_t*)m.w.q.data_ptr();
-  e.block_scalers = m.w.scal.data_ptr();
-  e.block_scalers_t = opt_ptr(m.w.scal_t);
-  e.quantized_data_t = (const uint8_t*)opt_ptr(m.w.q_t);
-  e.lora_a = m.a.data_ptr();
-  e.lora_b = m.b.data_ptr();
-  e.bias = opt_ptr(m.bias);
-  e.y = y.data_ptr();
-  e.N = m.w.N;
-  e.rank = (int)m.a.size(0);
-  e.scale = (float)m.scale;
-}
-
 GroupOut group_forward(const Tensor& x, std::vector<Member>& ms, bool gated, bool keep) {
   const int n = (int)ms.size();
   TORCH_CHECK_VALUE(n >= 1 && n <= TTAMD_GROUP_MAX, "lora_group_fwd: a group has 1 to ", TTAMD_GROUP_MAX, " members, got ", n);
@@ -451,6 +457,11 @@ GroupOut group_forward(const Tensor& x, std::vector<Member>& ms, bool gated, boo
     r_total += ms[i].a.size(0);
   }
   if (keep) o.h_cat = at::empty({M, r_total}, o.x2.options());
+  if (gated) o.act = at::empty_like(o.ys[0]);
+  if (ttamd_lora_few_fwd_applies(arr, n, M, K, gated)) {
+    check(ttamd_lora_few_fwd_bf16(o.x2.data_ptr(), arr, n, opt_ptr(o.h_cat), opt_ptr(o.act), M, K, stream_of(x)), "lora_few_fwd");
+    return o;
+  }
   const size_t h_bytes = keep ? 0 : align256(M * r_total * 2);
   const size_t hidden = ttamd_lora_group_hidden_workspace_bytes(arr, n, M, K), fwd = ttamd_lora_group_fwd_workspace_bytes(arr, n, M, K);
   const size_t bytes = hidden > fwd ? hidden : fwd;
@@ -460,7 +471,6 @@ GroupOut group_forward(const Tensor& x, std::vector<Member>& ms, bool gated, boo
   void* s = stream_of(x);
   check(ttamd_lora_group_hidden_bf16(o.x2.data_ptr(), arr, n, h_cat, M, K, ws, bytes, s), "lora_group_hidden");
   if (gated) {
-    o.act = at::empty_like(o.ys[0]);
     check(ttamd_nf4_lora_group_swiglu_fwd_bf16(o.x2.data_ptr(), arr, n, h_cat, o.act.data_ptr(), M, K, ws, bytes, s),
           "lora_group_fwd");
   } else {

@@ -179,6 +179,26 @@ extern "C" int ttamd_nf4_lora_group_swiglu_fwd_bf16(const void* x, const ttamd_l
   return ttamd_swiglu_fwd_bf16(members[0].y, members[1].y, act, M * members[0].N, stream);
 }
 
+// A handful of tokens: the members' hidden activations and outputs from one launch (or one per launch shape).
+extern "C" int ttamd_lora_few_fwd_applies(const ttamd_lora_group_member* members, int n_members, int64_t M, int64_t K, int swiglu) {
+  Decoded d;
+  if (decode("lora_few_fwd_applies", members, n_members, M, K, false, d) != TTAMD_OK) return 0;
+  if (swiglu && (n_members != 2 || members[0].N != members[1].N)) return 0;
+  return few_forms_hidden(d.gm, swiglu != 0) ? 1 : 0;
+}
+
+extern "C" int ttamd_lora_few_fwd_bf16(const void* x, const ttamd_lora_group_member* members, int n_members, void* h_cat, void* act,
+                                       int64_t M, int64_t K, void* stream) {
+  Decoded d;
+  if (int rc = decode("lora_few_fwd", members, n_members, M, K, false, d)) return rc;
+  TT_REQUIRE(x && aligned16(x) && aligned16(h_cat) && aligned16(act), "lora_few_fwd: x must be non-null, x, h_cat and act 16-byte aligned");
+  TT_REQUIRE(!act || (n_members == 2 && members[0].N == members[1].N),
+             "lora_few_fwd: act belongs to the gate and the up projection, two members of equal width");
+  if (!few_forms_hidden(d.gm, act != nullptr))
+    return fail(TTAMD_EUNSUPPORTED, "lora_few_fwd: shape not served (M=%lld K=%lld)", (long long)M, (long long)K);
+  return run_few_with_hidden(x, d.gm, d.sk.lora_a, h_cat, act, reinterpret_cast<hipStream_t>(stream));
+}
+
 extern "C" size_t ttamd_lora_group_bwd_workspace_bytes(const ttamd_lora_group_member* members, int n_members, int64_t M, int64_t K) {
   Decoded d;
   if (decode("lora_group_bwd_workspace_bytes", members, n_members, M, K, false, d) != TTAMD_OK) return 0;

@@ -4,22 +4,31 @@
 //
 // With so few rows the work is streaming the packed weight once: 0.5625 bytes per weight element against 2 for a
 // dense bf16 weight.  A workgroup owns 16 or 32 weight rows and the whole contraction, expands the codes in registers
-// exactly as the large-M kernel does (byte -> fp32 pair from an LDS table, times the fp32 block scaler, one rounding to
+// exactly as the large-M kernel does (byte -> pair of code points from an LDS table, times the fp32 block scaler, one rounding to
 // bf16 - the bits of ttamd_nf4_dequantize) and feeds v_mfma_f32_16x16x32_bf16 with the weight rows as the row operand
 // and 16-token tiles of x as the column operand.  A lane reads 16 contiguous bytes of codes (32 elements of
 // its row: the four lane groups of a row cover one 64-byte piece) and uses one dword of them per MFMA; x is small and
 // comes from the cache.  The waves' partial sums meet in LDS in a fixed order.
 //
-//  * nf4_few_kernel (at most 16 tokens, generation): the waves take 128-wide chunks of K in turn, one chunk each at a
-//    time.  Neighbouring waves then read neighbouring pieces of the same rows; groups of four chunks per wave, which
-//    put more bytes in flight, were slower at every size.  Only the lanes of tokens that exist ask for x.  The adapter
-//    is one more MFMA step whose operands are requested ahead of the loop, and the gate / up pair of a feed-forward
-//    shares a workgroup, so that silu(gate) * up leaves the same launch.
+//  * nf4_few_kernel (at most 16 tokens, generation): the waves take 128-wide chunks of K in turn, one chunk in flight each while
+//    the one before it is multiplied (more in flight gained nothing).  What bounded its first form was neither HBM nor
+//    arithmetic but the address unit - operands loaded straight into MFMA lanes, where neighbouring lanes are different rows,
+//    cost it 64 cycles a load instead of 16, and a block scaler's load as much as its 32 codes' - and one wave's sum over
+//    the others at the end (1.3 us).  Now codes, x and lora_a come by direct-to-LDS loads in row order, a workgroup's
+//    scalers in one pass ahead of the loop, the table holds fp16 pairs (a code point is exact in fp16), which the multiply
+//    converts on the way, and every thread finishes outputs.  The hidden product h = x . lora_a^T can ride along as
+//    further row tiles of the same loop, where that beats a launch of its own.
+//    us, weights from HBM, hidden product included, before -> now at 1 / 13 tokens: 4096 x 4096 12.5 / 14.2 -> 6.7 / 7.6, 14336 x 4096 21.3 /
+//    25.7 -> 14.9 / 16.7, 4096 x 14336 22.1 / 30.8 -> 15.6 / 20.4, 2048 x 2048 9.1 / 11.1 -> 5.4 / 5.9, gate / up pair of 14336 x 4096 38.0 / 43.1 ->
+//    26.6 / 31.2.  A read of the same bytes in the same row pieces takes 3.1, 6.3, 6.6 and (the pair) 10.3: the pair is bound by
+//    the expansion (VALU 10.9 us, LDS 11.7 of 22 us busy without the hidden product).
 //  * nf4_small_m_kernel (17 - 64 tokens): groups of U chunks per wave, two or four token tiles.
 #include "common.h"
 #include "group.h"
 #include "nf4_math.h"
 #include "swiglu_math.h"
+
+#define TT_LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
 
 namespace ttamd {
 namespace {
@@ -44,6 +53,8 @@ struct SmallMArgs {
   const uint8_t* codes;    // [N, K/2]
   const float* bscal;      // [N, K/64]
   const uint16_t* h;       // [M, R] bf16 (rows ldh elements apart) or null
+  const uint16_t* lora_a;  // [R, K] bf16 where the launch forms h itself
+  uint16_t* h_out;         // and where it leaves it (rows ldh elements apart), or null
   const uint16_t* lora_b;  // [N, R] bf16 or null
   const uint16_t* bias;    // [N] bf16 or null
   const uint16_t* cscale;  // [N] bf16 or null
@@ -258,204 +269,422 @@ __global__ __launch_bounds__(64 * MAXW) void nf4_small_m_kernel(const SmallMGrou
 }
 
 constexpr int kFewTokens = 16;
+// The launch shapes below address x, lora_a and the codes of a row tile with 32-bit byte offsets.
+constexpr int64_t kFewMaxK = int64_t(1) << 26;
+constexpr int kFewHiddenRank = 32;  // most ranks of a member whose hidden product a launch forms itself
 
-// RT tiles of 16 weight rows per workgroup, at most MAXW waves.  PAIR: tile 0 belongs to grp.m[0] (gate), tile 1 to grp.m[1]
-// (up projection, the same width), and act = bf16(bf16(silu(y_0)) * y_1) is written as well.
+// One NF4 code byte's two code points (exact in bf16 and so in fp16) times a block scaler, each one fp32 rounding: the
+// conversion rides in the multiply (adding -0 changes no product, signed zeros included).
+__device__ __forceinline__ float scaled_lo(uint32_t pair, float s) {
+  float r = 0.f;
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(pair), "v"(s), "s"(-0.0f));
+#endif
+  return r;
+}
+__device__ __forceinline__ float scaled_hi(uint32_t pair, float s) {
+  float r = 0.f;
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(pair), "v"(s), "s"(-0.0f));
+#endif
+  return r;
+}
+
+// LDS of a few-token workgroup: the code table, the block scalers of its rows over a segment of the contraction, and per wave
+// one stage: 128 columns of x (MQ groups of four tokens), of its row tiles' codes and of its members' lora_a.
+template <int RT, int NT, int MQ>
+struct FewLayout {
+  static constexpr int kCopies = NT > 0 ? 1 : 16;  // of the code table
+  static constexpr int kLut = 1024 * kCopies;
+  static constexpr int kSegment = 16384 / RT;  // columns; a multiple of 128 times the most waves, so that it does not move the waves' chunks
+  static constexpr int kStage = (MQ + RT + 4 * NT) * 1024;
+  __host__ __device__ static int scalers(int K) {  // an odd row stride: the rows of a tile on different banks
+    const int kb = (K < kSegment ? K : kSegment) >> 6;
+    return (RT * 16 * (kb | 1) * 4 + 15) & ~15;
+  }
+  static int bytes(int K, int waves) { return kLut + scalers(K) + waves * kStage; }
+};
+
+// RT tiles of 16 weight rows per workgroup, at most MAXW waves, tokens in MQ groups of four.  PAIR: the even tiles belong to grp.m[0]
+// (gate), the odd ones to the same rows of grp.m[1] (up projection, the same width), and act = bf16(bf16(silu(y_0)) * y_1) is
+// written as well.
+// NA > 0: h = x . lora_a^T is formed here, NA tiles of 16 ranks per member beside the row tiles (the workgroup's own copy: the
+// members' first workgroups also write it to m.h_out where that is asked for); otherwise it is read from m.h.
 // ONE: the launch has one member, and its arguments sit at fixed places (found through `which` they cost two dependent
 // scalar loads before the first request: 0.4 us of a launch of 6 - 8).
-template <int RT, int MAXW, bool PAIR, bool ONE>
+template <int RT, int MAXW, int MQ, int NA, bool PAIR, bool ONE>
 __global__ __launch_bounds__(64 * MAXW) void nf4_few_kernel(const SmallMGroup grp, uint16_t* __restrict__ act) {
-  static_assert(!PAIR || RT == 2, "a pair is two row tiles");
+#if defined(__HIP_DEVICE_COMPILE__)  // LDS address-space casts
+  static_assert(!PAIR || RT % 2 == 0, "a pair is two row tiles of equal rows");
+  constexpr int NT = NA * (PAIR ? 2 : 1);  // rank tiles
+  using L = FewLayout<RT, NT, MQ>;
   int which = 0;  // uniform over the workgroup
   if constexpr (!PAIR && !ONE) {
 #pragma unroll
     for (int q = 0; q < kGroupMax - 1; ++q)
       if (q < grp.n - 1 && (int)blockIdx.x >= grp.wg_end[q]) which = q + 1;
   }
-  __shared__ float2 lut[256];
-  __shared__ float red[(MAXW - 1) * RT * 256];
+  extern __shared__ __attribute__((aligned(16))) char few_smem[];
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int nw = blockDim.x >> 6;
   const int i = lane & 15, g = lane >> 4;
-  const int M = grp.m[which].M, K = grp.m[which].K;
+  const int M = grp.m[which].M, K = grp.m[which].K, KB = K >> 6;
   const int wg = (int)blockIdx.x - (!PAIR && !ONE && which ? grp.wg_end[which - 1] : 0);
-  auto member = [&](int rt) -> const SmallMArgs& { return grp.m[PAIR ? rt : which]; };
-  auto first_row = [&](int rt) { return PAIR ? 16 * wg : 16 * (RT * wg + rt); };  // N % (16 RT) == 0: every row exists
+  auto member = [&](int rt) -> const SmallMArgs& { return grp.m[PAIR ? rt & 1 : which]; };
+  auto first_row = [&](int rt) { return PAIR ? 16 * (wg * (RT / 2) + (rt >> 1)) : 16 * (RT * wg + rt); };  // every row exists
+  float* const scal = reinterpret_cast<float*>(few_smem + L::kLut);
+  const int scal_bytes = L::scalers(K);
+  char* const stage = few_smem + L::kLut + scal_bytes + wave * L::kStage;
+  const uint32_t lds_scal = (uint32_t)(uintptr_t)TT_LDS_PTR(scal), lds_stage = (uint32_t)(uintptr_t)TT_LDS_PTR(stage);
 
-  const bool token = i < M;
-  const uint16_t* xrow = grp.m[which].x + (int64_t)(token ? i : 0) * K + 32 * g;
-  const uint8_t* crow[RT];
-  const float* srow[RT];
+  // ---- requests: direct-to-LDS loads, 64 pieces of 16 bytes each.  Four neighbouring lanes ask for 64 contiguous bytes: the
+  //      address unit takes them at once, where the lanes of an MFMA operand (neighbours are different rows) cost it four
+  //      times as long; that unit was what bounded this kernel.  Piece p of row r of x and lora_a (16 pieces per 128 columns)
+  //      goes to slot p ^ r, piece p of row r of the codes (4) to slot p ^ (r / 4) % 4: operand reads then meet no bank twice.
+  auto dma16 = [&](uint32_t voff, const void* base, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "s"(lds) : "memory", "m0");
+  };
+  uint32_t x_off[MQ], a_off[NT > 0 ? NA * 4 : 1];
+  const int r4 = lane >> 4, p16 = lane & 15, cr = lane >> 2, cp = (lane & 3) ^ ((lane >> 4) & 3);
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    const int64_t n = first_row(rt) + i;
-    crow[rt] = member(rt).codes + ((n * K) >> 1) + 16 * g;
-    srow[rt] = member(rt).bscal + n * (K >> 6) + (g >> 1);
+  for (int d = 0; d < MQ; ++d) {
+    const int r = 4 * d + r4;
+    x_off[d] = (uint32_t)(r < M ? r : M - 1) * (uint32_t)K * 2u + ((p16 ^ r) << 4);  // rows beyond M repeat the last one: never stored
   }
-  u32x4_t cd[RT], xb[4];
-  float sc[RT];
-  auto request = [&](int c) {
-    const bool in = c * 128 + 32 * g < K;  // the last chunk of a K that is an odd multiple of 64 is half a chunk
+  if constexpr (NT > 0) {
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-      cd[rt] = u32x4_t{0, 0, 0, 0};
-      sc[rt] = 0.f;
-      if (in) {
-        cd[rt] = *reinterpret_cast<const u32x4_t*>(crow[rt] + (int64_t)c * 64);
-        sc[rt] = srow[rt][2 * c];
+    for (int d = 0; d < NA * 4; ++d) {
+      const int r = 4 * d + r4;  // ranks beyond R of any member repeat one: zeroed where they would count
+      a_off[d] = (uint32_t)r * (uint32_t)K * 2u + ((p16 ^ (r & 15)) << 4);
+    }
+  }
+  const uint32_t c_off = (uint32_t)cr * (uint32_t)(K >> 1) + (cp << 4);
+  auto request = [&](int c) {
+    const bool half = c * 128 + 64 >= K;  // the last chunk of a K that is an odd multiple of 64: its second half repeats the first
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+      dma16(half ? c_off - ((cp & 2) << 4) : c_off, member(rt).codes + (((int64_t)first_row(rt) * K) >> 1) + (int64_t)c * 64,
+            lds_stage + (MQ + rt) * 1024);
+#pragma unroll
+    for (int d = 0; d < MQ; ++d)
+      dma16(half ? x_off[d] - (((p16 ^ (4 * d + r4)) & 8) << 4) : x_off[d], reinterpret_cast<const char*>(grp.m[which].x) + (int64_t)c * 256,
+            lds_stage + d * 1024);
+    if constexpr (NT > 0) {
+#pragma unroll
+      for (int a = 0; a < NT; ++a) {
+        const SmallMArgs& ma = member(a / NA);
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+          const int e = 4 * (a % NA) + d;
+          uint32_t off = a_off[e];
+          if (4 * e + r4 >= ma.R) off = (p16 ^ ((4 * e + r4) & 15)) << 4;
+          if (half) off -= ((p16 ^ ((4 * e + r4) & 15)) & 8) << 4;
+          dma16(off, reinterpret_cast<const char*>(ma.lora_a) + (int64_t)c * 256, lds_stage + (MQ + RT + 4 * a) * 1024 + d * 1024);
+        }
       }
     }
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      xb[s] = u32x4_t{0, 0, 0, 0};
-      if (in && token) xb[s] = *reinterpret_cast<const u32x4_t*>(xrow + c * 128 + 8 * s);
+  };
+  constexpr int kBatch = RT + MQ + 4 * NT;
+  const int stride = (K < L::kSegment ? KB : L::kSegment >> 6) | 1;
+  auto request_scalers = [&](int first, int n) {  // blocks [first, first + n) of every row
+    for (int r = wave; r < 16 * RT; r += nw) {
+      const float* base = member(PAIR ? r >> 4 : 0).bscal + (int64_t)(first_row(r >> 4) + (r & 15)) * KB + first;
+      for (int j = 0; j < n; j += 64)
+        if (j + lane < n)
+          asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"((uint32_t)(j + lane) * 4u), "s"(base),
+                       "s"(lds_scal + (uint32_t)(r * stride + j) * 4u) : "memory", "m0");
     }
   };
   const int n_chunks = (K + 127) >> 7;
-  // The first chunk and wave 0's adapter operands are asked for before the code table is built: a workgroup lives for
-  // little more than one trip to memory, and neither the table nor a second trip at the end must stand in its way.
-  int c = wave;
-  if (c < n_chunks) request(c);
-  auto adapter = [&](int rt, int r0, u32x4_t& hv, u32x4_t& bv) {  // ranks r0 + 8 g .. + 7 (R % 8 == 0)
-    const SmallMArgs& a = member(rt);
-    hv = bv = u32x4_t{0, 0, 0, 0};
-    if (r0 + 8 * g < a.R) {
-      bv = *reinterpret_cast<const u32x4_t*>(a.lora_b + (int64_t)(first_row(rt) + i) * a.R + r0 + 8 * g);
-      if (token) hv = *reinterpret_cast<const u32x4_t*>(a.h + (int64_t)i * a.ldh + r0 + 8 * g);
-    }
-  };
-  u32x4_t hv[RT], bv[RT];
-  if (wave == 0) {
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) adapter(rt, 0, hv[rt], bv[rt]);
-  }
-  for (int e = t; e < 256; e += blockDim.x)
-    lut[e] = make_float2(round_to_bf16(nf4_code_value(e >> 4)), round_to_bf16(nf4_code_value(e & 15)));
-  f32x4_t acc[RT][4];  // four chains
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-    for (int s = 0; s < 4; ++s) acc[rt][s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  __syncthreads();
-  while (c < n_chunks) {
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) {
-        u32x4_t wf;
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          const float2 p = lut[(cd[rt][s] >> (8 * b)) & 0xffu];
-          wf[b] = pack_pair(p.x * sc[rt], p.y * sc[rt]);
-        }
-        acc[rt][s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf), __builtin_bit_cast(bf16x8_t, xb[s]),
-                                                             acc[rt][s], 0, 0, 0);
-      }
-    c += nw;
-    if (c < n_chunks) request(c);
-  }
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-#pragma unroll
-    for (int s = 1; s < 4; ++s) acc[rt][0] += acc[rt][s];
-    if (wave == 0) {
-      // adapter: sum_r bf16(h[m][r] * lscale) * lora_b[n][r], the operands the large-M kernel feeds its MFMA
-      const float ls = member(rt).lscale;
-      for (int r0 = 0; r0 < member(rt).R; r0 += 32) {
-        if (r0 > 0) adapter(rt, r0, hv[rt], bv[rt]);
-        u32x4_t hs;
-#pragma unroll
-        for (int d = 0; d < 4; ++d) hs[d] = pack_pair(lo_of(hv[rt][d]) * ls, hi_of(hv[rt][d]) * ls);
-        acc[rt][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, bv[rt]), __builtin_bit_cast(bf16x8_t, hs),
-                                                             acc[rt][0], 0, 0, 0);
-      }
+
+  // The first requests leave before the code table is built: a workgroup lives for little more than one trip to memory.
+  const int seg_chunks = L::kSegment >> 7;
+  request_scalers(0, KB < L::kSegment >> 6 ? KB : L::kSegment >> 6);
+  int c = wave;  // the host gives a launch no more waves than there are chunks
+  request(c);
+  uint32_t* const lut = reinterpret_cast<uint32_t*>(few_smem);
+  typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+  for (int e = t; e < 256; e += blockDim.x) {
+    const half2_t p = {(_Float16)round_to_bf16(nf4_code_value(e >> 4)), (_Float16)round_to_bf16(nf4_code_value(e & 15))};
+    const uint32_t v = __builtin_bit_cast(uint32_t, p);
+    if constexpr (L::kCopies == 1) {
+      lut[e] = v;
     } else {
 #pragma unroll
-      for (int v = 0; v < 4; ++v) red[((wave - 1) * RT + rt) * 256 + v * 64 + lane] = acc[rt][0][v];
+      for (int j = 0; j < L::kCopies / 4; ++j)
+        reinterpret_cast<u32x4_t*>(lut)[e * (L::kCopies / 4) + ((j + e) & (L::kCopies / 4 - 1))] = u32x4_t{v, v, v, v};
+    }
+  }
+  const char* const lut_lane = reinterpret_cast<const char*>(lut) + (L::kCopies > 1 ? (lane & (L::kCopies - 1)) * 4 : 0);
+  constexpr int kShift = L::kCopies == 1 ? 2 : 6;  // entry e lies at e << kShift
+  auto pair_of = [&](uint32_t codes, int b) {
+    const uint32_t off = (8 * b >= kShift ? codes >> (8 * b - kShift) : codes << (kShift - 8 * b)) & (0xffu << kShift);
+    return *reinterpret_cast<const uint32_t*>(lut_lane + off);
+  };
+  constexpr int kChains = 2;  // the same in every instance: a row's bits do not depend on the launch's shape
+  f32x4_t acc[RT][kChains], ah[NT > 0 ? NT : 1][kChains];
+#pragma unroll
+  for (int s = 0; s < kChains; ++s) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) acc[rt][s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int a = 0; a < (NT > 0 ? NT : 1); ++a) ah[a][s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  // the scalers are a wave's oldest requests: its first chunk may stay in flight across the barrier
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kBatch) : "memory");
+
+  const int xr = i & (4 * MQ - 1);
+  const int x_at = xr * 256, a_at = (MQ + RT) * 1024 + i * 256, c_at = MQ * 1024 + i * 64 + ((g ^ ((i >> 2) & 3)) << 4);
+  for (int first = 0;;) {  // segments of the contraction
+    const int end = n_chunks < first + seg_chunks ? n_chunks : first + seg_chunks;
+    for (; c < end; c += nw) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      // the stage goes to registers and is asked for again
+      u32x4_t cd[RT], xb[4], ab[NT > 0 ? NT : 1][4];
+      float sc[RT];
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {
+        cd[rt] = *reinterpret_cast<const u32x4_t*>(stage + c_at + rt * 1024);
+        sc[rt] = scal[(16 * rt + i) * stride + 2 * (c - first) + (g >> 1)];  // beyond K: any value, times zero
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        xb[s] = *reinterpret_cast<const u32x4_t*>(stage + x_at + (((4 * g + s) ^ xr) << 4));
+        if constexpr (NT > 0) {
+#pragma unroll
+          for (int a = 0; a < NT; ++a) ab[a][s] = *reinterpret_cast<const u32x4_t*>(stage + a_at + a * 4096 + (((4 * g + s) ^ i) << 4));
+        }
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (c + nw < end) request(c + nw);
+      if (c * 128 + 64 >= K && g >= 2) {  // half a chunk: nothing of its second half counts, whatever lies there
+#pragma unroll
+        for (int s = 0; s < 4; ++s) xb[s] = u32x4_t{0, 0, 0, 0};
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) sc[rt] = 0.f;
+        if constexpr (NT > 0) {
+#pragma unroll
+          for (int a = 0; a < NT; ++a)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) ab[a][s] = u32x4_t{0, 0, 0, 0};
+        }
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const bf16x8_t xv = __builtin_bit_cast(bf16x8_t, xb[s]);
+        if constexpr (NT > 0) {
+#pragma unroll
+          for (int a = 0; a < NT; ++a)
+            ah[a][s % kChains] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, ab[a][s]), xv, ah[a][s % kChains], 0, 0, 0);
+        }
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+          u32x4_t wf;
+#pragma unroll
+          for (int b = 0; b < 4; ++b) {
+            const uint32_t p = pair_of(cd[rt][s], b);
+            wf[b] = pack_pair(scaled_lo(p, sc[rt]), scaled_hi(p, sc[rt]));
+          }
+          acc[rt][s % kChains] =
+              __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf), xv, acc[rt][s % kChains], 0, 0, 0);
+        }
+      }
+    }
+    first += seg_chunks;
+    if (first >= n_chunks) break;
+    __syncthreads();  // every wave is done with the segment's scalers
+    request_scalers(2 * first, KB - 2 * first < (L::kSegment >> 6) ? KB - 2 * first : L::kSegment >> 6);
+    if (c < n_chunks) request(c);
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  }
+
+  // ---- the waves' partial sums meet in LDS, [tile][lane][v] at the head of each wave's stage, and are added in wave order
+  constexpr int kSteps = NA > 0 ? (NA + 1) / 2 : 2;  // MFMA steps of the adapter, 32 ranks each (the ranks of a group add up to at most 64)
+  u32x2_t bv[RT][2 * kSteps], hv[PAIR ? 2 : 1][2 * kSteps];  // wave 0: ranks 16 a + 4 g .. + 3 of its rows' lora_b and of its token's h
+  if (wave == 0) {
+#pragma unroll
+    for (int a = 0; a < 2 * kSteps; ++a) {
+      const int r = 16 * a + 4 * g;
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) {
+        bv[rt][a] = u32x2_t{0, 0};
+        if (r < member(rt).R) bv[rt][a] = *reinterpret_cast<const u32x2_t*>(member(rt).lora_b + (int64_t)(first_row(rt) + i) * member(rt).R + r);
+      }
+#pragma unroll
+      for (int u = 0; u < (PAIR ? 2 : 1); ++u) {
+        hv[u][a] = u32x2_t{0, 0};
+        if (NA == 0 && i < M && r < member(u).R) hv[u][a] = *reinterpret_cast<const u32x2_t*>(member(u).h + (int64_t)i * member(u).ldh + r);
+      }
+    }
+  }
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) acc[rt][0] += acc[rt][1];
+  auto leave = [&](int tile, const f32x4_t& v) { *reinterpret_cast<f32x4_t*>(stage + tile * 1024 + lane * 16) = v; };
+  if (wave > 0) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) leave(rt, acc[rt][0]);
+  }
+  if constexpr (NT > 0) {
+#pragma unroll
+    for (int a = 0; a < NT; ++a) {
+      ah[a][0] += ah[a][1];
+      if (wave > 0) leave(RT + a, ah[a][0]);
+    }
+    __syncthreads();
+    if (wave == 0) {  // h, rounded to bf16: rank 16 (a % NA) + 4 g + v of token i
+#pragma unroll
+      for (int a = 0; a < NT; ++a) {
+        for (int w = 1; w < nw; ++w) ah[a][0] += *reinterpret_cast<const f32x4_t*>(stage + w * L::kStage + (RT + a) * 1024 + lane * 16);
+        const SmallMArgs& ma = member(a / NA);
+        const int r = 16 * (a % NA) + 4 * g;
+        if (r < ma.R) hv[a / NA][a % NA] = u32x2_t{pack_pair(ah[a][0][0], ah[a][0][1]), pack_pair(ah[a][0][2], ah[a][0][3])};
+        if (ma.h_out && wg == 0 && i < M && r < ma.R)
+          *reinterpret_cast<u32x2_t*>(ma.h_out + (int64_t)i * ma.ldh + r) = hv[a / NA][a % NA];
+      }
+    }
+  }
+  if (wave == 0) {
+    // adapter: sum_r bf16(h[m][r] * lscale) * lora_b[n][r], the operands the large-M kernel feeds its MFMA
+    auto scaled = [&](uint32_t d, float ls) { return pack_pair(lo_of(d) * ls, hi_of(d) * ls); };
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      const int u = PAIR ? rt & 1 : 0;
+      const float ls = member(rt).lscale;
+#pragma unroll
+      for (int q = 0; q < kSteps; ++q) {
+        if (32 * q >= member(rt).R) break;
+        const u32x4_t b = {bv[rt][2 * q].x, bv[rt][2 * q].y, bv[rt][2 * q + 1].x, bv[rt][2 * q + 1].y};
+        const u32x4_t h = {scaled(hv[u][2 * q].x, ls), scaled(hv[u][2 * q].y, ls), scaled(hv[u][2 * q + 1].x, ls), scaled(hv[u][2 * q + 1].y, ls)};
+        acc[rt][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, b), __builtin_bit_cast(bf16x8_t, h), acc[rt][0], 0, 0, 0);
+      }
+      leave(rt, acc[rt][0]);
     }
   }
   __syncthreads();
-  if (wave != 0) return;
-  // acc[rt][0][v] = the wave's share of y[i][first_row(rt) + 4 g + v]
-  u32x2_t out[RT];
+  // every thread finishes one output (PAIR: one of each member) at a time: one wave alone took 1.3 us over sixteen waves' sums
+  const char* const parts = few_smem + L::kLut + scal_bytes;
+  for (int e = t; e < 256 * (PAIR ? RT / 2 : RT); e += blockDim.x) {
+    const int tile = e >> 8, token = (e >> 2) & 15, row = 4 * ((e >> 6) & 3) + (e & 3);
+    if (token >= M) continue;
+    uint32_t out[PAIR ? 2 : 1];
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    const SmallMArgs& a = member(rt);
-    const int nb = first_row(rt) + 4 * g;
-    float o[4];
+    for (int u = 0; u < (PAIR ? 2 : 1); ++u) {
+      const int rt = PAIR ? 2 * tile + u : tile;
+      const SmallMArgs& a = member(u);
+      const char* p = parts + rt * 1024 + (e & 255) * 4;
+      const int n = first_row(rt) + row;
+      float o = *reinterpret_cast<const float*>(p);
+      if (nw == MAXW) {
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      o[v] = acc[rt][0][v];
-      for (int w = 0; w < nw - 1; ++w) o[v] += red[(w * RT + rt) * 256 + v * 64 + lane];
+        for (int w = 1; w < MAXW; ++w) o += *reinterpret_cast<const float*>(p + w * L::kStage);
+      } else {
+        for (int w = 1; w < nw; ++w) o += *reinterpret_cast<const float*>(p + w * L::kStage);
+      }
+      if (a.bias) o += bf16_bits_to_f32(a.bias[n]);
+      if (a.cscale) o *= bf16_bits_to_f32(a.cscale[n]);
+      out[u] = pack_pair(o, 0.f);
+      a.y[(int64_t)token * a.N + n] = (uint16_t)out[u];
+      if (PAIR && u == 1) act[(int64_t)token * a.N + n] = (uint16_t)swiglu_gate_pair(out[0], out[PAIR ? 1 : 0]);
     }
-    if (a.bias) {
-      const u32x2_t bb = *reinterpret_cast<const u32x2_t*>(a.bias + nb);
-      o[0] += lo_of(bb.x); o[1] += hi_of(bb.x); o[2] += lo_of(bb.y); o[3] += hi_of(bb.y);
-    }
-    if (a.cscale) {
-      const u32x2_t cc = *reinterpret_cast<const u32x2_t*>(a.cscale + nb);
-      o[0] *= lo_of(cc.x); o[1] *= hi_of(cc.x); o[2] *= lo_of(cc.y); o[3] *= hi_of(cc.y);
-    }
-    out[rt].x = pack_pair(o[0], o[1]);
-    out[rt].y = pack_pair(o[2], o[3]);
-    if (token) *reinterpret_cast<u32x2_t*>(a.y + (int64_t)i * a.N + nb) = out[rt];
   }
-  if constexpr (PAIR) {
-    u32x2_t p;
-    p.x = swiglu_gate_pair(out[0].x, out[1].x);
-    p.y = swiglu_gate_pair(out[0].y, out[1].y);
-    if (token) *reinterpret_cast<u32x2_t*>(act + (int64_t)i * grp.m[0].N + 16 * wg + 4 * g) = p;
-  }
+#endif
 }
 
 // Launch shape at most 16 tokens.  The waves fix the order in which a row's products are summed and depend on the
 // layer alone, so that a row gets the same bits alone, in a batch of up to 16 tokens and inside a group; row tiles do not
-// enter the sums.  Measured over 48 layers of 256 - 28672 rows and 1024 - 28672 columns (us, weights from HBM, launch gap included):
-//  * up to 4096 rows a CU has one workgroup, which wants all the waves: one token, sixteen and eight waves: 4096 x 4096 7.5 and 7.9,
-//    4096 x 14336 15.8 and 18.9.  Layers below 8192 rows that are no wider than their input keep sixteen, too: a query projection
-//    then shares a launch with its key / value members.
-//  * up to 12288 rows eight: one token, sixteen / eight / four: 6912 x 2560 9.4 / 7.7 / 8.7, 8192 x 8192 18.9 / 17.1 / 22.0, 12288 x 2048
-//    11.3 / 7.9 / 8.5.  With two row tiles, which halve the reads of x, where those weigh and the layer is no wider than 8192 (16
-//    tokens, one and two tiles: 8192 x 28672 83.8 and 58.8, 8192 x 4096 14.8 and 13.4, but 8192 x 2048 9.1 and 9.9; 12 tokens, 12288 x 4096
-//    18.4 and 19.5).
-//  * beyond, three workgroups of eight waves per CU do not hold the layer any more: four (one token, eight and four: 14336 x 4096
-//    17.0 and 15.6, 16384 x 1024 7.9 and 6.9), unless the contraction is long (28672 x 8192 46.8 and 49.3); two tiles from 5 tokens on
-//    where x is large enough (14336 x 4096 at 8 tokens 21.2 and 18.4, 16384 x 1024 7.7 and 8.7).
+// enter the sums.  Measured over 27 layers of 256 - 28672 rows and 1024 - 28672 columns (us, weights from HBM, launch gap included):
+//  * eight waves (4096 x 4096 at 1 / 13 tokens, h formed inside: four 8.7 / 9.3, eight 6.7 / 7.9, sixteen 7.6 / 8.8; 2048 x 8192 at 13: 14.6 /
+//    11.1 / 12.3), four where the layer has workgroups to spare and a short contraction (gate / up pair of 14336 x 4096, eight and
+//    four: 21.8 and 20.6);
+//  * two row tiles, which share the reads of x and lora_a, from 8192 rows on (8192 x 2048 at 13 tokens: one 7.9, two 7.0; 14336 x 4096 at one
+//    token with its h: 17.8 and 14.9), but one where four waves at a few tokens read h instead (the same layer 13.9, two 16.1).
 struct FewConfig {
   int rt, waves;
   bool operator==(const FewConfig& o) const { return rt == o.rt && waves == o.waves; }
 };
-FewConfig few_config(int64_t M, int64_t N, int64_t K) {
-  if (N <= 4096 || (N < 8192 && N <= K)) return {1, 16};
-  if (N <= 12288) return {N <= 8192 && M * K >= 40960 ? 2 : 1, 8};
-  return {M > 4 && M * K >= 16384 ? 2 : 1, K < 8192 ? 4 : 8};
+int few_waves(int64_t N, int64_t K) { return N > 12288 && K < 8192 ? 4 : 8; }
+FewConfig few_config(int64_t M, int64_t N, int64_t K, bool hidden) {
+  const int waves = few_waves(N, K);
+  return {N >= 8192 && (hidden || waves == 8 || M > 4) ? 2 : 1, waves};
+}
+FewConfig few_pair_config(int64_t N, int64_t K, bool hidden) {
+  const int waves = few_waves(N, K);
+  return {hidden && waves == 4 ? 4 : 2, waves};
+}
+// Whether a launch of these workgroups forms its members' h = x . lora_a^T itself, instead of a launch or two ahead of it (4 - 6.5 us,
+// and as many launches for the host).  Every workgroup then reads its members' lora_a, rank_tiles tiles of 16 ranks: at 128 MB
+// for the launch still the better way (4096 x 14336: one token 15.6 against 20.2 us, 13 tokens 20.4 against 22.0; at 235 MB, 8192 x
+// 28672, no longer), and several tiles only where the LDS they take (`bytes` a workgroup) leaves room for every workgroup at once
+// (gate / up pair of 8192 x 2048, 512 workgroups in two rounds: 15.1 against 12.1; in one round, 2816 x 1024: 6.8 against 8.7).
+bool few_hidden(int64_t workgroups, int rank_tiles, int64_t K, int bytes) {
+  if (rank_tiles > 1 && workgroups > 256 * (160 * 1024 / bytes)) return false;
+  return workgroups * rank_tiles * 32 * K <= int64_t(128) << 20;
+}
+int few_bytes(int rt, int rank_tiles, int64_t M, int64_t K, int waves) {
+  const int cols = 16384 / rt, kb = (int)(K < cols ? K : cols) >> 6, n_chunks = (int)((K + 127) >> 7);
+  return 1024 + 64 * rt * (kb | 1) + (n_chunks < waves ? n_chunks : waves) * ((M <= 4 ? 1 : 4) + rt + 4 * rank_tiles) * 1024;
 }
 
-template <int RT, int MAXW, bool PAIR>
-int launch_few(SmallMGroup& g, void* act, hipStream_t s) {
-  int wgs = 0;
-  for (int i = 0; i < (PAIR ? 1 : g.n); ++i) {
-    wgs += g.m[i].N / (PAIR ? 16 : 16 * RT);
-    g.wg_end[i] = wgs;
+template <int RT, int MAXW, int MQ, int NA, bool PAIR, bool ONE>
+int launch_few(const SmallMGroup& g, unsigned wgs, uint16_t* act, hipStream_t s) {
+  constexpr int NT = NA * (PAIR ? 2 : 1);
+  using L = FewLayout<RT, NT, MQ>;
+  const int K = g.m[0].K, n_chunks = (K + 127) >> 7, waves = n_chunks < MAXW ? n_chunks : MAXW;
+  static bool attr_set[64] = {};  // the LDS limit is a per-device attribute of the function
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;
+  if (dev < 0 || !attr_set[dev]) {
+    const int most = L::bytes(L::kSegment, MAXW);
+    static_assert(FewLayout<RT, NT, MQ>::kLut + 16 * RT * (16384 / RT / 64 + 1) * 4 + MAXW * FewLayout<RT, NT, MQ>::kStage <= 160 * 1024,
+                  "the LDS of a CU");
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&nf4_few_kernel<RT, MAXW, MQ, NA, PAIR, ONE>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, most);
+    if (e != hipSuccess) return fail(TTAMD_ELAUNCH, "nf4_few: cannot reserve %d bytes of LDS: %s", most, hipGetErrorString(e));
+    if (dev >= 0) attr_set[dev] = true;
   }
-  const int n_chunks = (g.m[0].K + 127) >> 7;
-  const dim3 grid((unsigned)wgs), block(64 * (n_chunks < MAXW ? n_chunks : MAXW));
-  if (!PAIR && g.n == 1)
-    nf4_few_kernel<RT, MAXW, PAIR, true><<<grid, block, 0, s>>>(g, nullptr);
-  else
-    nf4_few_kernel<RT, MAXW, PAIR, false><<<grid, block, 0, s>>>(g, reinterpret_cast<uint16_t*>(act));
+  nf4_few_kernel<RT, MAXW, MQ, NA, PAIR, ONE><<<dim3(wgs), dim3(64 * waves), L::bytes(K, waves), s>>>(g, act);
   return check_launch("nf4_few");
 }
 
-int dispatch_few(SmallMGroup& g, const FewConfig& c, void* pair_act, hipStream_t s) {
-  if (pair_act) {
-    if (c.waves == 16) return launch_few<2, 16, true>(g, pair_act, s);
-    return c.waves == 8 ? launch_few<2, 8, true>(g, pair_act, s) : launch_few<2, 4, true>(g, pair_act, s);
+template <int RT, int MAXW, int MQ, int NA>
+int launch_few_members(SmallMGroup& g, hipStream_t s) {
+  int wgs = 0;
+  for (int i = 0; i < g.n; ++i) {
+    wgs += g.m[i].N / (16 * RT);
+    g.wg_end[i] = wgs;
   }
-  if (c.waves == 16) return launch_few<1, 16, false>(g, nullptr, s);
-  if (c.waves == 8) return c.rt == 2 ? launch_few<2, 8, false>(g, nullptr, s) : launch_few<1, 8, false>(g, nullptr, s);
-  return c.rt == 2 ? launch_few<2, 4, false>(g, nullptr, s) : launch_few<1, 4, false>(g, nullptr, s);
+  return g.n == 1 ? launch_few<RT, MAXW, MQ, NA, false, true>(g, wgs, nullptr, s) : launch_few<RT, MAXW, MQ, NA, false, false>(g, wgs, nullptr, s);
+}
+
+// rank_tiles: of a member, where the launch forms h; 0 where it reads it
+template <int MQ, int NA>
+int dispatch_few_members(SmallMGroup& g, const FewConfig& c, hipStream_t s) {
+  if (c.rt == 1) {
+    if constexpr (MQ == 1 && NA == 0) {
+      if (c.waves == 4) return launch_few_members<1, 4, MQ, NA>(g, s);
+    }
+    return launch_few_members<1, 8, MQ, NA>(g, s);
+  }
+  return c.waves == 8 ? launch_few_members<2, 8, MQ, NA>(g, s) : launch_few_members<2, 4, MQ, NA>(g, s);
+}
+int dispatch_few(SmallMGroup& g, const FewConfig& c, int rank_tiles, hipStream_t s) {
+  const bool one = g.m[0].M <= 4;  // group of four tokens
+  switch (rank_tiles) {
+    case 0: return one ? dispatch_few_members<1, 0>(g, c, s) : dispatch_few_members<4, 0>(g, c, s);
+    case 1: return one ? dispatch_few_members<1, 1>(g, c, s) : dispatch_few_members<4, 1>(g, c, s);
+    default: return one ? dispatch_few_members<1, 2>(g, c, s) : dispatch_few_members<4, 2>(g, c, s);
+  }
+}
+int dispatch_few_pair(const SmallMGroup& g, const FewConfig& c, bool hidden, uint16_t* act, hipStream_t s) {
+  const unsigned wgs = g.m[0].N / (8 * c.rt);
+  const bool one = g.m[0].M <= 4;
+  if (hidden) {
+    if (c.rt == 4) return launch_few<4, 4, 1, 1, true, false>(g, wgs, act, s);  // few_pair_hidden: at most four tokens
+    return one ? launch_few<2, 8, 1, 1, true, false>(g, wgs, act, s) : launch_few<2, 8, 4, 1, true, false>(g, wgs, act, s);
+  }
+  if (c.waves == 4) return one ? launch_few<2, 4, 1, 0, true, false>(g, wgs, act, s) : launch_few<2, 4, 4, 0, true, false>(g, wgs, act, s);
+  return one ? launch_few<2, 8, 1, 0, true, false>(g, wgs, act, s) : launch_few<2, 8, 4, 0, true, false>(g, wgs, act, s);
 }
 
 // Shape of a launch of 17 - 64 tokens: token tiles, row tiles per workgroup, chunks in flight per wave, most waves.  It fixes
@@ -536,50 +765,112 @@ int run_small_m(const void* x, const uint8_t* codes, const void* bscal, const vo
   a.y = reinterpret_cast<uint16_t*>(y);
   a.M = (int)M; a.N = (int)N; a.K = (int)K; a.R = R; a.ldh = ldh;
   a.lscale = lscale;
-  if (M <= kFewTokens) return dispatch_few(g, few_config(M, N, K), nullptr, s);
+  if (M <= kFewTokens && K < kFewMaxK) return dispatch_few(g, few_config(M, N, K, false), 0, s);
   return dispatch_small_m(g, small_m_config(M, N, K), s);
 }
 
-// The members of a group (same x, M, K) in as few launches as their launch shapes allow: consecutive members with
-// the same shape share one.  act != nullptr (two members of equal width): *act_done says whether the launch wrote
-// act = silu(y_0) * y_1 too.
-int run_small_m_group(const void* x, const GroupGemm& gg, const void* h_cat, void* act, bool* act_done, hipStream_t s) {
+namespace {
+int small_m_args(SmallMArgs (&all)[kGroupMax], const void* x, const GroupGemm& gg, const void* h_cat) {
   TT_REQUIRE(gg.M > 0 && gg.M <= small_m_limit(), "nf4_small_m: M (%lld) out of range", (long long)gg.M);
-  SmallMArgs all[kGroupMax] = {};
   for (int j = 0; j < gg.n; ++j) {
     TT_REQUIRE(gg.N[j] / 16 < (int64_t(1) << 27) && gg.N[j] * gg.K < (int64_t(1) << 40), "nf4_small_m: weight too large");
     SmallMArgs& a = all[j];
     a.x = reinterpret_cast<const uint16_t*>(x);
     a.codes = gg.codes[j];
     a.bscal = gg.bscal[j];
-    a.h = reinterpret_cast<const uint16_t*>(h_cat) + gg.r_off[j];
+    a.h = h_cat ? reinterpret_cast<const uint16_t*>(h_cat) + gg.r_off[j] : nullptr;
     a.lora_b = gg.lora_b[j];
     a.bias = gg.bias[j];
     a.y = gg.y[j];
     a.M = (int)gg.M; a.N = (int)gg.N[j]; a.K = (int)gg.K; a.R = gg.rank[j]; a.ldh = gg.r_off[gg.n];
     a.lscale = gg.scale[j];
   }
-  const bool few = gg.M <= kFewTokens;
+  return TTAMD_OK;
+}
+// members [i, j) share a launch
+template <typename Same>
+int run_of(const GroupGemm& gg, int i, Same same) {
+  int j = i + 1;
+  while (j < gg.n && same(i, j)) ++j;
+  return j;
+}
+bool same_few(const GroupGemm& gg, int i, int j, bool hidden) {
+  return few_config(gg.M, gg.N[j], gg.K, hidden) == few_config(gg.M, gg.N[i], gg.K, hidden);
+}
+int rank_tiles_of(const GroupGemm& gg, int i, int j) {
+  int most = 0;
+  for (int q = i; q < j; ++q) most = gg.rank[q] > most ? gg.rank[q] : most;
+  return (most + 15) / 16;
+}
+}  // namespace
+
+// The members of a group (same x, M, K) in as few launches as their launch shapes allow: consecutive members with
+// the same shape share one.  act != nullptr (two members of equal width): *act_done says whether the launch wrote
+// act = silu(y_0) * y_1 too.
+int run_small_m_group(const void* x, const GroupGemm& gg, const void* h_cat, void* act, bool* act_done, hipStream_t s) {
+  SmallMArgs all[kGroupMax] = {};
+  if (int rc = small_m_args(all, x, gg, h_cat)) return rc;
+  const bool few = gg.M <= kFewTokens && gg.K < kFewMaxK;
   if (act && few && gg.n == 2 && gg.N[0] == gg.N[1]) {
     SmallMGroup g = {};
     g.m[0] = all[0];
     g.m[1] = all[1];
     g.n = 2;
     *act_done = true;
-    return dispatch_few(g, few_config(gg.M, gg.N[0], gg.K), act, s);
+    return dispatch_few_pair(g, few_pair_config(gg.N[0], gg.K, false), false, reinterpret_cast<uint16_t*>(act), s);
   }
-  int i = 0;
-  while (i < gg.n) {
+  for (int i = 0; i < gg.n;) {
     SmallMGroup g = {};
-    int j = i;
-    auto same = [&](int q) {
-      return few ? few_config(gg.M, gg.N[q], gg.K) == few_config(gg.M, gg.N[i], gg.K)
-                 : small_m_config(gg.M, gg.N[q], gg.K) == small_m_config(gg.M, gg.N[i], gg.K);
-    };
-    for (; j < gg.n && same(j); ++j) g.m[j - i] = all[j];
+    const int j = run_of(gg, i, [&](int p, int q) {
+      return few ? same_few(gg, p, q, false) : small_m_config(gg.M, gg.N[q], gg.K) == small_m_config(gg.M, gg.N[p], gg.K);
+    });
+    for (int q = i; q < j; ++q) g.m[q - i] = all[q];
     g.n = j - i;
-    if (int rc = few ? dispatch_few(g, few_config(gg.M, gg.N[i], gg.K), nullptr, s) : dispatch_small_m(g, small_m_config(gg.M, gg.N[i], gg.K), s))
-      return rc;
+    if (int rc = few ? dispatch_few(g, few_config(gg.M, gg.N[i], gg.K, false), 0, s) : dispatch_small_m(g, small_m_config(gg.M, gg.N[i], gg.K), s)) return rc;
+    i = j;
+  }
+  return TTAMD_OK;
+}
+
+bool few_forms_hidden(const GroupGemm& gg, bool gated) {
+  if (gg.M > kFewTokens || gg.K >= kFewMaxK) return false;
+  for (int i = 0; i < gg.n; ++i)
+    if (gg.rank[i] < 8 || gg.rank[i] > kFewHiddenRank) return false;
+  if (gated) {
+    const FewConfig c = few_pair_config(gg.N[0], gg.K, true);
+    return rank_tiles_of(gg, 0, 2) == 1 && (c.rt == 2 || gg.M <= 4) && few_hidden(gg.N[0] / (8 * c.rt), 2, gg.K, few_bytes(c.rt, 2, gg.M, gg.K, c.waves));
+  }
+  for (int i = 0; i < gg.n;) {
+    const int j = run_of(gg, i, [&](int p, int q) { return same_few(gg, p, q, true); });
+    int64_t wgs = 0;
+    for (int q = i; q < j; ++q) wgs += gg.N[q] / (16 * few_config(gg.M, gg.N[q], gg.K, true).rt);
+    const FewConfig c = few_config(gg.M, gg.N[i], gg.K, true);
+    const int tiles = rank_tiles_of(gg, i, j);
+    if (!few_hidden(wgs, tiles, gg.K, few_bytes(c.rt, tiles, gg.M, gg.K, c.waves))) return false;
+    i = j;
+  }
+  return true;
+}
+
+int run_few_with_hidden(const void* x, const GroupGemm& gg, const uint16_t* const* lora_a, void* h_cat, void* act, hipStream_t s) {
+  SmallMArgs all[kGroupMax] = {};
+  if (int rc = small_m_args(all, x, gg, nullptr)) return rc;
+  for (int q = 0; q < gg.n; ++q) {
+    all[q].lora_a = lora_a[q];
+    all[q].h_out = h_cat ? reinterpret_cast<uint16_t*>(h_cat) + gg.r_off[q] : nullptr;
+  }
+  SmallMGroup g = {};
+  if (act) {
+    g.m[0] = all[0];
+    g.m[1] = all[1];
+    g.n = 2;
+    return dispatch_few_pair(g, few_pair_config(gg.N[0], gg.K, true), true, reinterpret_cast<uint16_t*>(act), s);
+  }
+  for (int i = 0; i < gg.n;) {
+    const int j = run_of(gg, i, [&](int p, int q) { return same_few(gg, p, q, true); });
+    for (int q = i; q < j; ++q) g.m[q - i] = all[q];
+    g.n = j - i;
+    if (int rc = dispatch_few(g, few_config(gg.M, gg.N[i], gg.K, true), rank_tiles_of(gg, i, j), s)) return rc;
     i = j;
   }
   return TTAMD_OK;
