@@ -61,6 +61,22 @@ def test_few_token_forward(kind, qp, n, k, group, bias, m):
     assert bool(((got.double() - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("kind,qp", [("8da4w", torch.float32), ("8da4w", torch.bfloat16), ("4w", torch.bfloat16)])
+@pytest.mark.parametrize("n,k,group", [(2048, 4128, 32), (2048, 4608, 256), (8192, 96, 32), (8256, 1536, 64), (320, 16384, 128), (2112, 32768, 256), (2112, 33024, 256)])
+@pytest.mark.parametrize("m", [1, 2, 4, 5, 8, 16])
+def test_streaming_launch_shapes(kind, qp, n, k, group, m):
+    """Eight and sixteen waves, one and two row tiles, the largest activation a workgroup quantises and the next, a last chunk of
+    one to three groups of 32: within the bound above, and a row's bits do not depend on the batch around it."""
+    layer = _layer(kind, n, k, group, False, qp)
+    x = torch.randn(m, k, generator=torch.Generator().manual_seed(m)).to(torch.bfloat16).to(DEV)
+    with torch.no_grad():
+        got, first = layer(x), layer(x[:1].contiguous())
+    xd, w = _operands(layer, x)
+    want, size = xd @ w.t(), xd.abs() @ w.abs().t()
+    assert bool(((got.double() - want).abs() <= want.abs() * 2.0 ** -8 + size * (k * 2.0 ** -23)).all())
+    assert torch.equal(got[:1], first)
+
+
 @pytest.mark.parametrize("m", [5, 20])  # the streaming and the tiled kernel
 def test_scales_at_the_top_of_the_range_expand_to_the_dense_weights_bits(m):
     """One-hot rows read single weights: (q - 8) * scale is finite for every code but 0, while 8 * scale is not."""

@@ -9,24 +9,27 @@
 //
 // Two kernels, by the number of tokens:
 //  * int4_stream_kernel (at most 16): bound by the weight stream.  A workgroup owns 16 or 32 weight rows and the whole
-//    contraction; its waves take 128-wide chunks of K in turn (one chunk in flight per wave: neighbouring waves then read
-//    neighbouring pieces of the rows, which beats two or four chunks per wave at every size).
-//    The lane that feeds an MFMA holds 32 consecutive k of one row (whole 128-byte lines of int8 weight per row), x
-//    comes from the cache - only the lanes of tokens that exist ask for it.  Partial sums meet in LDS in wave order.
+//    contraction; its waves take 128-wide chunks of K in turn, one in flight each while the one before it is multiplied.
+//    Neighbouring waves then read neighbouring pieces of the rows.  The lane that feeds an MFMA holds 32 consecutive k of one
+//    row; a chunk's codes, scales and x come by direct-to-LDS loads in row order and are read from there.  Partial sums
+//    meet in LDS in wave order.
 //  * int4_tile_kernel (more): the few-token kernel would read all of x in every workgroup (at 75 tokens nine times the
 //    bytes of its weight rows).  Four waves own 64 weight rows between them and share 128-wide chunks of up to 128
 //    tokens through a double LDS buffer; a weight fragment is expanded once per 128 tokens.  Launches of few tiles cut
 //    the contraction into slices (fp32 slabs, added in slice order by int4_reduce_kernel).
 //
 // Measured against dequantise + library GEMM (us, weights from HBM, launch gaps included; int8 / uint4):
-//   14336 x 4096:  1 token 60 / 60 -> 22 / 20, 16 tokens 59 / 60 -> 28 / 21, 75 tokens 63 / 65 -> 38 / 33, 256 tokens 83 / 82 -> 67 / 69
-//   4096 x 14336:  1 token 58 / 58 -> 23 / 19, 75 tokens 79 / 78 -> 38 / 32, 256 tokens 93 / 92 -> 74 / 66
-//   1024 x 4096:   1 token 20 / 20 ->  8 /  7, 256 tokens 21 / 21 -> 17 / 16
-// A launch's fixed part is about 6 us of these; what goes beyond it streams int8 weight at 3.6 TB/s.  Above 256 tokens the
-// two m-tiles' expansion and their slabs cost what the dense copy costs, and the library's larger tiles win.
+//   14336 x 4096:  1 token 60 / 60 -> 17.7 / 16.1, 16 tokens 59 / 60 -> 25 / 17.8, 75 tokens 63 / 65 -> 38 / 33, 256 tokens 83 / 82 -> 67 / 69
+//   4096 x 14336:  1 token 58 / 58 -> 16.5 / 15.3, 75 tokens 79 / 78 -> 38 / 32, 256 tokens 93 / 92 -> 74 / 66
+//   1024 x 4096:   1 token 20 / 20 -> 6.1 / 5.9, 256 tokens 21 / 21 -> 17 / 16
+// (at most 16 tokens with loads straight into the MFMA lanes and one wave's sum at the end: 26.4 / 19.0, 21.9 / 19.5 and 9.0 / 7.3 at
+// one token; a read of the same bytes takes 14 / 6.5).  Above 256 tokens the two m-tiles' expansion and their slabs cost what
+// the dense copy costs, and the library's larger tiles win.
 #include "common.h"
 #include "fq_math.h"
 #include "nf4_math.h"
+
+#define TT_LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
 
 namespace ttamd {
 namespace {
@@ -203,99 +206,198 @@ __device__ __forceinline__ void quantise_tokens(const Int4Args& a, const u32x4_t
   __syncthreads();
 }
 
-// RT tiles of 16 weight rows per workgroup (they share a wave's fragments of x), at most MAXW waves (DYN: exactly).
-template <int FMT, int RT, int MAXW, bool DYN>
+// One wave's stage of a streaming workgroup in LDS: 128 columns of x (MQ groups of four tokens; none where the workgroup
+// quantised x itself), of the codes of RT row tiles, and of their scales and zero points.
+template <int FMT, int RT, int MQ>
+struct StreamStage {
+  static constexpr int kX = MQ * 1024;
+  static constexpr int kCodes = FMT == kUint4 ? 1024 : 2048;
+  static constexpr int kScales = FMT == kInt8F32 ? 512 : FMT == kUint4 ? 256 : 0;  // bf16 scales go to registers
+  static constexpr int kBytes = kX + RT * (kCodes + kScales);
+};
+
+// RT tiles of 16 weight rows per workgroup (they share a wave's fragments of x), at most MAXW waves (DYN: exactly).  Dynamic
+// LDS: DYN: the quantised x; then the waves' stages.  Everything a chunk needs comes by direct-to-LDS loads in row order
+// (four neighbouring lanes ask for one row's neighbouring bytes: the address unit takes them together; straight into the
+// lanes of an MFMA operand, whose neighbours are different rows, it was what bounded the kernel).
+template <int FMT, int RT, int MAXW, bool DYN, int MQ>
 __global__ __launch_bounds__(64 * MAXW) void int4_stream_kernel(const Int4Args a) {
-  __shared__ float red[(MAXW - 1) * RT * 256];
-  __shared__ __attribute__((aligned(16))) uint16_t xq[DYN ? kDynPieces * 8 * 64 * MAXW : 8];
+#if defined(__HIP_DEVICE_COMPILE__)  // LDS address-space casts
+  using S = StreamStage<FMT, RT, DYN ? 0 : MQ>;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
   __shared__ float ext[2][DYN ? kDynPieces * MAXW : 1];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nw = blockDim.x >> 6;
   const int i = lane & 15, g = lane >> 4;
   const int n0 = (int)blockIdx.x * (16 * RT);  // N % 64 == 0: every row of the workgroup exists
-  const bool token = i < a.M;
-  const uint16_t* xrow = (DYN ? xq : a.x) + (int64_t)(token ? i : 0) * a.K + 32 * g;
+  uint16_t* const xq = reinterpret_cast<uint16_t*>(smem);
+  const int xq_bytes = DYN ? a.M * a.K * 2 : 0;
+  char* const stages = smem + ((xq_bytes + 1023) & ~1023);
+  char* const stage = stages + wave * S::kBytes;
+  const uint32_t lds = (uint32_t)(uintptr_t)TT_LDS_PTR(stage);
+  auto dma16 = [&](uint32_t voff, const void* base, uint32_t at) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "s"(at) : "memory", "m0");
+  };
+  auto dma4 = [&](uint32_t voff, const void* base, uint32_t at) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(base), "s"(at) : "memory", "m0");
+  };
   const int n_chunks = (a.K + 127) >> 7;
-  WeightPiece<FMT> w[RT];
+  // Piece p of row r goes to slot p ^ (a function of r) such that an operand's 16 lanes read disjoint banks.  int8: 8 pieces
+  // a row and chunk, 8 rows an instruction; uint4: 4 and 16; x: 16 and 4.  Pieces beyond K repeat one of the first 32
+  // columns (K % 32 == 0: they exist); what they hold is zeroed where it would count.
+  float sc_next[RT], z_next[RT];  // bf16 scales
   auto request = [&](int c) {
-    const int k = c * 128 + 32 * g;
+    const int left = a.K - c * 128;  // columns, at least 32
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
-      if (k < a.K)  // K % 32 == 0
-        w[rt].load(a, n0 + 16 * rt + i, k);
-      else
-        w[rt].clear();
+      const int64_t row0 = n0 + 16 * rt;
+      if constexpr (FMT == kUint4) {
+        const int r = lane >> 2;
+        int p = (lane & 3) ^ ((r >> 2) & 3);
+        p = 32 * p < left ? p : 0;
+        dma16((uint32_t)r * (uint32_t)(a.K >> 1) + 16 * p, a.q + ((row0 * a.K) >> 1) + (int64_t)c * 64, lds + S::kX + rt * S::kCodes);
+      } else {
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+          const int r = 8 * d + (lane >> 3);
+          int p = (lane & 7) ^ (r >> 1);
+          p = 16 * p < left ? p : p & 1;
+          dma16((uint32_t)r * (uint32_t)a.K + 16 * p, a.q + row0 * a.K + (int64_t)c * 128, lds + S::kX + rt * S::kCodes + d * 1024);
+        }
+      }
+      if constexpr (FMT == kUint4) {  // [K / g, N]: 16 rows are 64 contiguous bytes; slot i + 16 g
+        const int k = c * 128 + (32 * g < left ? 32 * g : 0);
+        dma4((uint32_t)(((k >> a.log2_group) * (int64_t)a.N + i) * 4), reinterpret_cast<const uint32_t*>(a.scale) + row0,
+             lds + S::kX + RT * S::kCodes + rt * S::kScales);
+      } else {
+        const int64_t groups = a.K >> a.log2_group;
+        if constexpr (FMT == kInt8F32) {  // [N, K / g]; slot 4 row + group of 32
+          const int k = c * 128 + (32 * (lane & 3) < left ? 32 * (lane & 3) : 0);
+          const uint32_t off = (uint32_t)(((lane >> 2) * groups + (k >> a.log2_group)) * 4);
+          dma4(off, reinterpret_cast<const float*>(a.scale) + row0 * groups, lds + S::kX + RT * S::kCodes + rt * S::kScales);
+          if (a.zero) dma4(off, reinterpret_cast<const float*>(a.zero) + row0 * groups, lds + S::kX + RT * S::kCodes + rt * S::kScales + 256);
+        } else {
+          const int64_t at = (row0 + i) * groups + ((c * 128 + (32 * g < left ? 32 * g : 0)) >> a.log2_group);
+          sc_next[rt] = bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(a.scale)[at]);
+          z_next[rt] = a.zero ? bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(a.zero)[at]) : 0.f;
+        }
+      }
+    }
+    if constexpr (!DYN) {
+#pragma unroll
+      for (int d = 0; d < MQ; ++d) {
+        const int r = 4 * d + (lane >> 4), row = r < a.M ? r : a.M - 1;  // rows beyond M repeat the last one: never stored
+        int p = (lane & 15) ^ r;
+        p = 8 * p < left ? p : p & 3;
+        dma16((uint32_t)row * (uint32_t)a.K * 2u + 16 * p, reinterpret_cast<const char*>(a.x) + (int64_t)c * 256, lds + d * 1024);
+      }
     }
   };
   int c = wave;
   if constexpr (DYN) {
-    u32x4_t raw[kDynPieces];  // asked for ahead of the weights, which then stay in flight while it is quantised
+    // x is asked for ahead of the weights, which then stay in flight while it is quantised; a thread's pieces are brought by
+    // its own wave
+    const int total = a.M * (a.K >> 3);
+#pragma unroll
+    for (int j = 0; j < kDynPieces; ++j) {
+      const int first = (j * MAXW + wave) * 64;
+      if (first < total) dma16((uint32_t)(first + lane < total ? first + lane : first) * 16u, a.x, (uint32_t)(uintptr_t)TT_LDS_PTR(smem) + first * 16);
+    }
+    if (c < n_chunks) {
+      request(c);
+      if (FMT == kInt8F32 && a.zero)
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * RT) : "memory");
+      else
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((FMT == kInt8F32 ? 3 : 2) * RT) : "memory");
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    u32x4_t raw[kDynPieces];
 #pragma unroll
     for (int j = 0; j < kDynPieces; ++j) {
       const int piece = j * 64 * MAXW + (int)threadIdx.x;
       raw[j] = u32x4_t{0, 0, 0, 0};
-      if (piece < a.M * (a.K >> 3)) raw[j] = reinterpret_cast<const u32x4_t*>(a.x)[piece];
+      if (piece < total) raw[j] = reinterpret_cast<const u32x4_t*>(xq)[piece];
     }
-    if (c < n_chunks) request(c);
     quantise_tokens<64 * MAXW>(a, raw, xq, ext);
   } else {
     if (c < n_chunks) request(c);
   }
-  f32x4_t acc[RT][4];
+  constexpr int kChains = 2;
+  f32x4_t acc[RT][kChains];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-    for (int s = 0; s < 4; ++s) acc[rt][s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < kChains; ++s) acc[rt][s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  while (c < n_chunks) {
+  const int xr = i & (4 * MQ - 1);  // DYN: tokens beyond M read the first one
+  const uint16_t* xrow = xq + (int64_t)(i < a.M ? i : 0) * a.K + 32 * g;
+  for (; c < n_chunks; c += nw) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // the stage goes to registers and is asked for again
+    WeightPiece<FMT> w[RT];
     u32x4_t xb[4];
-    const bool in = c * 128 + 32 * g < a.K;
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      const char* codes = stage + S::kX + rt * S::kCodes;
+      const char* scales = stage + S::kX + RT * S::kCodes + rt * S::kScales;
+      if constexpr (FMT == kUint4) {
+        w[rt].codes = *reinterpret_cast<const u32x4_t*>(codes + i * 64 + ((g ^ ((i >> 2) & 3)) << 4));
+        w[rt].sz = *reinterpret_cast<const uint32_t*>(scales + lane * 4);
+      } else {
+#pragma unroll
+        for (int d = 0; d < 2; ++d) w[rt].v[d] = *reinterpret_cast<const u32x4_t*>(codes + i * 128 + (((2 * g + d) ^ (i >> 1)) << 4));
+        if constexpr (FMT == kInt8F32) {
+          w[rt].sc = *reinterpret_cast<const float*>(scales + i * 16 + g * 4);
+          w[rt].z = a.zero ? *reinterpret_cast<const float*>(scales + 256 + i * 16 + g * 4) : 0.f;
+        } else {
+          w[rt].sc = sc_next[rt];
+          w[rt].z = z_next[rt];
+        }
+      }
+    }
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      xb[s] = u32x4_t{0, 0, 0, 0};
-      if (in && token) xb[s] = *reinterpret_cast<const u32x4_t*>(xrow + c * 128 + 8 * s);
+      if constexpr (DYN)
+        xb[s] = *reinterpret_cast<const u32x4_t*>(xrow + c * 128 + 8 * s);
+      else
+        xb[s] = *reinterpret_cast<const u32x4_t*>(stage + xr * 256 + (((4 * g + s) ^ xr) << 4));
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (c + nw < n_chunks) request(c + nw);
+    if (c * 128 + 32 * g >= a.K) {  // nothing beyond K counts, whatever lies there
+#pragma unroll
+      for (int s = 0; s < 4; ++s) xb[s] = u32x4_t{0, 0, 0, 0};
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt) w[rt].clear();
     }
 #pragma unroll
     for (int s = 0; s < 4; ++s)
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
-        acc[rt][s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w[rt].operand(s)),
-                                                             __builtin_bit_cast(bf16x8_t, xb[s]), acc[rt][s], 0, 0, 0);
-    c += nw;
-    if (c < n_chunks) request(c);
+        acc[rt][s % kChains] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w[rt].operand(s)),
+                                                                       __builtin_bit_cast(bf16x8_t, xb[s]), acc[rt][s % kChains], 0, 0, 0);
   }
+  // partial sums, [tile][lane][v] at the head of each wave's stage, added in wave order by all threads
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-#pragma unroll
-    for (int s = 1; s < 4; ++s) acc[rt][0] += acc[rt][s];
-    if (wave > 0) {
-#pragma unroll
-      for (int v = 0; v < 4; ++v) red[((wave - 1) * RT + rt) * 256 + v * 64 + lane] = acc[rt][0][v];
-    }
-  }
+  for (int rt = 0; rt < RT; ++rt) *reinterpret_cast<f32x4_t*>(stage + rt * 1024 + lane * 16) = acc[rt][0] + acc[rt][1];
   __syncthreads();
-  if (wave != 0) return;
+  for (int e = threadIdx.x; e < 256 * RT; e += blockDim.x) {
+    const int token = (e >> 2) & 15, n = n0 + 16 * (e >> 8) + 4 * ((e >> 6) & 3) + (e & 3);
+    if (token >= a.M) continue;
+    const char* p = stages + (e >> 8) * 1024 + (e & 255) * 4;
+    float o = *reinterpret_cast<const float*>(p);
+    if (nw == MAXW) {
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    // acc[rt][0][v] = the wave's share of y[i][n0 + 16 rt + 4 g + v]
-    float o[4];
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      o[v] = acc[rt][0][v];
-      for (int q = 0; q < nw - 1; ++q) o[v] += red[(q * RT + rt) * 256 + v * 64 + lane];
+      for (int q = 1; q < MAXW; ++q) o += *reinterpret_cast<const float*>(p + q * S::kBytes);
+    } else {
+      for (int q = 1; q < nw; ++q) o += *reinterpret_cast<const float*>(p + q * S::kBytes);
     }
-    if (!token) continue;
-    const int nb = n0 + 16 * rt + 4 * g;
-    if (a.bias) {
-      const u32x2_t b = *reinterpret_cast<const u32x2_t*>(a.bias + nb);
-      o[0] += lo_of(b.x); o[1] += hi_of(b.x); o[2] += lo_of(b.y); o[3] += hi_of(b.y);
-    }
-    u32x2_t out;
-    out.x = pack_pair(o[0], o[1]);
-    out.y = pack_pair(o[2], o[3]);
-    *reinterpret_cast<u32x2_t*>(a.y + (int64_t)i * a.N + nb) = out;
+    if (a.bias) o += bf16_bits_to_f32(a.bias[n]);
+    a.y[(int64_t)token * a.N + n] = (uint16_t)pack_pair(o, 0.f);
   }
+#endif
 }
 
 // Four waves, 64 weight rows, 16 MT tokens; blockIdx = (row tile, token tile, slice of the contraction).
@@ -445,43 +547,54 @@ void launch_tile(const Int4Args& a, int mt, dim3 grid, hipStream_t s) {
   }
 }
 
-template <int FMT, int RT, int MAXW>
-void launch_stream(const Int4Args& a, bool dyn, hipStream_t s) {
-  const int n_chunks = (a.K + 127) >> 7;
-  if constexpr (FMT != kUint4) {
-    if (dyn) {
-      int4_stream_kernel<FMT, RT, MAXW, true><<<dim3(a.N / (16 * RT)), dim3(64 * MAXW), 0, s>>>(a);
-      return;
-    }
+template <int FMT, int RT, int MAXW, bool DYN, int MQ>
+int launch_stream(const Int4Args& a, hipStream_t s) {
+  using S = StreamStage<FMT, RT, DYN ? 0 : MQ>;
+  const int n_chunks = (a.K + 127) >> 7, waves = DYN || n_chunks > MAXW ? MAXW : n_chunks;
+  const int head = DYN ? (a.M * a.K * 2 + 1023) & ~1023 : 0;
+  constexpr int kMost = (DYN ? 64 * MAXW * kDynPieces * 16 + 1023 : 0) + MAXW * S::kBytes;
+  static_assert(kMost + 2 * 4 * kDynPieces * MAXW <= 160 * 1024, "the LDS of a CU");
+  static_assert(S::kBytes >= RT * 1024, "the partial sums fit a stage");
+  static bool attr_set[64] = {};  // the LDS limit is a per-device attribute of the function
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;
+  if (dev < 0 || !attr_set[dev]) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&int4_stream_kernel<FMT, RT, MAXW, DYN, MQ>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, kMost);
+    if (e != hipSuccess) return fail(TTAMD_ELAUNCH, "int4_linear: cannot reserve %d bytes of LDS: %s", kMost, hipGetErrorString(e));
+    if (dev >= 0) attr_set[dev] = true;
   }
-  int4_stream_kernel<FMT, RT, MAXW, false><<<dim3(a.N / (16 * RT)), dim3(64 * (n_chunks < MAXW ? n_chunks : MAXW)), 0, s>>>(a);
+  int4_stream_kernel<FMT, RT, MAXW, DYN, MQ><<<dim3(a.N / (16 * RT)), dim3(64 * waves), head + waves * S::kBytes, s>>>(a);
+  return check_launch("int4_linear");
+}
+template <int FMT, int RT, int MAXW>
+int launch_stream(const Int4Args& a, bool dyn, hipStream_t s) {
+  if constexpr (FMT != kUint4) {
+    if (dyn) return launch_stream<FMT, RT, MAXW, true, 1>(a, s);
+  }
+  return a.M <= 4 ? launch_stream<FMT, RT, MAXW, false, 1>(a, s) : launch_stream<FMT, RT, MAXW, false, 4>(a, s);
 }
 
 // Waves of the int8 launch of at most 16 tokens, and whether it can quantise these activations itself: they fit the pieces
 // its threads hold, and no wave's piece crosses a row.
-int int8_stream_waves(int64_t N) { return N >= 8192 ? 4 : 8; }
+int int8_stream_waves(int64_t N, int64_t K) { return N >= 2048 && N < 8192 && K >= 4096 ? 16 : 8; }
 bool quantises_in_stream(int64_t M, int64_t N, int64_t K) {
-  return M <= kDynMaxTokens && (M == 1 || K % 512 == 0) && K <= 32768 && M * K <= int8_stream_waves(N) * 64 * kDynPieces * 8;
+  return M <= kDynMaxTokens && (M == 1 ? K <= int8_stream_waves(N, K) * 64 * kDynPieces * 8 : K % 512 == 0 && M * K <= 16384);
 }
 
 // dyn: x is not quantised yet (quantises_in_stream holds)
 template <int FMT>
 int launch(Int4Args& a, bool dyn, void* workspace, size_t workspace_bytes, hipStream_t s) {
   if (a.M <= kStreamTokens) {
-    // Measured (weights from HBM, us, launch gap included).  Wide layers have workgroups to spare: few waves each, and
-    // two row tiles where the reads of x weigh (int8 14336 x 4096 at 1 / 16 tokens: four waves and two tiles 21.2 / 27.8,
-    // sixteen and one 27 / 37; uint4 at 1 / 16 tokens: one tile 19.6 / 23, two 20.4 / 21.1).  Narrow ones need the waves (uint4
-    // 4096 x 14336 at 1 token: sixteen 20.0, eight 20.9; at 16 tokens 25 and 21.6).
+    // Measured (weights from HBM, us, launch gap included).  The waves fix the order of a row's sums and depend on the layer
+    // alone.  int8 at one token, eight and sixteen: 4096 x 4096 8.5 and 8.0, 4096 x 14336 17.5 and 16.5, but 1024 x 4096 6.1 and 6.6; a wide
+    // layer has workgroups enough for eight, and two row tiles from two tokens on (14336 x 4096 at 1 / 4 tokens: one 17.7 / 26.1,
+    // two 17.5 / 20.6; 8192 x 2048 at one 7.0 and 7.6).  uint4: narrow layers sixteen (4096 x 14336 16.4 and 15.3), wide eight (9728 x 3584
+    // 11.5 and 15.7).
     const bool wide = a.N >= 8192;
-    if constexpr (FMT == kUint4) {
-      if (wide && a.M > 8) launch_stream<FMT, 2, 8>(a, dyn, s);
-      else if (wide || a.M > 8) launch_stream<FMT, 1, 8>(a, dyn, s);
-      else launch_stream<FMT, 1, 16>(a, dyn, s);
-    } else {
-      if (wide) launch_stream<FMT, 2, 4>(a, dyn, s);
-      else launch_stream<FMT, 1, 8>(a, dyn, s);
-    }
-    return check_launch("int4_linear");
+    if constexpr (FMT == kUint4) return wide ? launch_stream<FMT, 1, 8>(a, dyn, s) : launch_stream<FMT, 1, 16>(a, dyn, s);
+    if (wide && a.M > 1) return launch_stream<FMT, 2, 8>(a, dyn, s);
+    return int8_stream_waves(a.N, a.K) == 16 ? launch_stream<FMT, 1, 16>(a, dyn, s) : launch_stream<FMT, 1, 8>(a, dyn, s);
   }
   const Slicing sl = slicing(a.M, a.N, a.K);
   const int mt = tile_mt(a.M);
