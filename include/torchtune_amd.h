@@ -77,6 +77,11 @@ size_t ttamd_nf4_quantize_workspace_bytes(int64_t numel, int block_size);
 int ttamd_nf4_quantize(const void* w, int dtype, int64_t numel, int block_size, int scaler_block_size,
                        uint8_t* quantized_data, int8_t* quantized_scalers, void* quantization_factor,
                        void* scaler_mean, void* workspace, size_t workspace_bytes, void* stream);
+/* The same, and the sixteen code values in `dtype` into code_values (NULL: not wanted): torchao's NF4Tensor carries them as a
+ * tensor (`nf4`), and a copy of them from the host would wait for the quantisation. */
+int ttamd_nf4_quantize_with_codes(const void* w, int dtype, int64_t numel, int block_size, int scaler_block_size, uint8_t* quantized_data,
+                                  int8_t* quantized_scalers, void* quantization_factor, void* scaler_mean, void* code_values, void* workspace,
+                                  size_t workspace_bytes, void* stream);
 
 /*
  * NF4Tensor.get_original_weight() / NF4Tensor.to(dtype): replaces the torchao dequantisation chain reached from

@@ -189,3 +189,15 @@ def test_one_dimensional_tensor_round_trip():
     assert a.shape == flat.shape and a.get_original_weight().shape == flat.shape
     assert torch.equal(a.quantized_data, b.quantized_data) and torch.equal(a.quantized_scalers, b.quantized_scalers)
     assert torch.equal(a.get_original_weight(), b.get_original_weight().view(-1))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows", [1, 129, 8192, 8193])  # workgroups of 8192 elements: one and a part, the most whose sums pass 3 reads itself, one more
+@pytest.mark.parametrize("bs,sbs", [(64, 8), (512, 2)])
+def test_mean_of_the_block_maxima(dtype, rows, bs, sbs):
+    """Every maximum enters the mean once: the fp64 sum of these values is exact (magnitudes within 2^9 of each other)."""
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    w = torch.randn(rows * 8192 + (1024 if rows == 129 else 0), device=DEV, generator=g).mul_(0.02).to(dtype)
+    t = to_nf4(w, bs, sbs)
+    sums = w.view(-1, bs).abs().amax(dim=1).double()
+    assert bits_equal(t.scaler_mean.cpu().reshape(1), (sums.sum() / sums.numel()).float().to(dtype).cpu().reshape(1))

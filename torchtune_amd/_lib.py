@@ -27,6 +27,10 @@ SIGNATURES = {
     "ttamd_version": (_int, []),
     "ttamd_last_error": (ctypes.c_char_p, []),
     "ttamd_nf4_quantize_workspace_bytes": (_size, [_i64, _int]),
+    "ttamd_nf4_quantize_with_codes": (
+        _int,
+        [_c_void_p, _int, _i64, _int, _int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _size, _c_void_p],
+    ),
     "ttamd_nf4_quantize": (
         _int,
         [_c_void_p, _int, _i64, _int, _int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _size, _c_void_p],

@@ -60,7 +60,7 @@ __device__ __forceinline__ void store1(void* base, int64_t i, float v) {
 //   their own, and one comparison (nf4_math.h says why that is exact);
 // * a thread's four chunks are all requested before the first is used.
 // 9 vector-ALU instructions per bf16 element (about 15 and a byte read from a 1.3 KB table before): 14336 x 4096 in bf16
-// takes 25 us = 6.0 TB/s, what a streaming copy reaches; quantising and dequantising it 101 -> 82 us.
+// takes 25 us = 6.0 TB/s, what a streaming copy reaches; quantising and dequantising it, with the passes below, 59 us.
 // An absmax outside the range where the shared reciprocal is exact (zero, denormal, huge, infinite, NaN) takes the
 // division and the search of the 16 codes.
 // ---------------------------------------------------------------------------------------------------
@@ -79,7 +79,7 @@ template <bool BF16, int LPB>
 __global__ __launch_bounds__(256) void nf4_quantize_blocks_kernel(const u32x4_t* __restrict__ w, int64_t n_chunks, int lpb_arg,
                                                                   int log2_lpb, uint32_t fast_low, uint32_t fast_high,
                                                                   uint32_t* __restrict__ qdata, float* __restrict__ absmax,
-                                                                  const Nf4BinTable<BF16> table) {
+                                                                  double* __restrict__ partial, const Nf4BinTable<BF16> table) {
   constexpr int U = kQuantChunksPerThread;
   constexpr int V = BF16 ? 1 : 2;  // 128-bit words per chunk
   __shared__ uint32_t tab[Nf4BinTable<BF16>::kWords];
@@ -93,8 +93,10 @@ __global__ __launch_bounds__(256) void nf4_quantize_blocks_kernel(const u32x4_t*
     for (int h = 0; h < V; ++h) raw[u][h] = w[V * at + h];
   }
   if (threadIdx.x < Nf4BinTable<BF16>::kWords) tab[threadIdx.x] = table.words[threadIdx.x];
+  __shared__ double wave_sum[4];
   __syncthreads();
   const int lpb = LPB ? LPB : lpb_arg;
+  double sum = 0.0;  // of the maxima of this lane's blocks
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int64_t chunk = chunk0 + u * 256;
@@ -125,7 +127,10 @@ __global__ __launch_bounds__(256) void nf4_quantize_blocks_kernel(const u32x4_t*
     }
     if (chunk >= n_chunks) continue;  // a whole block of lanes: n_chunks is a multiple of lpb
     const float m = bits_f32(m_bits);
-    if ((threadIdx.x & (lpb - 1)) == 0) absmax[chunk >> log2_lpb] = m;
+    if ((threadIdx.x & (lpb - 1)) == 0) {
+      absmax[chunk >> log2_lpb] = m;
+      sum += (double)m;
+    }
     float v[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -155,7 +160,13 @@ __global__ __launch_bounds__(256) void nf4_quantize_blocks_kernel(const u32x4_t*
     }
     qdata[chunk] = packed;
   }
+  for (int off = lpb; off < kWave; off <<= 1) sum += __shfl_xor(sum, off, kWave);
+  if ((threadIdx.x & (kWave - 1)) == 0) wave_sum[threadIdx.x >> 6] = sum;
+  __syncthreads();
+  if (threadIdx.x == 0) partial[blockIdx.x] = (wave_sum[0] + wave_sum[1]) + (wave_sum[2] + wave_sum[3]);
 }
+
+int64_t quantize_workgroups(int64_t n_chunks) { return (n_chunks + 256 * kQuantChunksPerThread - 1) / (256 * kQuantChunksPerThread); }
 
 // The table, filled and verified once per process.
 template <bool BF16>
@@ -166,14 +177,14 @@ struct Nf4BinTableHost {
 };
 
 template <bool BF16>
-void launch_quantize_blocks(const void* w, int64_t n_chunks, int lpb, int log2_lpb, uint8_t* qdata, float* absmax, hipStream_t s) {
+void launch_quantize_blocks(const void* w, int64_t n_chunks, int lpb, int log2_lpb, uint8_t* qdata, float* absmax, double* partial,
+                            hipStream_t s) {
   static const Nf4BinTableHost<BF16> host;
   const uint32_t low = host.ok ? Nf4FastRange<BF16>::low : 0u, high = host.ok ? Nf4FastRange<BF16>::high : 0u;
-  const int64_t per_wg = 256 * kQuantChunksPerThread;
-  const dim3 grid((unsigned)((n_chunks + per_wg - 1) / per_wg));
+  const dim3 grid((unsigned)quantize_workgroups(n_chunks));
   auto launch = [&](auto kernel) {
     kernel<<<grid, dim3(256), 0, s>>>(reinterpret_cast<const u32x4_t*>(w), n_chunks, lpb, log2_lpb, low, high,
-                                      reinterpret_cast<uint32_t*>(qdata), absmax, host.table);
+                                      reinterpret_cast<uint32_t*>(qdata), absmax, partial, host.table);
   };
   if (lpb == 8)
     launch(nf4_quantize_blocks_kernel<BF16, 8>);
@@ -182,43 +193,49 @@ void launch_quantize_blocks(const void* w, int64_t n_chunks, int lpb, int log2_l
 }
 
 // ---------------------------------------------------------------------------------------------------
-// quantise, pass 2: mean of the block absmaxes.  Summed in fp64 in a fixed order (256 partial sums, each
-// a fixed strided walk followed by a fixed LDS tree, added by pass 3) so the result does not depend on scheduling; for
-// realistic dynamic ranges the fp64 sum is exact.  mean = dtype(float(sum / n)).
+// quantise, pass 2: mean of the block absmaxes.  Summed in fp64 in a fixed order (pass 1 leaves one sum per workgroup, pass 3 adds
+// them by a fixed strided walk and a fixed LDS tree) so the result does not depend on scheduling; for realistic dynamic
+// ranges the fp64 sum is exact.  mean = dtype(float(sum / n)).  Every workgroup of pass 3 reads all the sums: 57 KB of them at
+// 14336 x 4096, where a launch that summed the maxima took 5.4 us and reading the sums takes 3 (the quantisation 38.7 -> 37.7, that of
+// 4096 x 4096 19.5 -> 16.8; fewer workgroups in pass 3 read less and are slower, 43.6 with 256); beyond kDirectPartials they are added up to
+// kMeanPartials by a launch of its own first (28672 x 8192 134 -> 124).
 // ---------------------------------------------------------------------------------------------------
 constexpr int kMeanPartials = 256;
+constexpr int64_t kDirectPartials = 8192;
 
-__device__ __forceinline__ double block_sum_256(double s, double* sh) {
-  sh[threadIdx.x] = s;
+__device__ __forceinline__ double block_sum_256(double s, double* sh) {  // sh: four
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) s += __shfl_xor(s, off, kWave);
+  if ((threadIdx.x & (kWave - 1)) == 0) sh[threadIdx.x >> 6] = s;
   __syncthreads();
-  for (int off = 128; off > 0; off >>= 1) {
-    if ((int)threadIdx.x < off) sh[threadIdx.x] += sh[threadIdx.x + off];
-    __syncthreads();
-  }
-  return sh[0];
+  return (sh[0] + sh[1]) + (sh[2] + sh[3]);
 }
 
-__global__ __launch_bounds__(256) void nf4_absmax_partial_sum_kernel(const float* __restrict__ absmax, int64_t n_blocks,
-                                                                     double* __restrict__ partial) {
-  __shared__ double sh[256];
+__global__ __launch_bounds__(256) void nf4_partial_sum_kernel(const double* __restrict__ sums, int64_t n, double* __restrict__ partial) {
+  __shared__ double sh[4];
   double s = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n_blocks; i += (int64_t)kMeanPartials * 256)
-    s += (double)absmax[i];
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)kMeanPartials * 256) s += sums[i];
   s = block_sum_256(s, sh);
   if (threadIdx.x == 0) partial[blockIdx.x] = s;
 }
 
 // ---------------------------------------------------------------------------------------------------
 // quantise, pass 3: double quantisation of the block scalers.  One wave per scaler block of SB blocks.  Every workgroup
-// finishes the mean for itself (256 partial sums in the same order: the same bits), which saves a launch of one workgroup.
+// finishes the mean for itself (the partial sums in the same order: the same bits), which saves a launch of one workgroup.
+// The first also writes the sixteen code values where they are asked for.
 // ---------------------------------------------------------------------------------------------------
 template <bool BF16>
 __global__ __launch_bounds__(256) void nf4_quantize_scalers_kernel(const float* __restrict__ absmax,
-                                                                   const double* __restrict__ partial, int64_t n_blocks,
+                                                                   const double* __restrict__ partial, int n_partial, int64_t n_blocks,
                                                                    int64_t n_sb, int SB, int8_t* __restrict__ qscalers,
-                                                                   void* __restrict__ qfactor, void* __restrict__ scaler_mean) {
-  __shared__ double sh[256];
-  const float mean = Arith<BF16>::rnd((float)(block_sum_256(partial[threadIdx.x], sh) / (double)n_blocks));
+                                                                   void* __restrict__ qfactor, void* __restrict__ scaler_mean,
+                                                                   void* __restrict__ code_values) {
+  __shared__ double sh[4];
+  double sum = 0.0;
+#pragma unroll 8
+  for (int i = threadIdx.x; i < n_partial; i += 256) sum += partial[i];
+  const float mean = Arith<BF16>::rnd((float)(block_sum_256(sum, sh) / (double)n_blocks));
+  if (code_values && blockIdx.x == 0 && threadIdx.x < 16) store1<BF16>(code_values, threadIdx.x, kNF4Dev[threadIdx.x]);
   if (blockIdx.x == 0 && threadIdx.x == 0) store1<BF16>(scaler_mean, 0, mean);
   const int64_t sb = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (sb >= n_sb) return;  // whole wave leaves together
@@ -319,12 +336,12 @@ int log2_exact(int64_t v) {
 
 struct QuantWorkspace {
   float* absmax;    // [n_blocks]
-  double* partial;  // [kMeanPartials]
+  double* partial;  // [kMeanPartials], then one per workgroup of pass 1
 };
 
-size_t quant_ws_bytes(int64_t n_blocks) {
+size_t quant_ws_bytes(int64_t numel, int64_t n_blocks) {
   size_t absmax_bytes = ((size_t)n_blocks * sizeof(float) + 255) & ~size_t(255);
-  return absmax_bytes + kMeanPartials * sizeof(double) + 256;
+  return absmax_bytes + (kMeanPartials + (size_t)quantize_workgroups(numel / 8)) * sizeof(double) + 256;
 }
 
 int check_nf4_shape(int64_t numel, int block_size, int scaler_block_size) {
@@ -347,12 +364,13 @@ using namespace ttamd;
 
 extern "C" size_t ttamd_nf4_quantize_workspace_bytes(int64_t numel, int block_size) {
   if (numel <= 0 || block_size <= 0) return 0;
-  return quant_ws_bytes(numel / block_size);
+  return quant_ws_bytes(numel, numel / block_size);
 }
 
-extern "C" int ttamd_nf4_quantize(const void* w, int dtype, int64_t numel, int block_size, int scaler_block_size,
-                                  uint8_t* quantized_data, int8_t* quantized_scalers, void* quantization_factor,
-                                  void* scaler_mean, void* workspace, size_t workspace_bytes, void* stream) {
+extern "C" int ttamd_nf4_quantize_with_codes(const void* w, int dtype, int64_t numel, int block_size, int scaler_block_size,
+                                             uint8_t* quantized_data, int8_t* quantized_scalers, void* quantization_factor,
+                                             void* scaler_mean, void* code_values, void* workspace,
+                                             size_t workspace_bytes, void* stream) {
   if (int rc = check_nf4_shape(numel, block_size, scaler_block_size)) return rc;
   TT_REQUIRE(dtype == TTAMD_BF16 || dtype == TTAMD_F32, "nf4_quantize: unknown dtype code %d", dtype);
   TT_REQUIRE(w && quantized_data && quantized_scalers && quantization_factor && scaler_mean && workspace,
@@ -361,9 +379,9 @@ extern "C" int ttamd_nf4_quantize(const void* w, int dtype, int64_t numel, int b
              "nf4_quantize: w/workspace must be 16-byte aligned and quantized_data 4-byte aligned");
   const int64_t n_blocks = numel / block_size;
   const int64_t n_sb = n_blocks / scaler_block_size;
-  if (workspace_bytes < quant_ws_bytes(n_blocks))
+  if (workspace_bytes < quant_ws_bytes(numel, n_blocks))
     return fail(TTAMD_EWORKSPACE, "nf4_quantize: workspace has %zu bytes, needs %zu", workspace_bytes,
-                quant_ws_bytes(n_blocks));
+                quant_ws_bytes(numel, n_blocks));
   QuantWorkspace ws;
   ws.absmax = reinterpret_cast<float*>(workspace);
   size_t absmax_bytes = ((size_t)n_blocks * sizeof(float) + 255) & ~size_t(255);
@@ -377,16 +395,27 @@ extern "C" int ttamd_nf4_quantize(const void* w, int dtype, int64_t numel, int b
   const int64_t grid3 = (n_sb + 3) / 4;
   auto run = [&](auto bf16) {
     constexpr bool BF16 = decltype(bf16)::value;
-    launch_quantize_blocks<BF16>(w, n_chunks, lpb, log2_exact(lpb), quantized_data, ws.absmax, s);
-    nf4_absmax_partial_sum_kernel<<<dim3(kMeanPartials), dim3(256), 0, s>>>(ws.absmax, n_blocks, ws.partial);
+    const int64_t sums = quantize_workgroups(n_chunks);
+    double* const by_workgroup = ws.partial + kMeanPartials;
+    launch_quantize_blocks<BF16>(w, n_chunks, lpb, log2_exact(lpb), quantized_data, ws.absmax, by_workgroup, s);
+    const bool direct = sums <= kDirectPartials;
+    if (!direct) nf4_partial_sum_kernel<<<dim3(kMeanPartials), dim3(256), 0, s>>>(by_workgroup, sums, ws.partial);
     nf4_quantize_scalers_kernel<BF16><<<dim3((unsigned)grid3), dim3(256), 0, s>>>(
-        ws.absmax, ws.partial, n_blocks, n_sb, scaler_block_size, quantized_scalers, quantization_factor, scaler_mean);
+        ws.absmax, direct ? by_workgroup : ws.partial, direct ? (int)sums : kMeanPartials, n_blocks, n_sb, scaler_block_size,
+        quantized_scalers, quantization_factor, scaler_mean, code_values);
   };
   if (dtype == TTAMD_BF16)
     run(std::true_type{});
   else
     run(std::false_type{});
   return check_launch("nf4_quantize");
+}
+
+extern "C" int ttamd_nf4_quantize(const void* w, int dtype, int64_t numel, int block_size, int scaler_block_size,
+                                  uint8_t* quantized_data, int8_t* quantized_scalers, void* quantization_factor,
+                                  void* scaler_mean, void* workspace, size_t workspace_bytes, void* stream) {
+  return ttamd_nf4_quantize_with_codes(w, dtype, numel, block_size, scaler_block_size, quantized_data, quantized_scalers,
+                                       quantization_factor, scaler_mean, nullptr, workspace, workspace_bytes, stream);
 }
 
 extern "C" int ttamd_nf4_dequantize(const uint8_t* quantized_data, const int8_t* quantized_scalers,

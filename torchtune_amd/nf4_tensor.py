@@ -195,8 +195,8 @@ class NF4Tensor(torch.Tensor):
         home = tensor.device
         dev = _compute_device(tensor)
         w = tensor.detach().to(dev)
-        qdata, qscalers, qfactor, mean = ops.nf4_quantize(w, block_size, scaler_block_size)
-        nf4 = torch.tensor(NF4_TABLE, dtype=tensor.dtype, device=dev)
+        # the code values come from the quantisation's launches: a copy from the host would wait for them
+        qdata, qscalers, qfactor, mean, nf4 = ops.nf4_quantize(w, block_size, scaler_block_size, code_values=True)
         inner = [qscalers, qfactor, mean, qdata, nf4]
         if home != dev:
             inner = [t.to(home) for t in inner]

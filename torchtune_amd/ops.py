@@ -62,9 +62,9 @@ def _workspace(nbytes: int, device: torch.device) -> torch.Tensor:
 # ---------------------------------------------------------------------------------------------------
 # NF4 codec
 # ---------------------------------------------------------------------------------------------------
-def nf4_quantize(w: torch.Tensor, block_size: int, scaler_block_size: int):
+def nf4_quantize(w: torch.Tensor, block_size: int, scaler_block_size: int, code_values: bool = False):
     """-> (quantized_data u8 [numel/2], quantized_scalers i8 [n_blocks], quantization_factor dtype [n_sb],
-    scaler_mean dtype 0-dim)"""
+    scaler_mean dtype 0-dim), and the sixteen code values in dtype where they are asked for"""
     _need_gpu(w, "nf4_quantize")
     code = _code(w.dtype, "nf4_quantize")
     w = w.detach().contiguous()
@@ -82,15 +82,16 @@ def nf4_quantize(w: torch.Tensor, block_size: int, scaler_block_size: int):
     qscalers = torch.empty(n_blocks, dtype=torch.int8, device=dev)
     qfactor = torch.empty(n_blocks // scaler_block_size, dtype=w.dtype, device=dev)
     mean = torch.empty((), dtype=w.dtype, device=dev)
+    codes = torch.empty(16, dtype=w.dtype, device=dev) if code_values else None
     ws_bytes = lib.ttamd_nf4_quantize_workspace_bytes(numel, block_size)
     ws = _workspace(ws_bytes, dev)
     with torch.cuda.device(dev):
-        rc = lib.ttamd_nf4_quantize(
+        rc = lib.ttamd_nf4_quantize_with_codes(
             w.data_ptr(), code, numel, block_size, scaler_block_size, qdata.data_ptr(), qscalers.data_ptr(),
-            qfactor.data_ptr(), mean.data_ptr(), ws.data_ptr(), ws.numel(), _stream(w),
+            qfactor.data_ptr(), mean.data_ptr(), _ptr(codes), ws.data_ptr(), ws.numel(), _stream(w),
         )
     _lib.check(rc, "nf4_quantize")
-    return qdata, qscalers, qfactor, mean
+    return (qdata, qscalers, qfactor, mean, codes) if code_values else (qdata, qscalers, qfactor, mean)
 
 
 def nf4_dequantize(
