@@ -108,3 +108,25 @@ def test_a_weight_quantizer_that_does_more_is_called(how):
     finally:
         if handle is not None:
             handle.remove()
+
+
+# tiles of 64, 128 and 256 rows with a last row tile of one row and a last column tile of half its width, fewer steps than the
+# ring has stages and more, slices of unequal length
+@pytest.mark.parametrize("M,N,K", [(1, 64, 64), (65, 320, 192), (1025, 3520, 2048), (1025, 6464, 192), (1025, 6464, 1024), (129, 512, 4160),
+                                   (1000, 2048, 8256), (2049, 2560, 128)])
+@pytest.mark.parametrize("kind", [0, 1])
+def test_tile_heights(kind, M, N, K):
+    lib = _lib.load()
+    torch.manual_seed(M + N + K + kind)
+    a = torch.randn(M, K, device="cuda").bfloat16()
+    b = torch.randn((N, K) if kind == 0 else (K, N), device="cuda").bfloat16()
+    bias = torch.randn(N, device="cuda").bfloat16() if kind == 0 else None
+    c = torch.full((M + 1, N), 7.0, device="cuda").bfloat16()  # one row beyond the product
+    need = lib.ttamd_gemm_mid_workspace_bytes(M, N, K)
+    ws = torch.empty(max(need, 1), device="cuda", dtype=torch.uint8)
+    status = lib.ttamd_gemm_mid_bf16(kind, a.data_ptr(), b.data_ptr(), bias.data_ptr() if kind == 0 else None, c.data_ptr(), M, N, K,
+                                     ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream)
+    assert status == 0
+    want = a.double() @ (b.double().t() if kind == 0 else b.double())
+    _close(c[:M], want + bias.double() if kind == 0 else want, K)
+    assert bool((c[M] == 7).all())
