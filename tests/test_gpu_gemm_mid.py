@@ -130,3 +130,20 @@ def test_tile_heights(kind, M, N, K):
     want = a.double() @ (b.double().t() if kind == 0 else b.double())
     _close(c[:M], want + bias.double() if kind == 0 else want, K)
     assert bool((c[M] == 7).all())
+
+
+# weight gradients on tiles of 256 x 256 whose last row and column of tiles hold 64 of 256: tokens of one part-filled step,
+# around one step, an odd number of steps, more than the ring has stages
+@pytest.mark.parametrize("tokens", [1, 31, 32, 33, 97, 1001, 1024])
+def test_weight_gradients_on_wide_tiles(tokens):
+    lib = _lib.load()
+    N, K = 4160, 2624
+    assert lib.ttamd_gemm_mid_workspace_bytes(N, K, tokens) == 0
+    torch.manual_seed(tokens)
+    gy = torch.randn(tokens, N, device="cuda").bfloat16()
+    x = torch.randn(tokens, K, device="cuda").bfloat16()
+    c = torch.full((N + 1, K), 7.0, device="cuda").bfloat16()  # one row beyond the product
+    assert lib.ttamd_gemm_mid_bf16(2, gy.data_ptr(), x.data_ptr(), None, c.data_ptr(), N, K, tokens, None, 0,
+                                   torch.cuda.current_stream().cuda_stream) == 0
+    _close(c[:N], gy.double().t() @ x.double(), tokens)
+    assert bool((c[N] == 7).all())

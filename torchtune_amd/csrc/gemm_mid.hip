@@ -14,15 +14,18 @@
 // matrix pipes) for workgroups: 256 rows where they fill the CUs (1000 x 8192 x 2048 44.4 -> 33.3 us, of which the matrix
 // pipes take 21 at the 1.6 GHz that the card holds under them), 128 below (1000 x 2048 x 8192 in two slices 50.8 -> 41.7),
 // 64 where the chip would be half idle (1000 x 2048 x 2048 21.1 -> 15.1).  The 64-row tile takes half a CU's LDS: two run there.
-// gemm_mid_pair_kernel (kind 2, and kind 1 over a short contraction of many tiles): four waves per tile of 128 x 128, two workgroups per CU,
-// steps of 32.  Both operands of kind 2 lie across the contraction, in lines of 256 bytes, and its contraction (the tokens) is
-// short where its tiles are many: two independent workgroups hide each other's first loads and last stores (8192 x 2048
-// outputs over 1000 tokens 52.6 us, eight waves 55 - 65).
+// gemm_mid_pair_kernel (kind 2, and kind 1 over a short contraction of many tiles): four waves per tile of 128 x 128, two
+// workgroups per CU, steps of 32.  Both operands of kind 2 lie across the contraction, in lines of 256 bytes, and its
+// contraction (the tokens) is short: two independent workgroups hide each other's first loads and last stores (8192 x 2048
+// outputs over 1000 tokens 52.6 us, on tiles as gemm_mid_kernel's 55 - 65).  Weight gradients of more outputs run on the
+// 256 x 256 tiles of gemm_tn.hip (31.3 us there).
 // Launches of few tiles cut the contraction into slices (fp32 slabs, added in slice order by gemm_mid_reduce_kernel).
 // Over 380 products of kinds 0 and 1 (40 - 8192 rows, 256 - 14336 columns) these two take 0.84 of the time of the four-wave
 // kernel alone, and the sums are closer to the exact ones (2.7e-7 against 3.9e-7 over 8192 indices in two slices): two chains
-// of half the length.  A training pass of a 1B-shaped layer over 1000 tokens with its 21 products: 825 -> 735 us.
+// of half the length.  A training pass of a 1B-shaped layer over 1000 tokens with its 21 products: 825 -> 735 us, with the wide
+// tiles for its weight gradients 714 (host-bound there).
 #include "common.h"
+#include "group.h"
 #include "nf4_math.h"
 
 #include <type_traits>
@@ -473,7 +476,7 @@ __global__ __launch_bounds__(256) void gemm_mid_reduce_kernel(const float* __res
 struct MidPlan {
   int64_t tiles_m, tiles;
   int slices, steps;
-  int rows;  // of a tile of gemm_mid_kernel; 0: gemm_mid_pair_kernel
+  int rows;  // of a tile of gemm_mid_kernel (kind 2: 256, gemm_tn_kernel); 0: gemm_mid_pair_kernel
 };
 // gemm_mid_pair_kernel, and the most slices of either kernel (the workspace is sized before the kind is known): the split with
 // the least of (steps of one workgroup) + (slabs written and read, one more launch), with the times measured on this kernel:
@@ -508,10 +511,21 @@ MidPlan plan_pair(int64_t M, int64_t N, int64_t K) {
 // (512 of the kernels that run two per CU), for its steps and for how full the chip is (its clock falls with the load), and for
 // the slabs.  The terms are fitted to 760 products (40 - 8192 rows, the widths of seven model shapes), every tile and split of
 // each measured; on 380 others the pick is 0.7 % slower than the fastest on average.
+// Kind 2: gemm_mid_pair_kernel, or the 256 x 256 tiles of gemm_tn.hip, by the same kind of model (fitted to 260 products, 0.1 %
+// slower than the faster one on average).  The wide tiles win from about half a round of them on (1000 tokens of 8192 x 2048
+// 51.5 -> 31.3 us, 4096 x 4096 44.4 -> 30.6, of 2048 x 2048 15.1 and 21.9).
 MidPlan plan_mid(int kind, int64_t M, int64_t N, int64_t K) {
   const MidPlan pair = plan_pair(M, N, K);
-  if (kind == 2) return pair;
   MidPlan p = pair;
+  if (kind == 2) {
+    // whole contractions only: a slice's sums are shorter chains, and with few tiles the 256 x 256 ones are fewer still
+    const double k = (double)((K + 31) / 32), tiles = (double)(((M + 255) / 256) * ((N + 255) / 256)), whole = ceil(tiles / 256),
+                 rounds = (double)((pair.tiles + 255) / 256);
+    const double wide = 0.2 + 7.26 * whole + k * (0.44 * whole + 0.25 * tiles / 256);
+    const double narrow = 3.8 + 1.6 * rounds + k * (rounds > 1 ? 0.04 * rounds : 0.095) + 0.265 * k * (double)pair.tiles / 256;
+    if (pair.slices == 1 && wide < narrow) p.rows = 256;
+    return p;
+  }
   double best = 1e30;
   if (kind == 1) {
     const double k = (double)((K + 31) / 32), rounds = (double)((pair.tiles + 255) / 256);
@@ -606,10 +620,11 @@ extern "C" int ttamd_gemm_mid_bf16(int kind, const void* a, const void* b, const
       return fail(TTAMD_EWORKSPACE, "gemm_mid: workspace of %zu bytes, %zu needed", workspace_bytes, need);
     TT_REQUIRE(aligned16(workspace), "gemm_mid: the workspace must be 16-byte aligned");
   }
-  const MidPlan p = plan_mid(kind, M, N, K);
+  const MidPlan p = kind == 2 && bias ? plan_pair(M, N, K) : plan_mid(kind, M, N, K);  // the wide tiles add no bias
   MidArgs g = {reinterpret_cast<const uint16_t*>(a), reinterpret_cast<const uint16_t*>(b), reinterpret_cast<const uint16_t*>(bias),
                reinterpret_cast<uint16_t*>(c), reinterpret_cast<float*>(workspace), (int)M, (int)N, (int)K, (int)p.tiles_m, (int)p.tiles, 0, p.slices, p.steps};
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (kind == 2 && p.rows) return run_gemm_tn(a, b, c, K, M, N, s);
   const int rc = p.rows ? (kind == 0 ? launch_rows<false>(g, p.rows, s) : launch_rows<true>(g, p.rows, s))
                  : kind == 1 ? launch_pair<false, false>(g, s)  // whole
                  : p.slices > 1 ? launch_pair<true, true>(g, s) : launch_pair<true, false>(g, s);

@@ -106,7 +106,8 @@ __device__ __forceinline__ void tn_locate(const TnArgs& g, int id, int& which, i
 
 // acc[j][i][v] = C[n][k], n = n0 + 128 wm + 16 i + l15, k = k0 + 64 wn + 16 j + 4 g4 + v.  Each wave transposes its
 // 128 x 64 band through LDS (128 KiB for the eight waves) and writes whole 128-byte row segments.
-__device__ __forceinline__ void tn_store_tile(const f32x4_t (&acc)[kTnNT][kTnMT], char* smem, uint16_t* C, int K, int n0, int k0) {
+template <bool EDGES>
+__device__ __forceinline__ void tn_store_tile(const f32x4_t (&acc)[kTnNT][kTnMT], char* smem, uint16_t* C, int N, int K, int n0, int k0) {
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wv >> 2, wn = wv & 3;
@@ -128,9 +129,11 @@ __device__ __forceinline__ void tn_store_tile(const f32x4_t (&acc)[kTnNT][kTnMT]
   const int c = lane & 7;
   uint16_t* crow = C + k0 + wn * 64 + 8 * c;
   const int nrow0 = n0 + 128 * wm;
+  if (EDGES && k0 + wn * 64 + 8 * c >= K) return;
 #pragma unroll 8
   for (int t = 0; t < 16; ++t) {
     const int r = 8 * t + (lane >> 3);
+    if (EDGES && nrow0 + r >= N) continue;
     const u32x4_t v = *reinterpret_cast<const u32x4_t*>(band + r * 128 + ((c ^ (r & 7)) << 4));
     *reinterpret_cast<u32x4_t*>(crow + (int64_t)(nrow0 + r) * K) = v;
   }
@@ -139,6 +142,12 @@ __device__ __forceinline__ void tn_store_tile(const f32x4_t (&acc)[kTnNT][kTnMT]
 // Steps [begin, end) of slice `slice` of `slices` over nk steps (every slice non-empty when slices <= nk).
 __device__ __forceinline__ int tn_slice_begin(int slice, int slices, int nk) { return (int)(((int64_t)slice * nk) / slices); }
 
+__device__ __constant__ u32x4_t kTnZero = {0, 0, 0, 0};
+
+// EDGES: M, N and K need not be whole steps and tiles (N and K multiples of 64).  Rows beyond M come as zeros, columns beyond
+// N and K repeat the tile's first ones and are not stored.  A kernel of its own: the whole tiles keep their instruction count
+// (8192 x 2048 outputs: 992 tokens 31.4 us, with edges 1000 32.2).
+template <bool EDGES>
 __global__ __launch_bounds__(512) void gemm_tn_kernel(const TnArgs g) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int MT = kTnMT, NT = kTnNT;
@@ -149,7 +158,7 @@ __global__ __launch_bounds__(512) void gemm_tn_kernel(const TnArgs g) {
   const int wm = wv >> 2, wn = wv & 3;
   const int l15 = lane & 15, g4 = lane >> 4;
 
-  const int nk_all = g.M >> 5;  // steps of 32 rows
+  const int nk_all = (g.M + 31) >> 5;  // steps of 32 rows
   int id = blockIdx.x, t_begin = 0, nk = nk_all;  // this workgroup runs steps [t_begin, nk)
   int slab = -1;
   if (id >= g.full_tiles) {
@@ -173,8 +182,9 @@ __global__ __launch_bounds__(512) void gemm_tn_kernel(const TnArgs g) {
   for (int d = 0; d < 2; ++d) {
     const int rl = 4 * wv + 2 * d + (lane >> 5);
     const int chunk = (lane & 31) ^ ((rl & 3) << 1) ^ (((rl >> 3) & 1) << 3);
-    a_off[d] = (uint32_t)rl * (uint32_t)N * 2u + (uint32_t)n0 * 2u + (uint32_t)chunk * 16u;
-    b_off[d] = (uint32_t)rl * (uint32_t)g.K * 2u + (uint32_t)k0 * 2u + (uint32_t)chunk * 16u;
+    const int a_chunk = EDGES && n0 + 8 * chunk >= N ? 0 : chunk, b_chunk = EDGES && k0 + 8 * chunk >= g.K ? 0 : chunk;
+    a_off[d] = (uint32_t)rl * (uint32_t)N * 2u + (uint32_t)n0 * 2u + (uint32_t)a_chunk * 16u;
+    b_off[d] = (uint32_t)rl * (uint32_t)g.K * 2u + (uint32_t)k0 * 2u + (uint32_t)b_chunk * 16u;
   }
   // The two requests of an operand name their LDS destinations through the instruction's offset field, which moves the
   // global address along with the LDS address: one M0 write per operand and step.  The second request therefore carries
@@ -198,6 +208,19 @@ __global__ __launch_bounds__(512) void gemm_tn_kernel(const TnArgs g) {
   };
   auto issue = [&](int t, int stage) {  // past the end: the last step again (the waits count a fixed number in flight)
     const int tk = t < nk ? t : nk - 1;
+    if (EDGES && 32 * (tk + 1) > g.M) {  // the last step, part-filled (the unrolled loop below stops short of it)
+      const uint32_t st = lds0 + stage * kTnStage + wv * 2048;
+      const char* const ab = reinterpret_cast<const char*>(A) + (int64_t)tk * a_step;
+      const char* const bb = reinterpret_cast<const char*>(g.B) + (int64_t)tk * b_step;
+      const char* const zero = reinterpret_cast<const char*>(&kTnZero);
+#pragma unroll
+      for (int d = 0; d < 2; ++d) {
+        const bool in = 32 * tk + 4 * wv + 2 * d + (lane >> 5) < g.M;
+        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(in ? ab + a_off[d] : zero), "s"(st + 1024u * d) : "memory", "m0");
+        asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(in ? bb + b_off[d] : zero), "s"(st + 16384u + 1024u * d) : "memory", "m0");
+      }
+      return;
+    }
     request(a_base + (int64_t)tk * a_step, b_base + (int64_t)tk * b_step, stage);
   };
 
@@ -384,7 +407,7 @@ __global__ __launch_bounds__(512) void gemm_tn_kernel(const TnArgs g) {
   }
   // ---- epilogue
   __syncthreads();
-  tn_store_tile(acc, smem, C, g.K, n0, k0);
+  tn_store_tile<EDGES>(acc, smem, C, N, g.K, n0, k0);
 #endif
 }
 
@@ -414,7 +437,7 @@ __global__ __launch_bounds__(512) void gemm_tn_reduce_kernel(const TnArgs g) {
         for (int e = 0; e < 4; ++e) acc[j][i][e] += v[e];
       }
   }
-  tn_store_tile(acc, smem, g.C[which], g.K, n0, k0);
+  tn_store_tile<false>(acc, smem, g.C[which], g.N[which], g.K, n0, k0);
 #endif
 }
 
@@ -456,6 +479,7 @@ TnPlan plan_tn(int64_t tiles, int64_t nk) {
 }
 size_t tn_slab_bytes(const TnPlan& p) { return (size_t)p.tail_tiles * (p.slices > 1 ? p.slices : 0) * 256 * 256 * sizeof(float); }
 
+template <bool EDGES = false>
 int launch_gemm_tn(TnArgs& g, void* workspace, size_t workspace_bytes, hipStream_t s) {
   const int64_t tiles = (int64_t)g.tiles_n * g.tiles_k;
   TnPlan plan = plan_tn(tiles, g.M >> 5);
@@ -471,13 +495,13 @@ int launch_gemm_tn(TnArgs& g, void* workspace, size_t workspace_bytes, hipStream
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;
   if (dev < 0 || !attr_set[dev]) {
-    for (const void* fn : {reinterpret_cast<const void*>(&gemm_tn_kernel), reinterpret_cast<const void*>(&gemm_tn_reduce_kernel)}) {
+    for (const void* fn : {reinterpret_cast<const void*>(&gemm_tn_kernel<EDGES>), reinterpret_cast<const void*>(&gemm_tn_reduce_kernel)}) {
       hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kTnLds);
       if (e != hipSuccess) return fail(TTAMD_ELAUNCH, "gemm_tn: cannot reserve %d bytes of LDS: %s", kTnLds, hipGetErrorString(e));
     }
     if (dev >= 0) attr_set[dev] = true;
   }
-  gemm_tn_kernel<<<dim3((unsigned)units), dim3(512), kTnLds, s>>>(g);
+  gemm_tn_kernel<EDGES><<<dim3((unsigned)units), dim3(512), kTnLds, s>>>(g);
   if (int rc = check_launch("gemm_tn")) return rc;
   if (plan.slices > 1) {
     gemm_tn_reduce_kernel<<<dim3((unsigned)plan.tail_tiles), dim3(512), kTnLds, s>>>(g);
@@ -486,6 +510,19 @@ int launch_gemm_tn(TnArgs& g, void* workspace, size_t workspace_bytes, hipStream
   return TTAMD_OK;
 }
 }  // namespace
+
+int ttamd::run_gemm_tn(const void* a, const void* b, void* c, int64_t M, int64_t N, int64_t K, hipStream_t s) {
+  TnArgs g = {};
+  g.n = 1;
+  g.A[0] = reinterpret_cast<const uint16_t*>(a);
+  g.C[0] = reinterpret_cast<uint16_t*>(c);
+  g.N[0] = (int)N;
+  g.B = reinterpret_cast<const uint16_t*>(b);
+  g.M = (int)M; g.K = (int)K;
+  g.tiles_n = g.tile_end[0] = (int)((N + 255) / 256);
+  g.tiles_k = (int)((K + 255) / 256);
+  return gemm_tn_applies(M, N, K) ? launch_gemm_tn<false>(g, nullptr, 0, s) : launch_gemm_tn<true>(g, nullptr, 0, s);
+}
 
 extern "C" size_t ttamd_gemm_tn_workspace_bytes(int64_t M, int64_t n_total, int64_t K) {
   if (M < 32 || n_total <= 0 || K <= 0 || n_total % 256 != 0 || K % 256 != 0) return 0;

@@ -84,6 +84,8 @@ size_t dense_group_dx_workspace_bytes(const GroupDx& d);
 int run_gemm_dense_group_dx(const GroupDx& d, const void* gh_cat, void* gx, void* workspace, hipStream_t s,
                             const void* tiles_fwd = nullptr, bool paired = false);
 
+// C[N, K] = A[M, N]^T . B[M, K], N and K multiples of 64 and any M (gemm_tn.hip); 16-byte aligned operands.
+int run_gemm_tn(const void* a, const void* b, void* c, int64_t M, int64_t N, int64_t K, hipStream_t s);
 // nf4_small_m.hip: y[i] = x . D(W_i)^T (+ bias) + scale . h_i . lora_b[i]^T for a handful of tokens
 int small_m_limit();
 // the forward of M tokens on an [N, K] weight runs the few-token kernel (sliced_ok: a slicing workspace is at hand)
