@@ -243,21 +243,31 @@ TILED_GEMM = True
 TILED_GEMM_MIN_ROWS = 2048
 TILED_GEMM_MIN_TILES = 256
 TN_GEMM_MIN_TILES = 192
-# Most products (rows * N * K) of a linear whose matmuls run on ``ttamd_gemm_mid_bf16``.  Up to here the two libraries are
-# level on the GPU (three products at 200 tokens of 14336 x 4096: 164 us, vendor library 199; 500 tokens of 8192 x 2048: 85
-# and 96; 1000 tokens: 142 and 132), while a vendor call takes 31 us of host time, of ours 5; above it the vendor's larger
-# tiles win (500 tokens of 4096 x 14336: 287 and 255; 1000: 481 and 384).
+# Most products (rows * N * K) of a linear whose matmuls run on ``ttamd_gemm_mid_bf16``, below 2048 rows.  Up to 2^34 the library's
+# kernels are faster than the vendor's (three products, us: 200 tokens of 14336 x 4096 141 and 210, 500 of 8192 x 2048 73 and 100,
+# 1000 of 2048 x 2048 45 and 56, of 2048 x 8192 110 and 126), and a vendor call takes 31 us of host time, of ours 5.
 MID_GEMM_MAX = 1 << 34
-# The same bound from 2048 rows on.  The kernels are not built for tall products (four 64 x 64 wave tiles, LDS bound): the
-# vendor's larger tiles win on the GPU from about 8 * 2^30 on, by 5 % at first and 10 - 25 % from 13 * 2^30 (three products, us,
-# these kernels and the vendor's: 2600 tokens of 2048 x 2048 103 and 108, 3300 122 and 117, 4096 142 and 118; 5200 of
-# 2816 x 1024 160 and 127).  Whole layers gain from the vendor only where they are not host bound with it: layer of dim 2048 at 4096
-# tokens 1768 -> 1718 us forward + backward, of dim 1024 at 5200 932 -> 955.  Narrow weights (N * K up to 2^20) keep the bound
-# above: their weight gradient, few tiles over a long contraction, is where the vendor loses (16384 tokens of 1024 x 1024
-# 158 and 171, 65536 of 256 x 1024 221 and 335).
+# The same bound for a weight with at least as many outputs as inputs whose forward fills the rounds of 256 x 128 tiles on the 256
+# CUs to ``MID_GEMM_MIN_FILL``: the most that was measured (983 tokens of 14336 x 4096 349 and 392 us, 1701 of 8192 x 2048 164
+# and 181; layer of dim 4096 forward + backward at 500 tokens 1454 -> 1313 us, at 700 1707 -> 1653, at 1900 3006 -> 2860).  With
+# emptier rounds the vendor's choice of tiles wins (1290 tokens of dim 2560, fill 0.63: 1071 and 1124), and with fewer outputs
+# than inputs it does at some lengths (1101 tokens of 4096 x 14336: 440 and 468).
+MID_GEMM_MAX_WIDE = 112 << 30
+MID_GEMM_MIN_FILL = 0.65
+# The same bound from 2048 rows on: the vendor's larger tiles win the forward and the grad-input of tall products from about
+# 14 * 2^30 on (three products, us, these kernels and the vendor's: 2600 tokens of 2048 x 2048 87 and 101, 3300 103 and 111, 4096
+# 124 and 117; 5200 of 2816 x 1024 143 and 127).  Narrow weights (N * K up to 2^20) keep the bound above: their weight gradient,
+# few tiles over a long contraction, is where the vendor loses (16384 tokens of 1024 x 1024 156 and 175, 65536 of 256 x 1024
+# 219 and 357).
 MID_GEMM_MAX_TALL = 14 << 30
 # the weight gradients of a group's members (they share fq(x)) as one launch; False: one launch per member (A/B timing)
 TN_GROUP_GEMM = True
+
+
+def _round_fill(rows: int, cols: int) -> float:
+    """How full the rounds of 256 x 128 output tiles on the 256 CUs are."""
+    tiles = max(1, -(-rows // 256) * -(-cols // 128))
+    return tiles / (256 * -(-tiles // 256))
 
 
 class _TiledFakeQuantLinearFn(torch.autograd.Function):
@@ -507,8 +517,8 @@ class FakeQuantizedLinear(nn.Linear):
                 and ops.tiled_weight_shape_ok(self.out_features, self.in_features, c.group_size))
 
     def _mid_ok(self, x: torch.Tensor) -> bool:
-        """The products run on the library's 128 x 128-tile kernels (``ttamd_gemm_mid_bf16``) instead of the vendor library:
-        the sizes below ``_tiled_ok``'s where they take about as long on the GPU and the vendor calls' host time counts.
+        """The products run on the library's kernels for smaller tiles (``ttamd_gemm_mid_bf16``) instead of the vendor library:
+        the sizes below ``_tiled_ok``'s where they are faster on the GPU, or level there and the vendor calls' host time counts.
         The weight's fake quantizer is then read, not called, so one that does more when called keeps the dense product."""
         q, w, b = self.weight_fake_quantizer, self.weight, self.bias
         if q is None or not _runs_as_written(q):
@@ -520,7 +530,11 @@ class FakeQuantizedLinear(nn.Linear):
         if type(x) is not torch.Tensor or type(w) is not nn.Parameter or (b is not None and (type(b) is not nn.Parameter or b.dtype != torch.bfloat16)):
             return False
         N, K = w.shape
-        most = MID_GEMM_MAX_TALL if x.numel() >= 2048 * K and N * K > 1 << 20 else MID_GEMM_MAX
+        most = MID_GEMM_MAX
+        if x.numel() >= 2048 * K:
+            most = MID_GEMM_MAX_TALL if N * K > 1 << 20 else MID_GEMM_MAX
+        elif x.numel() * N > MID_GEMM_MAX and N >= K and _round_fill(x.numel() // K, N) >= MID_GEMM_MIN_FILL:
+            most = MID_GEMM_MAX_WIDE
         return (0 < x.numel() * N <= most and N * K < 1 << 30 and N >= 256 and N % 64 == 0 and K % 64 == 0 and x.shape[-1] == K)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
