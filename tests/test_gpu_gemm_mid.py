@@ -151,7 +151,7 @@ def test_weight_gradients_on_wide_tiles(tokens):
 
 def test_products_below_2048_rows():
     for M, N, K, mid in [(1000, 14336, 4096, True), (2047, 14336, 4096, True), (1000, 4096, 14336, False), (2047, 15360, 4096, False),
-                         (1290, 6912, 2560, False)]:
+                         (1290, 6912, 2560, False), (2000, 800064, 64, False)]:
         layer = FakeQuantizedLinear(K, N, False, None, FakeQuantizeConfig(torch.int4, group_size=32), device="cuda", dtype=torch.bfloat16)
         assert layer._mid_ok(torch.empty(M, K, device="cuda", dtype=torch.bfloat16)) is mid, (M, N, K)
     test_linear_and_gradients(701, 9728, 3584, False)

@@ -533,7 +533,8 @@ class FakeQuantizedLinear(nn.Linear):
         most = MID_GEMM_MAX
         if x.numel() >= 2048 * K:
             most = MID_GEMM_MAX_TALL if N * K > 1 << 20 else MID_GEMM_MAX
-        elif x.numel() * N > MID_GEMM_MAX and N >= K and _round_fill(x.numel() // K, N) >= MID_GEMM_MIN_FILL:
+        elif (x.numel() * N > MID_GEMM_MAX and N >= K and x.numel() // K * N < 1 << 30  # the kernels' 32-bit offsets
+              and _round_fill(x.numel() // K, N) >= MID_GEMM_MIN_FILL):
             most = MID_GEMM_MAX_WIDE
         return (0 < x.numel() * N <= most and N * K < 1 << 30 and N >= 256 and N % 64 == 0 and K % 64 == 0 and x.shape[-1] == K)
 
