@@ -388,8 +388,7 @@ int ttamd_nf4_lora_group_swiglu_fwd_bf16(const void* x, const ttamd_lora_group_m
 /* A handful of tokens (at most 16): every member's h and y (and act, the gated product of a gate / up pair, where it is not
  * NULL) in as few launches as there are launch shapes, usually one; h_cat receives the hidden activations or is NULL where no
  * backward wants them.  Ranks of at most 32.  ttamd_lora_few_fwd_applies says whether this is the better way for a shape
- * (the call returns TTAMD_EUNSUPPORTED where it does not).  Same roundings as the calls above (h and y once each to bf16);
- * the fp32 sums of h run in another order. */
+ * (the call returns TTAMD_EUNSUPPORTED where it does not).  The same bits as the calls above. */
 int ttamd_lora_few_fwd_applies(const ttamd_lora_group_member* members, int n_members, int64_t M, int64_t K, int swiglu);
 int ttamd_lora_few_fwd_bf16(const void* x, const ttamd_lora_group_member* members, int n_members, void* h_cat, void* act, int64_t M,
                             int64_t K, void* stream);

@@ -724,3 +724,62 @@ def test_few_tokens_with_the_hidden_product_inside(M, Ns, K, ranks, bias):
         off += r
     if gated:
         assert torch.equal(act, ops.swiglu_fwd(*ys))
+
+
+def _few_layers(shapes, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    layers = []
+    for n, k, r in shapes:
+        torch.set_default_dtype(BF)
+        try:
+            with torch.device(DEV):
+                lin = LoRALinear(k, n, rank=r, alpha=2.0 * r, quantize_base=True)
+        finally:
+            torch.set_default_dtype(torch.float32)
+        with torch.no_grad():
+            lin.weight.copy_(torch.randn(n, k, device=DEV, generator=g).mul_(0.02).to(BF))
+            lin.lora_a.weight.copy_(torch.randn(r, k, device=DEV, generator=g).mul_(k ** -0.5).to(BF))
+            lin.lora_b.weight.copy_(torch.randn(n, r, device=DEV, generator=g).mul_(0.5).to(BF))
+        for p in lin.parameters():
+            p.requires_grad_(False)
+        layers.append(lin)
+    return layers
+
+
+@pytest.mark.parametrize("K,Ns,ranks", [(2048, (8192, 8192), (8, 8)), (4096, (14336, 14336), (16, 16)), (1024, (2816, 2816), (16, 8)), (4096, (4096, 1024, 1024), (16, 16, 16)),
+                                        (2560, (6912, 6912), (8, 16)), (1536, (8960, 8960), (32, 32)), (3072, (8192, 8192), (24, 8)), (4096, (8192, 1024), (8, 32)),
+                                        (14336, (4096, 64), (32, 16))])
+def test_a_row_has_the_same_bits_alone_in_a_batch_and_in_a_group(K, Ns, ranks, monkeypatch):
+    """Up to 16 tokens, over the launches that form the hidden product and those that read it: a layer on its own, in a group,
+    through the Python node with its two stages, and one row of a batch alone."""
+    from torchtune_amd.modules.peft import lora
+
+    layers = _few_layers([(n, K, r) for n, r in zip(Ns, ranks)], K)
+    x = torch.randn(16, K, device=DEV, generator=torch.Generator(device=DEV).manual_seed(3)).to(BF)
+    with torch.no_grad():
+        whole = [lin(x) for lin in layers]
+        for m in (1, 4, 5, 16):
+            rows = x[:m].contiguous()
+            for lin, y, z in zip(layers, whole, lora_linear_group(rows, layers)):
+                assert torch.equal(z, y[:m]) and torch.equal(lin(rows), y[:m])
+            if len(layers) == 2 and Ns[0] == Ns[1]:
+                assert torch.equal(lora_swiglu_group(rows, *layers), layer_ops.swiglu(whole[0][:m].contiguous(), whole[1][:m].contiguous()))
+        monkeypatch.setattr(lora, "ONE_CALL_PER_DIRECTION", False)
+        for lin, y in zip(layers, whole):
+            for m in (1, 16):
+                assert torch.equal(lin(x[:m].contiguous()), y[:m])
+
+
+@pytest.mark.parametrize("M", [1, 5])
+@pytest.mark.parametrize("N,parts", [(2048, 16), (8192, 8), (12352, 4)])
+def test_few_token_sums_run_in_four_chains_per_part(N, parts, M):
+    """Every weight is 1, every activation 1 but a first one of 2^40 and, where its chain ends, one of -2^40: what the chain adds
+    in between is absorbed, at most 32 values for each of the chain's chunks, and the result falls short by as much."""
+    K = 4096
+    codes = torch.full((N * K // 2,), 255, device=DEV, dtype=torch.uint8)
+    scal = torch.ones(N * K // 64, device=DEV)
+    x = torch.ones(M, K, device=DEV, dtype=BF)
+    chunks = K // 128 // parts
+    x[:, 0], x[:, (chunks - 1) * parts * 128] = 2.0 ** 40, -(2.0 ** 40)
+    y = ops.nf4_lora_linear_fwd(x, codes, scal, N, torch.zeros(M, 8, device=DEV, dtype=BF), torch.zeros(N, 8, device=DEV, dtype=BF), 1.0).float()
+    assert bool((y <= K).all()) and bool((y >= K - 2 - 32 * chunks - 16).all())  # 16: a bf16 step of the result

@@ -91,13 +91,19 @@ int small_m_limit();
 // the forward of M tokens on an [N, K] weight runs the few-token kernel (sliced_ok: a slicing workspace is at hand)
 bool small_m_applies(int64_t M, int64_t N, int64_t K, bool sliced_ok);
 int run_small_m_group(const void* x, const GroupGemm& g, const void* h_cat, void* act, bool* act_done, hipStream_t s);
-// the same with h_i = x . lora_a[i]^T formed inside the launches (gated: two members of equal width, act is written too), where
-// that is the better way; h_cat receives it, or is null
+// the same with h_i = x . lora_a[i]^T formed inside the launches (gated: two members of equal width, act is written too), the
+// same bits, where that is the better way; h_cat receives it, or is null
 bool few_forms_hidden(const GroupGemm& g, bool gated);
 int run_few_with_hidden(const void* x, const GroupGemm& g, const uint16_t* const* lora_a, void* h_cat, void* act, hipStream_t s);
 
 // lora_skinny.hip
 size_t group_hidden_ws_bytes(int64_t M, int64_t K, int r_total);
+// How h = x . lora_a^T of at most 32 tokens is summed over K (by K alone): in `splits` runs of 64-wide chunks, or (0) by the
+// sixteen waves of one workgroup
+struct HiddenOrder {
+  int splits, chunks_per_split;
+};
+HiddenOrder hidden_order(int64_t K);
 // h_cat[:, r_off[i] : r_off[i + 1]] = x . lora_a[i]^T for every member, in one pass over x
 int run_group_hidden(const uint16_t* x, const GroupSkinny& g, uint16_t* h_cat, float* ws, hipStream_t s);
 size_t group_lora_bwd_ws_bytes(const GroupSkinny& g);

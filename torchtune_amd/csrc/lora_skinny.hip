@@ -1307,6 +1307,11 @@ int check_skinny(const char* who, int64_t M, int64_t N, int64_t K, int rank) {
 
 size_t group_hidden_ws_bytes(int64_t M, int64_t K, int r_total) { return nt_part_bytes(M, K, r_total, false); }
 
+HiddenOrder hidden_order(int64_t K) {
+  const NtPlan p = plan_nt(1, K, false);  // the same plan up to 32 tokens: one row tile
+  return p.few ? HiddenOrder{0, 0} : HiddenOrder{p.splits, p.chunks_per_split};
+}
+
 int run_group_hidden(const uint16_t* x, const GroupSkinny& g, uint16_t* h_cat, float* ws, hipStream_t s) {
   NtBatch b = {};
   b.M = (int)g.M;

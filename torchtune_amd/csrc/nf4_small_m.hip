@@ -18,15 +18,17 @@
 //    scalers in one pass ahead of the loop, the table holds fp16 pairs (a code point is exact in fp16), which the multiply
 //    converts on the way, and every thread finishes outputs.  The hidden product h = x . lora_a^T can ride along as
 //    further row tiles of the same loop, where that beats a launch of its own.
-//    us, weights from HBM, hidden product included, before -> now at 1 / 13 tokens: 4096 x 4096 12.5 / 14.2 -> 6.7 / 7.6, 14336 x 4096 21.3 /
-//    25.7 -> 14.9 / 16.7, 4096 x 14336 22.1 / 30.8 -> 15.6 / 20.4, 2048 x 2048 9.1 / 11.1 -> 5.4 / 5.9, gate / up pair of 14336 x 4096 38.0 / 43.1 ->
-//    26.6 / 31.2.  A read of the same bytes in the same row pieces takes 3.1, 6.3, 6.6 and (the pair) 10.3: the pair is bound by
+//    us, weights from HBM, hidden product included, before -> now at 1 / 13 tokens: 4096 x 4096 12.5 / 14.2 -> 7.9 / 8.4, 14336 x 4096 21.3 /
+//    25.7 -> 17.0 / 19.7, 4096 x 14336 22.1 / 30.8 -> 19.3 / 23.3, 2048 x 2048 9.1 / 11.1 -> 5.6 / 6.1, gate / up pair of 14336 x 4096 38.0 / 43.1 ->
+//    31.0 / 31.5.  A read of the same bytes in the same row pieces takes 3.1, 6.3, 6.6 and (the pair) 10.3: the pair is bound by
 //    the expansion (VALU 10.9 us, LDS 11.7 of 22 us busy without the hidden product).
 //  * nf4_small_m_kernel (17 - 64 tokens): groups of U chunks per wave, two or four token tiles.
 #include "common.h"
 #include "group.h"
 #include "nf4_math.h"
 #include "swiglu_math.h"
+
+#include <type_traits>
 
 #define TT_LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
 
@@ -68,6 +70,7 @@ struct SmallMGroup {
   SmallMArgs m[kGroupMax];
   int wg_end[kGroupMax];
   int n;
+  int splits, chunks_per_split;  // where the launch forms h: how its sums run (hidden_order)
 };
 
 constexpr int kSmMaxWaves = 16;
@@ -290,34 +293,68 @@ __device__ __forceinline__ float scaled_hi(uint32_t pair, float s) {
   return r;
 }
 
-// LDS of a few-token workgroup: the code table, the block scalers of its rows over a segment of the contraction, and per wave
-// one stage: 128 columns of x (MQ groups of four tokens), of its row tiles' codes and of its members' lora_a.
-template <int RT, int NT, int MQ>
-struct FewLayout {
-  static constexpr int kCopies = NT > 0 ? 1 : 16;  // of the code table
-  static constexpr int kLut = 1024 * kCopies;
-  static constexpr int kSegment = 16384 / RT;  // columns; a multiple of 128 times the most waves, so that it does not move the waves' chunks
-  static constexpr int kStage = (MQ + RT + 4 * NT) * 1024;
-  __host__ __device__ static int scalers(int K) {  // an odd row stride: the rows of a tile on different banks
-    const int kb = (K < kSegment ? K : kSegment) >> 6;
-    return (RT * 16 * (kb | 1) * 4 + 15) & ~15;
-  }
-  static int bytes(int K, int waves) { return kLut + scalers(K) + waves * kStage; }
-};
+// How h = x . lora_a^T of at most 16 tokens is summed, wherever it is formed: the order of the adapters' own launch
+// (lora_skinny.hip), which is the same for every such token count, for a member alone and in a group.
+//   K <= kNtFewK (splits == 0): 64-wide chunks go round sixteen waves, two chains each (the halves of every chunk); the chains of
+//     a wave, then the waves in order.
+//   beyond: splits of chunks_per_split chunks, dealt to four waves in turn, one chain each; the waves of a split in order,
+//     then the splits.
+// In a chunk lane group g holds columns 16 g .. + 15, the first eight for one MFMA, the others for the next.
+// A launch that forms h itself meets that order by one of three forms:
+//   kWaves (splits == 0): the 128-wide chunk that a wave has staged for its weight rows is a chunk of two of the sixteen waves.
+//   kPaired (sixteen parts of a row's sum, eight chunks per split): the two parts of a wave are two 128-wide chunks apart, which
+//     makes them the two chunks of two chains.
+//   kGather (the others): the chunks of a chain, a and a + 4, are staged side by side, x a second time with them; a wave forms
+//     whole splits.
+enum HiddenForm { kReads, kWaves, kPaired, kGather };
+
+// LDS of a few-token workgroup: the code table, the block scalers of its rows over a segment of the contraction, the splits'
+// sums of h, and per wave one stage: 128 columns of x (MQ groups of four tokens), of its row tiles' codes, and of its
+// members' lora_a (kGather: and of x again).  At the end a stage holds the wave's partial sums.
+constexpr int few_lut_bytes(int nt) { return nt > 0 ? 1024 : 16 * 1024; }  // one or sixteen copies of the code table
+// Columns of a segment: whole rounds of the waves' chunks and splits, so that it does not move either.
+constexpr int few_segment(int rt, int nt, int mq, int form) {
+  return nt == 2 && mq == 4 ? 4096 : form == kPaired && mq == 4 ? 8192 : 16384 / rt;
+}
+constexpr int few_stage_bytes(int rt, int sets, int nt, int mq, int form) {
+  const int staged = mq + rt + (form == kGather ? mq : 0) + 4 * nt, left = sets * rt;
+  return (staged > left ? staged : left) * 1024;
+}
+constexpr int few_scaler_bytes(int rt, int nt, int mq, int form, int K) {  // an odd row stride: the rows of a tile on different banks
+  const int segment = few_segment(rt, nt, mq, form), kb = (K < segment ? K : segment) >> 6;
+  return (rt * 16 * (kb | 1) * 4 + 15) & ~15;
+}
+// fp32 [split][sums of a split][rank tile][4 ranks][token][4]; kPaired: of its first two chains, its third, its fourth
+constexpr int few_split_sums(int form) { return form == kPaired ? 3 : form == kGather ? 1 : 0; }
+constexpr int few_split_bytes(int rt, int nt, int mq, int form, int splits) {
+  const int most = few_segment(rt, nt, mq, form) / 512;
+  return (splits < most ? splits : most) * few_split_sums(form) * nt * 64 * 4 * mq;
+}
+constexpr int few_bytes(int rt, int sets, int nt, int mq, int form, int K, int splits, int waves) {
+  return few_lut_bytes(nt) + few_scaler_bytes(rt, nt, mq, form, K) + few_split_bytes(rt, nt, mq, form, splits) +
+         waves * few_stage_bytes(rt, sets, nt, mq, form);
+}
 
 // RT tiles of 16 weight rows per workgroup, at most MAXW waves, tokens in MQ groups of four.  PAIR: the even tiles belong to grp.m[0]
 // (gate), the odd ones to the same rows of grp.m[1] (up projection, the same width), and act = bf16(bf16(silu(y_0)) * y_1) is
 // written as well.
-// NA > 0: h = x . lora_a^T is formed here, NA tiles of 16 ranks per member beside the row tiles (the workgroup's own copy: the
-// members' first workgroups also write it to m.h_out where that is asked for); otherwise it is read from m.h.
+// SETS: a row's chunks are summed in MAXW SETS parts of four chains each (part c % (MAXW SETS) takes chunk c), added in order; a
+// wave has the parts wave and wave + 8, kPaired: 4 (wave / 2) + wave % 2 and the one two further on.
+// FORM != kReads: h = x . lora_a^T is formed here, NA tiles of 16 ranks per member beside the row tiles (the workgroup's own
+// copy: the members' first workgroups also write it to m.h_out where that is asked for); otherwise it is read from m.h.
 // ONE: the launch has one member, and its arguments sit at fixed places (found through `which` they cost two dependent
 // scalar loads before the first request: 0.4 us of a launch of 6 - 8).
-template <int RT, int MAXW, int MQ, int NA, bool PAIR, bool ONE>
-__global__ __launch_bounds__(64 * MAXW) void nf4_few_kernel(const SmallMGroup grp, uint16_t* __restrict__ act) {
+// Registers: two workgroups per CU, but one of eight waves where LDS has no room for a second.
+template <int RT, int MAXW, int SETS, int MQ, int NA, int FORM, bool PAIR, bool ONE>
+__global__ __launch_bounds__(64 * MAXW, MAXW == 8 && NA * (PAIR ? 2 : 1) <= 1 && (FORM < kPaired || MQ == 1) ? 4 : 2) void nf4_few_kernel(const SmallMGroup grp, uint16_t* __restrict__ act) {
 #if defined(__HIP_DEVICE_COMPILE__)  // LDS address-space casts
   static_assert(!PAIR || RT % 2 == 0, "a pair is two row tiles of equal rows");
-  constexpr int NT = NA * (PAIR ? 2 : 1);  // rank tiles
-  using L = FewLayout<RT, NT, MQ>;
+  static_assert(MAXW == 8 || (MAXW == 4 && SETS == 1), "the parts of a row's sum");
+  constexpr int NT = NA * (PAIR ? 2 : 1), kNA = NA > 0 ? NA : 1;  // rank tiles, of a member
+  constexpr bool GATHER = FORM == kGather, PAIRED = FORM == kPaired, SPLITS = GATHER || PAIRED;
+  static_assert((NA > 0) == (FORM != kReads) && (!PAIRED || (MAXW == 8 && SETS == 2)), "the forms");
+  constexpr int kStage = few_stage_bytes(RT, SETS, NT, MQ, FORM), kSegment = few_segment(RT, NT, MQ, FORM);
+  constexpr int kX2 = (MQ + RT) * 1024, kA = kX2 + (GATHER ? MQ * 1024 : 0);  // of a stage: x again, lora_a
   int which = 0;  // uniform over the workgroup
   if constexpr (!PAIR && !ONE) {
 #pragma unroll
@@ -333,9 +370,11 @@ __global__ __launch_bounds__(64 * MAXW) void nf4_few_kernel(const SmallMGroup gr
   const int wg = (int)blockIdx.x - (!PAIR && !ONE && which ? grp.wg_end[which - 1] : 0);
   auto member = [&](int rt) -> const SmallMArgs& { return grp.m[PAIR ? rt & 1 : which]; };
   auto first_row = [&](int rt) { return PAIR ? 16 * (wg * (RT / 2) + (rt >> 1)) : 16 * (RT * wg + rt); };  // every row exists
-  float* const scal = reinterpret_cast<float*>(few_smem + L::kLut);
-  const int scal_bytes = L::scalers(K);
-  char* const stage = few_smem + L::kLut + scal_bytes + wave * L::kStage;
+  float* const scal = reinterpret_cast<float*>(few_smem + few_lut_bytes(NT));
+  const int n_splits = SPLITS ? grp.splits : 0, per_split = grp.chunks_per_split;
+  char* const split_sums = few_smem + few_lut_bytes(NT) + few_scaler_bytes(RT, NT, MQ, FORM, K);
+  char* const stages = split_sums + few_split_bytes(RT, NT, MQ, FORM, n_splits);
+  char* const stage = stages + wave * kStage;
   const uint32_t lds_scal = (uint32_t)(uintptr_t)TT_LDS_PTR(scal), lds_stage = (uint32_t)(uintptr_t)TT_LDS_PTR(stage);
 
   // ---- requests: direct-to-LDS loads, 64 pieces of 16 bytes each.  Four neighbouring lanes ask for 64 contiguous bytes: the
@@ -345,48 +384,61 @@ __global__ __launch_bounds__(64 * MAXW) void nf4_few_kernel(const SmallMGroup gr
   auto dma16 = [&](uint32_t voff, const void* base, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "s"(lds) : "memory", "m0");
   };
-  uint32_t x_off[MQ], a_off[NT > 0 ? NA * 4 : 1];
-  const int r4 = lane >> 4, p16 = lane & 15, cr = lane >> 2, cp = (lane & 3) ^ ((lane >> 4) & 3);
+  const int r4 = lane >> 4, cr = lane >> 2, cp = (lane & 3) ^ ((lane >> 4) & 3);
+  uint32_t piece[4];  // byte offset of the lane's piece of row 4 d + r4 (and of the rows 16 further on)
+  uint32_t x_row[MQ];
+#pragma unroll
+  for (int d = 0; d < 4; ++d) piece[d] = (uint32_t)((lane & 15) ^ (4 * d + r4)) << 4;
 #pragma unroll
   for (int d = 0; d < MQ; ++d) {
     const int r = 4 * d + r4;
-    x_off[d] = (uint32_t)(r < M ? r : M - 1) * (uint32_t)K * 2u + ((p16 ^ r) << 4);  // rows beyond M repeat the last one: never stored
+    x_row[d] = (uint32_t)(r < M ? r : M - 1) * (uint32_t)K * 2u;  // rows beyond M repeat the last one: never stored
   }
-  if constexpr (NT > 0) {
+  const uint32_t a_lane = (uint32_t)r4 * (uint32_t)K * 2u;
+  auto request_x = [&](int64_t col_bytes, int to, auto at) {
 #pragma unroll
-    for (int d = 0; d < NA * 4; ++d) {
-      const int r = 4 * d + r4;  // ranks beyond R of any member repeat one: zeroed where they would count
-      a_off[d] = (uint32_t)r * (uint32_t)K * 2u + ((p16 ^ (r & 15)) << 4);
-    }
-  }
-  const uint32_t c_off = (uint32_t)cr * (uint32_t)(K >> 1) + (cp << 4);
-  auto request = [&](int c) {
-    const bool half = c * 128 + 64 >= K;  // the last chunk of a K that is an odd multiple of 64: its second half repeats the first
+    for (int d = 0; d < MQ; ++d) dma16(x_row[d] + at(piece[d]), reinterpret_cast<const char*>(grp.m[which].x) + col_bytes, lds_stage + to + d * 1024);
+  };
+  auto request_a = [&](int64_t col_bytes, auto at) {
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
-      dma16(half ? c_off - ((cp & 2) << 4) : c_off, member(rt).codes + (((int64_t)first_row(rt) * K) >> 1) + (int64_t)c * 64,
-            lds_stage + (MQ + rt) * 1024);
+    for (int a = 0; a < NT; ++a) {
+      const SmallMArgs& ma = member(a / kNA);
 #pragma unroll
-    for (int d = 0; d < MQ; ++d)
-      dma16(half ? x_off[d] - (((p16 ^ (4 * d + r4)) & 8) << 4) : x_off[d], reinterpret_cast<const char*>(grp.m[which].x) + (int64_t)c * 256,
-            lds_stage + d * 1024);
-    if constexpr (NT > 0) {
-#pragma unroll
-      for (int a = 0; a < NT; ++a) {
-        const SmallMArgs& ma = member(a / NA);
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-          const int e = 4 * (a % NA) + d;
-          uint32_t off = a_off[e];
-          if (4 * e + r4 >= ma.R) off = (p16 ^ ((4 * e + r4) & 15)) << 4;
-          if (half) off -= ((p16 ^ ((4 * e + r4) & 15)) & 8) << 4;
-          dma16(off, reinterpret_cast<const char*>(ma.lora_a) + (int64_t)c * 256, lds_stage + (MQ + RT + 4 * a) * 1024 + d * 1024);
-        }
+      for (int d = 0; d < 4; ++d) {
+        const int row = 16 * (a % kNA) + 4 * d;  // R % 8 == 0: four rows exist or none; beyond R the first ones again, which do not count
+        dma16(a_lane + at(piece[d]), reinterpret_cast<const char*>(ma.lora_a) + (row < ma.R ? (int64_t)row * K * 2 : 0) + col_bytes,
+              lds_stage + kA + a * 4096 + d * 1024);
       }
     }
   };
-  constexpr int kBatch = RT + MQ + 4 * NT;
-  const int stride = (K < L::kSegment ? KB : L::kSegment >> 6) | 1;
+  const uint32_t c_off = (uint32_t)cr * (uint32_t)(K >> 1) + (cp << 4);
+  auto half_of = [&](int c) { return c * 128 + 64 >= K; };  // the last chunk of a K that is an odd multiple of 64: its second half repeats the first
+  auto request_codes = [&](int c) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+      dma16(half_of(c) ? c_off - ((cp & 2) << 4) : c_off, member(rt).codes + (((int64_t)first_row(rt) * K) >> 1) + (int64_t)c * 64,
+            lds_stage + (MQ + rt) * 1024);
+  };
+  auto request_operands = [&](int c) {
+    const uint32_t mask = half_of(c) ? 0x70u : 0xf0u;
+    auto at = [&](uint32_t p) { return p & mask; };
+    request_x((int64_t)c * 256, 0, at);
+    if constexpr (NT > 0 && !GATHER) request_a((int64_t)c * 256, at);
+  };
+  auto request = [&](int c) {
+    request_codes(c);
+    request_operands(c);
+  };
+  // GATHER: chain w of split sp; its chunks are chunk_of and, where that exists, four further on
+  auto chunk_of = [&](int sp, int w) { return sp * per_split + w; };
+  auto chunks_end = [&](int sp) { return (sp + 1) * per_split < KB ? (sp + 1) * per_split : KB; };
+  auto request_chain = [&](int sp, int w) {
+    const uint32_t second = chunk_of(sp, w) + 4 < chunks_end(sp) ? 512u : 0u;  // otherwise the second repeats the first
+    auto at = [&](uint32_t p) { return (p & 0x70u) | ((p << 2) & second); };
+    request_x((int64_t)chunk_of(sp, w) * 128, kX2, at);
+    request_a((int64_t)chunk_of(sp, w) * 128, at);
+  };
+  const int stride = (K < kSegment ? KB : kSegment >> 6) | 1;
   auto request_scalers = [&](int first, int n) {  // blocks [first, first + n) of every row
     for (int r = wave; r < 16 * RT; r += nw) {
       const float* base = member(PAIR ? r >> 4 : 0).bscal + (int64_t)(first_row(r >> 4) + (r & 15)) * KB + first;
@@ -399,171 +451,337 @@ __global__ __launch_bounds__(64 * MAXW) void nf4_few_kernel(const SmallMGroup gr
   const int n_chunks = (K + 127) >> 7;
 
   // The first requests leave before the code table is built: a workgroup lives for little more than one trip to memory.
-  const int seg_chunks = L::kSegment >> 7;
-  request_scalers(0, KB < L::kSegment >> 6 ? KB : L::kSegment >> 6);
-  int c = wave;  // the host gives a launch no more waves than there are chunks
-  request(c);
+  constexpr int seg_chunks = kSegment >> 7, seg_splits = kSegment / 512;
+  request_scalers(0, KB < kSegment >> 6 ? KB : kSegment >> 6);
+  const int start = PAIRED ? 4 * (wave >> 1) + (wave & 1) : wave;  // the wave's first chunk of a segment
+  request(start);  // the host gives a launch no more waves than there are chunks (kPaired: at least seventeen chunks)
+  if constexpr (GATHER) {
+    if (wave < n_splits) request_chain(wave, 0);
+  }
   uint32_t* const lut = reinterpret_cast<uint32_t*>(few_smem);
+  constexpr int kCopies = few_lut_bytes(NT) / 1024;
   typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
   for (int e = t; e < 256; e += blockDim.x) {
     const half2_t p = {(_Float16)round_to_bf16(nf4_code_value(e >> 4)), (_Float16)round_to_bf16(nf4_code_value(e & 15))};
     const uint32_t v = __builtin_bit_cast(uint32_t, p);
-    if constexpr (L::kCopies == 1) {
+    if constexpr (kCopies == 1) {
       lut[e] = v;
     } else {
 #pragma unroll
-      for (int j = 0; j < L::kCopies / 4; ++j)
-        reinterpret_cast<u32x4_t*>(lut)[e * (L::kCopies / 4) + ((j + e) & (L::kCopies / 4 - 1))] = u32x4_t{v, v, v, v};
+      for (int j = 0; j < kCopies / 4; ++j)
+        reinterpret_cast<u32x4_t*>(lut)[e * (kCopies / 4) + ((j + e) & (kCopies / 4 - 1))] = u32x4_t{v, v, v, v};
     }
   }
-  const char* const lut_lane = reinterpret_cast<const char*>(lut) + (L::kCopies > 1 ? (lane & (L::kCopies - 1)) * 4 : 0);
-  constexpr int kShift = L::kCopies == 1 ? 2 : 6;  // entry e lies at e << kShift
+  const char* const lut_lane = reinterpret_cast<const char*>(lut) + (kCopies > 1 ? (lane & (kCopies - 1)) * 4 : 0);
+  constexpr int kShift = kCopies == 1 ? 2 : 6;  // entry e lies at e << kShift
   auto pair_of = [&](uint32_t codes, int b) {
     const uint32_t off = (8 * b >= kShift ? codes >> (8 * b - kShift) : codes << (kShift - 8 * b)) & (0xffu << kShift);
     return *reinterpret_cast<const uint32_t*>(lut_lane + off);
   };
-  constexpr int kChains = 2;  // the same in every instance: a row's bits do not depend on the launch's shape
-  f32x4_t acc[RT][kChains], ah[NT > 0 ? NT : 1][kChains];
+  constexpr int kHSets = SPLITS ? 1 : 8 / MAXW;  // pairs of h's sixteen parts that a wave forms
+  // h: kWaves [][set][half of a chunk][chain]; kPaired [][0][chain][0]; kGather [][0][0][0] the split's sum so far
+  f32x4_t acc[RT][SETS][4], ah[NT > 0 ? NT : 1][kHSets][2][2];
 #pragma unroll
-  for (int s = 0; s < kChains; ++s) {
+  for (int s = 0; s < 4; ++s) {
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) acc[rt][s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-    for (int a = 0; a < (NT > 0 ? NT : 1); ++a) ah[a][s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      for (int u = 0; u < SETS; ++u) acc[rt][u][s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int a = 0; a < (NT > 0 ? NT : 1); ++a)
+#pragma unroll
+      for (int u = 0; u < kHSets; ++u) ah[a][u][s >> 1][s & 1] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
-  // the scalers are a wave's oldest requests: its first chunk may stay in flight across the barrier
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kBatch) : "memory");
+  // the scalers are a wave's oldest requests: its first chunk (and chain) may stay in flight across the barrier
+  if (GATHER && wave >= n_splits)
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(RT + MQ) : "memory");
+  else
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(RT + MQ + (GATHER ? MQ : 0) + 4 * NT) : "memory");
 
-  const int xr = i & (4 * MQ - 1);
-  const int x_at = xr * 256, a_at = (MQ + RT) * 1024 + i * 256, c_at = MQ * 1024 + i * 64 + ((g ^ ((i >> 2) & 3)) << 4);
+  constexpr int kTokens = 4 * MQ;
+  const int xr = i & (kTokens - 1);
+  const int c_at = MQ * 1024 + i * 64 + ((g ^ ((i >> 2) & 3)) << 4);
+  // piece p of this lane's token and rank
+  auto read_x = [&](int from, int p) { return *reinterpret_cast<const u32x4_t*>(stage + from + xr * 256 + ((p ^ xr) << 4)); };
+  auto read_a = [&](int a, int p) { return *reinterpret_cast<const u32x4_t*>(stage + kA + a * 4096 + i * 256 + ((p ^ i) << 4)); };
+  auto mfma = [&](const u32x4_t& rows, const u32x4_t& cols, const f32x4_t& sum) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, rows), __builtin_bit_cast(bf16x8_t, cols), sum, 0, 0, 0);
+  };
+  // what this thread has of h where splits are added, elements t, t + 64 MAXW, .. of [rank tile][4 ranks][token][4]
+  constexpr int kHElements = NT * 16 * kTokens, kHOwn = (kHElements + 64 * MAXW - 1) / (64 * MAXW);
+  float h_sum[kHOwn > 0 ? kHOwn : 1];
+#pragma unroll
+  for (int j = 0; j < (kHOwn > 0 ? kHOwn : 1); ++j) h_sum[j] = 0.f;
+
   for (int first = 0;;) {  // segments of the contraction
     const int end = n_chunks < first + seg_chunks ? n_chunks : first + seg_chunks;
-    for (; c < end; c += nw) {
+    const int first_split = first / seg_chunks * seg_splits, end_split = n_splits < first_split + seg_splits ? n_splits : first_split + seg_splits;
+    // One chunk of the weight rows and (GATHER) one chain of h.  set: the part of the sums that they belong to.
+    int c = first + start, sp = first_split + wave, w = 0;
+    auto step = [&](auto which_set) {
+      constexpr int set = decltype(which_set)::value;
+      const int next = PAIRED ? (set == 0 ? c + 2 : c + 14) : c + nw;
+      const bool has = c < end;
+      const int chunk = GATHER && sp < end_split ? chunk_of(sp, w) : 0, stop = GATHER && sp < end_split ? chunks_end(sp) : 0;
+      const bool chain = GATHER && chunk < stop;
+      const bool half = half_of(c);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       // the stage goes to registers and is asked for again
-      u32x4_t cd[RT], xb[4], ab[NT > 0 ? NT : 1][4];
+      u32x4_t cd[RT], xb[4], xh[4], ab[NT > 0 ? NT : 1][4];
       float sc[RT];
+      const bool forms = NT > 0 && (GATHER ? chain : has);
+      auto multiply_h = [&]() {
+        if (!forms) return;
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt) {
-        cd[rt] = *reinterpret_cast<const u32x4_t*>(stage + c_at + rt * 1024);
-        sc[rt] = scal[(16 * rt + i) * stride + 2 * (c - first) + (g >> 1)];  // beyond K: any value, times zero
-      }
+        for (int a = 0; a < NT; ++a) {
+          if constexpr (GATHER) {
+            f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
+            sum = mfma(ab[a][1], xh[1], mfma(ab[a][0], xh[0], sum));
+            if (chunk + 4 < stop) sum = mfma(ab[a][3], xh[3], mfma(ab[a][2], xh[2], sum));
+            ah[a][0][0][0] = w == 0 ? sum : ah[a][0][0][0] + sum;
+          } else if constexpr (PAIRED) {
 #pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        xb[s] = *reinterpret_cast<const u32x4_t*>(stage + x_at + (((4 * g + s) ^ xr) << 4));
-        if constexpr (NT > 0) {
+            for (int b = 0; b < 2; ++b) {
+              if (set == 0) ah[a][0][b][0] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+              if (b == 0 || !half) ah[a][0][b][0] = mfma(ab[a][2 * b + 1], xh[2 * b + 1], mfma(ab[a][2 * b], xh[2 * b], ah[a][0][b][0]));
+            }
+          } else {
+            constexpr int hs = set % kHSets;
 #pragma unroll
-          for (int a = 0; a < NT; ++a) ab[a][s] = *reinterpret_cast<const u32x4_t*>(stage + a_at + a * 4096 + (((4 * g + s) ^ i) << 4));
+            for (int s = 0; s < 4; ++s)
+              if (s < 2 || !half) ah[a][hs][s >> 1][s & 1] = mfma(ab[a][s], xh[s], ah[a][hs][s >> 1][s & 1]);
+          }
         }
+      };
+      auto read_h = [&]() {
+        if (!forms) return;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {  // half s / 2 of the 128 columns, MFMA s % 2 of it
+          const int p = 8 * (s >> 1) + 2 * g + (s & 1);
+          xh[s] = read_x(GATHER ? kX2 : 0, p);
+#pragma unroll
+          for (int a = 0; a < NT; ++a) ab[a][s] = read_a(a, p);
+        }
+      };
+      constexpr bool kHFirst = NT > 0 && RT > 1;  // all operands at once do not fit the registers of two workgroups per CU
+      if constexpr (kHFirst) {
+        read_h();
+        multiply_h();
+        asm volatile("" ::: "memory");
       }
+      if (has) {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+          cd[rt] = *reinterpret_cast<const u32x4_t*>(stage + c_at + rt * 1024);
+          sc[rt] = scal[(16 * rt + i) * stride + 2 * (c - first) + (g >> 1)];  // beyond K: any value, times zero
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s) xb[s] = read_x(0, 4 * g + s);
+      }
+      if constexpr (!kHFirst) read_h();
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      if (c + nw < end) request(c + nw);
-      if (c * 128 + 64 >= K && g >= 2) {  // half a chunk: nothing of its second half counts, whatever lies there
-#pragma unroll
-        for (int s = 0; s < 4; ++s) xb[s] = u32x4_t{0, 0, 0, 0};
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) sc[rt] = 0.f;
-        if constexpr (NT > 0) {
-#pragma unroll
-          for (int a = 0; a < NT; ++a)
-#pragma unroll
-            for (int s = 0; s < 4; ++s) ab[a][s] = u32x4_t{0, 0, 0, 0};
-        }
+      if (next < end) request(next);
+      const int nsp = w == 3 ? sp + nw : sp, nwv = (w + 1) & 3;
+      if constexpr (GATHER) {
+        if (nsp < end_split && chunk_of(nsp, nwv) < chunks_end(nsp)) request_chain(nsp, nwv);
       }
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const bf16x8_t xv = __builtin_bit_cast(bf16x8_t, xb[s]);
-        if constexpr (NT > 0) {
+      if constexpr (!kHFirst) multiply_h();
+      if constexpr (GATHER) {
+        if (sp < end_split && w == 3 && i < kTokens) {
 #pragma unroll
           for (int a = 0; a < NT; ++a)
-            ah[a][s % kChains] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, ab[a][s]), xv, ah[a][s % kChains], 0, 0, 0);
+            *reinterpret_cast<f32x4_t*>(split_sums + ((sp - first_split) * NT + a) * kTokens * 64 + (g * kTokens + i) * 16) = ah[a][0][0][0];
+        }
+        sp = __builtin_amdgcn_readfirstlane(nsp);
+        w = __builtin_amdgcn_readfirstlane(nwv);
+      }
+      if (has) {
+        if (half) {  // nothing of its second half counts, whatever lies there
+#pragma unroll
+          for (int s = 0; s < 4; ++s) xb[s] = g >= 2 ? u32x4_t{0, 0, 0, 0} : xb[s];
+#pragma unroll
+          for (int rt = 0; rt < RT; ++rt) sc[rt] = g >= 2 ? 0.f : sc[rt];
         }
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
-          u32x4_t wf;
+          uint32_t pairs[4][4];  // all reads of a tile's chunk in flight together
 #pragma unroll
-          for (int b = 0; b < 4; ++b) {
-            const uint32_t p = pair_of(cd[rt][s], b);
-            wf[b] = pack_pair(scaled_lo(p, sc[rt]), scaled_hi(p, sc[rt]));
+          for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) pairs[s][b] = pair_of(cd[rt][s], b);
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            u32x4_t wf;
+#pragma unroll
+            for (int b = 0; b < 4; ++b) wf[b] = pack_pair(scaled_lo(pairs[s][b], sc[rt]), scaled_hi(pairs[s][b], sc[rt]));
+            acc[rt][set % SETS][s] = mfma(wf, xb[s], acc[rt][set % SETS][s]);
           }
-          acc[rt][s % kChains] =
-              __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf), xv, acc[rt][s % kChains], 0, 0, 0);
+        }
+      }
+      c = next;
+    };
+    while (c < end || (GATHER && sp < end_split)) {  // a segment is an even number of rounds: sets do not shift
+      const int split = c >> 2;
+      step(std::integral_constant<int, 0>());
+      if constexpr (SETS > 1 || (NT > 0 && kHSets > 1)) {
+        if (c < end || (GATHER && sp < end_split)) step(std::integral_constant<int, 1>());
+      }
+      if constexpr (PAIRED) {  // chains 0 and 1 of the split, or 2 and 3
+        if (i < kTokens) {
+#pragma unroll
+          for (int a = 0; a < NT; ++a) {
+            char* const to = split_sums + ((split - first_split) * 3 * NT + a) * kTokens * 64 + (g * kTokens + i) * 16;
+            if (wave & 1) {
+              *reinterpret_cast<f32x4_t*>(to + NT * kTokens * 64) = ah[a][0][0][0];
+              *reinterpret_cast<f32x4_t*>(to + 2 * NT * kTokens * 64) = ah[a][0][1][0];
+            } else {
+              *reinterpret_cast<f32x4_t*>(to) = ah[a][0][0][0] + ah[a][0][1][0];
+            }
+          }
+        }
+      }
+    }
+    if constexpr (SPLITS) {
+      __syncthreads();  // the segment's splits are in LDS
+#pragma unroll
+      for (int j = 0; j < kHOwn; ++j) {
+        const int e = t + j * 64 * MAXW;
+        if (e < kHElements) {
+          const float* const from = reinterpret_cast<const float*>(split_sums) + e;
+          constexpr int kSums = few_split_sums(FORM);
+          int n = end_split - first_split;
+          const bool last_of_one = PAIRED && 4 * (end_split - 1) + 1 >= n_chunks;  // the last split has no third and fourth chain
+          if (last_of_one) --n;
+#pragma unroll 4
+          for (int q = 0; q < n; ++q) {
+            float sum = from[kSums * q * kHElements];
+            if constexpr (PAIRED) sum = (sum + from[(3 * q + 1) * kHElements]) + from[(3 * q + 2) * kHElements];
+            h_sum[j] += sum;
+          }
+          if (last_of_one) h_sum[j] += from[kSums * n * kHElements];
         }
       }
     }
     first += seg_chunks;
     if (first >= n_chunks) break;
-    __syncthreads();  // every wave is done with the segment's scalers
-    request_scalers(2 * first, KB - 2 * first < (L::kSegment >> 6) ? KB - 2 * first : L::kSegment >> 6);
-    if (c < n_chunks) request(c);
+    __syncthreads();  // every wave is done with the segment's scalers (and splits)
+    request_scalers(first * 2, KB - 2 * first < (kSegment >> 6) ? KB - 2 * first : kSegment >> 6);
+    if (first + start < n_chunks) request(first + start);
+    if constexpr (GATHER) {
+      if (first / seg_chunks * seg_splits + wave < n_splits) request_chain(first / seg_chunks * seg_splits + wave, 0);
+    }
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
   }
 
-  // ---- the waves' partial sums meet in LDS, [tile][lane][v] at the head of each wave's stage, and are added in wave order
+  // ---- the parts of the sums meet in LDS, [part][tile][lane][v] at the head of each wave's stage, and are added in order
   constexpr int kSteps = NA > 0 ? (NA + 1) / 2 : 2;  // MFMA steps of the adapter, 32 ranks each (the ranks of a group add up to at most 64)
-  u32x2_t bv[RT][2 * kSteps], hv[PAIR ? 2 : 1][2 * kSteps];  // wave 0: ranks 16 a + 4 g .. + 3 of its rows' lora_b and of its token's h
+  u32x4_t bv[RT][kSteps], hv[PAIR ? 2 : 1][kSteps];  // wave 0: ranks 32 q + 8 g .. + 7 of its rows' lora_b and of its token's h
   if (wave == 0) {
 #pragma unroll
-    for (int a = 0; a < 2 * kSteps; ++a) {
-      const int r = 16 * a + 4 * g;
+    for (int q = 0; q < kSteps; ++q) {
+      const int r = 32 * q + 8 * g;
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
-        bv[rt][a] = u32x2_t{0, 0};
-        if (r < member(rt).R) bv[rt][a] = *reinterpret_cast<const u32x2_t*>(member(rt).lora_b + (int64_t)(first_row(rt) + i) * member(rt).R + r);
+        bv[rt][q] = u32x4_t{0, 0, 0, 0};
+        if (r < member(rt).R) bv[rt][q] = *reinterpret_cast<const u32x4_t*>(member(rt).lora_b + (int64_t)(first_row(rt) + i) * member(rt).R + r);
       }
+      if constexpr (NA == 0) {
 #pragma unroll
-      for (int u = 0; u < (PAIR ? 2 : 1); ++u) {
-        hv[u][a] = u32x2_t{0, 0};
-        if (NA == 0 && i < M && r < member(u).R) hv[u][a] = *reinterpret_cast<const u32x2_t*>(member(u).h + (int64_t)i * member(u).ldh + r);
+        for (int u = 0; u < (PAIR ? 2 : 1); ++u) {
+          hv[u][q] = u32x4_t{0, 0, 0, 0};
+          if (i < M && r < member(u).R) hv[u][q] = *reinterpret_cast<const u32x4_t*>(member(u).h + (int64_t)i * member(u).ldh + r);
+        }
       }
     }
   }
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) acc[rt][0] += acc[rt][1];
-  auto leave = [&](int tile, const f32x4_t& v) { *reinterpret_cast<f32x4_t*>(stage + tile * 1024 + lane * 16) = v; };
-  if (wave > 0) {
+  for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) leave(rt, acc[rt][0]);
-  }
+    for (int u = 0; u < SETS; ++u)
+#pragma unroll
+      for (int s = 1; s < 4; ++s) acc[rt][u][0] += acc[rt][u][s];
+  auto leave = [&](int u, int rt) { *reinterpret_cast<f32x4_t*>(stage + (u * RT + rt) * 1024 + lane * 16) = acc[rt][u][0]; };
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int u = 0; u < SETS; ++u)
+      if (u > 0 || wave > 0) leave(u, rt);
   if constexpr (NT > 0) {
+    // h in bf16, [rank tile][token][16 ranks], over the code table (every wave is past its last chunk)
+    char* const h_tile = few_smem;
+    static_assert(NT * 16 * 32 <= few_lut_bytes(NT), "h lies where the code table was");
+    auto h_done = [&](int e, float sum) {  // element e of [rank tile][4 ranks][token][4]
+      const int a = e / (16 * kTokens), token = (e >> 2) & (kTokens - 1), r = 4 * ((e / (4 * kTokens)) & 3) + (e & 3);
+      const uint16_t bits = f32_to_bf16_bits(sum);
+      *reinterpret_cast<uint16_t*>(h_tile + (a * 16 + token) * 32 + r * 2) = bits;
+      const SmallMArgs& ma = member(a / NA);
+      const int rank = 16 * (a % NA) + r;
+      if (ma.h_out && wg == 0 && token < M && rank < ma.R) ma.h_out[(int64_t)token * ma.ldh + rank] = bits;
+    };
+    if constexpr (SPLITS) {
 #pragma unroll
-    for (int a = 0; a < NT; ++a) {
-      ah[a][0] += ah[a][1];
-      if (wave > 0) leave(RT + a, ah[a][0]);
+      for (int j = 0; j < kHOwn; ++j)
+        if (t + j * 64 * MAXW < kHElements) h_done(t + j * 64 * MAXW, h_sum[j]);
+    } else {
+      // part 2 wave + b + 8 u of sixteen, behind the wave's partial sums
+      constexpr int kAt = SETS * RT * 1024;
+      static_assert(kAt + kHSets * 2 * kHElements * 4 <= kStage, "the parts of h fit a stage");
+#pragma unroll
+      for (int a = 0; a < NT; ++a)
+#pragma unroll
+        for (int u = 0; u < kHSets; ++u)
+#pragma unroll
+          for (int b = 0; b < 2; ++b)
+            if (i < kTokens)
+              *reinterpret_cast<f32x4_t*>(stage + kAt + ((u * 2 + b) * kHElements + a * 16 * kTokens) * 4 + (g * kTokens + i) * 16) = ah[a][u][b][0] + ah[a][u][b][1];
+      __syncthreads();
+      const int parts = KB < 16 ? KB : 16;
+      for (int e = t; e < kHElements; e += blockDim.x) {
+        auto part = [&](int q) {
+          const int from = (q % (2 * MAXW)) >> 1, slot = 2 * (q / (2 * MAXW)) + (q & 1);
+          return *reinterpret_cast<const float*>(stages + from * kStage + kAt + (slot * kHElements + e) * 4);
+        };
+        float sum = part(0);
+        if (parts == 16) {
+#pragma unroll
+          for (int q = 1; q < 16; ++q) sum += part(q);
+        } else {
+          for (int q = 1; q < parts; ++q) sum += part(q);
+        }
+        h_done(e, sum);
+      }
     }
     __syncthreads();
-    if (wave == 0) {  // h, rounded to bf16: rank 16 (a % NA) + 4 g + v of token i
+    if (wave == 0) {
 #pragma unroll
-      for (int a = 0; a < NT; ++a) {
-        for (int w = 1; w < nw; ++w) ah[a][0] += *reinterpret_cast<const f32x4_t*>(stage + w * L::kStage + (RT + a) * 1024 + lane * 16);
-        const SmallMArgs& ma = member(a / NA);
-        const int r = 16 * (a % NA) + 4 * g;
-        if (r < ma.R) hv[a / NA][a % NA] = u32x2_t{pack_pair(ah[a][0][0], ah[a][0][1]), pack_pair(ah[a][0][2], ah[a][0][3])};
-        if (ma.h_out && wg == 0 && i < M && r < ma.R)
-          *reinterpret_cast<u32x2_t*>(ma.h_out + (int64_t)i * ma.ldh + r) = hv[a / NA][a % NA];
-      }
+      for (int u = 0; u < (PAIR ? 2 : 1); ++u)
+#pragma unroll
+        for (int q = 0; q < kSteps; ++q) {
+          const int r = 32 * q + 8 * g;
+          hv[u][q] = u32x4_t{0, 0, 0, 0};
+          if (i < M && r < member(u).R) hv[u][q] = *reinterpret_cast<const u32x4_t*>(h_tile + ((u * NA + (r >> 4)) * 16 + i) * 32 + (r & 15) * 2);
+        }
     }
   }
   if (wave == 0) {
     // adapter: sum_r bf16(h[m][r] * lscale) * lora_b[n][r], the operands the large-M kernel feeds its MFMA
-    auto scaled = [&](uint32_t d, float ls) { return pack_pair(lo_of(d) * ls, hi_of(d) * ls); };
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
-      const int u = PAIR ? rt & 1 : 0;
       const float ls = member(rt).lscale;
 #pragma unroll
       for (int q = 0; q < kSteps; ++q) {
         if (32 * q >= member(rt).R) break;
-        const u32x4_t b = {bv[rt][2 * q].x, bv[rt][2 * q].y, bv[rt][2 * q + 1].x, bv[rt][2 * q + 1].y};
-        const u32x4_t h = {scaled(hv[u][2 * q].x, ls), scaled(hv[u][2 * q].y, ls), scaled(hv[u][2 * q + 1].x, ls), scaled(hv[u][2 * q + 1].y, ls)};
-        acc[rt][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, b), __builtin_bit_cast(bf16x8_t, h), acc[rt][0], 0, 0, 0);
+        u32x4_t h;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) h[d] = pack_pair(lo_of(hv[PAIR ? rt & 1 : 0][q][d]) * ls, hi_of(hv[PAIR ? rt & 1 : 0][q][d]) * ls);
+        acc[rt][0][0] = mfma(bv[rt][q], h, acc[rt][0][0]);
       }
-      leave(rt, acc[rt][0]);
+      leave(0, rt);
     }
   }
   __syncthreads();
   // every thread finishes one output (PAIR: one of each member) at a time: one wave alone took 1.3 us over sixteen waves' sums
-  const char* const parts = few_smem + L::kLut + scal_bytes;
+  const int parts = SETS * MAXW < n_chunks ? SETS * MAXW : n_chunks;
   for (int e = t; e < 256 * (PAIR ? RT / 2 : RT); e += blockDim.x) {
     const int tile = e >> 8, token = (e >> 2) & 15, row = 4 * ((e >> 6) & 3) + (e & 3);
     if (token >= M) continue;
@@ -572,14 +790,17 @@ __global__ __launch_bounds__(64 * MAXW) void nf4_few_kernel(const SmallMGroup gr
     for (int u = 0; u < (PAIR ? 2 : 1); ++u) {
       const int rt = PAIR ? 2 * tile + u : tile;
       const SmallMArgs& a = member(u);
-      const char* p = parts + rt * 1024 + (e & 255) * 4;
       const int n = first_row(rt) + row;
-      float o = *reinterpret_cast<const float*>(p);
-      if (nw == MAXW) {
+      auto part = [&](int q) {
+        const int from = PAIRED ? 2 * (q >> 2) + (q & 1) : q % MAXW, set = PAIRED ? (q >> 1) & 1 : q / MAXW;
+        return *reinterpret_cast<const float*>(stages + from * kStage + (set * RT + rt) * 1024 + (e & 255) * 4);
+      };
+      float o = part(0);
+      if (parts == SETS * MAXW) {
 #pragma unroll
-        for (int w = 1; w < MAXW; ++w) o += *reinterpret_cast<const float*>(p + w * L::kStage);
+        for (int q = 1; q < SETS * MAXW; ++q) o += part(q);
       } else {
-        for (int w = 1; w < nw; ++w) o += *reinterpret_cast<const float*>(p + w * L::kStage);
+        for (int q = 1; q < parts; ++q) o += part(q);
       }
       if (a.bias) o += bf16_bits_to_f32(a.bias[n]);
       if (a.cscale) o *= bf16_bits_to_f32(a.cscale[n]);
@@ -591,100 +812,145 @@ __global__ __launch_bounds__(64 * MAXW) void nf4_few_kernel(const SmallMGroup gr
 #endif
 }
 
-// Launch shape at most 16 tokens.  The waves fix the order in which a row's products are summed and depend on the
-// layer alone, so that a row gets the same bits alone, in a batch of up to 16 tokens and inside a group; row tiles do not
-// enter the sums.  Measured over 27 layers of 256 - 28672 rows and 1024 - 28672 columns (us, weights from HBM, launch gap included):
-//  * eight waves (4096 x 4096 at 1 / 13 tokens, h formed inside: four 8.7 / 9.3, eight 6.7 / 7.9, sixteen 7.6 / 8.8; 2048 x 8192 at 13: 14.6 /
-//    11.1 / 12.3), four where the layer has workgroups to spare and a short contraction (gate / up pair of 14336 x 4096, eight and
-//    four: 21.8 and 20.6);
+// Launch shape at most 16 tokens.  The waves and their sets fix the order in which a row's products are summed (parts of four
+// chains: sixteen up to 4096 rows and, below 8192, where the layer is no wider than its input, four beyond 12288 rows over
+// less than 8192 columns, otherwise eight) and depend on the layer alone, so that a row gets the same bits alone, in a
+// batch of up to 16 tokens and inside a group; row tiles do not enter the sums.  Measured over 27 layers of 256 - 28672 rows
+// and 1024 - 28672 columns (us, weights from HBM, launch gap included):
+//  * eight waves (4096 x 4096 at 1 / 13 tokens, h in the launch's own order: four 8.7 / 9.3, eight 6.7 / 7.9, sixteen 7.6 / 8.8; 2048 x 8192
+//    at 13: 14.6 / 11.1 / 12.3), four where the layer has workgroups to spare and a short contraction (gate / up pair of 14336 x 4096,
+//    eight and four: 21.8 and 20.6);
 //  * two row tiles, which share the reads of x and lora_a, from 8192 rows on (8192 x 2048 at 13 tokens: one 7.9, two 7.0; 14336 x 4096 at one
-//    token with its h: 17.8 and 14.9), but one where four waves at a few tokens read h instead (the same layer 13.9, two 16.1).
+//    token with its h, in the launch's own order: 17.8 and 14.9), but one where four waves at a few tokens read h instead (the
+//    same layer 13.9, two 16.1).
 struct FewConfig {
-  int rt, waves;
-  bool operator==(const FewConfig& o) const { return rt == o.rt && waves == o.waves; }
+  int rt, waves, sets;
+  bool operator==(const FewConfig& o) const { return rt == o.rt && waves == o.waves && sets == o.sets; }
 };
 int few_waves(int64_t N, int64_t K) { return N > 12288 && K < 8192 ? 4 : 8; }
+int few_sets(int64_t N, int64_t K) { return N <= 4096 || (N < 8192 && N <= K) ? 2 : 1; }
 FewConfig few_config(int64_t M, int64_t N, int64_t K, bool hidden) {
   const int waves = few_waves(N, K);
-  return {N >= 8192 && (hidden || waves == 8 || M > 4) ? 2 : 1, waves};
+  return {N >= 8192 && (hidden || waves == 8 || M > 4) ? 2 : 1, waves, few_sets(N, K)};
 }
 FewConfig few_pair_config(int64_t N, int64_t K, bool hidden) {
   const int waves = few_waves(N, K);
-  return {hidden && waves == 4 ? 4 : 2, waves};
+  return {hidden && waves == 4 ? 4 : 2, waves, few_sets(N, K)};
 }
-// Whether a launch of these workgroups forms its members' h = x . lora_a^T itself, instead of a launch or two ahead of it (4 - 6.5 us,
-// and as many launches for the host).  Every workgroup then reads its members' lora_a, rank_tiles tiles of 16 ranks: at 128 MB
-// for the launch still the better way (4096 x 14336: one token 15.6 against 20.2 us, 13 tokens 20.4 against 22.0; at 235 MB, 8192 x
-// 28672, no longer), and several tiles only where the LDS they take (`bytes` a workgroup) leaves room for every workgroup at once
-// (gate / up pair of 8192 x 2048, 512 workgroups in two rounds: 15.1 against 12.1; in one round, 2816 x 1024: 6.8 against 8.7).
-bool few_hidden(int64_t workgroups, int rank_tiles, int64_t K, int bytes) {
-  if (rank_tiles > 1 && workgroups > 256 * (160 * 1024 / bytes)) return false;
+constexpr int kFewMostLds = 160 * 1024;
+HiddenForm few_form(const FewConfig& c, int64_t K) {
+  const HiddenOrder o = hidden_order(K);
+  return o.splits == 0 ? kWaves : c.sets == 2 && o.chunks_per_split == 8 ? kPaired : kGather;
+}
+// Whether a launch of these workgroups forms its members' h = x . lora_a^T itself, instead of a launch or two ahead of it; the
+// bits are the same.  Every workgroup then reads its members' lora_a, rank_tiles tiles of 16 ranks: at 128 MB for the launch
+// still the better way (us with its h, against reading it: 4096 x 14336 at one token 19.3 and 21.1, at 13 tokens 23.3 and 22.2 but two
+// launches fewer; at 235 MB, 8192 x 28672, no longer), and several tiles only where the LDS they take leaves room for every
+// workgroup at once (gate / up pair of 8192 x 2048, 512 workgroups in two rounds: 15.1 against 12.1; in one round, 2816 x 1024:
+// 7.3 against 9.3).  In the order of the adapters' launch h takes 0.4 us of a launch more over 2048 columns and 1 - 3.5 over
+// 4096 - 14336 than in the order that suits the launch (4096 x 4096 6.9 -> 7.9, 2048 x 8192 9.1 -> 11.2; reading it 11.1 and 13.4);
+// the gate / up pair of 14336 x 4096 takes 31.0 with it and 27.3 with two launches ahead, in a layer outside a graph 77 and 82.
+bool few_hidden(int64_t workgroups, const FewConfig& c, int rank_tiles, int64_t M, int64_t K) {
+  const int n_chunks = (int)((K + 127) >> 7), waves = n_chunks < c.waves ? n_chunks : c.waves;
+  const int bytes = few_bytes(c.rt, c.sets, rank_tiles, M <= 4 ? 1 : 4, few_form(c, K), (int)K, hidden_order(K).splits, waves);
+  if (bytes > kFewMostLds || (rank_tiles > 1 && workgroups > 256 * (kFewMostLds / bytes))) return false;
   return workgroups * rank_tiles * 32 * K <= int64_t(128) << 20;
 }
-int few_bytes(int rt, int rank_tiles, int64_t M, int64_t K, int waves) {
-  const int cols = 16384 / rt, kb = (int)(K < cols ? K : cols) >> 6, n_chunks = (int)((K + 127) >> 7);
-  return 1024 + 64 * rt * (kb | 1) + (n_chunks < waves ? n_chunks : waves) * ((M <= 4 ? 1 : 4) + rt + 4 * rank_tiles) * 1024;
-}
 
-template <int RT, int MAXW, int MQ, int NA, bool PAIR, bool ONE>
+template <int RT, int MAXW, int SETS, int MQ, int NA, int FORM, bool PAIR, bool ONE>
 int launch_few(const SmallMGroup& g, unsigned wgs, uint16_t* act, hipStream_t s) {
   constexpr int NT = NA * (PAIR ? 2 : 1);
-  using L = FewLayout<RT, NT, MQ>;
   const int K = g.m[0].K, n_chunks = (K + 127) >> 7, waves = n_chunks < MAXW ? n_chunks : MAXW;
+  constexpr int kSegment = few_segment(RT, NT, MQ, FORM);
+  constexpr int kMost = few_bytes(RT, SETS, NT, MQ, FORM, kSegment, kSegment / 512, MAXW);
+  static_assert(kMost <= kFewMostLds, "the LDS of a CU");
   static bool attr_set[64] = {};  // the LDS limit is a per-device attribute of the function
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;
   if (dev < 0 || !attr_set[dev]) {
-    const int most = L::bytes(L::kSegment, MAXW);
-    static_assert(FewLayout<RT, NT, MQ>::kLut + 16 * RT * (16384 / RT / 64 + 1) * 4 + MAXW * FewLayout<RT, NT, MQ>::kStage <= 160 * 1024,
-                  "the LDS of a CU");
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&nf4_few_kernel<RT, MAXW, MQ, NA, PAIR, ONE>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, most);
-    if (e != hipSuccess) return fail(TTAMD_ELAUNCH, "nf4_few: cannot reserve %d bytes of LDS: %s", most, hipGetErrorString(e));
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&nf4_few_kernel<RT, MAXW, SETS, MQ, NA, FORM, PAIR, ONE>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, kMost);
+    if (e != hipSuccess) return fail(TTAMD_ELAUNCH, "nf4_few: cannot reserve %d bytes of LDS: %s", kMost, hipGetErrorString(e));
     if (dev >= 0) attr_set[dev] = true;
   }
-  nf4_few_kernel<RT, MAXW, MQ, NA, PAIR, ONE><<<dim3(wgs), dim3(64 * waves), L::bytes(K, waves), s>>>(g, act);
+  nf4_few_kernel<RT, MAXW, SETS, MQ, NA, FORM, PAIR, ONE>
+      <<<dim3(wgs), dim3(64 * waves), few_bytes(RT, SETS, NT, MQ, FORM, K, g.splits, waves), s>>>(g, act);
   return check_launch("nf4_few");
 }
 
-template <int RT, int MAXW, int MQ, int NA>
+template <int RT, int MAXW, int SETS, int MQ, int NA, int FORM>
 int launch_few_members(SmallMGroup& g, hipStream_t s) {
   int wgs = 0;
   for (int i = 0; i < g.n; ++i) {
     wgs += g.m[i].N / (16 * RT);
     g.wg_end[i] = wgs;
   }
-  return g.n == 1 ? launch_few<RT, MAXW, MQ, NA, false, true>(g, wgs, nullptr, s) : launch_few<RT, MAXW, MQ, NA, false, false>(g, wgs, nullptr, s);
+  return g.n == 1 ? launch_few<RT, MAXW, SETS, MQ, NA, FORM, false, true>(g, wgs, nullptr, s)
+                  : launch_few<RT, MAXW, SETS, MQ, NA, FORM, false, false>(g, wgs, nullptr, s);
 }
 
-// rank_tiles: of a member, where the launch forms h; 0 where it reads it
-template <int MQ, int NA>
+// The shapes that few_config and few_form give.  NA: rank tiles of a member, where the launch forms h.
+template <int MQ, int NA, int FORM>
 int dispatch_few_members(SmallMGroup& g, const FewConfig& c, hipStream_t s) {
-  if (c.rt == 1) {
-    if constexpr (MQ == 1 && NA == 0) {
-      if (c.waves == 4) return launch_few_members<1, 4, MQ, NA>(g, s);
+  if (c.rt == 1 && c.sets == 2) return launch_few_members<1, 8, 2, MQ, NA, FORM>(g, s);
+  if constexpr (FORM == kPaired) {
+    return fail(TTAMD_EUNSUPPORTED, "nf4_few: no such launch");
+  } else {
+    if (c.rt == 1) {
+      if constexpr (MQ == 1 && NA == 0) {
+        if (c.waves == 4) return launch_few_members<1, 4, 1, MQ, NA, FORM>(g, s);
+      }
+      return launch_few_members<1, 8, 1, MQ, NA, FORM>(g, s);
     }
-    return launch_few_members<1, 8, MQ, NA>(g, s);
+    if constexpr (MQ == 4 || NA > 0) {
+      if (c.waves == 4) return launch_few_members<2, 4, 1, MQ, NA, FORM>(g, s);
+    }
+    if constexpr (MQ == 4 && NA == 2 && FORM == kGather)
+      return fail(TTAMD_EUNSUPPORTED, "nf4_few: no room for the operands of h");  // few_hidden
+    else
+      return launch_few_members<2, 8, 1, MQ, NA, FORM>(g, s);
   }
-  return c.waves == 8 ? launch_few_members<2, 8, MQ, NA>(g, s) : launch_few_members<2, 4, MQ, NA>(g, s);
 }
-int dispatch_few(SmallMGroup& g, const FewConfig& c, int rank_tiles, hipStream_t s) {
+template <int NA>
+int dispatch_few_forming(SmallMGroup& g, const FewConfig& c, hipStream_t s) {
   const bool one = g.m[0].M <= 4;  // group of four tokens
-  switch (rank_tiles) {
-    case 0: return one ? dispatch_few_members<1, 0>(g, c, s) : dispatch_few_members<4, 0>(g, c, s);
-    case 1: return one ? dispatch_few_members<1, 1>(g, c, s) : dispatch_few_members<4, 1>(g, c, s);
-    default: return one ? dispatch_few_members<1, 2>(g, c, s) : dispatch_few_members<4, 2>(g, c, s);
+  switch (few_form(c, g.m[0].K)) {
+    case kWaves: return one ? dispatch_few_members<1, NA, kWaves>(g, c, s) : dispatch_few_members<4, NA, kWaves>(g, c, s);
+    case kPaired: return one ? dispatch_few_members<1, NA, kPaired>(g, c, s) : dispatch_few_members<4, NA, kPaired>(g, c, s);
+    default: return one ? dispatch_few_members<1, NA, kGather>(g, c, s) : dispatch_few_members<4, NA, kGather>(g, c, s);
   }
 }
+// rank_tiles: of a member, where the launch forms h; 0 where it reads it
+int dispatch_few(SmallMGroup& g, const FewConfig& c, int rank_tiles, hipStream_t s) {
+  if (rank_tiles == 0) return g.m[0].M <= 4 ? dispatch_few_members<1, 0, kReads>(g, c, s) : dispatch_few_members<4, 0, kReads>(g, c, s);
+  return rank_tiles == 1 ? dispatch_few_forming<1>(g, c, s) : dispatch_few_forming<2>(g, c, s);
+}
+template <int MQ>
+int dispatch_few_pair_reading(const SmallMGroup& g, const FewConfig& c, unsigned wgs, uint16_t* act, hipStream_t s) {
+  if (c.waves == 4) return launch_few<2, 4, 1, MQ, 0, kReads, true, false>(g, wgs, act, s);
+  return c.sets == 2 ? launch_few<2, 8, 2, MQ, 0, kReads, true, false>(g, wgs, act, s) : launch_few<2, 8, 1, MQ, 0, kReads, true, false>(g, wgs, act, s);
+}
+// few_pair_forms: more than four tokens only over short contractions, and not with four row tiles
+template <int FORM>
+int dispatch_few_pair_forming(const SmallMGroup& g, const FewConfig& c, unsigned wgs, uint16_t* act, hipStream_t s) {
+  if constexpr (FORM == kWaves) {
+    if (g.m[0].M > 4) return c.sets == 2 ? launch_few<2, 8, 2, 4, 1, FORM, true, false>(g, wgs, act, s) : launch_few<2, 8, 1, 4, 1, FORM, true, false>(g, wgs, act, s);
+  }
+  if (c.sets == 2) return launch_few<2, 8, 2, 1, 1, FORM, true, false>(g, wgs, act, s);
+  if constexpr (FORM == kPaired)
+    return fail(TTAMD_EUNSUPPORTED, "nf4_few: no such launch");
+  else
+    return c.rt == 4 ? launch_few<4, 4, 1, 1, 1, FORM, true, false>(g, wgs, act, s) : launch_few<2, 8, 1, 1, 1, FORM, true, false>(g, wgs, act, s);
+}
+bool few_pair_forms(const FewConfig& c, int64_t M, int64_t K) { return M <= 4 || (c.rt == 2 && few_form(c, K) == kWaves); }
 int dispatch_few_pair(const SmallMGroup& g, const FewConfig& c, bool hidden, uint16_t* act, hipStream_t s) {
   const unsigned wgs = g.m[0].N / (8 * c.rt);
-  const bool one = g.m[0].M <= 4;
-  if (hidden) {
-    if (c.rt == 4) return launch_few<4, 4, 1, 1, true, false>(g, wgs, act, s);  // few_pair_hidden: at most four tokens
-    return one ? launch_few<2, 8, 1, 1, true, false>(g, wgs, act, s) : launch_few<2, 8, 4, 1, true, false>(g, wgs, act, s);
+  if (!hidden) return g.m[0].M <= 4 ? dispatch_few_pair_reading<1>(g, c, wgs, act, s) : dispatch_few_pair_reading<4>(g, c, wgs, act, s);
+  switch (few_form(c, g.m[0].K)) {
+    case kWaves: return dispatch_few_pair_forming<kWaves>(g, c, wgs, act, s);
+    case kPaired: return dispatch_few_pair_forming<kPaired>(g, c, wgs, act, s);
+    default: return dispatch_few_pair_forming<kGather>(g, c, wgs, act, s);
   }
-  if (c.waves == 4) return one ? launch_few<2, 4, 1, 0, true, false>(g, wgs, act, s) : launch_few<2, 4, 4, 0, true, false>(g, wgs, act, s);
-  return one ? launch_few<2, 8, 1, 0, true, false>(g, wgs, act, s) : launch_few<2, 8, 4, 0, true, false>(g, wgs, act, s);
 }
 
 // Shape of a launch of 17 - 64 tokens: token tiles, row tiles per workgroup, chunks in flight per wave, most waves.  It fixes
@@ -833,20 +1099,19 @@ int run_small_m_group(const void* x, const GroupGemm& gg, const void* h_cat, voi
 }
 
 bool few_forms_hidden(const GroupGemm& gg, bool gated) {
-  if (gg.M > kFewTokens || gg.K >= kFewMaxK) return false;
+  if (gg.M > kFewTokens || gg.K >= kFewMaxK || hidden_order(gg.K).chunks_per_split > 8) return false;
   for (int i = 0; i < gg.n; ++i)
     if (gg.rank[i] < 8 || gg.rank[i] > kFewHiddenRank) return false;
   if (gated) {
     const FewConfig c = few_pair_config(gg.N[0], gg.K, true);
-    return rank_tiles_of(gg, 0, 2) == 1 && (c.rt == 2 || gg.M <= 4) && few_hidden(gg.N[0] / (8 * c.rt), 2, gg.K, few_bytes(c.rt, 2, gg.M, gg.K, c.waves));
+    return rank_tiles_of(gg, 0, 2) == 1 && few_pair_forms(c, gg.M, gg.K) && few_hidden(gg.N[0] / (8 * c.rt), c, 2, gg.M, gg.K);
   }
   for (int i = 0; i < gg.n;) {
     const int j = run_of(gg, i, [&](int p, int q) { return same_few(gg, p, q, true); });
-    int64_t wgs = 0;
-    for (int q = i; q < j; ++q) wgs += gg.N[q] / (16 * few_config(gg.M, gg.N[q], gg.K, true).rt);
     const FewConfig c = few_config(gg.M, gg.N[i], gg.K, true);
-    const int tiles = rank_tiles_of(gg, i, j);
-    if (!few_hidden(wgs, tiles, gg.K, few_bytes(c.rt, tiles, gg.M, gg.K, c.waves))) return false;
+    int64_t wgs = 0;
+    for (int q = i; q < j; ++q) wgs += gg.N[q] / (16 * c.rt);
+    if (!few_hidden(wgs, c, rank_tiles_of(gg, i, j), gg.M, gg.K)) return false;
     i = j;
   }
   return true;
@@ -859,7 +1124,10 @@ int run_few_with_hidden(const void* x, const GroupGemm& gg, const uint16_t* cons
     all[q].lora_a = lora_a[q];
     all[q].h_out = h_cat ? reinterpret_cast<uint16_t*>(h_cat) + gg.r_off[q] : nullptr;
   }
+  const HiddenOrder order = hidden_order(gg.K);
   SmallMGroup g = {};
+  g.splits = order.splits;
+  g.chunks_per_split = order.chunks_per_split;
   if (act) {
     g.m[0] = all[0];
     g.m[1] = all[1];
