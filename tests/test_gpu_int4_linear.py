@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from torchtune_amd import ops
+from torchtune_amd import _lib, ops
 from torchtune_amd.qat import Int8DynActInt4WeightLinear, WeightOnlyInt4Linear
 
 pytestmark = pytest.mark.gpu
@@ -120,3 +120,25 @@ def test_calls_the_kernels_do_not_serve_keep_the_dense_weight():
     # odd widths run as before
     narrow = _layer("8da4w", 200, 256, 32, False, torch.float32)
     assert not ops.int4_linear_applies(5, 200, 256, 32) and narrow(x.detach()).shape == (5, 200)
+
+
+@pytest.mark.parametrize("m", [1, 5])
+@pytest.mark.parametrize("int8,n,parts", [(True, 1024, 8), (True, 4096, 16), (True, 8192, 8), (False, 1024, 16), (False, 8192, 8)])
+def test_streaming_sums_run_in_four_chains_per_wave(int8, n, parts, m):
+    """Every weight is 1, every activation 1 but a first one of 2^40 and, where its chain ends, one of -2^40: what the chain adds
+    in between is absorbed, at most 32 values for each of the chain's chunks, and the result falls short by as much."""
+    lib, k = _lib.load(), 4096
+    chunks = k // 128 // parts
+    x = torch.ones(m, k, device=DEV, dtype=torch.bfloat16)
+    x[:, 0], x[:, (chunks - 1) * parts * 128] = 2.0 ** 40, -(2.0 ** 40)
+    y = torch.empty(m, n, device=DEV, dtype=torch.bfloat16)
+    stream = torch.cuda.current_stream().cuda_stream
+    if int8:
+        q, scale = torch.ones(n, k, device=DEV, dtype=torch.int8), torch.ones(n, k // 128, device=DEV)
+        status = lib.ttamd_int8_group_linear_bf16(x.data_ptr(), q.data_ptr(), scale.data_ptr(), None, _lib.TTAMD_F32, 128, None, y.data_ptr(), m, n, k, None, 0, stream)
+    else:
+        q = torch.full((n, k // 2), 0x99, device=DEV, dtype=torch.uint8)  # (9 - 8) * scale + zero
+        scale = torch.tensor([1.0, 0.0], device=DEV, dtype=torch.bfloat16).repeat(k // 128 * n)
+        status = lib.ttamd_uint4_group_linear_bf16(x.data_ptr(), q.data_ptr(), scale.data_ptr(), 128, None, y.data_ptr(), m, n, k, None, 0, stream)
+    assert status == 0
+    assert bool((y.float() <= k).all()) and bool((y.float() >= k - 2 - 32 * chunks - 16).all())  # 16: a bf16 step of the result

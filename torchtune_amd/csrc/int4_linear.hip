@@ -324,12 +324,11 @@ __global__ __launch_bounds__(64 * MAXW) void int4_stream_kernel(const Int4Args a
   } else {
     if (c < n_chunks) request(c);
   }
-  constexpr int kChains = 2;
-  f32x4_t acc[RT][kChains];
+  f32x4_t acc[RT][4];  // four chains
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-    for (int s = 0; s < kChains; ++s) acc[rt][s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < 4; ++s) acc[rt][s] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   const int xr = i & (4 * MQ - 1);  // DYN: tokens beyond M read the first one
   const uint16_t* xrow = xq + (int64_t)(i < a.M ? i : 0) * a.K + 32 * g;
@@ -376,12 +375,12 @@ __global__ __launch_bounds__(64 * MAXW) void int4_stream_kernel(const Int4Args a
     for (int s = 0; s < 4; ++s)
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
-        acc[rt][s % kChains] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w[rt].operand(s)),
-                                                                       __builtin_bit_cast(bf16x8_t, xb[s]), acc[rt][s % kChains], 0, 0, 0);
+        acc[rt][s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w[rt].operand(s)),
+                                                             __builtin_bit_cast(bf16x8_t, xb[s]), acc[rt][s], 0, 0, 0);
   }
   // partial sums, [tile][lane][v] at the head of each wave's stage, added in wave order by all threads
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) *reinterpret_cast<f32x4_t*>(stage + rt * 1024 + lane * 16) = acc[rt][0] + acc[rt][1];
+  for (int rt = 0; rt < RT; ++rt) *reinterpret_cast<f32x4_t*>(stage + rt * 1024 + lane * 16) = ((acc[rt][0] + acc[rt][1]) + acc[rt][2]) + acc[rt][3];
   __syncthreads();
   for (int e = threadIdx.x; e < 256 * RT; e += blockDim.x) {
     const int token = (e >> 2) & 15, n = n0 + 16 * (e >> 8) + 4 * ((e >> 6) & 3) + (e & 3);
