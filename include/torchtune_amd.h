@@ -425,6 +425,10 @@ int ttamd_nf4_group_bwd_dx_ws_bf16(const ttamd_lora_group_member* members, int n
 size_t ttamd_gemm_mid_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int ttamd_gemm_mid_bf16(int kind, const void* a, const void* b, const void* bias, void* c, int64_t M, int64_t N, int64_t K,
                         void* workspace, size_t workspace_bytes, void* stream);
+/* How that call runs a product (bias: one comes with it): rows of an output tile (0: tiles of 128 x 128 on four waves; kind 2 with
+ * 256: tiles of 256 x 256), slices of the contraction (a workspace of slices * M * N * 4 bytes serves where there are
+ * several), and the most contraction indices that one chain of fp32 sums runs over.  Needs no GPU. */
+int ttamd_gemm_mid_plan(int kind, int bias, int64_t M, int64_t N, int64_t K, int* tile_rows, int* slices, int* chain);
 
 /*
  * One expansion for both directions of a group.  ttamd_nf4_group_fwd_leaves_tiles says what the group's forward call

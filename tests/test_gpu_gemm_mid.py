@@ -1,5 +1,7 @@
 """Fake-quantised linears below the sizes of the 256 x 256-tile kernels: the three products of ``ttamd_gemm_mid_bf16`` through
 ``FakeQuantizedLinear``, against fp32 matmuls of the same fake-quantised operands."""
+import ctypes
+
 import pytest
 import torch
 import torch.nn.functional as F
@@ -149,9 +151,60 @@ def test_weight_gradients_on_wide_tiles(tokens):
     assert bool((c[N] == 7).all())
 
 
+def _plan(kind, M, N, K, bias=0):
+    tile_rows, slices, chain = (ctypes.c_int() for _ in range(3))
+    assert _lib.load().ttamd_gemm_mid_plan(kind, bias, M, N, K, ctypes.byref(tile_rows), ctypes.byref(slices), ctypes.byref(chain)) == 0
+    return tile_rows.value, slices.value, chain.value
+
+
 def test_products_below_2048_rows():
     for M, N, K, mid in [(1000, 14336, 4096, True), (2047, 14336, 4096, True), (1000, 4096, 14336, False), (2047, 15360, 4096, False),
                          (1290, 6912, 2560, False), (2000, 800064, 64, False)]:
         layer = FakeQuantizedLinear(K, N, False, None, FakeQuantizeConfig(torch.int4, group_size=32), device="cuda", dtype=torch.bfloat16)
         assert layer._mid_ok(torch.empty(M, K, device="cuda", dtype=torch.bfloat16)) is mid, (M, N, K)
     test_linear_and_gradients(701, 9728, 3584, False)
+
+
+@pytest.mark.parametrize("kind,M,N,K,rows", [(1, 368, 2048, 2048, 64), (0, 1053, 1024, 2816, 64), (0, 660, 3584, 9728, 128), (1, 1254, 2048, 8192, 128)])
+def test_chains_that_end_before_the_contraction_does(kind, M, N, K, rows):
+    """Every operand is 1 but one of 2^40 at the head of a chain and one of -2^40 at the head of the next: each absorbs the ones
+    that follow it in its chain.  In one chain the second would restore the first, and half as many would be lost."""
+    tile_rows, slices, chain = _plan(kind, M, N, K)
+    assert (tile_rows, slices) == (rows, 1) and chain < K // 2
+    a = torch.ones(M, K, device="cuda", dtype=torch.bfloat16)
+    a[:, 0], a[:, 2 * chain] = 2.0 ** 40, -(2.0 ** 40)  # a step is 64 indices, the first 32 of them in this half's chains
+    b = torch.ones((N, K) if kind == 0 else (K, N), device="cuda", dtype=torch.bfloat16)
+    c = torch.empty(M, N, device="cuda", dtype=torch.bfloat16)
+    assert _lib.load().ttamd_gemm_mid_bf16(kind, a.data_ptr(), b.data_ptr(), None, c.data_ptr(), M, N, K, None, 0,
+                                           torch.cuda.current_stream().cuda_stream) == 0
+    lost = K - c.float()
+    last = min(chain, K // 2 - chain)  # of the second chain
+    assert bool((lost <= chain + last + K / 128).all()) and bool((lost >= chain + last - 64 - K / 128).all())  # 128: a bf16 step
+    torch.manual_seed(M + N + K)
+    a, b = torch.randn(M, K, device="cuda").bfloat16(), torch.randn_like(b.float()).bfloat16()
+    assert _lib.load().ttamd_gemm_mid_bf16(kind, a.data_ptr(), b.data_ptr(), None, c.data_ptr(), M, N, K, None, 0,
+                                           torch.cuda.current_stream().cuda_stream) == 0
+    _close(c, a.double() @ (b.double().t() if kind == 0 else b.double()), K)
+
+
+# every launch that the plan can choose, by the plan's own word: (kind, M, N, K) -> rows of a tile, split / whole / ended chains
+@pytest.mark.parametrize("kind,M,N,K,rows,form", [
+    (0, 65, 320, 192, 64, "whole"), (0, 129, 512, 4160, 64, "split"), (0, 193, 320, 704, 64, "ended"), (0, 1025, 3520, 2048, 128, "whole"),
+    (0, 1000, 2048, 8256, 128, "split"), (0, 193, 8256, 4160, 128, "ended"), (0, 1025, 6464, 192, 256, "whole"),
+    (1, 65, 320, 192, 64, "whole"), (1, 129, 512, 4160, 64, "split"), (1, 193, 320, 704, 64, "ended"), (1, 1025, 3520, 2048, 128, "whole"),
+    (1, 1000, 2048, 8256, 128, "split"), (1, 193, 8256, 4160, 128, "ended"), (1, 1025, 6464, 1024, 256, "whole"), (1, 1025, 6464, 192, 0, "whole"),
+    (2, 64, 64, 513, 0, "split"), (2, 128, 576, 65, 0, "whole"), (2, 4160, 2624, 33, 256, "whole"), (2, 8192, 2048, 1001, 256, "whole"),
+    (2, 8192, 2048, 1024, 256, "whole")])
+def test_every_launch(kind, M, N, K, rows, form):
+    tile_rows, slices, chain = _plan(kind, M, N, K)
+    halves = 2 if kind < 2 and tile_rows else 1
+    assert (tile_rows, "split" if slices > 1 else "ended" if halves * chain < K else "whole") == (rows, form)
+    torch.manual_seed(M + N + K + kind)
+    a = torch.randn((K, M) if kind == 2 else (M, K), device="cuda").bfloat16()
+    b = torch.randn((N, K) if kind == 0 else (K, N), device="cuda").bfloat16()
+    c = torch.full((M + 1, N), 7.0, device="cuda").bfloat16()  # one row beyond the product
+    ws = torch.empty(max(4 * slices * M * N if slices > 1 else 0, 1), device="cuda", dtype=torch.uint8)
+    assert _lib.load().ttamd_gemm_mid_bf16(kind, a.data_ptr(), b.data_ptr(), None, c.data_ptr(), M, N, K, ws.data_ptr(), ws.numel(),
+                                           torch.cuda.current_stream().cuda_stream) == 0
+    _close(c[:M], (a.double().t() if kind == 2 else a.double()) @ (b.double().t() if kind == 0 else b.double()), K)
+    assert bool((c[M] == 7).all())

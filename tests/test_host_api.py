@@ -647,3 +647,23 @@ def test_small_bf16_products_of_few_tiles_are_sliced_within_one_workgroup_per_cu
             for K in (64, 1024, 4096, 14336):
                 slices = lib.ttamd_gemm_mid_workspace_bytes(M, N, K) // (4 * M * N)
                 assert slices == 0 or tiles > 128 or tiles * slices <= 256, (M, N, K)
+
+
+
+def _gemm_mid_plan(kind, M, N, K, bias=0):
+    tile_rows, slices, chain = (ctypes.c_int() for _ in range(3))
+    assert _lib.load().ttamd_gemm_mid_plan(kind, bias, M, N, K, ctypes.byref(tile_rows), ctypes.byref(slices), ctypes.byref(chain)) == 0
+    return tile_rows.value, slices.value, chain.value
+
+
+def test_chains_of_small_bf16_products_are_no_longer_than_the_four_wave_kernels():
+    """The split of the four-wave kernel is what the workspace query counts; a chain of it runs over one slice."""
+    lib = _lib.load()
+    widths = (256, 512, 1024, 1536, 2048, 2816, 3584, 4096, 8192, 9728, 14336)
+    for M in (48, 60, 129, 333, 368, 500, 660, 1000, 1290, 1400, 1528, 1900, 2047):
+        for N in widths:
+            for K in widths:
+                split = max(1, lib.ttamd_gemm_mid_workspace_bytes(M, N, K) // (4 * M * N))
+                most = 32 * max(-(-(K // 32) // split), 2)
+                for kind in (0, 1, 2):
+                    assert _gemm_mid_plan(kind, M, N, K)[2] <= most, (kind, M, N, K)

@@ -21,8 +21,8 @@
 // 256 x 256 tiles of gemm_tn.hip (31.3 us there).
 // Launches of few tiles cut the contraction into slices (fp32 slabs, added in slice order by gemm_mid_reduce_kernel).
 // Over 380 products of kinds 0 and 1 (40 - 8192 rows, 256 - 14336 columns) these two take 0.84 of the time of the four-wave
-// kernel alone, and the sums are closer to the exact ones (2.7e-7 against 3.9e-7 over 8192 indices in two slices): two chains
-// of half the length.  A training pass of a 1B-shaped layer over 1000 tokens with its 21 products: 825 -> 735 us, with the wide
+// kernel alone; where both cut the contraction alike the sums are closer to the exact ones (2.7e-7 against 3.9e-7 over 8192
+// indices in two slices): two chains of half the length.  A training pass of a 1B-shaped layer over 1000 tokens with its 21 products: 825 -> 735 us, with the wide
 // tiles for its weight gradients 714 (host-bound there).
 #include "common.h"
 #include "group.h"
@@ -59,6 +59,7 @@ struct MidArgs {
   int M, N, K;
   int tiles_m, tiles, per_xcd;
   int slices, steps_per_slice;
+  int chain;             // FOLD: steps of a chain, even
 };
 
 constexpr int kMidCols = 128;  // columns of a tile
@@ -76,7 +77,8 @@ struct MidShape {
   static constexpr int a_loads = MT / 2, b_loads = 2, loads = a_loads + b_loads;  // per wave and step, 1 KiB each
 };
 
-template <bool B_COL, bool SPLIT, int MT, int WGS>
+// FOLD: the chains end after g.chain steps and are added up in registers (not with 256 rows: they fill the registers).
+template <bool B_COL, bool SPLIT, int MT, int WGS, bool FOLD>
 __global__ __launch_bounds__(512, 2 * WGS) void gemm_mid_kernel(const MidArgs g) {
 #if defined(__HIP_DEVICE_COMPILE__)
   using S = MidShape<MT, WGS>;
@@ -194,14 +196,36 @@ __global__ __launch_bounds__(512, 2 * WGS) void gemm_mid_kernel(const MidArgs g)
         if (more) issue(t + S::stages, old, d);
     }
   };
+  f32x4_t ended[FOLD ? 4 : 1][MT];  // the chains that have ended
+  int left = FOLD ? g.chain : 0;    // steps of the present one
+  auto fold = [&](bool last) {
+    if constexpr (FOLD) {
+      left -= 2;
+      if (left > 0 && !last) return;
+      left = g.chain;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+          ended[j][i] += acc[j][i];
+          acc[j][i] = last ? ended[j][i] : f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+  };
+#pragma unroll
+  for (int j = 0; j < (FOLD ? 4 : 1); ++j)
+#pragma unroll
+    for (int i = 0; i < MT; ++i) ended[j][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   int t = t_begin;
   for (; t + 1 + S::stages < t_end; t += 2) {
     step(t, 0, std::true_type());
     step(t + 1, 1, std::true_type());
+    fold(false);
   }
   for (; t < t_end; t += 2) {
     step(t, 0, std::false_type());
     if (t + 1 < t_end) step(t + 1, 1, std::false_type());
+    fold(t + 2 >= t_end);
   }
 
   // ---- the two halves of each step's contraction: a wave keeps the columns 32 kg .. + 31 of its 64 and hands over the rest
@@ -476,7 +500,8 @@ __global__ __launch_bounds__(256) void gemm_mid_reduce_kernel(const float* __res
 struct MidPlan {
   int64_t tiles_m, tiles;
   int slices, steps;
-  int rows;  // of a tile of gemm_mid_kernel (kind 2: 256, gemm_tn_kernel); 0: gemm_mid_pair_kernel
+  int rows;   // of a tile of gemm_mid_kernel (kind 2: 256, gemm_tn_kernel); 0: gemm_mid_pair_kernel
+  int chain;  // steps of a chain, below `steps` where a whole contraction's chains are ended early
 };
 // gemm_mid_pair_kernel, and the most slices of either kernel (the workspace is sized before the kind is known): the split with
 // the least of (steps of one workgroup) + (slabs written and read, one more launch), with the times measured on this kernel:
@@ -504,9 +529,13 @@ MidPlan plan_pair(int64_t M, int64_t N, int64_t K) {
       p.slices = (int)slices;
     }
   }
+  p.chain = p.steps;
   return p;
 }
 
+// No fp32 chain is longer than the split of plan_pair would make it, which one whole contraction in nine is (3696 products of
+// kinds 0 and 1, 48 - 2047 rows): gemm_mid_kernel at 64 and 128 rows then ends its chains there, at 3 % of its time on average,
+// and the others are no candidates (1183 x 3584 x 9728, from 256 rows to 128: 126 -> 140 us).
 // Kinds 0 and 1: the kernel, tile height and split with the least modelled time in us, a term for each round of 256 workgroups
 // (512 of the kernels that run two per CU), for its steps and for how full the chip is (its clock falls with the load), and for
 // the slabs.  The terms are fitted to 760 products (40 - 8192 rows, the widths of seven model shapes), every tile and split of
@@ -527,11 +556,9 @@ MidPlan plan_mid(int kind, int64_t M, int64_t N, int64_t K) {
     return p;
   }
   double best = 1e30;
-  if (kind == 1) {
+  if (kind == 1 && pair.slices == 1) {
     const double k = (double)((K + 31) / 32), rounds = (double)((pair.tiles + 255) / 256);
     best = 1.54 + 2.19 * rounds + k * (rounds > 1 ? 0.15 * rounds : 0.19) + 0.07 * k * (double)pair.tiles / 256;
-    p.slices = 1;
-    p.steps = (int)((K + 31) / 32);
   }
   const int64_t nk = K / kMidStep;
   for (const int rows : {64, 128, 256}) {
@@ -544,18 +571,23 @@ MidPlan plan_mid(int kind, int64_t M, int64_t N, int64_t K) {
                  : rows == 128 ? rounds * (5.04 + 0.32 * k) + 0.14 * k * fill
                                : rounds * (8.72 + 0.32 * k) + 0.26 * k * fill;
       if (slices > 1) t += rows == 64 ? 2.23 + 2.71 * slabs : 3.84 + 1.84 * slabs;
-      if (t < best) {
+      const bool fold = steps > pair.steps;
+      if (t < best && !(fold && (rows == 256 || slices > 1))) {
         best = t;
         p.rows = rows;
         p.tiles_m = tiles_m;
         p.tiles = tiles;
         p.steps = (int)steps;
         p.slices = (int)slices;
+        p.chain = !fold ? (int)steps : pair.steps > 3 ? pair.steps / 2 * 2 : 2;
       }
     }
   }
   return p;
 }
+
+// the wide tiles of kind 2 add no bias
+MidPlan plan_of(int kind, bool bias, int64_t M, int64_t N, int64_t K) { return kind == 2 && bias ? plan_pair(M, N, K) : plan_mid(kind, M, N, K); }
 
 // the LDS limit is a per-device attribute of the function
 int reserve_lds(const void* fn, int bytes, bool (&set)[64]) {
@@ -568,19 +600,20 @@ int reserve_lds(const void* fn, int bytes, bool (&set)[64]) {
   return 0;
 }
 
-template <bool B_COL, bool SPLIT, int MT, int WGS>
+template <bool B_COL, bool SPLIT, int MT, int WGS, bool FOLD = false>
 int launch_mid(MidArgs& g, hipStream_t s) {
   static bool set[64] = {};
   using S = MidShape<MT, WGS>;
-  if (int rc = reserve_lds(reinterpret_cast<const void*>(&gemm_mid_kernel<B_COL, SPLIT, MT, WGS>), S::lds, set)) return rc;
+  if (int rc = reserve_lds(reinterpret_cast<const void*>(&gemm_mid_kernel<B_COL, SPLIT, MT, WGS, FOLD>), S::lds, set)) return rc;
   g.per_xcd = (g.tiles * g.slices + 7) / 8;
-  gemm_mid_kernel<B_COL, SPLIT, MT, WGS><<<dim3(8u * g.per_xcd), dim3(512), S::lds, s>>>(g);
+  gemm_mid_kernel<B_COL, SPLIT, MT, WGS, FOLD><<<dim3(8u * g.per_xcd), dim3(512), S::lds, s>>>(g);
   return check_launch("gemm_mid");
 }
 
 template <bool B_COL>
 int launch_rows(MidArgs& g, int rows, hipStream_t s) {
   if (rows == 256) return launch_mid<B_COL, false, 8, 1>(g, s);
+  if (g.slices == 1 && g.chain < g.steps_per_slice) return rows == 128 ? launch_mid<B_COL, false, 4, 1, true>(g, s) : launch_mid<B_COL, false, 2, 2, true>(g, s);
   if (rows == 128) return g.slices > 1 ? launch_mid<B_COL, true, 4, 1>(g, s) : launch_mid<B_COL, false, 4, 1>(g, s);
   return g.slices > 1 ? launch_mid<B_COL, true, 2, 2>(g, s) : launch_mid<B_COL, false, 2, 2>(g, s);
 }
@@ -605,6 +638,15 @@ extern "C" size_t ttamd_gemm_mid_workspace_bytes(int64_t M, int64_t N, int64_t K
   return p.slices > 1 ? (size_t)p.slices * M * N * sizeof(float) : 0;
 }
 
+extern "C" int ttamd_gemm_mid_plan(int kind, int bias, int64_t M, int64_t N, int64_t K, int* tile_rows, int* slices, int* chain) {
+  TT_REQUIRE(kind >= 0 && kind <= 2 && M > 0 && N > 0 && K > 0 && tile_rows && slices && chain, "gemm_mid_plan: bad argument");
+  const MidPlan p = plan_of(kind, bias != 0, M, N, K);
+  *tile_rows = p.rows;
+  *slices = p.slices;
+  *chain = 32 * p.chain;
+  return TTAMD_OK;
+}
+
 extern "C" int ttamd_gemm_mid_bf16(int kind, const void* a, const void* b, const void* bias, void* c, int64_t M, int64_t N, int64_t K,
                                    void* workspace, size_t workspace_bytes, void* stream) {
   TT_REQUIRE(kind >= 0 && kind <= 2, "gemm_mid: unknown kind %d", kind);
@@ -614,15 +656,15 @@ extern "C" int ttamd_gemm_mid_bf16(int kind, const void* a, const void* b, const
              "gemm_mid: bad shape M=%lld N=%lld K=%lld", (long long)M, (long long)N, (long long)K);
   // per-lane byte offsets inside the kernels are 32-bit
   TT_REQUIRE(M * N < (int64_t(1) << 30) && M * K < (int64_t(1) << 30) && N * K < (int64_t(1) << 30), "gemm_mid: operands too large");
-  const size_t need = ttamd_gemm_mid_workspace_bytes(M, N, K);
+  const MidPlan p = plan_of(kind, bias != nullptr, M, N, K);
+  const size_t need = p.slices > 1 ? (size_t)p.slices * M * N * sizeof(float) : 0;
   if (need) {
     if (!workspace || workspace_bytes < need)
       return fail(TTAMD_EWORKSPACE, "gemm_mid: workspace of %zu bytes, %zu needed", workspace_bytes, need);
     TT_REQUIRE(aligned16(workspace), "gemm_mid: the workspace must be 16-byte aligned");
   }
-  const MidPlan p = kind == 2 && bias ? plan_pair(M, N, K) : plan_mid(kind, M, N, K);  // the wide tiles add no bias
   MidArgs g = {reinterpret_cast<const uint16_t*>(a), reinterpret_cast<const uint16_t*>(b), reinterpret_cast<const uint16_t*>(bias),
-               reinterpret_cast<uint16_t*>(c), reinterpret_cast<float*>(workspace), (int)M, (int)N, (int)K, (int)p.tiles_m, (int)p.tiles, 0, p.slices, p.steps};
+               reinterpret_cast<uint16_t*>(c), reinterpret_cast<float*>(workspace), (int)M, (int)N, (int)K, (int)p.tiles_m, (int)p.tiles, 0, p.slices, p.steps, p.chain};
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (kind == 2 && p.rows) return run_gemm_tn(a, b, c, K, M, N, s);
   const int rc = p.rows ? (kind == 0 ? launch_rows<false>(g, p.rows, s) : launch_rows<true>(g, p.rows, s))
