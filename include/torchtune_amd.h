@@ -420,7 +420,7 @@ int ttamd_nf4_group_bwd_dx_ws_bf16(const ttamd_lora_group_member* members, int n
  * fake-quantised linear at short sequences (F.linear and its autograd on torchao's FakeQuantizedLinear; the recipes reach
  * it from recipes/qat_single_device.py).  kind 0: c[M,N] = a[M,K] . b[N,K]^T (+ bias [N] or NULL); 1: c[M,N] = a[M,K] . b[K,N];
  * 2: c[M,N] = a[K,M]^T . b[K,N].  N % 64 == 0; kinds 0 and 1: K % 64 == 0; kind 2: M % 64 == 0, any K.  workspace:
- * ttamd_gemm_mid_workspace_bytes(M, N, K) bytes (0: may be NULL).
+ * ttamd_gemm_mid_workspace_bytes(M, N, K) bytes serve every kind (0: may be NULL); ttamd_gemm_mid_plan knows of kinds that need none.
  */
 size_t ttamd_gemm_mid_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int ttamd_gemm_mid_bf16(int kind, const void* a, const void* b, const void* bias, void* c, int64_t M, int64_t N, int64_t K,

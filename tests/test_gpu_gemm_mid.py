@@ -6,7 +6,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from torchtune_amd import _lib, ops
+from torchtune_amd import _host, _lib, ops
 from torchtune_amd.qat import FakeQuantizeConfig, FakeQuantizedLinear, FakeQuantizer
 
 pytestmark = pytest.mark.gpu
@@ -208,3 +208,16 @@ def test_every_launch(kind, M, N, K, rows, form):
                                            torch.cuda.current_stream().cuda_stream) == 0
     _close(c[:M], (a.double().t() if kind == 2 else a.double()) @ (b.double().t() if kind == 0 else b.double()), K)
     assert bool((c[M] == 7).all())
+
+
+def test_a_linear_allocates_no_slabs_that_its_products_do_not_write():
+    """1400 tokens of 2048 -> 8192: the four-wave kernel would cut the grad-input into four slices of 11 MB; it runs whole."""
+    M, N, K = 1400, 8192, 2048
+    assert _plan(1, M, K, N)[1] == 1 and _lib.load().ttamd_gemm_mid_workspace_bytes(M, K, N) == 4 * 4 * M * K
+    w = torch.randn(N, K, device="cuda").mul_(0.02).bfloat16()
+    x, gy = torch.randn(M, K, device="cuda").bfloat16().requires_grad_(), torch.randn(M, N, device="cuda").bfloat16()
+    y = _host.load().straight_through_linear(x, w, w, None)
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    torch.autograd.grad(y, x, gy)
+    assert torch.cuda.max_memory_allocated() - before < 2 * 2 * M * K  # the gradient itself: 2 bytes an element

@@ -745,7 +745,9 @@ Tensor gemm_mid(int kind, const Tensor& a_in, const Tensor& b_in, const Tensor& 
   TORCH_CHECK_VALUE((kind == 0 ? b.size(1) : b.size(0)) == K, "gemm_mid: ", a.sizes(), " and ", b.sizes(), " do not fit");
   const c10::DeviceGuard guard(a.device());
   Tensor c = at::empty({M, N}, a.options());
-  const size_t bytes = ttamd_gemm_mid_workspace_bytes(M, N, K);
+  int rows = 0, slices = 1, chain = 0;  // the workspace query counts slices that no launch of this kind may make
+  if (M > 0 && N > 0 && K > 0) check(ttamd_gemm_mid_plan(kind, bias.defined(), M, N, K, &rows, &slices, &chain), "gemm_mid");
+  const size_t bytes = slices > 1 ? (size_t)slices * M * N * sizeof(float) : 0;
   const Tensor ws = bytes ? scratch(bytes, a) : Tensor();
   check(ttamd_gemm_mid_bf16(kind, a.data_ptr(), b.data_ptr(), opt_ptr(bias), c.data_ptr(), M, N, K, opt_ptr(ws), bytes, stream_of(a)), "gemm_mid");
   return c;
