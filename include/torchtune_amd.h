@@ -37,6 +37,7 @@ extern "C" {
 #define TTAMD_BF16 0
 #define TTAMD_F32 1
 
+#define TTAMD_FEW_TOKENS 16 /* most tokens of ttamd_lora_few_fwd_bf16 */
 #define TTAMD_GROUP_MAX 4 /* most members of a group of linears with a common input (ttamd_lora_group_*) */
 
 #define TTAMD_OK 0

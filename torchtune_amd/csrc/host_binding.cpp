@@ -322,6 +322,15 @@ void fill(ttamd_lora_group_member& e, const Member& m, const Tensor& y) {
   e.scale = (float)m.scale;
 }
 
+// The call for a handful of tokens, where it serves these members: its rule and the launch in one crossing of the ABI.  What it
+// refuses, the calls for any number of tokens serve or name the fault of.
+bool few_forward(const Tensor& x2, const ttamd_lora_group_member* members, int n, const Tensor& h_cat, const Tensor& act) {
+  const int status = ttamd_lora_few_fwd_bf16(x2.data_ptr(), members, n, opt_ptr(h_cat), opt_ptr(act), x2.size(0), x2.size(1), stream_of(x2));
+  if (status == TTAMD_EUNSUPPORTED || status == TTAMD_EINVAL) return false;
+  check(status, "lora_few_fwd");
+  return true;
+}
+
 struct LinearOut {
   Tensor x2, h, y;
 };
@@ -337,11 +346,10 @@ LinearOut linear_forward(const Tensor& x, Member m, bool keep) {
   const int rank = (int)m.a.size(0);
   o.y = at::empty(with_last(x, m.w.N), o.x2.options());
   if (keep) o.h = at::empty({M, rank}, o.x2.options());
-  ttamd_lora_group_member one;
-  fill(one, m, o.y);
-  if (ttamd_lora_few_fwd_applies(&one, 1, M, K, 0)) {
-    check(ttamd_lora_few_fwd_bf16(o.x2.data_ptr(), &one, 1, opt_ptr(o.h), nullptr, M, K, stream_of(x)), "lora_few_fwd");
-    return o;
+  if (M <= TTAMD_FEW_TOKENS) {
+    ttamd_lora_group_member one;
+    fill(one, m, o.y);
+    if (few_forward(o.x2, &one, 1, o.h, Tensor())) return o;
   }
   const size_t h_bytes = keep ? 0 : align256(M * rank * 2);
   const Tensor ws = scratch(h_bytes + ttamd_qlora_linear_fwd_workspace_bytes(M, m.w.N, K, rank), o.x2);
@@ -458,10 +466,7 @@ GroupOut group_forward(const Tensor& x, std::vector<Member>& ms, bool gated, boo
   }
   if (keep) o.h_cat = at::empty({M, r_total}, o.x2.options());
   if (gated) o.act = at::empty_like(o.ys[0]);
-  if (ttamd_lora_few_fwd_applies(arr, n, M, K, gated)) {
-    check(ttamd_lora_few_fwd_bf16(o.x2.data_ptr(), arr, n, opt_ptr(o.h_cat), opt_ptr(o.act), M, K, stream_of(x)), "lora_few_fwd");
-    return o;
-  }
+  if (M <= TTAMD_FEW_TOKENS && few_forward(o.x2, arr, n, o.h_cat, o.act)) return o;
   const size_t h_bytes = keep ? 0 : align256(M * r_total * 2);
   const size_t hidden = ttamd_lora_group_hidden_workspace_bytes(arr, n, M, K), fwd = ttamd_lora_group_fwd_workspace_bytes(arr, n, M, K);
   const size_t bytes = hidden > fwd ? hidden : fwd;

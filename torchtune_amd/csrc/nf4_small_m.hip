@@ -271,7 +271,7 @@ __global__ __launch_bounds__(64 * MAXW) void nf4_small_m_kernel(const SmallMGrou
   }
 }
 
-constexpr int kFewTokens = 16;
+constexpr int kFewTokens = TTAMD_FEW_TOKENS;
 // The launch shapes below address x, lora_a and the codes of a row tile with 32-bit byte offsets.
 constexpr int64_t kFewMaxK = int64_t(1) << 26;
 constexpr int kFewHiddenRank = 32;  // most ranks of a member whose hidden product a launch forms itself
