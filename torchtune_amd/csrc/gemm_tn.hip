@@ -482,7 +482,7 @@ size_t tn_slab_bytes(const TnPlan& p) { return (size_t)p.tail_tiles * (p.slices 
 template <bool EDGES = false>
 int launch_gemm_tn(TnArgs& g, void* workspace, size_t workspace_bytes, hipStream_t s) {
   const int64_t tiles = (int64_t)g.tiles_n * g.tiles_k;
-  TnPlan plan = plan_tn(tiles, g.M >> 5);
+  TnPlan plan = EDGES ? TnPlan{(int)tiles, 0, 1} : plan_tn(tiles, g.M >> 5);  // the reduction stores whole tiles of whole steps
   if (plan.slices > 1 && (workspace == nullptr || workspace_bytes < tn_slab_bytes(plan))) plan = TnPlan{(int)tiles, 0, 1};
   TT_REQUIRE(plan.slices == 1 || aligned16(workspace), "gemm_tn: workspace must be 16-byte aligned");
   g.full_tiles = plan.full_tiles;
