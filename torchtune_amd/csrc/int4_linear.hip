@@ -591,9 +591,12 @@ int launch(Int4Args& a, bool dyn, void* workspace, size_t workspace_bytes, hipSt
     // two 17.5 / 20.6; 8192 x 2048 at one 7.0 and 7.6).  uint4: narrow layers sixteen (4096 x 14336 16.4 and 15.3), wide eight (9728 x 3584
     // 11.5 and 15.7).
     const bool wide = a.N >= 8192;
-    if constexpr (FMT == kUint4) return wide ? launch_stream<FMT, 1, 8>(a, dyn, s) : launch_stream<FMT, 1, 16>(a, dyn, s);
-    if (wide && a.M > 1) return launch_stream<FMT, 2, 8>(a, dyn, s);
-    return int8_stream_waves(a.N, a.K) == 16 ? launch_stream<FMT, 1, 16>(a, dyn, s) : launch_stream<FMT, 1, 8>(a, dyn, s);
+    if constexpr (FMT == kUint4) {
+      return wide ? launch_stream<FMT, 1, 8>(a, dyn, s) : launch_stream<FMT, 1, 16>(a, dyn, s);
+    } else {
+      if (wide && a.M > 1) return launch_stream<FMT, 2, 8>(a, dyn, s);
+      return int8_stream_waves(a.N, a.K) == 16 ? launch_stream<FMT, 1, 16>(a, dyn, s) : launch_stream<FMT, 1, 8>(a, dyn, s);
+    }
   }
   const Slicing sl = slicing(a.M, a.N, a.K);
   const int mt = tile_mt(a.M);

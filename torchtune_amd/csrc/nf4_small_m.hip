@@ -311,7 +311,9 @@ enum HiddenForm { kReads, kWaves, kPaired, kGather };
 // LDS of a few-token workgroup: the code table, the block scalers of its rows over a segment of the contraction, the splits'
 // sums of h, and per wave one stage: 128 columns of x (MQ groups of four tokens), of its row tiles' codes, and of its
 // members' lora_a (kGather: and of x again).  At the end a stage holds the wave's partial sums.
-constexpr int few_lut_bytes(int nt) { return nt > 0 ? 1024 : 16 * 1024; }  // one or sixteen copies of the code table
+// Sixteen copies of the code table where h is read (wide layers at one token: 14336 x 4096 18.1 us against 19.2 with one copy, their
+// pair 25.6 and 26.9; narrow ones level), one where it is formed: LDS has the operands of h to hold.
+constexpr int few_lut_bytes(int nt) { return nt > 0 ? 1024 : 16 * 1024; }
 // Columns of a segment: whole rounds of the waves' chunks and splits, so that it does not move either.
 constexpr int few_segment(int rt, int nt, int mq, int form) {
   return nt == 2 && mq == 4 ? 4096 : form == kPaired && mq == 4 ? 8192 : 16384 / rt;
@@ -843,9 +845,10 @@ HiddenForm few_form(const FewConfig& c, int64_t K) {
   return o.splits == 0 ? kWaves : c.sets == 2 && o.chunks_per_split == 8 ? kPaired : kGather;
 }
 // Whether a launch of these workgroups forms its members' h = x . lora_a^T itself, instead of a launch or two ahead of it; the
-// bits are the same.  Every workgroup then reads its members' lora_a, rank_tiles tiles of 16 ranks: at 128 MB for the launch
-// still the better way (us with its h, against reading it: 4096 x 14336 at one token 19.3 and 21.1, at 13 tokens 23.3 and 22.2 but two
-// launches fewer; at 235 MB, 8192 x 28672, no longer), and several tiles only where the LDS they take leaves room for every
+// bits are the same.  Every workgroup then reads its members' lora_a, rank_tiles tiles of 16 ranks: up to 128 MiB for the launch
+// the better way (us with its h, against reading it, at one token: 8192 x 8192, 128 MiB, 18.3 and 19.2, 4096 x 14336 19.3 and 21.1; at
+// 13 tokens 21.3 and 20.0, 23.3 and 22.2, but two launches fewer), not beyond (4096 x 20480, 160 MiB, 26.2 and 25.4, 10240 x 8192
+// 30.0 and 23.9, 8192 x 12288, 192 MiB, 25.8 and 24.2); several tiles only where the LDS they take leaves room for every
 // workgroup at once (gate / up pair of 8192 x 2048, 512 workgroups in two rounds: 15.1 against 12.1; in one round, 2816 x 1024:
 // 7.3 against 9.3).  In the order of the adapters' launch h takes 0.4 us of a launch more over 2048 columns and 1 - 3.5 over
 // 4096 - 14336 than in the order that suits the launch (4096 x 4096 6.9 -> 7.9, 2048 x 8192 9.1 -> 11.2; reading it 11.1 and 13.4);
