@@ -249,8 +249,8 @@ TN_GEMM_MIN_TILES = 192
 MID_GEMM_MAX = 1 << 34
 # The same bound for a weight with at least as many outputs as inputs whose forward fills the rounds of 256 x 128 tiles on the 256
 # CUs to ``MID_GEMM_MIN_FILL``: the range over which whole layers were measured (983 tokens of 14336 x 4096 340 and 394 us, 1701 of
-# 8192 x 2048 164 and 181; layer of dim 4096 forward + backward at 500 tokens 1454 -> 1313 us, at 700 1707 -> 1653, at 1900 3006 ->
-# 2860).  It is not where the vendor begins to win: three products above it are level or faster here, too (2047 tokens of
+# 8192 x 2048 164 and 181; layer of dim 4096 forward + backward at 500 tokens 1240 and 1381 us, at 700 1572 and 1592, at 1900 2695 and
+# 2844).  It is not where the vendor begins to win: three products above it are level or faster here, too (2047 tokens of
 # 16384 x 4096 606 and 673, of 28672 x 4096 1110 and 1157, of 28672 x 8192 2172 and 2247, but 1500 of that 1802 and 1743); those calls
 # keep the kernels, and so the bits, that they had.  With emptier rounds the vendor's choice of tiles wins (1290 tokens of dim 2560,
 # fill 0.63: 1071 and 1124), and with fewer outputs than inputs it does at some lengths (1101 tokens of 4096 x 14336: 440 and 468).
