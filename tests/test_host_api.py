@@ -667,3 +667,20 @@ def test_chains_of_small_bf16_products_are_no_longer_than_the_four_wave_kernels(
                 most = 32 * max(-(-(K // 32) // split), 2)
                 for kind in (0, 1, 2):
                     assert _gemm_mid_plan(kind, M, N, K)[2] <= most, (kind, M, N, K)
+
+
+def _few_applies(M, N, K, rank):
+    member = (_lib.LoraGroupMember * 1)()
+    for field in ("quantized_data", "block_scalers", "lora_a", "lora_b", "y"):
+        setattr(member[0], field, 1 << 16)  # only looked at for alignment
+    member[0].N, member[0].rank, member[0].scale = N, rank, 1.0
+    return _lib.load().ttamd_lora_few_fwd_applies(member, 1, M, K, 0)
+
+
+def test_a_few_token_launch_is_there_for_every_contraction_or_for_none():
+    """Two row tiles, two rank tiles and more than four tokens have no launch that forms h beyond 2048 columns: its operands do
+    not fit a CU's LDS at every length, and the rule says no also where they would."""
+    N = 8192
+    for K in range(2112, 4224, 64):
+        assert _few_applies(5, N, K, 32) == 0 and _few_applies(16, N, K, 24) == 0, K
+    assert _few_applies(5, N, 2048, 32) == 1 and _few_applies(4, N, 2112, 32) == 1 and _few_applies(5, N, 2112, 16) == 1

@@ -854,9 +854,13 @@ HiddenForm few_form(const FewConfig& c, int64_t K) {
 // 4096 - 14336 than in the order that suits the launch (4096 x 4096 6.9 -> 7.9, 2048 x 8192 9.1 -> 11.2; reading it 11.1 and 13.4);
 // the gate / up pair of 14336 x 4096 takes 31.0 with it and 27.3 with two launches ahead, in a layer outside a graph 77 and 82.
 bool few_hidden(int64_t workgroups, const FewConfig& c, int rank_tiles, int64_t M, int64_t K) {
+  const HiddenForm form = few_form(c, K);
+  const int mq = M <= 4 ? 1 : 4, segment = few_segment(c.rt, rank_tiles, mq, form);
+  // the launch is there for every contraction or for none (launch_few)
+  if (few_bytes(c.rt, c.sets, rank_tiles, mq, form, segment, segment / 512, c.waves) > kFewMostLds) return false;
   const int n_chunks = (int)((K + 127) >> 7), waves = n_chunks < c.waves ? n_chunks : c.waves;
-  const int bytes = few_bytes(c.rt, c.sets, rank_tiles, M <= 4 ? 1 : 4, few_form(c, K), (int)K, hidden_order(K).splits, waves);
-  if (bytes > kFewMostLds || (rank_tiles > 1 && workgroups > 256 * (kFewMostLds / bytes))) return false;
+  const int bytes = few_bytes(c.rt, c.sets, rank_tiles, mq, form, (int)K, hidden_order(K).splits, waves);
+  if (rank_tiles > 1 && workgroups > 256 * (kFewMostLds / bytes)) return false;
   return workgroups * rank_tiles * 32 * K <= int64_t(128) << 20;
 }
 
