@@ -113,7 +113,8 @@ def test_a_weight_quantizer_that_does_more_is_called(how):
 
 
 # tiles of 64, 128 and 256 rows with a last row tile of one row and a last column tile of half its width, fewer steps than the
-# ring has stages and more, slices of unequal length
+# ring has stages and more, slices of unequal length (at kind 1 two of them are the four-wave kernel's; test_every_launch asserts
+# which launch a product gets)
 @pytest.mark.parametrize("M,N,K", [(1, 64, 64), (65, 320, 192), (1025, 3520, 2048), (1025, 6464, 192), (1025, 6464, 1024), (129, 512, 4160),
                                    (1000, 2048, 8256), (2049, 2560, 128)])
 @pytest.mark.parametrize("kind", [0, 1])
@@ -135,7 +136,7 @@ def test_tile_heights(kind, M, N, K):
 
 
 # weight gradients on tiles of 256 x 256 whose last row and column of tiles hold 64 of 256: tokens of one part-filled step,
-# around one step, an odd number of steps, more than the ring has stages
+# around one step, an odd number of steps, more than the ring has stages (widths that are whole tiles: test_every_launch)
 @pytest.mark.parametrize("tokens", [1, 31, 32, 33, 97, 1001, 1024])
 def test_weight_gradients_on_wide_tiles(tokens):
     lib = _lib.load()

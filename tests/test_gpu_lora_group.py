@@ -783,3 +783,23 @@ def test_few_token_sums_run_in_four_chains_per_part(N, parts, M):
     x[:, 0], x[:, (chunks - 1) * parts * 128] = 2.0 ** 40, -(2.0 ** 40)
     y = ops.nf4_lora_linear_fwd(x, codes, scal, N, torch.zeros(M, 8, device=DEV, dtype=BF), torch.zeros(N, 8, device=DEV, dtype=BF), 1.0).float()
     assert bool((y <= K).all()) and bool((y >= K - 2 - 32 * chunks - 16).all())  # 16: a bf16 step of the result
+
+
+@pytest.mark.parametrize("M", [1, 4, 5, 16])
+@pytest.mark.parametrize("N,K,r", [(64, 64, 8), (64, 576, 16), (8192, 1088, 32), (64, 2048, 16), (64, 2112, 24), (4096, 4160, 16), (8192, 4160, 8),
+                                   (12352, 4224, 16), (1024, 8256, 32), (8192, 8256, 16), (64, 16448, 16), (128, 33088, 32)])
+def test_the_hidden_product_inside_has_the_bits_of_the_adapters_launch(N, K, r, M):
+    """Fewer chunks than waves, half a chunk at the end, a last split of one to eight chunks, several segments, each form of the
+    order and both row tilings: the sums of h are those of the launch of its own, to the bit."""
+    from torchtune_amd import _lib
+
+    g = torch.Generator(device=DEV).manual_seed(M + N + K + r)
+    x = torch.randn(M, K, device=DEV, generator=g).to(BF)
+    m = ops.GroupMember(torch.randint(0, 256, (N * K // 2,), device=DEV, generator=g, dtype=torch.uint8), torch.rand(N * K // 64, device=DEV, generator=g),
+                        None, torch.randn(r, K, device=DEV, generator=g).mul_(K ** -0.5).to(BF), torch.randn(N, r, device=DEV, generator=g).to(BF),
+                        None, 2.0, N)
+    y, h = torch.empty(M, N, device=DEV, dtype=BF), torch.full((M, r), float("nan"), device=DEV, dtype=BF)
+    arr, keep = ops._group_array("test", [m], K, [y], M)
+    assert _lib.load().ttamd_lora_few_fwd_applies(arr, 1, M, K, 0) == 1
+    _lib.check(_lib.load().ttamd_lora_few_fwd_bf16(x.data_ptr(), arr, 1, h.data_ptr(), None, M, K, torch.cuda.current_stream().cuda_stream), "lora_few_fwd")
+    assert torch.equal(h, ops.lora_hidden(x, m.lora_a))
