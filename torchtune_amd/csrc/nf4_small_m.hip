@@ -311,8 +311,10 @@ enum HiddenForm { kReads, kWaves, kPaired, kGather };
 // LDS of a few-token workgroup: the code table, the block scalers of its rows over a segment of the contraction, the splits'
 // sums of h, and per wave one stage: 128 columns of x (MQ groups of four tokens), of its row tiles' codes, and of its
 // members' lora_a (kGather: and of x again).  At the end a stage holds the wave's partial sums.
-// Sixteen copies of the code table where h is read (wide layers at one token: 14336 x 4096 18.1 us against 19.2 with one copy, their
-// pair 25.6 and 26.9; narrow ones level), one where it is formed: LDS has the operands of h to hold.
+// Sixteen copies of the code table where h is read (us behind one another in a graph, sixteen and one: 14336 x 4096 at one token
+// 13.3 and 14.2, 9728 x 3584 10.2 and 11.2, 28672 x 8192 36.6 and 38.3; 4096 x 4096 level; their fill costs small layers 2 - 5 %, 2048 x
+// 2048 4.5 and 4.3, and their LDS a workgroup per CU at 28672 x 8192 from 8 tokens on, 45.7 and 41.3), one where it is formed: LDS
+// has the operands of h to hold.
 constexpr int few_lut_bytes(int nt) { return nt > 0 ? 1024 : 16 * 1024; }
 // Columns of a segment: whole rounds of the waves' chunks and splits, so that it does not move either.
 constexpr int few_segment(int rt, int nt, int mq, int form) {
