@@ -542,7 +542,8 @@ MidPlan plan_pair(int64_t M, int64_t N, int64_t K) {
 // each measured; on 380 others the pick is 0.7 % slower than the fastest on average.
 // Kind 2: gemm_mid_pair_kernel, or the 256 x 256 tiles of gemm_tn.hip, by the same kind of model (fitted to 260 products, 0.1 %
 // slower than the faster one on average).  The wide tiles win from about half a round of them on (1000 tokens of 8192 x 2048
-// 51.5 -> 31.3 us, 4096 x 4096 44.4 -> 30.6, of 2048 x 2048 15.1 and 21.9).
+// 51.5 -> 31.3 us, 4096 x 4096 44.4 -> 30.6, of 2048 x 2048 15.1 and 21.9).  Where the model has them less than 5 % ahead they are
+// up to 12 % behind (585 tokens of 4096 x 2048, 887 of 2560 x 3072 20.2 and 21.8) and seldom ahead (517 of 8192 x 1024, 18 %).
 MidPlan plan_mid(int kind, int64_t M, int64_t N, int64_t K) {
   const MidPlan pair = plan_pair(M, N, K);
   MidPlan p = pair;
@@ -552,7 +553,7 @@ MidPlan plan_mid(int kind, int64_t M, int64_t N, int64_t K) {
                  rounds = (double)((pair.tiles + 255) / 256);
     const double wide = 0.2 + 7.26 * whole + k * (0.44 * whole + 0.25 * tiles / 256);
     const double narrow = 3.8 + 1.6 * rounds + k * (rounds > 1 ? 0.04 * rounds : 0.095) + 0.265 * k * (double)pair.tiles / 256;
-    if (pair.slices == 1 && wide < narrow) p.rows = 256;
+    if (pair.slices == 1 && wide < 0.95 * narrow) p.rows = 256;
     return p;
   }
   double best = 1e30;

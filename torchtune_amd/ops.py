@@ -1242,6 +1242,13 @@ def dequantize_per_group_int4(q: torch.Tensor, scale: torch.Tensor, zeros: Optio
     return out
 
 
+def gemm_mid_plan(kind: int, M: int, N: int, K: int) -> Tuple[int, int, int]:
+    """How ``ttamd_gemm_mid_bf16`` runs a product without a bias: rows of an output tile, slices, indices of an fp32 chain."""
+    tile_rows, slices, chain = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    _lib.check(_lib.load().ttamd_gemm_mid_plan(kind, 0, M, N, K, ctypes.byref(tile_rows), ctypes.byref(slices), ctypes.byref(chain)), "gemm_mid_plan")
+    return tile_rows.value, slices.value, chain.value
+
+
 def int4_linear_applies(M: int, N: int, K: int, group_size: int) -> bool:
     """Sizes the kernels that stream a converted linear's integer weight serve."""
     return bool(_lib.load().ttamd_int4_linear_applies(M, N, K, group_size))
