@@ -222,3 +222,10 @@ def test_a_linear_allocates_no_slabs_that_its_products_do_not_write():
     before = torch.cuda.memory_allocated()
     torch.autograd.grad(y, x, gy)
     assert torch.cuda.max_memory_allocated() - before < 2 * 2 * M * K  # the gradient itself: 2 bytes an element
+
+
+def test_linears_whose_grad_input_part_fills_its_rounds_keep_the_dense_product():
+    """Tiles of 128 rows in a second round of 280 of 512: slower here than with the vendor's kernels."""
+    layer = FakeQuantizedLinear(3584, 9728, False, None, FakeQuantizeConfig(torch.int4, group_size=32), device="cuda", dtype=torch.bfloat16)
+    for M, mid in [(740, True), (1182, False), (1447, False), (1485, True)]:
+        assert layer._mid_ok(torch.empty(M, 3584, device="cuda", dtype=torch.bfloat16)) is mid, M

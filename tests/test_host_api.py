@@ -690,3 +690,11 @@ def test_weight_gradients_take_wide_tiles_only_well_ahead():
     """585 tokens of 4096 x 2048 and 887 of 2560 x 3072 took 8 - 12 % longer on 256 x 256 tiles, which a cost model has level."""
     assert ops.gemm_mid_plan(2, 4096, 2048, 585)[0] == 0 and ops.gemm_mid_plan(2, 2560, 3072, 887)[0] == 0
     assert ops.gemm_mid_plan(2, 8192, 2048, 1000)[0] == 256 and ops.gemm_mid_plan(2, 4096, 4096, 61)[0] == 256
+
+
+def test_wide_fake_quantised_linears_whose_grad_input_part_fills_its_rounds():
+    from torchtune_amd import qat
+
+    for rows, N, K, own in [(1182, 9728, 3584, False), (1411, 8192, 3072, False), (1155, 12288, 4096, False), (1485, 9728, 3584, True),
+                            (1571, 8192, 3072, True), (740, 9728, 3584, True), (1415, 8192, 2048, True), (1906, 14336, 4096, True)]:
+        assert qat._grad_input_rounds_ok(rows, N, K) is own, (rows, N, K)

@@ -256,6 +256,11 @@ MID_GEMM_MAX = 1 << 34
 # fill 0.63: 1071 and 1124), and with fewer outputs than inputs it does at some lengths (1101 tokens of 4096 x 14336: 440 and 468).
 MID_GEMM_MAX_WIDE = 112 << 30
 MID_GEMM_MIN_FILL = 0.65
+# And of that range the vendor keeps what leaves the grad-input on tiles of 128 rows in more than one round of 128 x 128 tiles, the
+# rounds less than this full (linear forward + backward, us, these kernels and the vendor's: 1182 tokens of 9728 x 3584 332 and
+# 315, 1375 of 8192 x 3072 263 and 250, 1155 of 12288 x 4096 417 and 392; level at 14336 x 4096, 1111 tokens 492 and 490).  Where the
+# grad-input takes tiles of 256 rows or fuller rounds it is ahead (1485 of 9728 x 3584 346 and 354, 1571 of 8192 x 3072 268 and 280).
+MID_GEMM_MIN_GRAD_FILL = 0.67
 # The same bound from 2048 rows on: the vendor's larger tiles win the forward and the grad-input of tall products from about
 # 14 * 2^30 on (three products, us, these kernels and the vendor's: 2600 tokens of 2048 x 2048 87 and 101, 3300 103 and 111, 4096
 # 124 and 117; 5200 of 2816 x 1024 143 and 127).  Narrow weights (N * K up to 2^20) keep the bound above: their weight gradient,
@@ -266,10 +271,15 @@ MID_GEMM_MAX_TALL = 14 << 30
 TN_GROUP_GEMM = True
 
 
-def _round_fill(rows: int, cols: int) -> float:
-    """How full the rounds of 256 x 128 output tiles on the 256 CUs are."""
-    tiles = max(1, -(-rows // 256) * -(-cols // 128))
+def _round_fill(rows: int, cols: int, tile_rows: int = 256) -> float:
+    """How full the rounds of ``tile_rows`` x 128 output tiles on the 256 CUs are."""
+    tiles = max(1, -(-rows // tile_rows) * -(-cols // 128))
     return tiles / (256 * -(-tiles // 256))
+
+
+def _grad_input_rounds_ok(rows: int, N: int, K: int) -> bool:
+    return (-(-rows // 128) * -(-K // 128) <= 256 or _round_fill(rows, K, 128) >= MID_GEMM_MIN_GRAD_FILL
+            or ops.gemm_mid_plan(1, rows, K, N)[0] != 128)
 
 
 class _TiledFakeQuantLinearFn(torch.autograd.Function):
@@ -536,7 +546,7 @@ class FakeQuantizedLinear(nn.Linear):
         if x.numel() >= 2048 * K:
             most = MID_GEMM_MAX_TALL if N * K > 1 << 20 else MID_GEMM_MAX
         elif (x.numel() * N > MID_GEMM_MAX and N >= K and x.numel() // K * N < 1 << 30  # the kernels' 32-bit offsets
-              and _round_fill(x.numel() // K, N) >= MID_GEMM_MIN_FILL):
+              and _round_fill(x.numel() // K, N) >= MID_GEMM_MIN_FILL and _grad_input_rounds_ok(x.numel() // K, N, K)):
             most = MID_GEMM_MAX_WIDE
         return (0 < x.numel() * N <= most and N * K < 1 << 30 and N >= 256 and N % 64 == 0 and K % 64 == 0 and x.shape[-1] == K)
 
