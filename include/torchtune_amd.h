@@ -258,6 +258,11 @@ int ttamd_nf4_linear_bwd_dx_bf16(const void* gy, const uint8_t* quantized_data, 
 size_t ttamd_nf4_gemm_workspace_bytes(int64_t M, int64_t n_out, int64_t k_contract);
 /* 1 when those bytes are the expanded weight of the many-token path, 0 when they are slices (or none) */
 int ttamd_nf4_gemm_expands_weight(int64_t M, int64_t n_out, int64_t k_contract);
+/* How those entry points run a product that neither the few-token kernel nor the expanded weight serves: rows of an output tile (64
+ * x 128 columns, 96, 128 or 256 x 256), slices of the contraction (given room for them: may_slice), and the most contraction
+ * indices that one chain of fp32 sums runs over.  by_128: the contraction may be taken 128 indices at a time (a group's
+ * grad-input: every member's N is a multiple of 128); forward: else the grad-input.  Needs no GPU. */
+int ttamd_nf4_gemm_plan(int64_t M, int64_t n_out, int64_t k_contract, int may_slice, int by_128, int forward, int* tile_rows, int* slices, int* chain);
 int ttamd_nf4_lora_linear_fwd_ws_bf16(const void* x, const uint8_t* quantized_data, const void* block_scalers,
                                       const void* block_scalers_t, const void* h, const void* lora_b, int rank, float scale,
                                       const void* bias, const void* col_scale, void* y, int64_t M, int64_t N, int64_t K,

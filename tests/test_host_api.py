@@ -669,6 +669,39 @@ def test_chains_of_small_bf16_products_are_no_longer_than_the_four_wave_kernels(
                     assert _gemm_mid_plan(kind, M, N, K)[2] <= most, (kind, M, N, K)
 
 
+def _nf4_gemm_plan(M, N, K, may_slice=1, by_128=1, forward=1):
+    rows, slices, chain = (ctypes.c_int() for _ in range(3))
+    rc = _lib.load().ttamd_nf4_gemm_plan(M, N, K, may_slice, by_128, forward, ctypes.byref(rows), ctypes.byref(slices), ctypes.byref(chain))
+    return (rows.value, slices.value, chain.value) if rc == 0 else None
+
+
+def test_plans_of_fused_nf4_products_keep_their_chains_and_fit_the_workspace():
+    """A contraction has as many chains of fp32 sums as slices of it, on tiles of 128 x 256, would fill the chip (at least 256
+    indices each, at most 16); the wave groups of a tile (4 on 64 rows, 2 on 96 and 128) are chains of their own.  The workspace
+    query covers every plan, and without one nothing is sliced."""
+    lib = _lib.load()
+    widths = (64, 256, 576, 1024, 2048, 2816, 4096, 8192, 9728, 14336)
+    for M in (33, 65, 129, 333, 500, 700, 1000, 1279, 1500, 2047):
+        for N in widths:
+            for K in widths:
+                tiles = -(-M // 128) * -(-N // 256)
+                chains = 1
+                if tiles <= 64 or (tiles <= 128 and K >= 4096):
+                    chains = max(1, min(256 // tiles, K // 256, 16))
+                for by_128, forward in ((0, 0), (1, 0), (1, 1)):
+                    plan = _nf4_gemm_plan(M, N, K, 1, by_128, forward)
+                    if plan is None:
+                        assert lib.ttamd_nf4_gemm_expands_weight(M, N, K)
+                        continue
+                    rows, slices, chain = plan
+                    step = 128 if rows == 64 else 64
+                    if chains > 1:
+                        assert chain <= -(-K // 64 // chains) * 64 + step, (M, N, K, plan, chains)
+                    need = slices * M * N * 4 if slices > 1 else 0
+                    assert not by_128 or lib.ttamd_nf4_gemm_workspace_bytes(M, N, K) >= need
+                    assert _nf4_gemm_plan(M, N, K, 0, by_128, forward)[1] == 1
+
+
 def _few_applies(M, N, K, rank):
     member = (_lib.LoraGroupMember * 1)()
     for field in ("quantized_data", "block_scalers", "lora_a", "lora_b", "y"):

@@ -155,6 +155,7 @@ SIGNATURES = {
         _int, [_c_void_p, _int, _i64, _i64, _int, _int, _c_void_p, _c_void_p, _c_void_p, _c_void_p]),
     "ttamd_dequantize_per_group_uint4": (_int, [_c_void_p, _c_void_p, _c_void_p, _int, _i64, _i64, _int, _c_void_p, _c_void_p]),
     "ttamd_gemm_mid_workspace_bytes": (_size, [_i64, _i64, _i64]),
+    "ttamd_nf4_gemm_plan": (_int, [_i64, _i64, _i64, _int, _int, _int, _c_void_p, _c_void_p, _c_void_p]),
     "ttamd_gemm_mid_plan": (_int, [_int, _int, _i64, _i64, _i64, _c_void_p, _c_void_p, _c_void_p]),
     "ttamd_gemm_mid_bf16": (_int, [_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _i64, _i64, _i64, _c_void_p, _size, _c_void_p]),
     "ttamd_int4_linear_applies": (_int, [_i64, _i64, _i64, _int]),

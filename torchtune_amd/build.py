@@ -20,7 +20,7 @@ LIB_DIR = PKG / "lib"
 LIB_PATH = LIB_DIR / "libtorchtune_amd.so"
 HOST_MODULE = "torchtune_amd_host"
 HOST_PATH = LIB_DIR / f"{HOST_MODULE}.so"
-SOURCES = ["capi.hip", "nf4_codec.hip", "fake_quant.hip", "int4_linear.hip", "nf4_gemm.hip", "nf4_gemm_rs.hip", "nf4_gemm_dense.hip", "gemm_tn.hip", "gemm_mid.hip", "nf4_small_m.hip", "lora_skinny.hip", "lora_group.hip", "qlora_linear.hip", "nf4_merge.hip", "neighbours.hip"]
+SOURCES = ["capi.hip", "nf4_codec.hip", "fake_quant.hip", "int4_linear.hip", "nf4_gemm.hip", "nf4_gemm_rs.hip", "nf4_gemm_mid.hip", "nf4_gemm_dense.hip", "gemm_tn.hip", "gemm_mid.hip", "nf4_small_m.hip", "lora_skinny.hip", "lora_group.hip", "qlora_linear.hip", "nf4_merge.hip", "neighbours.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -35,6 +35,7 @@ HIPCC_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wall",
     "-Wno-unused-function",
+    "-Wno-inline-asm",
 ]
 
 
@@ -61,7 +62,8 @@ def _compile_host(obj_dir: Path) -> Path:
 
     obj = obj_dir / "host_binding.o"
     cmd = [
-        shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function", "-D__HIP_PLATFORM_AMD__=1",
+        shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
+    "-Wno-inline-asm", "-D__HIP_PLATFORM_AMD__=1",
         "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-DTORCH_EXTENSION_NAME={HOST_MODULE}",
         *[f"-isystem{p}" for p in include_paths()], "-isystem/opt/rocm/include", f"-isystem{sysconfig.get_paths()['include']}",
         "-c", str(CSRC / "host_binding.cpp"), "-o", str(obj),
