@@ -544,6 +544,141 @@ __global__ __launch_bounds__(256) void skinny_tn_kernel(const TnBatch a) {
 }
 
 // ---------------------------------------------------------------------------------------------------
+// skinny_tn_whole: the same row contractions, finished: sixteen waves share all rows of 64 columns, their sums meet in LDS, and the
+// gradients leave rounded.  What bounds skinny_tn on few rows is not its bytes but its two launches and, for several groups of 16
+// ranks, the partial sums in between; without row splits there is neither.  Adapter backward (gh, gA, gB) of one linear, us, two
+// launches -> one: 2048 x 2048 at 700 tokens rank 8 14.8 -> 9.7, rank 32 19.4 -> 11.4; 4096 x 4096 at 1000 rank 48 38.5 -> 19.8;
+// 1024 x 1024 at 48 rank 8 11.5 -> 7.6; 2048 x 8192 at 2048 rank 16 22.7 -> 16.9.
+// ---------------------------------------------------------------------------------------------------
+constexpr int kTnWholeWaves = 16, kTnWholeCols = 64;
+constexpr int kTnWholePitch = 160;  // 128 + 32: four consecutive rows fall on disjoint banks
+constexpr int tn_whole_wave_lds(int rgm) { return 32 * kTnWholePitch + rgm * 32 * 32; }
+struct TnWholeOut {
+  uint16_t* ga[kMaxGroup];  // [rank i, Kc of problem 0]: problem 0's rows [r_off[i], r_off[i + 1])
+  uint16_t* gb[kMaxGroup];  // [Kc, rank i] of problem 1 + i, times scale[i]
+  float scale[kMaxGroup];
+  int r_off[kMaxGroup + 1];
+};
+
+template <int RGM>
+__global__ __launch_bounds__(64 * kTnWholeWaves) void skinny_tn_whole_kernel(const TnBatch a, const TnWholeOut o) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  extern __shared__ __attribute__((aligned(16))) char whole[];
+  int which = 0;  // uniform over the workgroup
+#pragma unroll
+  for (int q = 0; q < kTnMaxProblems - 1; ++q)
+    if (q < a.n - 1 && (int)blockIdx.x >= a.cg_end[q]) which = q + 1;
+  const TnProblem& P = a.p[which];
+  const uint16_t* __restrict__ G = P.G;
+  const uint16_t* __restrict__ X = P.X;
+  const int Kc = P.Kc, M = a.M, R = P.R, ldg = P.ldg;
+  const int rg = (R + 15) >> 4;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, i = lane & 15;
+  const int c0 = ((int)blockIdx.x - (which ? a.cg_end[which - 1] : 0)) * kTnWholeCols;
+
+  char* my = whole + wave * tn_whole_wave_lds(RGM);
+  // copy-in: X piece, instruction u (0..3): row 8 u + lane / 8, 16-byte chunk lane % 8; G as in skinny_tn
+  const uint16_t* xsrc = X + c0 + 8 * (lane & 7);  // Kc is a multiple of 64
+  char* xdst = my + (lane >> 3) * kTnWholePitch + 16 * (lane & 7);
+  const int gcol = 8 * (lane & 1);  // + 16 q;  R % 8 == 0: a lane's 8 columns are all in or all out
+  char* gdst = my + 32 * kTnWholePitch + (lane >> 1) * 32 + 16 * (lane & 1);  // + 1024 q
+  const uint32_t my_lds = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)my);
+  const uint32_t xrd = my_lds + (8 * g + (i >> 2)) * kTnWholePitch + 8 * (i & 3);
+  const uint32_t grd = my_lds + 32 * kTnWholePitch + (8 * g + (i >> 2)) * 32 + 8 * (i & 3);
+
+  f32x4_t acc[RGM][4];
+#pragma unroll
+  for (int q = 0; q < RGM; ++q)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[q][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  u32x4_t xv[4], gv[RGM];
+  auto fetch = [&](int m) {  // rows m .. m + 31 into registers
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int row = m + 8 * u + (lane >> 3);
+      xv[u] = u32x4_t{0, 0, 0, 0};
+      if (row < M) xv[u] = *reinterpret_cast<const u32x4_t*>(xsrc + (int64_t)row * Kc);
+    }
+    const int grow = m + (lane >> 1);
+#pragma unroll
+    for (int q = 0; q < RGM; ++q) {
+      gv[q] = u32x4_t{0, 0, 0, 0};
+      if (grow < M && gcol + 16 * q < R) gv[q] = *reinterpret_cast<const u32x4_t*>(G + (int64_t)grow * ldg + gcol + 16 * q);
+    }
+  };
+  int m = 32 * wave;
+  if (m < M) fetch(m);
+  for (; m < M; m += 32 * kTnWholeWaves) {
+    // the previous step's reads of this region are complete: they were waited for before its MFMAs
+#pragma unroll
+    for (int u = 0; u < 4; ++u) *reinterpret_cast<u32x4_t*>(xdst + 8 * u * kTnWholePitch) = xv[u];
+#pragma unroll
+    for (int q = 0; q < RGM; ++q) *reinterpret_cast<u32x4_t*>(gdst + 1024 * q) = gv[q];  // zeros beyond R
+    if (m + 32 * kTnWholeWaves < M) fetch(m + 32 * kTnWholeWaves);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the copy-in has landed (LDS operations of a wave complete in order)
+    u32x2_t ga[RGM], gb[RGM], xa[4], xb[4];
+#pragma unroll
+    for (int q = 0; q < RGM; ++q) {
+      ga[q] = lds_read_tr16(grd, 1024 * q);
+      gb[q] = lds_read_tr16(grd, 1024 * q + 4 * 32);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      xa[e] = lds_read_tr16(xrd, 32 * e);
+      xb[e] = lds_read_tr16(xrd, 32 * e + 4 * kTnWholePitch);
+    }
+    // waits that name the registers they release, so that no use can be scheduled ahead of them
+#pragma unroll
+    for (int q = 0; q < RGM; ++q) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(ga[q]), "+v"(gb[q]));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(xa[e]), "+v"(xb[e]));
+      const u32x4_t xop = {xa[e].x, xa[e].y, xb[e].x, xb[e].y};
+#pragma unroll
+      for (int q = 0; q < RGM; ++q) {
+        if (q < rg) {
+          const u32x4_t gop = {ga[q].x, ga[q].y, gb[q].x, gb[q].y};
+          acc[q][e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, gop), __builtin_bit_cast(bf16x8_t, xop), acc[q][e], 0, 0, 0);
+        }
+      }
+    }
+  }
+  // acc[q][e][v] = sum over this wave's rows of G[.][16 q + 4 g + v] * X[.][c0 + 16 e + i]; 16 columns of G at a time meet in
+  // the staging memory, and every thread finishes one output of them
+  float (*red)[16][64] = reinterpret_cast<float (*)[16][64]>(whole);
+  for (int q = 0; q < rg; ++q) {
+    __syncthreads();  // the staging regions (or the previous group's sums) are free
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        float val = acc[0][e][v];
+#pragma unroll
+        for (int qq = 1; qq < RGM; ++qq) val = q == qq ? acc[qq][e][v] : val;
+        red[wave][v * 4 + e][lane] = val;
+      }
+    __syncthreads();
+    float s = red[0][wave][lane];
+#pragma unroll
+    for (int w = 1; w < kTnWholeWaves; ++w) s += red[w][wave][lane];
+    const int r = 16 * q + 4 * g + (wave >> 2), col = c0 + 16 * (wave & 3) + i;
+    if (r >= R) continue;
+    if (which == 0) {
+      int mem = 0;
+#pragma unroll
+      for (int k = 1; k < kMaxGroup; ++k)
+        if (k < a.n - 1 && r >= o.r_off[k]) mem = k;
+      o.ga[mem][(int64_t)(r - o.r_off[mem]) * Kc + col] = f32_to_bf16_bits(s);
+    } else {
+      o.gb[which - 1][(int64_t)col * R + r] = f32_to_bf16_bits(s * o.scale[which - 1]);
+    }
+  }
+#endif
+}
+
+// ---------------------------------------------------------------------------------------------------
 // skinny_tn_gh: both products of a backward that read gy, from one pass over it (rank <= 16):
 //   part  [split][r][c] = sum_{m in split} H[m][r] * GY[m][c]                   gB, as skinny_tn
 //   part_h[cg][m][r]    = sum_{c in column group cg} GY[m][c] * Bm[c][r]        gh, before scale and rounding
@@ -1233,6 +1368,53 @@ size_t tn_part_bytes(int64_t M, int n, const int64_t* Kc, const int* R) {
   return (size_t)plan_tn(M, groups).splits * elems * sizeof(float);
 }
 
+// ---- gA and gB without row splits (skinny_tn_whole_kernel) ------------------------------------------------------------
+// Up to 2048 rows it was the faster way on every pair of ten (256 x 1024 to 14336 x 4096, rank 8 - 48: 0.5 - 0.9 of the time, level
+// where both products are 14336 wide); at 3000 4096 x 14336 rank 16 takes 39.1 instead of 38.0 us, at 8192 256 x 1024 25.9 instead of
+// 16.5.  Beyond 48 ranks the sums of a wave do not fit its registers: 1024 rows (23.2 -> 20.5; at 2048 25.8 -> 28.6).
+bool tn_whole_pays(const GroupSkinny& g) { return g.M <= (g.r_off[g.n] <= 48 ? 2048 : 1024); }
+
+template <int RGM>
+int launch_tn_whole(const TnBatch& b, const TnWholeOut& o, hipStream_t s) {
+  constexpr int kLds = kTnWholeWaves * tn_whole_wave_lds(RGM);
+  static_assert(kLds >= kTnWholeWaves * 16 * 64 * (int)sizeof(float) && kLds <= 160 * 1024, "the sums fit the staging memory");
+  static bool set[64] = {};  // the LDS limit is a per-device attribute of the function (a race only repeats the call)
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;
+  if (dev < 0 || !set[dev]) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&skinny_tn_whole_kernel<RGM>), hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+    if (e != hipSuccess) return fail(TTAMD_ELAUNCH, "skinny_tn: cannot reserve %d bytes of LDS: %s", kLds, hipGetErrorString(e));
+    if (dev >= 0) set[dev] = true;
+  }
+  skinny_tn_whole_kernel<RGM><<<dim3((unsigned)b.cg_end[b.n - 1]), dim3(64 * kTnWholeWaves), kLds, s>>>(b, o);
+  return check_launch("skinny_tn");
+}
+
+// b: M and problem 0 are set
+int run_tn_whole(TnBatch& b, const GroupSkinny& g, const uint16_t* h_cat, hipStream_t s) {
+  TnWholeOut o = {};
+  const int rt = g.r_off[g.n];
+  int64_t groups = 0;
+  const int rgm = (rt + 15) / 16;
+  b.n = 1 + g.n;
+  for (int i = 0; i < g.n; ++i) {
+    b.p[1 + i] = TnProblem{h_cat + g.r_off[i], g.gy[i], nullptr, (int)g.N[i], g.rank[i], rt};
+    o.ga[i] = g.ga[i];
+    o.gb[i] = g.gb[i];
+    o.scale[i] = g.scale[i];
+    o.r_off[i] = g.r_off[i];
+  }
+  o.r_off[g.n] = rt;
+  for (int i = 0; i < b.n; ++i) {
+    groups += b.p[i].Kc / kTnWholeCols;
+    b.cg_end[i] = (int)groups;
+  }
+  return rgm == 1   ? launch_tn_whole<1>(b, o, s)
+         : rgm == 2 ? launch_tn_whole<2>(b, o, s)
+         : rgm == 3 ? launch_tn_whole<3>(b, o, s)
+                    : launch_tn_whole<4>(b, o, s);
+}
+
 // ---- gh and gB from one pass over gy (skinny_tn_gh_kernel) ------------------------------------------------------------
 // Taken when every member is wide and of rank <= 16: the pass over gy that gh alone would need then costs more than the
 // partial sums the fused kernel writes and the launch of their reduction (measured on [8192, 14336] pairs: 88 us for the
@@ -1437,6 +1619,7 @@ int run_group_lora_bwd(const uint16_t* x, const uint16_t* h_cat, const GroupSkin
   TnBatch t = {};
   t.M = (int)g.M;
   t.p[0] = TnProblem{gh_cat, x, nullptr, (int)g.K, rt, rt};
+  if (tn_whole_pays(g)) return run_tn_whole(t, g, h_cat, s);
   TnSumBatch f = {};
   int sum_problem[kTnMaxSums], sum_row0[kTnMaxSums];
   for (int i = 0; i < g.n; ++i) {
