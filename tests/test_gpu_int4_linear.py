@@ -77,6 +77,42 @@ def test_streaming_launch_shapes(kind, qp, n, k, group, m):
     assert torch.equal(got[:1], first)
 
 
+@pytest.mark.parametrize("kind,qp", [("8da4w", torch.float32), ("8da4w", torch.bfloat16), ("4w", torch.bfloat16)])
+@pytest.mark.parametrize("n,k,group", [(8256, 1568, 32), (4160, 4128, 32), (16448, 2048, 128), (2112, 8288, 32), (256, 128, 64)])
+@pytest.mark.parametrize("m", [31, 64, 96, 113, 161, 192])
+def test_tiled_launch_shapes(kind, qp, n, k, group, m):
+    """More and fewer steps than the ring has stages, one to eight slices, a last step of one group of 32 that three of four wave
+    groups sit out, odd numbers of groups per row: within the bound above."""
+    layer = _layer(kind, n, k, group, False, qp)
+    x = torch.randn(m, k, generator=torch.Generator().manual_seed(m)).to(torch.bfloat16).to(DEV)
+    with torch.no_grad():
+        got = layer(x)
+    xd, w = _operands(layer, x)
+    want, size = xd @ w.t(), xd.abs() @ w.abs().t()
+    assert bool(((got.double() - want).abs() <= want.abs() * 2.0 ** -8 + size * (k * 2.0 ** -23)).all())
+
+
+@pytest.mark.parametrize("m", [5, 20])
+def test_every_scale_and_zero_point_expands_to_the_dense_weights_bits(m):
+    """One-hot rows read single weights: bf16 scales and zero points of every exponent, scales of both signs."""
+    layer = _layer("4w", 256, 512, 32, False, torch.bfloat16)
+    g = torch.Generator().manual_seed(m)
+    layer.weight.copy_(torch.randint(0, 256, layer.weight.shape, generator=g))
+    bits = torch.randint(0, 254 * 128, (16, 256, 2), generator=g)
+    bits[..., 1] = bits[..., 1] % (224 * 128) + 30 * 128  # a sum stays a normal number, the product with the scale need not
+    sign = torch.randint(0, 2, bits.shape, generator=g) * 2 ** 15
+    layer.scales_and_zeros.copy_((bits + sign).to(torch.int32).to(torch.uint16).view(torch.bfloat16))
+    dense = layer.dense_weight()
+    ok = dense.isfinite().t()
+    for first in range(0, 512, m):
+        k = torch.arange(first, first + m) % 512
+        x = torch.nn.functional.one_hot(k, 512).to(torch.bfloat16).to(DEV)
+        keep = ok.all(0)  # an infinite weight makes its row's other products NaN
+        with torch.no_grad():
+            assert torch.equal(layer(x)[:, keep], dense[:, k.to(DEV)].t()[:, keep])
+    assert int(keep.sum()) > 16
+
+
 @pytest.mark.parametrize("m", [5, 20])  # the streaming and the tiled kernel
 def test_scales_at_the_top_of_the_range_expand_to_the_dense_weights_bits(m):
     """One-hot rows read single weights: (q - 8) * scale is finite for every code but 0, while 8 * scale is not."""

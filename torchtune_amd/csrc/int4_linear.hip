@@ -14,20 +14,21 @@
 //    row; a chunk's codes, scales and x come by direct-to-LDS loads in row order and are read from there.  Partial sums
 //    meet in LDS in wave order.
 //  * int4_tile_kernel (more): the few-token kernel would read all of x in every workgroup (at 75 tokens nine times the
-//    bytes of its weight rows).  Four waves own 64 weight rows between them and share 128-wide chunks of up to 128
-//    tokens through a double LDS buffer; a weight fragment is expanded once per 128 tokens.  Launches of few tiles cut
-//    the contraction into slices (fp32 slabs, added in slice order by int4_reduce_kernel).
+//    bytes of its weight rows).  Eight waves share 64 weight rows and up to 128 tokens; a weight fragment is expanded once per 128
+//    tokens.  Launches of few tiles cut the contraction into slices (fp32 slabs, added in slice order by int4_reduce_kernel).
 //
 // Measured against dequantise + library GEMM (us, weights from HBM, launch gaps included; int8 / uint4):
-//   14336 x 4096:  1 token 60 / 60 -> 17.7 / 16.1, 16 tokens 59 / 60 -> 25 / 17.8, 75 tokens 63 / 65 -> 38 / 33, 256 tokens 83 / 82 -> 67 / 69
-//   4096 x 14336:  1 token 58 / 58 -> 16.5 / 15.3, 75 tokens 79 / 78 -> 38 / 32, 256 tokens 93 / 92 -> 74 / 66
-//   1024 x 4096:   1 token 20 / 20 -> 6.1 / 5.9, 256 tokens 21 / 21 -> 17 / 16
+//   14336 x 4096:  1 token 60 / 60 -> 17.7 / 15.0, 16 tokens 59 / 60 -> 25 / 16.7, 75 tokens 63 / 65 -> 31 / 26, 256 tokens 83 / 82 -> 59 / 54
+//   4096 x 14336:  1 token 58 / 58 -> 16.5 / 13.5, 75 tokens 79 / 78 -> 33 / 26, 256 tokens 93 / 92 -> 61 / 49
+//   1024 x 4096:   1 token 20 / 20 -> 6.1 / 5.1, 256 tokens 21 / 21 -> 16 / 14
 // (at most 16 tokens with loads straight into the MFMA lanes and one wave's sum at the end: 26.4 / 19.0, 21.9 / 19.5 and 9.0 / 7.3 at
-// one token; a read of the same bytes takes 14 / 6.5).  Above 256 tokens the two m-tiles' expansion and their slabs cost what
-// the dense copy costs, and the library's larger tiles win.
+// one token; a read of the same bytes takes 14 / 6.5).
 #include "common.h"
 #include "fq_math.h"
 #include "nf4_math.h"
+
+#include <algorithm>
+#include <type_traits>
 
 #define TT_LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
 
@@ -39,6 +40,8 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ uint32_t pack_pair(float lo, float hi) {
   bf16x2_t v;
@@ -48,6 +51,57 @@ __device__ __forceinline__ uint32_t pack_pair(float lo, float hi) {
 }
 __device__ __forceinline__ float lo_of(uint32_t d) { return bits_f32(d << 16); }
 __device__ __forceinline__ float hi_of(uint32_t d) { return bits_f32(d & 0xffff0000u); }
+
+// The eight uint4 codes of a dword (the even element in a byte's high nibble) as an MFMA operand: bf16(bf16((q - 8) * scale) + zero).
+// A nibble under the exponent of 1024 is the half 1024 + q (1024 + 16 q), two to a dword; q - 8 is exact from there on and
+// (q - 8) * scale is rounded to bf16 directly, whatever the scale (8 * scale overflows above 2^125).  A value rounded into the
+// upper half of a dword is its own fp32.  37 instructions, spelled out: the compiler makes 60 - 75 of the plain expressions (one
+// token of 14336 x 4096 18.1 us, 15.0 with these).
+__device__ __forceinline__ u32x4_t uint4_operand(uint32_t codes, float sc, float z) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const float sc16 = sc * 0.0625f;
+  uint32_t half[4];  // [0], [1]: bytes 0 and 2, [2], [3]: bytes 1 and 3; 16 (q - 8) of the even and q - 8 of the odd elements
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    const uint32_t c = codes >> (8 * b);
+    uint32_t even, odd;
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(even) : "v"(c), "s"(0x00f000f0u), "v"(0x64006400u));
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(odd) : "v"(c), "s"(0x000f000fu), "v"(0x64006400u));
+    asm("v_pk_add_f16 %0, %1, %2" : "=v"(half[2 * b]) : "v"(even), "s"(0xe480e480u));     // - 1152
+    asm("v_pk_add_f16 %0, %1, %2" : "=v"(half[2 * b + 1]) : "v"(odd), "s"(0xe408e408u));  // - 1032
+  }
+  u32x4_t w;
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    const uint32_t even = half[2 * (b & 1)], odd = half[2 * (b & 1) + 1];
+    float p0, p1, r0, r1;
+    if (b < 2) {
+      asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,0,0]" : "=v"(p0) : "v"(even), "v"(sc16));
+      asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,0,0]" : "=v"(p1) : "v"(odd), "v"(sc));
+    } else {
+      asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(p0) : "v"(even), "v"(sc16));
+      asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(p1) : "v"(odd), "v"(sc));
+    }
+    asm("v_cvt_pk_bf16_f32 %0, 0, %1" : "=v"(r0) : "v"(p0));
+    asm("v_cvt_pk_bf16_f32 %0, 0, %1" : "=v"(r1) : "v"(p1));
+    w[b] = pack_pair(r0 + z, r1 + z);
+  }
+  return w;
+#else
+  return u32x4_t{};
+#endif
+}
+
+// Eight int8 values of two dwords: bf16((q - zero) * scale)
+__device__ __forceinline__ u32x4_t int8_operand(uint32_t low, uint32_t high, float sc, float z) {
+  u32x4_t w;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const uint32_t two = (d < 2 ? low : high) >> (16 * (d & 1));
+    w[d] = pack_pair(((float)(int8_t)(two & 0xffu) - z) * sc, ((float)(int8_t)((two >> 8) & 0xffu) - z) * sc);
+  }
+  return w;
+}
 
 struct Int4Args {
   const uint16_t* x;     // [M, K] bf16
@@ -66,67 +120,21 @@ struct Int4Args {
 // How a weight is stored.
 enum Format { kInt8F32, kInt8Bf16, kUint4 };
 
-// 32 consecutive k of one weight row, as loaded.
+// 32 consecutive k of one weight row; operand(s): elements 8 s .. 8 s + 7 as an MFMA operand.
 template <int FMT>
-struct WeightPiece;
-
+struct WeightPiece {
+  u32x4_t v[2];
+  float sc, z;
+  __device__ __forceinline__ void clear() { v[0] = v[1] = u32x4_t{0, 0, 0, 0}; sc = z = 0.f; }
+  __device__ __forceinline__ u32x4_t operand(int s) const { return int8_operand(v[s >> 1][2 * (s & 1)], v[s >> 1][2 * (s & 1) + 1], sc, z); }
+};
 template <>
 struct WeightPiece<kUint4> {
   u32x4_t codes;
   uint32_t sz;
   __device__ __forceinline__ void clear() { codes = u32x4_t{0, 0, 0, 0}; sz = 0; }
-  __device__ __forceinline__ void load(const Int4Args& a, int n, int k) {
-    codes = *reinterpret_cast<const u32x4_t*>(a.q + (((int64_t)n * a.K + k) >> 1));
-    sz = reinterpret_cast<const uint32_t*>(a.scale)[(int64_t)(k >> a.log2_group) * a.N + n];
-  }
-  // elements 8 s .. 8 s + 7 as an MFMA operand: bf16(bf16((q - 8) * scale) + zero).  The first product is that of 16 (q - 8), a
-  // byte with the nibble on top, and scale / 16, both exact (8 * scale, which a fused multiply-add would subtract, overflows
-  // for scales above 2^125 whose small multiples do not).
-  __device__ __forceinline__ u32x4_t operand(int s) const {
-    const float sc = lo_of(sz) * 0.0625f, z = hi_of(sz);
-    const uint32_t c = codes[s] ^ 0x88888888u, high = c & 0xf0f0f0f0u, low = (c << 4) & 0xf0f0f0f0u;
-    u32x4_t w;
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      const uint32_t p = pack_pair((float)(int8_t)(high >> (8 * b)) * sc, (float)(int8_t)(low >> (8 * b)) * sc);
-      w[b] = pack_pair(lo_of(p) + z, hi_of(p) + z);
-    }
-    return w;
-  }
+  __device__ __forceinline__ u32x4_t operand(int s) const { return uint4_operand(codes[s], lo_of(sz), hi_of(sz)); }
 };
-
-template <bool QP_BF16>
-struct Int8Piece {
-  u32x4_t v[2];
-  float sc, z;
-  __device__ __forceinline__ void clear() { v[0] = v[1] = u32x4_t{0, 0, 0, 0}; sc = z = 0.f; }
-  __device__ __forceinline__ void load(const Int4Args& a, int n, int k) {
-    const u32x4_t* p = reinterpret_cast<const u32x4_t*>(a.q + (int64_t)n * a.K + k);
-    v[0] = p[0];
-    v[1] = p[1];
-    const int64_t gi = (int64_t)n * (a.K >> a.log2_group) + (k >> a.log2_group);
-    if constexpr (QP_BF16) {
-      sc = bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(a.scale)[gi]);
-      z = a.zero ? bf16_bits_to_f32(reinterpret_cast<const uint16_t*>(a.zero)[gi]) : 0.f;
-    } else {
-      sc = reinterpret_cast<const float*>(a.scale)[gi];
-      z = a.zero ? reinterpret_cast<const float*>(a.zero)[gi] : 0.f;
-    }
-  }
-  __device__ __forceinline__ u32x4_t operand(int s) const {  // bf16((q - zero) * scale)
-    u32x4_t w;
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      const uint32_t two = v[s >> 1][2 * (s & 1) + (d >> 1)] >> (16 * (d & 1));
-      w[d] = pack_pair(((float)(int8_t)(two & 0xffu) - z) * sc, ((float)(int8_t)((two >> 8) & 0xffu) - z) * sc);
-    }
-    return w;
-  }
-};
-template <>
-struct WeightPiece<kInt8F32> : Int8Piece<false> {};
-template <>
-struct WeightPiece<kInt8Bf16> : Int8Piece<true> {};
 
 constexpr int kStreamTokens = 16;
 
@@ -399,83 +407,236 @@ __global__ __launch_bounds__(64 * MAXW) void int4_stream_kernel(const Int4Args a
 #endif
 }
 
-// Four waves, 64 weight rows, 16 MT tokens; blockIdx = (row tile, token tile, slice of the contraction).
+// Eight waves, 64 weight rows, 32 MT tokens; blockIdx = (row tile, token tile, slice of the contraction).  A step is 128 k:
+// wave (kg, rg) multiplies the 32 k of its kg by the 32 weight rows of its rg and all tokens; the four kg's sums meet in LDS.
+//
+// What bounds it: the instructions of the expansion beside the matrix pipes.  Two waves per SIMD (one workgroup per CU at most sizes)
+// issue one instruction in 5.5 clocks each; of the 165 of a wave's step at 75 tokens 78 are the expansion's, 6 products, 7 reads of LDS
+// and 4 loads.  A step takes 0.5 - 0.6 us, 32 of them on 224 CUs for 14336 x 4096.
+//   * Four waves that expanded a fragment for 16-token products, read x from LDS for every 16 rows and went through registers
+//     to stage it took 35 us there at 75 tokens, in two slices and their sum; this takes 26 (uint4; int8 42 and 34), 44 and 27
+//     at 128, 71 and 54 at 256.
+//   * 32 x 32 x 16 products: one read of x from LDS serves 32 weight rows, and up to six other instructions ride under one.
+//   * The barrier lies between the two products of a step: with it ahead of both, a stage less was in flight, which three
+//     stages (int8 at 128 tokens) do not have to spare: 50 us, 41 now.
+template <int FMT, int MT>
+struct TileStage {
+  static constexpr int kX = MT * 8192;
+  static constexpr int kCodeRow = FMT == kUint4 ? 64 : 128;
+  static constexpr int kCodes = 64 * kCodeRow;
+  static constexpr int kScales = FMT == kUint4 ? 1024 : 2048;
+  static constexpr int kBytes = kX + kCodes + kScales;
+  static constexpr int kFit = (MT == 1 ? 80 : 160) * 1024 / kBytes, kStages = kFit < 6 ? kFit : 6;  // of 32 tokens two workgroups fit a CU
+  static constexpr int kLoads = MT + (FMT == kUint4 ? 1 : 2);  // a wave's loads per step
+  static constexpr int kSumRow = 272;  // bytes of a token's 64 partial sums, padded: 8 lanes of a write fall on all banks
+  static constexpr int kSums = 4 * 32 * MT * kSumRow;
+  static constexpr int kLds = kStages * kBytes > kSums ? kStages * kBytes : kSums;
+  static_assert(kStages >= 3 && kLds <= 160 * 1024, "the LDS of a CU");
+};
+
 template <int FMT, int MT, bool SPLIT>
-__global__ __launch_bounds__(256) void int4_tile_kernel(const Int4Args a) {
-  // 128 k of 16 MT tokens: token r's 16-byte piece p lies in slot p ^ (r % 16), so that the 16 lanes of a fragment read
-  // (16 tokens, one piece each) fall on disjoint banks
-  __shared__ u32x4_t xs[2][MT * 16 * 16];
-  const int t = threadIdx.x, lane = t & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int i = lane & 15, g = lane >> 4;
-  const int n = (int)blockIdx.x * 64 + 16 * wave + i;  // N % 64 == 0
-  const int m0 = (int)blockIdx.y * (16 * MT);
+__global__ __launch_bounds__(512, 2) void int4_tile_kernel(const Int4Args a) {
+#if defined(__HIP_DEVICE_COMPILE__)  // LDS address-space casts
+  using S = TileStage<FMT, MT>;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kg = wv >> 1, rg = wv & 1;
+  const int l31 = lane & 31, h = lane >> 5;
+  const int n0 = (int)blockIdx.x * 64;  // N % 64 == 0: every row of the workgroup exists
+  const int m0 = (int)blockIdx.y * (32 * MT);
   const int n_chunks = (a.K + 127) >> 7;
-  const int c_first = SPLIT ? (int)blockIdx.z * a.chunks_per_slice : 0;
-  const int c_end = SPLIT ? min(c_first + a.chunks_per_slice, n_chunks) : n_chunks;
+  const int t_begin = SPLIT ? (int)blockIdx.z * a.chunks_per_slice : 0;
+  const int t_end = SPLIT ? min(t_begin + a.chunks_per_slice, n_chunks) : n_chunks;
+  const int groups = a.K >> a.log2_group;
 
-  // thread t stages piece t % 16 of tokens t / 16 + 16 j
-  const int piece = t & 15, row = t >> 4;
-  const uint16_t* xsrc[MT];
+  // ---- loads into the ring.  Piece p (16 bytes) of row r goes to slot p ^ (a function of r) such that an operand's lanes read
+  // disjoint banks.  Pieces beyond K repeat one of the step's first 32 columns (K % 32 == 0: they exist); the waves that
+  // would multiply them sit the step out.
+  const uint32_t ring0 = (uint32_t)(uintptr_t)TT_LDS_PTR(smem);
+  uint32_t x_off[MT], c_off;
+  auto set_offsets = [&](int left) {
 #pragma unroll
-  for (int j = 0; j < MT; ++j) {
-    int m = m0 + 16 * j + row;
-    m = m < a.M ? m : a.M - 1;  // tokens beyond M repeat the last one and are never stored
-    xsrc[j] = a.x + (int64_t)m * a.K + 8 * piece;
-  }
-  const int slot = row * 16 + (piece ^ row);
-
-  f32x4_t acc[MT];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) acc[mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  u32x4_t xr[MT];
-  WeightPiece<FMT> w;
-  auto request = [&](int c) {
-    const int k = c * 128 + 32 * g;
-    if (k < a.K)
-      w.load(a, n, k);
-    else
-      w.clear();
-    const bool in = c * 128 + 8 * piece < a.K;
-#pragma unroll
-    for (int j = 0; j < MT; ++j) {
-      xr[j] = u32x4_t{0, 0, 0, 0};
-      if (in) xr[j] = *reinterpret_cast<const u32x4_t*>(xsrc[j] + c * 128);
+    for (int d = 0; d < MT; ++d) {
+      const int r = wv * 4 * MT + 4 * d + (lane >> 4);
+      int p = (lane & 15) ^ (r & 15);
+      p = 8 * p < left ? p : p & 3;
+      int row = m0 + r;
+      row = row < a.M ? row : a.M - 1;  // tokens beyond M repeat the last one and are never stored
+      x_off[d] = (uint32_t)row * (uint32_t)a.K * 2u + 16 * p;
+    }
+    // uint4: waves 0 - 3 bring the codes and 4 - 7 the scales; int8: all the codes, 0 - 3 the scales and 4 - 7 the zero points
+    if constexpr (FMT == kUint4) {
+      const int r = (wv & 3) * 16 + (lane >> 2);
+      int p = (lane & 3) ^ ((r >> 2) & 3);
+      p = 32 * p < left ? p : 0;
+      c_off = (uint32_t)r * (uint32_t)(a.K >> 1) + 16 * p;
+    } else {
+      const int r = wv * 8 + (lane >> 3);
+      int p = (lane & 7) ^ ((r >> 1) & 7);
+      p = 16 * p < left ? p : p & 1;
+      c_off = (uint32_t)r * (uint32_t)a.K + 16 * p;
     }
   };
-  request(c_first);
-#pragma unroll
-  for (int j = 0; j < MT; ++j) xs[0][j * 256 + slot] = xr[j];
-  __syncthreads();
-  int buf = 0;
-  for (int c = c_first; c < c_end; ++c) {
-    const WeightPiece<FMT> wc = w;
-    const bool more = c + 1 < c_end;
-    if (more) request(c + 1);
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const bf16x8_t wf = __builtin_bit_cast(bf16x8_t, wc.operand(s));
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-        acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            wf, __builtin_bit_cast(bf16x8_t, xs[buf][mt * 256 + i * 16 + ((4 * g + s) ^ i)]), acc[mt], 0, 0, 0);
+  set_offsets(128);
+  auto dma16 = [&](uint32_t voff, const void* base, uint32_t at) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "s"(at) : "memory", "m0");
+  };
+  auto dma4 = [&](uint32_t voff, const void* base, uint32_t at) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(base), "s"(at) : "memory", "m0");
+  };
+  const char* const codes0 = reinterpret_cast<const char*>(a.q) + (((int64_t)n0 * a.K) >> (FMT == kUint4 ? 1 : 0));
+  const char* const scales0 = reinterpret_cast<const char*>(FMT != kUint4 && wv >= 4 && a.zero ? a.zero : a.scale);
+  auto issue = [&](int c, uint32_t stage, int d) {  // load d of step c
+    const int left = a.K - c * 128;  // columns, at least 32
+    if (d < MT) {
+      if (d == 0 && left < 128) set_offsets(left);  // the last step
+      dma16(x_off[d], reinterpret_cast<const char*>(a.x) + (int64_t)c * 256, ring0 + stage + wv * (MT * 1024) + d * 1024);
+    } else if (FMT == kUint4 ? wv < 4 : d == MT) {
+      dma16(c_off, codes0 + (int64_t)c * (FMT == kUint4 ? 64 : 128), ring0 + stage + S::kX + wv * 1024);
+    } else if constexpr (FMT == kUint4) {  // [K / g, N]; slot 64 (32 of k) + row
+      const int k = c * 128 + (32 * (wv & 3) < left ? 32 * (wv & 3) : 0);
+      dma4(((uint32_t)(k >> a.log2_group) * (uint32_t)a.N + (uint32_t)(n0 + lane)) * 4u, scales0, ring0 + stage + S::kX + S::kCodes + (wv & 3) * 256);
+    } else {  // [N, K / g]; slot 4 row + (32 of k)
+      const int kb = lane & 3, k = c * 128 + (32 * kb < left ? 32 * kb : 0);
+      const uint32_t e = (uint32_t)(n0 + (wv & 3) * 16 + (lane >> 2)) * (uint32_t)groups + (uint32_t)(k >> a.log2_group);
+      const uint32_t off = FMT == kInt8F32 ? e * 4u : (e & ~1u) * 2u;  // bf16: the dword that it lies in (N * K / g is even)
+      dma4(off, scales0, ring0 + stage + S::kX + S::kCodes + wv * 256);
     }
-    buf ^= 1;
-    if (more) {
-#pragma unroll
-      for (int j = 0; j < MT; ++j) xs[buf][j * 256 + slot] = xr[j];
-    }
-    __syncthreads();
-  }
-  const int nb = (int)blockIdx.x * 64 + 16 * wave + 4 * g;
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    const int m = m0 + 16 * mt + i;
-    if (m >= a.M) continue;
-    if constexpr (SPLIT) {
-      *reinterpret_cast<f32x4_t*>(a.part + ((int64_t)blockIdx.z * a.M + m) * a.N + nb) = acc[mt];
+  };
+
+  // ---- operands.  Lane (l31, h) holds k 32 kg + 16 h + 8 s .. + 7 of row l31 for product s of a step.
+  constexpr int kDwords = FMT == kUint4 ? 2 : 4;
+  struct Weights {
+    uint32_t codes[kDwords];
+    float sc, z;
+  };
+  auto read_weights = [&](int c, uint32_t stage) {
+    Weights w;
+    const char* codes = smem + stage + (S::kX + (32 * rg + l31) * S::kCodeRow);
+    const char* scales = smem + stage + S::kX + S::kCodes;
+    if constexpr (FMT == kUint4) {
+      const u32x2_t v = *reinterpret_cast<const u32x2_t*>(codes + ((kg ^ ((l31 >> 2) & 3)) << 4) + 8 * h);
+      w.codes[0] = v.x;
+      w.codes[1] = v.y;
+      const uint32_t sz = *reinterpret_cast<const uint32_t*>(scales + (kg * 64 + 32 * rg + l31) * 4);
+      w.sc = lo_of(sz);
+      w.z = hi_of(sz);
     } else {
-      f32x4_t o = acc[mt];
+      const u32x4_t v = *reinterpret_cast<const u32x4_t*>(codes + (((2 * kg + h) ^ ((l31 >> 1) & 7)) << 4));
+#pragma unroll
+      for (int d = 0; d < 4; ++d) w.codes[d] = v[d];
+      const char* at = scales + (4 * (32 * rg + l31) + kg) * 4;
+      if constexpr (FMT == kInt8F32) {
+        w.sc = *reinterpret_cast<const float*>(at);
+        w.z = a.zero ? *reinterpret_cast<const float*>(at + 1024) : 0.f;
+      } else {
+        const uint32_t odd = ((uint32_t)(n0 + 32 * rg + l31) * (uint32_t)groups + (uint32_t)((c * 128 + 32 * kg) >> a.log2_group)) & 1u;
+        const uint32_t s2 = *reinterpret_cast<const uint32_t*>(at), z2 = *reinterpret_cast<const uint32_t*>(at + 1024);
+        w.sc = odd ? hi_of(s2) : lo_of(s2);
+        w.z = !a.zero ? 0.f : odd ? hi_of(z2) : lo_of(z2);
+      }
+    }
+    return w;
+  };
+  auto expand = [&](const Weights& w, int s) {
+    if constexpr (FMT == kUint4) return uint4_operand(w.codes[s], w.sc, w.z);
+    else return int8_operand(w.codes[2 * s], w.codes[2 * s + 1], w.sc, w.z);
+  };
+  int x_at[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) x_at[s] = l31 * 256 + (((4 * kg + 2 * h + s) ^ (l31 & 15)) << 4);
+  auto read_x = [&](uint32_t stage, int s, int i) {
+    return *reinterpret_cast<const bf16x8_t*>(smem + stage + x_at[s] + i * 8192);
+  };
+  auto landed = [&](int left) {  // this wave's loads but those of the newest `left` steps, and everybody is here
+    if (S::kStages > 5 && left >= 4) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(4 * S::kLoads) : "memory");
+    else if (S::kStages > 4 && left >= 3) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(3 * S::kLoads) : "memory");
+    else if (S::kStages > 3 && left >= 2) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * S::kLoads) : "memory");
+    else if (left >= 1) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(S::kLoads) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+
+  f32x16_t acc[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[i][v] = 0.f;
+  const int n_steps = t_end - t_begin;
+  const int filled = n_steps < S::kStages ? n_steps : S::kStages;
+  for (int p = 0; p < filled; ++p) {
+#pragma unroll
+    for (int d = 0; d < S::kLoads; ++d) issue(t_begin + p, p * S::kBytes, d);
+  }
+  landed(filled - 1 < S::kStages - 2 ? filled - 1 : S::kStages - 2);
+  bf16x8_t xf[2][MT];
+  u32x4_t wf[2];
+  Weights w = read_weights(t_begin, 0);
+#pragma unroll
+  for (int i = 0; i < MT; ++i) xf[0][i] = read_x(0, 0, i);
+  wf[0] = expand(w, 0);
+
+  // The barrier of step t stands between its two products: by then a wave has the step's operands in registers, so the loads of
+  // step t + stages may take its stage, and everybody's loads of step t + 1 have landed.  Beside the first product the weights
+  // of the second are expanded, beside the second those of the next step's first.
+  uint32_t stage = 0;
+  auto step = [&](int t, auto steady) {
+    constexpr bool kSteady = decltype(steady)::value;
+    const uint32_t here = stage;
+    stage = stage == (S::kStages - 1) * S::kBytes ? 0 : stage + S::kBytes;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) xf[1][i] = read_x(here, 1, i);
+    wf[1] = expand(w, 1);
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+      acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, wf[0]), xf[0][i], acc[i], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (kSteady) {
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S::kStages - 2) * S::kLoads) : "memory");
+    } else {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      landed(t_end - t - 2 < S::kStages - 2 ? t_end - t - 2 : S::kStages - 2);
+    }
+    w = read_weights(t + 1, stage);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) xf[0][i] = read_x(stage, 0, i);
+    if constexpr (kSteady) {
+#pragma unroll
+      for (int d = 0; d < S::kLoads; ++d) issue(t + S::kStages, here, d);
+    }
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+      acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, wf[1]), xf[1][i], acc[i], 0, 0, 0);
+    wf[0] = expand(w, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  int t = t_begin;
+  for (; t + S::kStages < t_end; ++t) step(t, std::true_type());
+  const int tail = a.K & 127;
+  const int t_stop = tail != 0 && 32 * kg >= tail && t_end == n_chunks ? t_end - 1 : t_end;
+  for (; t < t_stop; ++t) step(t, std::false_type());
+  if (t < t_end) landed(0);
+
+  // ---- the four kg's sums meet in LDS, in order
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      *reinterpret_cast<f32x4_t*>(smem + (kg * 32 * MT + 32 * i + l31) * S::kSumRow + (32 * rg + 8 * q + 4 * h) * 4) =
+          f32x4_t{acc[i][4 * q], acc[i][4 * q + 1], acc[i][4 * q + 2], acc[i][4 * q + 3]};
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < MT; ++j) {
+    const int token = 32 * j + ((int)threadIdx.x >> 4), quad = threadIdx.x & 15, m = m0 + token;
+    if (m >= a.M) continue;
+    f32x4_t o = *reinterpret_cast<const f32x4_t*>(smem + token * S::kSumRow + quad * 16);
+#pragma unroll
+    for (int q = 1; q < 4; ++q) o += *reinterpret_cast<const f32x4_t*>(smem + (q * 32 * MT + token) * S::kSumRow + quad * 16);
+    const int nb = n0 + 4 * quad;
+    if constexpr (SPLIT) {
+      *reinterpret_cast<f32x4_t*>(a.part + ((int64_t)blockIdx.z * a.M + m) * a.N + nb) = o;
+    } else {
       if (a.bias) {
         const u32x2_t b = *reinterpret_cast<const u32x2_t*>(a.bias + nb);
         o += f32x4_t{lo_of(b.x), hi_of(b.x), lo_of(b.y), hi_of(b.y)};
@@ -486,6 +647,7 @@ __global__ __launch_bounds__(256) void int4_tile_kernel(const Int4Args a) {
       *reinterpret_cast<u32x2_t*>(a.y + (int64_t)m * a.N + nb) = out;
     }
   }
+#endif
 }
 
 // y = bf16(sum of the slices in order + bias), four columns per thread
@@ -509,40 +671,65 @@ __global__ __launch_bounds__(256) void int4_reduce_kernel(const float* __restric
 constexpr int kMaxTokens = 256;
 constexpr int kMinRows = 256;
 
-// 16-token tiles per workgroup: as few rows of padding as the instantiated sizes allow (75 tokens on 14336 x 4096 int8: five
-// tiles 38 us, eight 48 us)
+// 32-token tiles per workgroup: as few rows of padding as token tiles of at most 128 allow
 int tile_mt(int64_t M) {
-  const int64_t wg_rows = (M + 127) / 128;
-  const int mt = (int)((M + 16 * wg_rows - 1) / (16 * wg_rows));
-  return mt <= 2 ? 2 : (mt == 7 ? 8 : mt);
+  const int64_t tiles = (M + 127) / 128;
+  return (int)((M + 32 * tiles - 1) / (32 * tiles));
 }
 
 struct Slicing {
   int slices, chunks;
 };
+// Slices of the contraction, by the time they take (us, fitted to all slicings of ten layers at 32 - 256 tokens): a round of
+// workgroups 4.2 and 0.43 + 0.05 per 32 tokens a step; the sum 1.8, 0.15 a slab and 0.65 a MB of slabs.  One workgroup fits a CU, of 32
+// tokens two, which take 1.5 times as long together.  75 tokens: 14336 x 4096 (224 row tiles) 26 whole, 33 in two slices, 4096 x 14336
+// (64) 75 whole, 28 in four, 33 in eight; 1024 x 4096 (16) 23 whole, 11 in eight, 13 in sixteen.  Beyond 512 workgroups only the slabs
+// grow.  A wave adds a quarter of its slice in one chain, which is at most as long as with 512 workgroups of one chain per slice.
 Slicing slicing(int64_t M, int64_t N, int64_t K) {
   const int64_t n_chunks = (K + 127) / 128;
-  const int64_t wgs = (N / 64) * ((M + 16 * tile_mt(M) - 1) / (16 * tile_mt(M)));
-  // two workgroups per CU and not one more: 64 tokens on 14336 x 4096 (224 row tiles, us, int8) 43 with one slice, 34 with
-  // two, 36 with three, 38 with four; on 4096 x 14336 (64 row tiles) 40 / 34 / 37 with four / eight / sixteen
-  int64_t s = wgs < 512 ? 512 / wgs : 1;
-  const int64_t most = n_chunks / 4 > 1 ? n_chunks / 4 : 1;
-  s = s < most ? s : most;
-  s = s < 16 ? s : 16;
-  const int64_t chunks = (n_chunks + s - 1) / s;
-  return {(int)((n_chunks + chunks - 1) / chunks), (int)chunks};
+  const int mt = tile_mt(M);
+  const int64_t wgs = (N / 64) * ((M + 32 * mt - 1) / (32 * mt));
+  int64_t fine = wgs < 512 ? 512 / wgs : 1;
+  fine = std::min({fine, std::max<int64_t>(n_chunks / 4, 1), int64_t(16)});
+  const int64_t longest = 4 * ((n_chunks + fine - 1) / fine);
+  Slicing best = {};
+  double best_us = 0;
+  for (int64_t s = 1; s <= 16 && s <= n_chunks && (s == 1 || wgs * s <= 512); ++s) {
+    const int64_t chunks = (n_chunks + s - 1) / s, slices = (n_chunks + chunks - 1) / chunks;
+    if (chunks > longest) continue;
+    const double rounds = mt > 1 || wgs * slices <= 256 ? (double)((wgs * slices + 255) / 256) : 1.5 * ((wgs * slices + 511) / 512);
+    double us = rounds * (4.2 + chunks * (0.43 + 0.05 * mt));
+    if (slices > 1) us += 1.8 + slices * (0.15 + 0.65e-6 * 4 * M * N);
+    if (best.slices == 0 || us < best_us) {
+      best = {(int)slices, (int)chunks};
+      best_us = us;
+    }
+  }
+  return best;
 }
 
+template <int FMT, int MT, bool SPLIT>
+int launch_tile(const Int4Args& a, dim3 grid, hipStream_t s) {
+  constexpr int kLds = TileStage<FMT, MT>::kLds;
+  static bool attr_set[64] = {};  // the LDS limit is a per-device attribute of the function
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = -1;
+  if (dev < 0 || !attr_set[dev]) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&int4_tile_kernel<FMT, MT, SPLIT>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+    if (e != hipSuccess) return fail(TTAMD_ELAUNCH, "int4_linear: cannot reserve %d bytes of LDS: %s", kLds, hipGetErrorString(e));
+    if (dev >= 0) attr_set[dev] = true;
+  }
+  int4_tile_kernel<FMT, MT, SPLIT><<<grid, dim3(512), kLds, s>>>(a);
+  return check_launch("int4_linear");
+}
 template <int FMT, bool SPLIT>
-void launch_tile(const Int4Args& a, int mt, dim3 grid, hipStream_t s) {
-  const dim3 block(256);
+int launch_tile(const Int4Args& a, int mt, dim3 grid, hipStream_t s) {
   switch (mt) {
-    case 2: int4_tile_kernel<FMT, 2, SPLIT><<<grid, block, 0, s>>>(a); break;
-    case 3: int4_tile_kernel<FMT, 3, SPLIT><<<grid, block, 0, s>>>(a); break;
-    case 4: int4_tile_kernel<FMT, 4, SPLIT><<<grid, block, 0, s>>>(a); break;
-    case 5: int4_tile_kernel<FMT, 5, SPLIT><<<grid, block, 0, s>>>(a); break;
-    case 6: int4_tile_kernel<FMT, 6, SPLIT><<<grid, block, 0, s>>>(a); break;
-    default: int4_tile_kernel<FMT, 8, SPLIT><<<grid, block, 0, s>>>(a); break;
+    case 1: return launch_tile<FMT, 1, SPLIT>(a, grid, s);
+    case 2: return launch_tile<FMT, 2, SPLIT>(a, grid, s);
+    case 3: return launch_tile<FMT, 3, SPLIT>(a, grid, s);
+    default: return launch_tile<FMT, 4, SPLIT>(a, grid, s);
   }
 }
 
@@ -589,7 +776,7 @@ int launch(Int4Args& a, bool dyn, void* workspace, size_t workspace_bytes, hipSt
     // alone.  int8 at one token, eight and sixteen: 4096 x 4096 8.5 and 8.0, 4096 x 14336 17.5 and 16.5, but 1024 x 4096 6.1 and 6.6; a wide
     // layer has workgroups enough for eight, and two row tiles from two tokens on (14336 x 4096 at 1 / 4 tokens: one 17.7 / 26.1,
     // two 17.5 / 20.6; 8192 x 2048 at one 7.0 and 7.6).  uint4: narrow layers sixteen (4096 x 14336 16.4 and 15.3), wide eight (9728 x 3584
-    // 11.5 and 15.7).
+    // 11.5 and 15.7; both pairs with an expansion of 60 instructions, with that of 37 13.5 and 10.3).
     const bool wide = a.N >= 8192;
     if constexpr (FMT == kUint4) {
       return wide ? launch_stream<FMT, 1, 8>(a, dyn, s) : launch_stream<FMT, 1, 16>(a, dyn, s);
@@ -600,19 +787,15 @@ int launch(Int4Args& a, bool dyn, void* workspace, size_t workspace_bytes, hipSt
   }
   const Slicing sl = slicing(a.M, a.N, a.K);
   const int mt = tile_mt(a.M);
-  const dim3 grid(a.N / 64, (a.M + 16 * mt - 1) / (16 * mt), sl.slices);
+  const dim3 grid(a.N / 64, (a.M + 32 * mt - 1) / (32 * mt), sl.slices);
   a.chunks_per_slice = sl.chunks;
-  if (sl.slices == 1) {
-    launch_tile<FMT, false>(a, mt, grid, s);
-    return check_launch("int4_linear");
-  }
+  if (sl.slices == 1) return launch_tile<FMT, false>(a, mt, grid, s);
   const size_t need = (size_t)sl.slices * a.M * a.N * sizeof(float);
   if (!workspace || workspace_bytes < need)
     return fail(TTAMD_EWORKSPACE, "int4_linear: workspace of %zu bytes, %zu needed", workspace_bytes, need);
   TT_REQUIRE(aligned16(workspace), "int4_linear: the workspace must be 16-byte aligned");
   a.part = reinterpret_cast<float*>(workspace);
-  launch_tile<FMT, true>(a, mt, grid, s);
-  if (int rc = check_launch("int4_linear")) return rc;
+  if (int rc = launch_tile<FMT, true>(a, mt, grid, s)) return rc;
   const int64_t quads = (int64_t)a.M * a.N / 4;
   int4_reduce_kernel<<<dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s>>>(a.part, sl.slices, quads, a.N / 4, a.bias, a.y);
   return check_launch("int4_linear: reduction");

@@ -635,10 +635,9 @@ def _int4_kernels_apply(x: torch.Tensor, weight: torch.Tensor, in_features: int,
     if bias is not None and (bias.dtype != torch.bfloat16 or not bias.is_cuda or (bias.requires_grad and torch.is_grad_enabled())):
         return False
     rows, N = x.numel() // in_features, weight.shape[0]
-    # More than 192 tokens are two tiles of rows, and a layer of more than 16384 outputs then has more than two workgroups per CU,
-    # which expand its weight twice: the dense copy and the library's larger tiles win (us at 200 tokens, these kernels and the
-    # two passes, int8 / uint4: 28672 x 8192 278 / 280 and 255 / 281, 20480 x 5120 161 / 145 and 130 / 136; at 192 tokens 117 / 104 and
-    # 132 / 136; 16384 x 4096 at 200 75 / 77 and 83 / 87).
+    # Wide layers of more than 192 tokens keep the dense weight, whose product they have always had: the line was drawn where tiles
+    # of 16 tokens per product lost to the two passes (us at 200 tokens, uint4: 28672 x 8192 280 and 255).  The present ones are
+    # ahead beyond it as well (205 and 296; int8 242 and 262).
     if rows > 192 and N > 16384:
         return False
     return weight.is_contiguous() and ops.int4_linear_applies(rows, N, in_features, groupsize)
