@@ -77,6 +77,30 @@ def test_streaming_launch_shapes(kind, qp, n, k, group, m):
     assert torch.equal(got[:1], first)
 
 
+@pytest.mark.parametrize("qp", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m", [4, 40])  # the streaming and the tiled kernel
+def test_zero_points_absent_or_anywhere_in_memory(qp, m):
+    """No zero points are zeros; those that start an element behind an aligned address are read as they are."""
+    lib, n, k, group = _lib.load(), 320, 1632, 32  # an odd number of groups per row
+    g = torch.Generator().manual_seed(m)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+    q = torch.randint(-8, 8, (n, k), generator=g, dtype=torch.int8).to(DEV)
+    scale = (torch.rand(n, k // group, generator=g) * 0.1).to(qp).to(DEV)
+    zero = torch.randint(-2, 3, (n * (k // group) + 2,), generator=g).to(qp).to(DEV)
+    zero[0] = zero[-1] = 100.0
+    stream = torch.cuda.current_stream().cuda_stream
+    ws = torch.empty(max(lib.ttamd_int4_linear_workspace_bytes(m, n, k), 16), dtype=torch.uint8, device=DEV)
+
+    def run(z):
+        y = torch.empty(m, n, device=DEV, dtype=torch.bfloat16)
+        assert lib.ttamd_int8_group_linear_bf16(x.data_ptr(), q.data_ptr(), scale.data_ptr(), z, _lib.TTAMD_F32 if qp is torch.float32 else _lib.TTAMD_BF16, group, None,
+                                                y.data_ptr(), m, n, k, ws.data_ptr(), ws.numel(), stream) == 0
+        return y
+
+    assert torch.equal(run(zero[1:].data_ptr()), run(zero[1:-1].clone().data_ptr()))
+    assert torch.equal(run(None), run(torch.zeros_like(scale).data_ptr()))
+
+
 @pytest.mark.parametrize("kind,qp", [("8da4w", torch.float32), ("8da4w", torch.bfloat16), ("4w", torch.bfloat16)])
 @pytest.mark.parametrize("n,k,group", [(8256, 1568, 32), (4160, 4128, 32), (16448, 2048, 128), (2112, 8288, 32), (256, 128, 64)])
 @pytest.mark.parametrize("m", [31, 64, 96, 113, 161, 192])

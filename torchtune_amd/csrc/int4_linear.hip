@@ -486,7 +486,11 @@ __global__ __launch_bounds__(512, 2) void int4_tile_kernel(const Int4Args a) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(base), "s"(at) : "memory", "m0");
   };
   const char* const codes0 = reinterpret_cast<const char*>(a.q) + (((int64_t)n0 * a.K) >> (FMT == kUint4 ? 1 : 0));
-  const char* const scales0 = reinterpret_cast<const char*>(FMT != kUint4 && wv >= 4 && a.zero ? a.zero : a.scale);
+  const char* scales0 = reinterpret_cast<const char*>(FMT != kUint4 && wv >= 4 && a.zero ? a.zero : a.scale);
+  // bf16 scales and zero points come as the dwords that they lie in (N * K / g is even); zero points may start in the middle of one
+  const uint32_t zero_shift = FMT == kInt8Bf16 ? (uint32_t)((uintptr_t)a.zero >> 1) & 1u : 0u;
+  const uint32_t my_shift = wv >= 4 ? zero_shift : 0u;
+  scales0 -= 2 * my_shift;
   auto issue = [&](int c, uint32_t stage, int d) {  // load d of step c
     const int left = a.K - c * 128;  // columns, at least 32
     if (d < MT) {
@@ -500,7 +504,7 @@ __global__ __launch_bounds__(512, 2) void int4_tile_kernel(const Int4Args a) {
     } else {  // [N, K / g]; slot 4 row + (32 of k)
       const int kb = lane & 3, k = c * 128 + (32 * kb < left ? 32 * kb : 0);
       const uint32_t e = (uint32_t)(n0 + (wv & 3) * 16 + (lane >> 2)) * (uint32_t)groups + (uint32_t)(k >> a.log2_group);
-      const uint32_t off = FMT == kInt8F32 ? e * 4u : (e & ~1u) * 2u;  // bf16: the dword that it lies in (N * K / g is even)
+      const uint32_t off = FMT == kInt8F32 ? e * 4u : ((e + my_shift) & ~1u) * 2u;
       dma4(off, scales0, ring0 + stage + S::kX + S::kCodes + wv * 256);
     }
   };
@@ -531,10 +535,10 @@ __global__ __launch_bounds__(512, 2) void int4_tile_kernel(const Int4Args a) {
         w.sc = *reinterpret_cast<const float*>(at);
         w.z = a.zero ? *reinterpret_cast<const float*>(at + 1024) : 0.f;
       } else {
-        const uint32_t odd = ((uint32_t)(n0 + 32 * rg + l31) * (uint32_t)groups + (uint32_t)((c * 128 + 32 * kg) >> a.log2_group)) & 1u;
+        const uint32_t e = (uint32_t)(n0 + 32 * rg + l31) * (uint32_t)groups + (uint32_t)((c * 128 + 32 * kg) >> a.log2_group);
         const uint32_t s2 = *reinterpret_cast<const uint32_t*>(at), z2 = *reinterpret_cast<const uint32_t*>(at + 1024);
-        w.sc = odd ? hi_of(s2) : lo_of(s2);
-        w.z = !a.zero ? 0.f : odd ? hi_of(z2) : lo_of(z2);
+        w.sc = e & 1u ? hi_of(s2) : lo_of(s2);
+        w.z = !a.zero ? 0.f : (e + zero_shift) & 1u ? hi_of(z2) : lo_of(z2);
       }
     }
     return w;
