@@ -923,7 +923,7 @@ def main() -> int:
                           and harness.GROUP_SHARED_INPUT and harness.SWIGLU_BWD_EPILOGUE and not qat else "")
                        + "; forward and grad-input calls)"
                        if timer.expanded_calls * 2 > calls else
-                       "nf4_gemm_rs_kernel (fused NF4-dequant + LoRA bf16 MFMA GEMM, forward and grad-input launches)"),
+                       "nf4_gemm_mid_kernel, nf4_gemm_rs16_kernel (fused NF4-dequant + LoRA bf16 MFMA GEMM, forward and grad-input launches)"),
             "achieved": round(achieved, 1),
             "peak": MFMA_BF16_PEAK_TFLOPS,
             "unit": "TFLOP/s",

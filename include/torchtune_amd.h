@@ -232,7 +232,7 @@ int ttamd_nf4_linear_bwd_dx_bf16(const void* gy, const uint8_t* quantized_data, 
 
 /*
  * The same two GEMMs for token counts between the few-token kernel and a full grid (17 - 64 tokens where the slices beat
- * the few-token kernel, see above, and 64 < M; at most 128 output tiles of 128 x 256): with a workspace the contraction is cut into up to 16 slices, one workgroup per tile per slice, fp32
+ * the few-token kernel, see above, and 64 < M): with a workspace the contraction may be cut into up to 16 slices where tiles are few, one workgroup per tile per slice, fp32
  * partial tiles in the workspace, and a second kernel adds the slices in a fixed order, then bias, column scale and
  * the rounding to bf16.  The plain entry points above are these with workspace = NULL (no slicing: a launch of few
  * tiles then leaves most of the chip idle).  The reference has no counterpart: it dequantises the weight and calls a

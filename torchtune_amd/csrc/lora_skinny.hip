@@ -11,7 +11,7 @@
 // contiguous bytes).  The last two contract over rows: bf16 MFMA as well, with both operands transposed on the way
 // through LDS (ds_read_b64_tr_b16).  Both split the contraction over many workgroups to
 // put enough loads in flight and combine the fp32 partial sums in a second, fixed-order pass, so results
-// are deterministic.  For wide layers of rank <= 16 the two products that read gy (gh and gB) come from one pass over
+// are deterministic (up to 2048 rows gA and gB are finished in one launch: skinny_tn_whole_kernel).  For wide layers of rank <= 16 the two products that read gy (gh and gB) come from one pass over
 // it (skinny_tn_gh_kernel).
 #include <atomic>
 #include "common.h"
