@@ -2,7 +2,9 @@
 validation works without a GPU, the shared rounding code matches the oracle exhaustively, and the Python surface
 mirrors the reference's (names, attributes, error messages)."""
 import ctypes
+import math
 import os
+import random
 import re
 import subprocess
 
@@ -675,31 +677,57 @@ def _nf4_gemm_plan(M, N, K, may_slice=1, by_128=1, forward=1):
     return (rows.value, slices.value, chain.value) if rc == 0 else None
 
 
+def _part_filled_slices(tiles, M, N, K):
+    whole = 64.0 * K / 4096
+    best, slices = whole / 1.2, 1
+    for sp in range(2, 9):
+        if K // sp < 1024:
+            break
+        cost = whole * -(-tiles * sp // 256) / sp + 6 + sp * M * N * 8 / 4e6
+        if cost < best:
+            best, slices = cost, sp
+    return slices
+
+
+def _longest_chain(M, N, K, room):
+    """Contraction indices of the longest chain of fp32 sums that an output may have: given room, a contraction of few tiles of 128 x
+    256 is cut into slices that fill the chip (at least 256 indices each, at most 16), one of a part-filled round into those that
+    fill its rounds; whole, it is two chains of half of it, or one where 256-row tiles take fewer than 5/9 of the rounds."""
+    columns = -(-N // 256)
+    tiles = -(-M // 128) * columns
+    slices = 1
+    if room and (tiles <= 64 or (tiles <= 128 and K >= 4096)):
+        slices = max(1, min(256 // tiles, K // 256, 16))
+    elif room and 128 < tiles < 256:
+        slices = _part_filled_slices(tiles, M, N, K)
+    if slices > 1:
+        return 64 * -(-K // 64 // slices)
+    rounds256, rounds128 = -(-(-(-M // 256) * columns) // 256), -(-tiles // 256)
+    return K if 9 * rounds256 < 5 * rounds128 else 64 * -(-K // 128)
+
+
 def test_plans_of_fused_nf4_products_keep_their_chains_and_fit_the_workspace():
-    """A contraction has as many chains of fp32 sums as slices of it, on tiles of 128 x 256, would fill the chip (at least 256
-    indices each, at most 16); the wave groups of a tile (4 on 64 rows, 2 on 96 and 128) are chains of their own.  The workspace
+    """No output's contraction runs in a longer chain of fp32 sums than above, with room for slices and without.  The workspace
     query covers every plan, and without one nothing is sliced."""
     lib = _lib.load()
-    widths = (64, 256, 576, 1024, 2048, 2816, 4096, 8192, 9728, 14336)
-    for M in (33, 65, 129, 333, 500, 700, 1000, 1279, 1500, 2047):
-        for N in widths:
-            for K in widths:
-                tiles = -(-M // 128) * -(-N // 256)
-                chains = 1
-                if tiles <= 64 or (tiles <= 128 and K >= 4096):
-                    chains = max(1, min(256 // tiles, K // 256, 16))
-                for by_128, forward in ((0, 0), (1, 0), (1, 1)):
-                    plan = _nf4_gemm_plan(M, N, K, 1, by_128, forward)
-                    if plan is None:
-                        assert lib.ttamd_nf4_gemm_expands_weight(M, N, K)
-                        continue
-                    rows, slices, chain = plan
-                    step = 128 if rows == 64 else 64
-                    if chains > 1:
-                        assert chain <= -(-K // 64 // chains) * 64 + step, (M, N, K, plan, chains)
-                    need = slices * M * N * 4 if slices > 1 else 0
-                    assert not by_128 or lib.ttamd_nf4_gemm_workspace_bytes(M, N, K) >= need
-                    assert _nf4_gemm_plan(M, N, K, 0, by_128, forward)[1] == 1
+    widths = (64, 256, 576, 1024, 2048, 2816, 4096, 8192, 9728, 14336, 28672)
+    sizes = [(M, N, K) for M in (33, 65, 129, 333, 500, 700, 1000, 1153, 1279, 1397, 1500, 2047, 4096) for N in widths for K in widths]
+    rng = random.Random(5)
+    for _ in range(4000):
+        M, N, K = (int(math.exp(rng.uniform(math.log(low), math.log(high)))) for low, high in ((17, 8192), (1, 512), (1, 512)))
+        sizes.append((M, 64 * N, 64 * K))
+    for M, N, K in sizes:
+        for by_128, forward in ((0, 0), (1, 0), (1, 1)):
+            plan = _nf4_gemm_plan(M, N, K, 1, by_128, forward)
+            if plan is None:
+                assert lib.ttamd_nf4_gemm_expands_weight(M, N, K) or M <= 64
+                continue
+            rows, slices, chain = plan
+            assert chain <= _longest_chain(M, N, K, True), (M, N, K, plan)
+            need = slices * M * N * 4 if slices > 1 else 0
+            assert not by_128 or M <= 32 or lib.ttamd_nf4_gemm_workspace_bytes(M, N, K) >= need
+            whole = _nf4_gemm_plan(M, N, K, 0, by_128, forward)
+            assert whole[1] == 1 and whole[2] <= _longest_chain(M, N, K, False), (M, N, K, whole)
 
 
 def _few_applies(M, N, K, rank):

@@ -983,11 +983,15 @@ size_t slabs_bytes(const NMidPlan& p, int64_t M, int64_t Nout, int64_t Kc) {
 // nf4_gemm_mid_kernel's way.  Time in us by rounds of the 256 CUs and 64-wide steps, fitted to products of 600 - 2047 rows: 14336 x
 // 4096 at 1000 tokens 108 against 124 on tiles of 128 rows, at 1500 (a second, part-filled round) 204 against 192; grad-input of
 // 4096 x 14336 at 900 112 and 127.
+// A 256-row tile adds the whole contraction in one chain, the other tiles' wave groups half of it each.  The longer chain is
+// admitted only where 256-row tiles take fewer than 5/9 of the rounds of 128-row ones (a round of theirs costs 1.8).
 bool wide_tiles_pay(int64_t M, int64_t Nout, int64_t Kc, double mid_cost) {
   if (nmid_min_chains(M, Nout, Kc) > 1) return false;
-  const int64_t tiles = ((M + 255) / 256) * ((Nout + kBN - 1) / kBN);
-  const double k = (double)(Kc / 64), rounds = (double)((tiles + 255) / 256),
-               wide = 2.4 + 13.0 * rounds + k * (1.07 * rounds + 0.47 * (double)tiles / 256);
+  const int64_t tiles_n = (Nout + kBN - 1) / kBN, tiles = ((M + 255) / 256) * tiles_n;
+  const int64_t rounds = (tiles + 255) / 256, rounds128 = (((M + 127) / 128) * tiles_n + 255) / 256;
+  if (9 * rounds >= 5 * rounds128) return false;
+  const double k = (double)(Kc / 64), r = (double)rounds;
+  const double wide = 2.4 + 13.0 * r + k * (1.07 * r + 0.47 * (double)tiles / 256);
   return mid_cost > 0.95 * wide;
 }
 
