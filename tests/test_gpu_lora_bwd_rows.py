@@ -52,3 +52,24 @@ def test_groups(M, Ns, ranks):
         _close(ga, gh[:, off:off + r].double().t() @ x.double())
         _close(gb, m.scale * (gy.double().t() @ h_cat[:, off:off + r].double()))
         off += r
+
+
+@pytest.mark.parametrize("M,r", [(2048, 8), (2048, 24), (2048, 48), (1024, 64)])
+def test_sums_of_32_rows_are_rounded_apart_from_the_others(M, r):
+    """Rows 512 apart are the same wave's: beside 2^24, whose neighbours are 2 apart, each 32 of them (0.3125, 10 together, every
+    partial sum of them exact) are added at once, not a few at a time.  A row of -2^24 then leaves their sum, which is off by at most half a
+    spacing for each addition at that size."""
+    steps = M // 512 - 1
+    column = torch.zeros(M, device=DEV)
+    column[0], column[32] = 2.0 ** 24, -(2.0 ** 24)
+    for s in range(steps):
+        column[512 * (s + 1):512 * (s + 1) + 32] = 0.3125
+    big = column[:, None].expand(M, 64).to(BF).contiguous()
+    ones = torch.ones(M, r, device=DEV, dtype=BF)
+    B = torch.zeros(64, r, device=DEV, dtype=BF)
+    B[0] = 1.0
+    one_hot = torch.nn.functional.one_hot(torch.zeros(M, dtype=torch.long, device=DEV), 64).to(BF)
+    _, _, gb = ops.lora_bwd(big, one_hot, ones, B, 1.0)
+    gh, ga, _ = ops.lora_bwd(one_hot, big, ones, B, 1.0)
+    assert torch.equal(gh, ones)
+    assert bool(((gb.double() - 10.0 * steps).abs() <= steps).all()) and bool(((ga.double() - 10.0 * steps).abs() <= steps).all())

@@ -547,8 +547,11 @@ __global__ __launch_bounds__(256) void skinny_tn_kernel(const TnBatch a) {
 // skinny_tn_whole: the same row contractions, finished: sixteen waves share all rows of 64 columns, their sums meet in LDS, and the
 // gradients leave rounded.  What bounds skinny_tn on few rows is not its bytes but its two launches and, for several groups of 16
 // ranks, the partial sums in between; without row splits there is neither.  Adapter backward (gh, gA, gB) of one linear, us, two
-// launches -> one: 2048 x 2048 at 700 tokens rank 8 14.8 -> 9.7, rank 32 19.4 -> 11.4; 4096 x 4096 at 1000 rank 48 38.5 -> 19.8;
-// 1024 x 1024 at 48 rank 8 11.5 -> 7.6; 2048 x 8192 at 2048 rank 16 22.7 -> 16.9.
+// launches -> one: 2048 x 2048 at 700 tokens rank 8 15.4 -> 10.2, rank 32 20.4 -> 12.8; 4096 x 4096 at 1000 rank 48 37.0 -> 19.9;
+// 1024 x 1024 at 48 rank 8 10.9 -> 7.0; 2048 x 8192 at 2048 rank 16 23.1 -> 19.2.
+// A wave adds up to four times 32 rows, and every 32 are a chain of their own, the waves' sums a tree: one chain per wave and the
+// waves one after the other, 0 - 3 % faster, had 1.08 - 1.14 times skinny_tn's rounding error at 700 - 2048 rows (2048 x 2048, of the
+// terms' absolute sum: 3.0e-9 at 700 and 2.2e-9 at 2048 in splits, 3.3e-9 and 2.5e-9 so, 3.0e-9 and 2.1e-9 as it is).
 // ---------------------------------------------------------------------------------------------------
 constexpr int kTnWholeWaves = 16, kTnWholeCols = 64;
 constexpr int kTnWholePitch = 160;  // 128 + 32: four consecutive rows fall on disjoint banks
@@ -640,7 +643,7 @@ __global__ __launch_bounds__(64 * kTnWholeWaves) void skinny_tn_whole_kernel(con
       for (int q = 0; q < RGM; ++q) {
         if (q < rg) {
           const u32x4_t gop = {ga[q].x, ga[q].y, gb[q].x, gb[q].y};
-          acc[q][e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, gop), __builtin_bit_cast(bf16x8_t, xop), acc[q][e], 0, 0, 0);
+          acc[q][e] += __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, gop), __builtin_bit_cast(bf16x8_t, xop), f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
         }
       }
     }
@@ -660,9 +663,14 @@ __global__ __launch_bounds__(64 * kTnWholeWaves) void skinny_tn_whole_kernel(con
         red[wave][v * 4 + e][lane] = val;
       }
     __syncthreads();
-    float s = red[0][wave][lane];
+    float sums[kTnWholeWaves];
 #pragma unroll
-    for (int w = 1; w < kTnWholeWaves; ++w) s += red[w][wave][lane];
+    for (int w = 0; w < kTnWholeWaves; ++w) sums[w] = red[w][wave][lane];
+#pragma unroll
+    for (int d = 1; d < kTnWholeWaves; d *= 2)
+#pragma unroll
+      for (int w = 0; w < kTnWholeWaves; w += 2 * d) sums[w] += sums[w + d];
+    const float s = sums[0];
     const int r = 16 * q + 4 * g + (wave >> 2), col = c0 + 16 * (wave & 3) + i;
     if (r >= R) continue;
     if (which == 0) {
