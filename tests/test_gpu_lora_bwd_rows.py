@@ -54,7 +54,7 @@ def test_groups(M, Ns, ranks):
         off += r
 
 
-@pytest.mark.parametrize("M,r", [(2048, 8), (2048, 24), (2048, 48), (1024, 64)])
+@pytest.mark.parametrize("M,r", [(2048, 8), (2048, 24), (2048, 48), (1024, 64), (2048, 64)])
 def test_sums_of_32_rows_are_rounded_apart_from_the_others(M, r):
     """Rows 512 apart are the same wave's: beside 2^24, whose neighbours are 2 apart, each 32 of them (0.3125, 10 together, every
     partial sum of them exact) are added at once, not a few at a time.  A row of -2^24 then leaves their sum, which is off by at most half a

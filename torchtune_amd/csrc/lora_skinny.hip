@@ -611,6 +611,9 @@ __global__ __launch_bounds__(64 * kTnWholeWaves) void skinny_tn_whole_kernel(con
       if (grow < M && gcol + 16 * q < R) gv[q] = *reinterpret_cast<const u32x4_t*>(G + (int64_t)grow * ldg + gcol + 16 * q);
     }
   };
+  // Beyond 48 ranks the next rows are fetched behind the products, not beside them, which would spill 29 registers (4096 x 4096
+  // rank 64 at 1000 tokens 28.7 us so, 22.9)
+  constexpr bool kAhead = RGM < 4;
   int m = 32 * wave;
   if (m < M) fetch(m);
   for (; m < M; m += 32 * kTnWholeWaves) {
@@ -619,7 +622,7 @@ __global__ __launch_bounds__(64 * kTnWholeWaves) void skinny_tn_whole_kernel(con
     for (int u = 0; u < 4; ++u) *reinterpret_cast<u32x4_t*>(xdst + 8 * u * kTnWholePitch) = xv[u];
 #pragma unroll
     for (int q = 0; q < RGM; ++q) *reinterpret_cast<u32x4_t*>(gdst + 1024 * q) = gv[q];  // zeros beyond R
-    if (m + 32 * kTnWholeWaves < M) fetch(m + 32 * kTnWholeWaves);
+    if (kAhead && m + 32 * kTnWholeWaves < M) fetch(m + 32 * kTnWholeWaves);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the copy-in has landed (LDS operations of a wave complete in order)
     u32x2_t ga[RGM], gb[RGM], xa[4], xb[4];
 #pragma unroll
@@ -647,6 +650,7 @@ __global__ __launch_bounds__(64 * kTnWholeWaves) void skinny_tn_whole_kernel(con
         }
       }
     }
+    if (!kAhead && m + 32 * kTnWholeWaves < M) fetch(m + 32 * kTnWholeWaves);
   }
   // acc[q][e][v] = sum over this wave's rows of G[.][16 q + 4 g + v] * X[.][c0 + 16 e + i]; 16 columns of G at a time meet in
   // the staging memory, and every thread finishes one output of them
@@ -1378,9 +1382,9 @@ size_t tn_part_bytes(int64_t M, int n, const int64_t* Kc, const int* R) {
 
 // ---- gA and gB without row splits (skinny_tn_whole_kernel) ------------------------------------------------------------
 // Up to 2048 rows it was the faster way on every pair of ten (256 x 1024 to 14336 x 4096, rank 8 - 48: 0.5 - 0.9 of the time, level
-// where both products are 14336 wide); at 3000 4096 x 14336 rank 16 takes 39.1 instead of 38.0 us, at 8192 256 x 1024 25.9 instead of
-// 16.5.  Beyond 48 ranks the sums of a wave do not fit its registers: 1024 rows (23.2 -> 20.5; at 2048 25.8 -> 28.6).
-bool tn_whole_pays(const GroupSkinny& g) { return g.M <= (g.r_off[g.n] <= 48 ? 2048 : 1024); }
+// where both products are 14336 wide; rank 64, adapter backward: 4096 x 4096 49.1 -> 22.9 us at 1024 rows, 56.7 -> 37.4 at 2048, 14336 x
+// 4096 87.9 -> 61.9 at 2048); at 3000 4096 x 14336 rank 16 takes 39.1 instead of 38.0 us, at 8192 256 x 1024 25.9 instead of 16.5.
+bool tn_whole_pays(const GroupSkinny& g) { return g.M <= 2048; }
 
 template <int RGM>
 int launch_tn_whole(const TnBatch& b, const TnWholeOut& o, hipStream_t s) {
