@@ -84,6 +84,52 @@ def test_grad_input(M, K, N, rows, sliced):
     _close(ops.nf4_linear_bwd_dx(gy, t.codes, t.scalers, K, transposed=t.transposed), gy.float() @ D)
 
 
+@pytest.mark.parametrize("M,N,K", [(520, 13312, 8192)])
+def test_without_a_workspace_the_plan_of_the_query_runs(M, N, K):
+    """Slices would be the better way, but there is no memory for them: the tiles are those that the query names, and a row has the
+    bits of the same tiles in a larger product.  Tiles of another kind add the contraction in other chains."""
+    assert _plan(M, N, K)[1] > 1 and _plan(M, N, K, may_slice=False)[0] == 256 and _plan(700, N, K)[0] == 256
+    t = _Weight(N, K, 1)
+    x = torch.randn(700, K, device=DEV, generator=t.g).to(BF)
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+
+    def run(rows):
+        y = torch.empty(rows, N, device=DEV, dtype=BF)
+        assert lib.ttamd_nf4_lora_linear_fwd_ws_bf16(x.data_ptr(), t.codes.data_ptr(), t.scalers.data_ptr(), t.transposed[1].data_ptr(), None, None, 0, 0.0,
+                                                     None, None, y.data_ptr(), rows, N, K, None, 0, stream) == 0
+        return y
+
+    assert torch.equal(run(M), run(700)[:M])
+    sliced = ops.nf4_lora_linear_fwd(x[:M], t.codes, t.scalers, N, block_scalers_t=t.transposed[1])
+    assert not torch.equal(sliced, run(M))
+    _close(sliced, x[:M].float() @ t.dense.t())
+
+
+@pytest.mark.parametrize("M,Ns,K", [(700, (3072, 3072), 3072), (333, (4096, 1024, 1024), 4096)])
+def test_groups_without_a_workspace(M, Ns, K):
+    """Members that slices would serve better, without memory for them: the bits of the members alone without a workspace."""
+    members = []
+    for i, n in enumerate(Ns):
+        t = _Weight(n, K, 3 * M + i)
+        A, B = ((torch.randn(s, device=DEV, generator=t.g) * 0.02).to(BF) for s in ((8, K), (n, 8)))
+        members.append(ops.GroupMember(t.codes, t.scalers, t.transposed, A, B, None, 2.0, n))
+    assert any(_plan(M, n, K)[1] > 1 for n in Ns)
+    x = torch.randn(M, K, device=DEV, generator=t.g).to(BF)
+    h = torch.randn(M, 8 * len(Ns), device=DEV, generator=t.g).to(BF)
+    ys = [torch.empty(M, n, device=DEV, dtype=BF) for n in Ns]
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    array = (_lib.LoraGroupMember * len(Ns))()
+    for e, m, y in zip(array, members, ys):
+        e.quantized_data, e.block_scalers, e.block_scalers_t = m.qdata.data_ptr(), m.block_scalers.data_ptr(), m.transposed[1].data_ptr()
+        e.lora_a, e.lora_b, e.y, e.N, e.rank, e.scale = m.lora_a.data_ptr(), m.lora_b.data_ptr(), y.data_ptr(), m.N, 8, m.scale
+    assert lib.ttamd_nf4_lora_group_fwd_bf16(x.data_ptr(), array, len(Ns), h.data_ptr(), M, K, None, 0, stream) == 0
+    for i, (m, y) in enumerate(zip(members, ys)):
+        hi, alone = h[:, 8 * i:8 * i + 8].contiguous(), torch.empty_like(y)
+        assert lib.ttamd_nf4_lora_linear_fwd_ws_bf16(x.data_ptr(), m.qdata.data_ptr(), m.block_scalers.data_ptr(), m.transposed[1].data_ptr(), hi.data_ptr(),
+                                                     m.lora_b.data_ptr(), 8, m.scale, None, None, alone.data_ptr(), M, m.N, K, None, 0, stream) == 0
+        assert torch.equal(y, alone)
+
+
 @pytest.mark.parametrize("M,K,Ns", [(65, 192, (128, 64, 64)), (200, 1088, (1088, 128, 192)), (333, 4096, (4096, 1024, 1024)), (700, 64, (8256, 4160)),
                                     (129, 2112, (4160, 64)), (300, 576, (320, 320))])
 @pytest.mark.parametrize("bias", [False, True])

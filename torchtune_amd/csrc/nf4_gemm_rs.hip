@@ -995,6 +995,23 @@ bool wide_tiles_pay(int64_t M, int64_t Nout, int64_t Kc, double mid_cost) {
   return mid_cost > 0.95 * wide;
 }
 
+// How a product runs that is neither a few tokens' nor on the expanded weight, with `scratch` bytes at hand for slices: on 256-row
+// tiles, or as mid says.
+struct FusedPlan {
+  bool wide;
+  NMidPlan mid;
+};
+FusedPlan fused_plan(int64_t M, int64_t Nout, int64_t Kc, size_t scratch, bool forward) {
+  FusedPlan f = {};
+  for (bool may_slice = scratch > 0;; may_slice = false) {
+    double cost;
+    f.mid = nmid_plan(M, Nout, Kc, may_slice, true, forward, &cost);
+    f.wide = wide_tiles_pay(M, Nout, Kc, cost);
+    if (f.wide) f.mid.slices = 1;
+    if (f.mid.slices == 1 || scratch >= (size_t)f.mid.slices * (size_t)M * (size_t)Nout * sizeof(float)) return f;
+  }
+}
+
 }  // namespace
 
 // Bytes of workspace run_gemm_rs can use: slices of the contraction for a small launch, or the expanded copy of the
@@ -1003,10 +1020,7 @@ size_t gemm_rs_workspace_bytes(int64_t M, int64_t Nout, int64_t Kc) {
   if (dense_path_applies(M, Nout, Kc)) return dense_workspace_bytes(M, Nout, Kc);
   size_t most = 0;
   for (const bool forward : {false, true}) {
-    double cost;
-    NMidPlan p = nmid_plan(M, Nout, Kc, true, true, forward, &cost);
-    if (wide_tiles_pay(M, Nout, Kc, cost)) p.slices = 1;
-    const size_t b = slabs_bytes(p, M, Nout, Kc);
+    const size_t b = slabs_bytes(fused_plan(M, Nout, Kc, SIZE_MAX, forward).mid, M, Nout, Kc);
     most = b > most ? b : most;
   }
   return most;
@@ -1015,12 +1029,14 @@ size_t gemm_rs_workspace_bytes(int64_t M, int64_t Nout, int64_t Kc) {
 extern "C" int ttamd_nf4_gemm_plan(int64_t M, int64_t n_out, int64_t k_contract, int may_slice, int by_128, int forward, int* tile_rows, int* slices, int* chain) {
   TT_REQUIRE(M > 0 && n_out > 0 && k_contract > 0 && n_out % 64 == 0 && k_contract % 64 == 0 && tile_rows && slices && chain, "nf4_gemm_plan: bad argument");
   if (dense_path_applies(M, n_out, k_contract)) return fail(TTAMD_EUNSUPPORTED, "nf4_gemm_plan: a product on the expanded weight");
+  FusedPlan f = {};
   double cost;
-  const NMidPlan p = nmid_plan(M, n_out, k_contract, may_slice != 0, by_128 != 0, forward != 0, &cost);
-  const bool wide = by_128 != 0 && wide_tiles_pay(M, n_out, k_contract, cost);
-  *tile_rows = wide ? 256 : p.rows;
-  *slices = wide ? 1 : p.slices;
-  *chain = wide ? (int)k_contract : 32 * (p.chain > 0 && p.chain < p.steps ? p.chain : p.steps);
+  if (by_128) f = fused_plan(M, n_out, k_contract, may_slice ? SIZE_MAX : 0, forward != 0);
+  else f.mid = nmid_plan(M, n_out, k_contract, may_slice != 0, false, forward != 0, &cost);
+  const NMidPlan& p = f.mid;
+  *tile_rows = f.wide ? 256 : p.rows;
+  *slices = p.slices;
+  *chain = f.wide ? (int)k_contract : 32 * (p.chain > 0 && p.chain < p.steps ? p.chain : p.steps);
   return TTAMD_OK;
 }
 
@@ -1060,19 +1076,13 @@ int run_gemm_rs(const void* X, const uint8_t* codes, const void* scal, int mode,
   g.lw_row_major = lw_row_major ? 1 : 0;
   g.ldlx = ldlx;
   g.lscale = lscale;
-  double cost;
-  NMidPlan p = nmid_plan(M, Nout, Kc, true, true, mode != 1, &cost);
-  if (wide_tiles_pay(M, Nout, Kc, cost)) return mode == 1 ? launch_rs16<1>(g, s) : mode == 2 ? launch_rs16<2>(g, s) : launch_rs16<0>(g, s);
-  if (p.slices > 1) {
-    if (workspace != nullptr && workspace_bytes >= (size_t)p.slices * (size_t)M * (size_t)Nout * sizeof(float)) {
-      TT_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 15u) == 0, "nf4_gemm: workspace must be 16-byte aligned");
-      g.part = reinterpret_cast<float*>(workspace);
-    } else {
-      p = nmid_plan(M, Nout, Kc, false, true, mode != 1, &cost);
-    }
-  }
-  const int rc = run_nf4_gemm_mid(mode, g, p, nullptr, nullptr, s);
-  return rc != TTAMD_OK || p.slices == 1 ? rc : launch_reduce(g, p.slices, s);
+  const FusedPlan f = fused_plan(M, Nout, Kc, workspace ? workspace_bytes : 0, mode != 1);
+  if (f.wide) return mode == 1 ? launch_rs16<1>(g, s) : mode == 2 ? launch_rs16<2>(g, s) : launch_rs16<0>(g, s);
+  const int slices = f.mid.slices;
+  TT_REQUIRE(slices == 1 || aligned16(workspace), "nf4_gemm: workspace must be 16-byte aligned");
+  g.part = slices > 1 ? reinterpret_cast<float*>(workspace) : nullptr;
+  const int rc = run_nf4_gemm_mid(mode, g, f.mid, nullptr, nullptr, s);
+  return rc != TTAMD_OK || slices == 1 ? rc : launch_reduce(g, slices, s);
 }
 
 namespace {
@@ -1101,37 +1111,37 @@ namespace {
 // Whether nf4_gemm_mid_kernel serves the members' forwards: then those on 64-row tiles share a launch and the others one, each
 // member with the slices and chains of a launch of its own (the same bits).  Launches of their own leave CUs idle and end in a
 // sum each: 4096 + 1024 + 1024 rows of 4096 at 333 tokens 63 us apart, 44 here.
-bool group_plan(const GroupGemm& d, NMidPlan (&p)[kGroupMax]) {
+bool group_plan(const GroupGemm& d, bool may_slice, NMidPlan (&p)[kGroupMax]) {
   if (d.n < 2 || d.M * d.K * 2 >= (int64_t(1) << 32) || d.K * 2 * 256 >= (int64_t(1) << 32)) return false;
   for (int i = 0; i < d.n; ++i) {
     if (!d.bscal_t[i] || d.N[i] * d.K / 2 >= (int64_t(1) << 32) || dense_path_applies(d.M, d.N[i], d.K)) return false;
-    double cost;
-    p[i] = nmid_plan(d.M, d.N[i], d.K, true, true, true, &cost);
-    if (wide_tiles_pay(d.M, d.N[i], d.K, cost)) return false;
+    const FusedPlan f = fused_plan(d.M, d.N[i], d.K, may_slice ? SIZE_MAX : 0, true);
+    if (f.wide) return false;
+    p[i] = f.mid;
   }
   return true;
 }
-}  // namespace
-
-size_t group_fwd_slices_bytes(const GroupGemm& d) {
-  NMidPlan p[kGroupMax];
-  if (!group_plan(d, p)) return 0;
+size_t group_slabs_bytes(const GroupGemm& d, const NMidPlan (&p)[kGroupMax]) {
   size_t bytes = 0;
   for (int i = 0; i < d.n; ++i)
     if (p[i].slices > 1) bytes += (size_t)p[i].slices * (size_t)d.M * (size_t)d.N[i] * sizeof(float);
   return bytes;
 }
+}  // namespace
 
-// The members' forwards in one launch or two (and, where some are sliced, one sum); *done = false where the rule above refuses it
-// or the memory for the slices is missing.
+size_t group_fwd_slices_bytes(const GroupGemm& d) {
+  NMidPlan p[kGroupMax];
+  return group_plan(d, true, p) ? group_slabs_bytes(d, p) : 0;
+}
+
+// The members' forwards in one launch or two (and, where some are sliced, one sum); *done = false where the rule above refuses it.
+// Without memory for the slices every member runs as a call of its own without a workspace does.
 int run_gemm_rs_group_fwd(const void* x, const GroupGemm& d, const void* h_cat, void* workspace, size_t workspace_bytes, bool* done, hipStream_t s) {
   NMidPlan p[kGroupMax];
-  *done = group_plan(d, p);
+  *done = group_plan(d, workspace != nullptr, p);
+  if (*done && workspace_bytes < group_slabs_bytes(d, p)) *done = group_plan(d, false, p);
   if (!*done) return TTAMD_OK;
-  const size_t need = group_fwd_slices_bytes(d);
-  *done = need == 0 || (workspace != nullptr && workspace_bytes >= need);
-  if (!*done) return TTAMD_OK;
-  TT_REQUIRE(need == 0 || aligned16(workspace), "nf4_lora_group_fwd: workspace must be 16-byte aligned");
+  TT_REQUIRE(aligned16(workspace), "nf4_lora_group_fwd: workspace must be 16-byte aligned");
   RsReduce r = {};
   int64_t part = 0;
   int sum_wgs = 0, sums = 0;
