@@ -1003,7 +1003,7 @@ struct FusedPlan {
 };
 FusedPlan fused_plan(int64_t M, int64_t Nout, int64_t Kc, size_t scratch, bool forward) {
   FusedPlan f = {};
-  for (bool may_slice = scratch > 0;; may_slice = false) {
+  for (bool may_slice = true;; may_slice = false) {  // an unsliced plan of the first needs no memory
     double cost;
     f.mid = nmid_plan(M, Nout, Kc, may_slice, true, forward, &cost);
     f.wide = wide_tiles_pay(M, Nout, Kc, cost);
