@@ -237,11 +237,14 @@ int ttamd_nf4_linear_bwd_dx_bf16(const void* gy, const uint8_t* quantized_data, 
  * the rounding to bf16.  The plain entry points above are these with workspace = NULL (no slicing: a launch of few
  * tiles then leaves most of the chip idle).  The reference has no counterpart: it dequantises the weight and calls a
  * dense GEMM (nf4_linear.py:67-70, lora.py:138).
- *   ttamd_nf4_gemm_workspace_bytes(M, n_out, k_contract): bytes to pass (0: the launch is not sliced); n_out /
- *     k_contract = N / K for the forward, K / N for the grad-input.
+ *   ttamd_nf4_gemm_workspace_bytes(M, n_out, k_contract): bytes to pass (0: none are used); n_out / k_contract = N / K for the
+ *     forward, K / N for the grad-input.  A slab of M * n_out floats for every slice, and at least one for every chain of fp32
+ *     sums that the contraction has: some plans (ttamd_nf4_gemm_plan) keep those in registers and write less or nothing.  The calls
+ *     for whole layers and for groups ask for what their plans write.
  *   ttamd_nf4_lora_linear_fwd_ws_bf16: col_scale NULL = ttamd_nf4_lora_linear_fwd_bf16, else = ttamd_nf4_dora_linear_fwd_bf16.
  *   ttamd_nf4_linear_bwd_dx_ws_bf16: slices only the variant with the transposed copies.
- * A workspace smaller than ttamd_nf4_gemm_workspace_bytes says, or NULL, runs the unsliced kernel.
+ * A workspace too small for the plan's slices, or NULL, runs the unsliced kernel, and the few-token kernel up to 64 tokens when it is
+ * smaller than ttamd_nf4_gemm_workspace_bytes says.
  *
  * Many tokens (M >= 2048 and at least 256 output tiles of 256 x 256, or M >= 1280 and more than 128 such tiles, where
  * the fused kernel would need a second round of its 128-row tiles, or M >= 1280 and at least 256 of them, where these
@@ -256,7 +259,7 @@ int ttamd_nf4_linear_bwd_dx_bf16(const void* gy, const uint8_t* quantized_data, 
  * caller that only ever runs many-token calls need not build them.
  */
 size_t ttamd_nf4_gemm_workspace_bytes(int64_t M, int64_t n_out, int64_t k_contract);
-/* 1 when those bytes are the expanded weight of the many-token path, 0 when they are slices (or none) */
+/* 1 when those bytes are the expanded weight of the many-token path, 0 when they are slabs (or none) */
 int ttamd_nf4_gemm_expands_weight(int64_t M, int64_t n_out, int64_t k_contract);
 /* How those entry points run a product that neither the few-token kernel nor the expanded weight serves: rows of an output tile (64
  * x 128 columns, 96, 128 or 256 x 256), slices of the contraction (given room for them: may_slice), and the most contraction

@@ -51,16 +51,48 @@ struct GroupDx {
   const uint16_t* lora_a[kGroupMax];   // [rank, K]
 };
 
-// nf4_gemm_rs.hip
+// How nf4_gemm_mid_kernel runs a product: tiles of 64 rows x 128 columns (steps of 128 contraction indices), of 96 or of 128 x 256
+// (steps of 64); slices of the contraction of `steps` steps each; chain > 0: chains of sums end after so many steps.
+struct NMidPlan {
+  int rows, slices, steps, chain;
+};
+// How a product of more than a few tokens runs: on the weight expanded once, on the fused 256-row tiles, or as mid says.  An entry
+// point plans once and hands the plan down.
+struct GemmPlan {
+  bool dense, wide;
+  NMidPlan mid;
+  size_t bytes;  // of memory that it writes
+};
+constexpr size_t kAnyScratch = SIZE_MAX;
+// nf4_gemm_rs.hip.  scratch: bytes at hand (kAnyScratch: as many as it asks for); forward: else the grad-input
+GemmPlan plan_gemm_rs(int64_t M, int64_t Nout, int64_t Kc, size_t scratch, bool forward);
+// workspace: p.bytes
 int run_gemm_rs(const void* X, const uint8_t* codes, const void* scal, int mode, const void* lX, int ldlx, const void* lW,
                 bool lw_row_major, int R, float lscale, const void* bias, const void* cscale, void* C, int64_t M, int64_t Nout,
-                int64_t Kc, void* workspace, size_t workspace_bytes, hipStream_t s);
+                int64_t Kc, const GemmPlan& p, void* workspace, hipStream_t s);
+// what callers of the per-kernel entry points bring (ttamd_nf4_gemm_workspace_bytes)
 size_t gemm_rs_workspace_bytes(int64_t M, int64_t Nout, int64_t Kc);
-// memory for the slices of a grouped launch of few tiles (0: it is not sliced)
-size_t group_dx_slices_bytes(const GroupDx& d);
-size_t group_fwd_slices_bytes(const GroupGemm& d);
-int run_gemm_rs_group_dx(const GroupDx& d, const void* gh_cat, void* gx, hipStream_t s, void* workspace = nullptr, size_t workspace_bytes = 0);
-int run_gemm_rs_group_fwd(const void* x, const GroupGemm& d, const void* h_cat, void* workspace, size_t workspace_bytes, bool* done, hipStream_t s);
+// the forward of M tokens runs the few-token kernel whatever memory there is
+bool few_tokens(int64_t M, int64_t Nout, int64_t Kc);
+// The grouped grad-input on the fused tiles
+GemmPlan plan_gemm_rs_group_dx(const GroupDx& d, size_t scratch);
+int run_gemm_rs_group_dx(const GroupDx& d, const void* gh_cat, void* gx, const GemmPlan& p, void* workspace, hipStream_t s);
+// The members' forwards: in one launch or two, or (one_launch false) one after the other in the same memory
+struct GroupFwdPlan {
+  bool one_launch;
+  GemmPlan member[kGroupMax];
+  size_t bytes;
+};
+GroupFwdPlan plan_gemm_rs_group_fwd(const GroupGemm& d, bool room);
+int run_gemm_rs_group_fwd(const void* x, const GroupGemm& d, const void* h_cat, const GroupFwdPlan& p, void* workspace, hipStream_t s);
+
+// nf4_gemm.hip: the checked layer calls on a plan of the caller's; plan null: the few-token kernel
+int run_lora_linear_fwd(const char* who, const void* x, const uint8_t* quantized_data, const void* block_scalers, const void* block_scalers_t,
+                        const void* h, const void* lora_b, int rank, float scale, const void* bias, const void* col_scale, void* y,
+                        int64_t M, int64_t N, int64_t K, const GemmPlan* plan, void* workspace, hipStream_t s);
+int run_linear_bwd_dx(const void* gy, const uint8_t* quantized_data, const void* block_scalers, const uint8_t* quantized_data_t,
+                      const void* block_scalers_t, const void* gh, const void* lora_a, int rank, void* gx, int64_t M, int64_t N,
+                      int64_t K, const GemmPlan& plan, void* workspace, hipStream_t s);
 
 // nf4_gemm_dense.hip: expand the weight once into scratch memory, then a plain bf16 GEMM (many tokens)
 bool dense_path_applies(int64_t M, int64_t Nout, int64_t Kc);
@@ -88,7 +120,7 @@ int run_gemm_dense_group_dx(const GroupDx& d, const void* gh_cat, void* gx, void
 int run_gemm_tn(const void* a, const void* b, void* c, int64_t M, int64_t N, int64_t K, hipStream_t s);
 // nf4_small_m.hip: y[i] = x . D(W_i)^T (+ bias) + scale . h_i . lora_b[i]^T for a handful of tokens
 int small_m_limit();
-// the forward of M tokens on an [N, K] weight runs the few-token kernel (sliced_ok: a slicing workspace is at hand)
+// the forward of M tokens on an [N, K] weight runs the few-token kernel (sliced_ok: the tiled kernel may cut its contraction)
 bool small_m_applies(int64_t M, int64_t N, int64_t K, bool sliced_ok);
 int run_small_m_group(const void* x, const GroupGemm& g, const void* h_cat, void* act, bool* act_done, hipStream_t s);
 // the same with h_i = x . lora_a[i]^T formed inside the launches (gated: two members of equal width, act is written too), the

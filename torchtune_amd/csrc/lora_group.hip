@@ -69,21 +69,32 @@ bool group_small_m(const Decoded& d, bool sliced_ok) {
   for (int i = 0; i < d.gm.n; ++i) n_max = d.gm.N[i] > n_max ? d.gm.N[i] : n_max;
   return small_m_applies(d.gm.M, n_max, d.gm.K, sliced_ok);
 }
+// with room for the tiles' slices or without: see few_tokens
+bool group_few_tokens(const Decoded& d, bool room) {
+  if (d.gm.M > small_m_limit()) return false;
+  if (!room || group_small_m(d, true)) return true;
+  for (int i = 0; i < d.gm.n; ++i)
+    if (gemm_rs_workspace_bytes(d.gm.M, d.gm.N[i], d.gm.K) > 0) return false;
+  return true;
+}
 
-// slices of the grouped launch or of the largest sliced member GEMM, or the expanded weight(s) of the many-token path
-size_t fwd_gemm_ws(const Decoded& d) {
-  const bool tiled = !group_small_m(d, true);
-  size_t w = tiled ? dense_group_fwd_workspace_bytes(d.gm) : 0;
-  if (tiled)
-    for (int i = 0; i < d.gm.n; ++i) {
-      const size_t b = gemm_rs_workspace_bytes(d.gm.M, d.gm.N[i], d.gm.K);
-      w = b > w ? b : w;
-    }
-  if (tiled) {
-    const size_t b = group_fwd_slices_bytes(d.gm);
-    w = b > w ? b : w;
-  }
-  return w;
+// How a group's forward runs, with room for what it asks for or without any: on the few-token kernel, on the members' weights
+// expanded once and side by side, or on the fused tiles
+struct FwdPlan {
+  bool few, dense;
+  GroupFwdPlan tiled;
+  size_t bytes;
+};
+FwdPlan fwd_plan(const Decoded& d, bool room) {
+  FwdPlan p = {};
+  p.few = group_few_tokens(d, room);
+  if (p.few) return p;
+  p.bytes = room ? dense_group_fwd_workspace_bytes(d.gm) : 0;
+  p.dense = p.bytes > 0;
+  if (p.dense) return p;
+  p.tiled = plan_gemm_rs_group_fwd(d.gm, room);
+  p.bytes = p.tiled.bytes;
+  return p;
 }
 
 }  // namespace
@@ -116,7 +127,7 @@ extern "C" int ttamd_lora_group_hidden_bf16(const void* x, const ttamd_lora_grou
 extern "C" size_t ttamd_lora_group_fwd_workspace_bytes(const ttamd_lora_group_member* members, int n_members, int64_t M, int64_t K) {
   Decoded d;
   if (decode("lora_group_fwd_workspace_bytes", members, n_members, M, K, false, d) != TTAMD_OK) return 0;
-  return align256(fwd_gemm_ws(d));
+  return align256(fwd_plan(d, true).bytes);
 }
 
 namespace {
@@ -127,35 +138,23 @@ int group_fwd(const char* who, const void* x, const ttamd_lora_group_member* mem
   if (int rc = decode(who, members, n_members, M, K, false, d)) return rc;
   TT_REQUIRE(x && h_cat && aligned16(x) && aligned16(h_cat), "%s: x and h_cat must be non-null and 16-byte aligned", who);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  // slices of the contraction for a member with few output tiles, when the caller brought the memory for them
-  const size_t gem = align256(fwd_gemm_ws(d));
-  const bool sliced = gem > 0 && workspace != nullptr && workspace_bytes >= gem;
-  if (group_small_m(d, sliced)) {
+  FwdPlan p = fwd_plan(d, true);
+  // without the memory that it asks for: up to 64 tokens the few-token kernel, else no slices
+  if (p.bytes > 0 && (workspace == nullptr || workspace_bytes < align256(p.bytes))) p = fwd_plan(d, false);
+  if (p.few) {
     bool done = false;
     const int rc = run_small_m_group(x, d.gm, h_cat, act, &done, s);
     if (act_done) *act_done = done;
     return rc;
   }
-  TT_REQUIRE(!sliced || aligned16(workspace), "%s: workspace must be 16-byte aligned", who);
+  TT_REQUIRE(p.bytes == 0 || aligned16(workspace), "%s: workspace must be 16-byte aligned", who);
   // many tokens: one launch over the members' concatenated output columns, every weight expanded once
-  if (sliced && dense_group_fwd_workspace_bytes(d.gm) > 0) {
+  if (p.dense) {
     const bool gated = act != nullptr && dense_group_gated_applies(d.gm);
     if (act_done) *act_done = gated;
     return run_gemm_dense_group_fwd(x, d.gm, h_cat, workspace, s, gated ? act : nullptr);
   }
-  // fewer tokens: one launch over the members' tiles where they make at most one round of them
-  bool one_launch = false;
-  if (int rc = run_gemm_rs_group_fwd(x, d.gm, h_cat, sliced ? workspace : nullptr, sliced ? workspace_bytes : 0, &one_launch, s)) return rc;
-  if (one_launch) return TTAMD_OK;
-  const int ldh = d.gm.r_off[d.gm.n];
-  for (int i = 0; i < d.gm.n; ++i) {
-    const void* sc = d.gm.bscal_t[i] ? d.gm.bscal_t[i] : d.gm.bscal[i];
-    if (int rc = run_gemm_rs(x, d.gm.codes[i], sc, d.gm.bscal_t[i] ? 2 : 0, reinterpret_cast<const uint16_t*>(h_cat) + d.gm.r_off[i], ldh,
-                             d.gm.lora_b[i], true, d.gm.rank[i], d.gm.scale[i], d.gm.bias[i], nullptr, d.gm.y[i], M, d.gm.N[i], K,
-                             sliced ? workspace : nullptr, sliced ? workspace_bytes : 0, s))
-      return rc;
-  }
-  return TTAMD_OK;
+  return run_gemm_rs_group_fwd(x, d.gm, h_cat, p.tiled, p.bytes ? workspace : nullptr, s);
 }
 }  // namespace
 
@@ -236,22 +235,32 @@ extern "C" int ttamd_lora_group_swiglu_bwd_bf16(const void* x, const void* h_cat
                             reinterpret_cast<uint16_t*>(gh_cat), reinterpret_cast<float*>(workspace), reinterpret_cast<hipStream_t>(stream), &sw);
 }
 
+namespace {
+// the grouped grad-input on the fused tiles
+int group_dx_fused(const Decoded& d, const void* gh_cat, void* gx, void* workspace, size_t workspace_bytes, void* stream) {
+  TT_REQUIRE(gh_cat && gx && aligned16(gh_cat) && aligned16(gx), "nf4_group_bwd_dx: gh_cat and gx must be non-null and 16-byte aligned");
+  for (int i = 0; i < d.dx.n; ++i)
+    TT_REQUIRE(d.dx.codes_t[i] && d.dx.scal_t[i] && aligned16(d.dx.codes_t[i]),
+               "nf4_group_bwd_dx: member %d: needs the transposed copies (ttamd_nf4_transpose_for_backward), 16-byte aligned", i);
+  return run_gemm_rs_group_dx(d.dx, gh_cat, gx, plan_gemm_rs_group_dx(d.dx, workspace ? workspace_bytes : 0), workspace,
+                              reinterpret_cast<hipStream_t>(stream));
+}
+}  // namespace
+
 extern "C" int ttamd_nf4_group_bwd_dx_bf16(const ttamd_lora_group_member* members, int n_members, const void* gh_cat, void* gx,
                                            int64_t M, int64_t K, void* stream) {
   Decoded d;
   if (int rc = decode("nf4_group_bwd_dx", members, n_members, M, K, false, d)) return rc;
-  TT_REQUIRE(gh_cat && gx && aligned16(gh_cat) && aligned16(gx), "nf4_group_bwd_dx: gh_cat and gx must be non-null and 16-byte aligned");
-  for (int i = 0; i < n_members; ++i)
-    TT_REQUIRE(d.dx.codes_t[i] && d.dx.scal_t[i] && aligned16(d.dx.codes_t[i]),
-               "nf4_group_bwd_dx: member %d: needs the transposed copies (ttamd_nf4_transpose_for_backward), 16-byte aligned", i);
-  return run_gemm_rs_group_dx(d.dx, gh_cat, gx, reinterpret_cast<hipStream_t>(stream));
+  return group_dx_fused(d, gh_cat, gx, nullptr, 0, stream);
 }
 
 extern "C" size_t ttamd_nf4_group_bwd_dx_workspace_bytes(const ttamd_lora_group_member* members, int n_members, int64_t M, int64_t K) {
   Decoded d;
   if (decode("nf4_group_bwd_dx_workspace_bytes", members, n_members, M, K, false, d) != TTAMD_OK) return 0;
-  const size_t expanded = dense_group_dx_workspace_bytes(d.dx);
-  return expanded > 0 ? expanded : group_dx_slices_bytes(d.dx);
+  if (const size_t expanded = dense_group_dx_workspace_bytes(d.dx)) return expanded;
+  for (int i = 0; i < n_members; ++i)
+    if (!d.dx.codes_t[i] || !d.dx.scal_t[i]) return 0;
+  return plan_gemm_rs_group_dx(d.dx, kAnyScratch).bytes;
 }
 
 extern "C" int ttamd_nf4_group_bwd_dx_ws_bf16(const ttamd_lora_group_member* members, int n_members, const void* gh_cat, void* gx,
@@ -259,14 +268,8 @@ extern "C" int ttamd_nf4_group_bwd_dx_ws_bf16(const ttamd_lora_group_member* mem
   Decoded d;
   if (int rc = decode("nf4_group_bwd_dx", members, n_members, M, K, false, d)) return rc;
   const size_t need = dense_group_dx_workspace_bytes(d.dx);
-  const size_t slices = need == 0 ? group_dx_slices_bytes(d.dx) : 0;
-  if (slices > 0 && workspace != nullptr && workspace_bytes >= slices) {
-    TT_REQUIRE(gh_cat && gx && aligned16(gh_cat) && aligned16(gx), "nf4_group_bwd_dx: gh_cat and gx must be non-null and 16-byte aligned");
-    for (int i = 0; i < n_members; ++i) TT_REQUIRE(aligned16(d.dx.codes_t[i]), "nf4_group_bwd_dx: member %d: the transposed copies must be 16-byte aligned", i);
-    return run_gemm_rs_group_dx(d.dx, gh_cat, gx, reinterpret_cast<hipStream_t>(stream), workspace, workspace_bytes);
-  }
-  if (need == 0 || workspace == nullptr || workspace_bytes < need)
-    return ttamd_nf4_group_bwd_dx_bf16(members, n_members, gh_cat, gx, M, K, stream);
+  if (need == 0) return group_dx_fused(d, gh_cat, gx, workspace, workspace_bytes, stream);
+  if (workspace == nullptr || workspace_bytes < need) return group_dx_fused(d, gh_cat, gx, nullptr, 0, stream);
   TT_REQUIRE(gh_cat && gx && aligned16(gh_cat) && aligned16(gx), "nf4_group_bwd_dx: gh_cat and gx must be non-null and 16-byte aligned");
   // members without transposed copies are expanded from the weight's own codes
   return run_gemm_dense_group_dx(d.dx, gh_cat, gx, workspace, reinterpret_cast<hipStream_t>(stream));

@@ -439,26 +439,35 @@ extern "C" int ttamd_nf4_block_scalers(const int8_t* quantized_scalers, const vo
   return check_launch("nf4_block_scalers");
 }
 
+namespace ttamd {
+int run_lora_linear_fwd(const char* who, const void* x, const uint8_t* quantized_data, const void* block_scalers, const void* block_scalers_t,
+                        const void* h, const void* lora_b, int rank, float scale, const void* bias, const void* col_scale, void* y,
+                        int64_t M, int64_t N, int64_t K, const GemmPlan* plan, void* workspace, hipStream_t s) {
+  if (int rc = check_gemm_args(who, x, quantized_data, block_scalers, y, M, N, K, rank, h, lora_b)) return rc;
+  TT_REQUIRE((bias == nullptr || (reinterpret_cast<uintptr_t>(bias) & 7u) == 0) &&
+                 (col_scale == nullptr || (reinterpret_cast<uintptr_t>(col_scale) & 7u) == 0),
+             "%s: bias / col_scale must be 8-byte aligned", who);
+  // a handful of tokens: stream the packed weight once (nf4_small_m.hip)
+  if (!plan) return run_small_m(x, quantized_data, block_scalers, h, rank, lora_b, rank, scale, bias, col_scale, y, M, N, K, s);
+  TT_REQUIRE(aligned16(block_scalers_t), "%s: block_scalers_t must be 16-byte aligned", who);
+  return run_gemm_rs(x, quantized_data, block_scalers_t ? block_scalers_t : block_scalers, block_scalers_t ? 2 : 0, h, rank, lora_b, true,
+                     rank, scale, bias, col_scale, y, M, N, K, *plan, workspace, s);
+}
+}  // namespace ttamd
+
 namespace {
 int lora_linear_fwd(const char* who, const void* x, const uint8_t* quantized_data, const void* block_scalers,
                     const void* block_scalers_t, const void* h, const void* lora_b, int rank, float scale, const void* bias,
                     const void* col_scale, void* y, int64_t M, int64_t N, int64_t K, void* workspace, size_t workspace_bytes,
                     void* stream) {
   if (int rc = check_gemm_args(who, x, quantized_data, block_scalers, y, M, N, K, rank, h, lora_b)) return rc;
-  TT_REQUIRE((bias == nullptr || (reinterpret_cast<uintptr_t>(bias) & 7u) == 0) &&
-                 (col_scale == nullptr || (reinterpret_cast<uintptr_t>(col_scale) & 7u) == 0),
-             "%s: bias / col_scale must be 8-byte aligned", who);
-  // a handful of tokens: stream the packed weight once (nf4_small_m.hip)
-  if (small_m_applies(M, N, K, workspace != nullptr && workspace_bytes > 0 && workspace_bytes >= gemm_rs_workspace_bytes(M, N, K)))
-    return run_small_m(x, quantized_data, block_scalers, h, rank, lora_b, rank, scale, bias, col_scale, y, M, N, K,
-                       reinterpret_cast<hipStream_t>(stream));
-  if (block_scalers_t) {
-    TT_REQUIRE(aligned16(block_scalers_t), "%s: block_scalers_t must be 16-byte aligned", who);
-    return run_gemm_rs(x, quantized_data, block_scalers_t, 2, h, rank, lora_b, true, rank, scale, bias, col_scale, y, M, N, K,
-                       workspace, workspace_bytes, reinterpret_cast<hipStream_t>(stream));
-  }
-  return run_gemm_rs(x, quantized_data, block_scalers, 0, h, rank, lora_b, true, rank, scale, bias, col_scale, y, M, N, K,
-                     workspace, workspace_bytes, reinterpret_cast<hipStream_t>(stream));
+  const size_t bytes = workspace ? workspace_bytes : 0;
+  // 17 - 64 tokens leave the few-token kernel only with all the memory that ttamd_nf4_gemm_workspace_bytes names
+  const bool few = M <= small_m_limit() && small_m_applies(M, N, K, bytes > 0 && bytes >= gemm_rs_workspace_bytes(M, N, K));
+  GemmPlan plan = {};
+  if (!few) plan = plan_gemm_rs(M, N, K, bytes, true);
+  return run_lora_linear_fwd(who, x, quantized_data, block_scalers, block_scalers_t, h, lora_b, rank, scale, bias, col_scale, y, M, N, K,
+                             few ? nullptr : &plan, workspace, reinterpret_cast<hipStream_t>(stream));
 }
 }  // namespace
 
@@ -513,22 +522,22 @@ extern "C" int ttamd_nf4_transpose_for_backward(const uint8_t* quantized_data, c
   return check_launch("nf4_transpose_for_backward");
 }
 
-extern "C" int ttamd_nf4_linear_bwd_dx_ws_bf16(const void* gy, const uint8_t* quantized_data, const void* block_scalers,
-                                               const uint8_t* quantized_data_t, const void* block_scalers_t, const void* gh,
-                                               const void* lora_a, int rank, void* gx, int64_t M, int64_t N, int64_t K,
-                                               void* workspace, size_t workspace_bytes, void* stream) {
+namespace ttamd {
+int run_linear_bwd_dx(const void* gy, const uint8_t* quantized_data, const void* block_scalers, const uint8_t* quantized_data_t,
+                      const void* block_scalers_t, const void* gh, const void* lora_a, int rank, void* gx, int64_t M, int64_t N,
+                      int64_t K, const GemmPlan& plan, void* workspace, hipStream_t s) {
   if (int rc = check_gemm_args("nf4_linear_bwd_dx", gy, quantized_data, block_scalers, gx, M, N, K, rank, gh, lora_a)) return rc;
   TT_REQUIRE((quantized_data_t == nullptr) == (block_scalers_t == nullptr),
              "nf4_linear_bwd_dx: the transposed codes and scalers must be given together");
   if (quantized_data_t != nullptr) {
     TT_REQUIRE(aligned16(quantized_data_t) && aligned16(block_scalers_t), "nf4_linear_bwd_dx: transposed copies must be 16-byte aligned");
-    return run_gemm_rs(gy, quantized_data_t, block_scalers_t, 1, gh, rank, lora_a, false, rank, 1.0f, nullptr, nullptr, gx, M, K, N,
-                       workspace, workspace_bytes, reinterpret_cast<hipStream_t>(stream));
+    return run_gemm_rs(gy, quantized_data_t, block_scalers_t, 1, gh, rank, lora_a, false, rank, 1.0f, nullptr, nullptr, gx, M, K, N, plan,
+                       workspace, s);
   }
   // no transposed copy, many tokens and room for the expanded weight: W^T is expanded from the weight's own codes
-  if (workspace != nullptr && dense_path_applies(M, K, N) && workspace_bytes >= dense_workspace_bytes(M, K, N))
+  if (plan.dense)
     return run_gemm_dense(gy, quantized_data, block_scalers, 3, gh, rank, lora_a, false, rank, 1.0f, nullptr, nullptr, gx, M, K, N,
-                          workspace, reinterpret_cast<hipStream_t>(stream));
+                          workspace, s);
   GemmArgs g;
   g.A = reinterpret_cast<const uint16_t*>(gy);
   g.qdata = quantized_data;
@@ -539,7 +548,18 @@ extern "C" int ttamd_nf4_linear_bwd_dx_ws_bf16(const void* gy, const uint8_t* qu
   g.C = reinterpret_cast<uint16_t*>(gx);
   g.M = (int)M; g.N = (int)N; g.K = (int)K; g.R = rank;
   g.lscale = 1.0f;
-  return dispatch_gemm<true>(g, reinterpret_cast<hipStream_t>(stream));
+  return dispatch_gemm<true>(g, s);
+}
+}  // namespace ttamd
+
+extern "C" int ttamd_nf4_linear_bwd_dx_ws_bf16(const void* gy, const uint8_t* quantized_data, const void* block_scalers,
+                                               const uint8_t* quantized_data_t, const void* block_scalers_t, const void* gh,
+                                               const void* lora_a, int rank, void* gx, int64_t M, int64_t N, int64_t K,
+                                               void* workspace, size_t workspace_bytes, void* stream) {
+  if (int rc = check_gemm_args("nf4_linear_bwd_dx", gy, quantized_data, block_scalers, gx, M, N, K, rank, gh, lora_a)) return rc;
+  const GemmPlan plan = plan_gemm_rs(M, K, N, workspace ? workspace_bytes : 0, false);
+  return run_linear_bwd_dx(gy, quantized_data, block_scalers, quantized_data_t, block_scalers_t, gh, lora_a, rank, gx, M, N, K, plan,
+                           workspace, reinterpret_cast<hipStream_t>(stream));
 }
 
 extern "C" int ttamd_nf4_linear_bwd_dx_swiglu_ws_bf16(const void* gy, const uint8_t* quantized_data, const void* block_scalers,

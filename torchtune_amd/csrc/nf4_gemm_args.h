@@ -56,11 +56,6 @@ struct RsMembers {
   int n;
 };
 
-// How nf4_gemm_mid_kernel runs a product: tiles of 64 rows x 128 columns (steps of 128 contraction indices), of 96 or of 128 x 256
-// (steps of 64); slices of the contraction of `steps` steps each; chain > 0: chains of sums end after so many steps.
-struct NMidPlan {
-  int rows, slices, steps, chain;
-};
 int nmid_cols(int rows);
 // the chains of sums that an output's contraction has at least
 int nmid_min_chains(int64_t M, int64_t Nout, int64_t Kc);

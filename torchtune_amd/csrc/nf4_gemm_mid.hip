@@ -30,7 +30,6 @@
 #include "nf4_gemm_args.h"
 #include "nf4_math.h"
 
-#include <cmath>
 #include <type_traits>
 
 namespace ttamd {
@@ -656,10 +655,11 @@ struct NMidTerms {
 };
 constexpr NMidTerms kTerms[] = {{64, 4.08, 2.90, 0.521, 0.156, 2.18, 2.08}, {96, 4.95, 4.08, 0.557, 0.227, 2.86, 1.25}, {128, 4.39, 5.21, 0.589, 0.326, 3.06, 1.13}};
 
-double launch_cost(const NMidTerms& c, int64_t items, int64_t steps, int64_t slabs, int64_t M, int64_t Nout) {
-  const double fill = (double)items / 256, rounds = (double)((items + 255) / 256), part = fill - floor(fill);
-  const double t = c.start + rounds * (c.round + c.step * (double)steps) + c.full_step * (floor(fill) + part * part) * (double)steps;
-  return slabs > 1 ? t + c.sum + c.slab * 1e-6 * (double)slabs * (double)M * (double)Nout : t;
+double launch_cost(const NMidTerms& c, int64_t items, int64_t steps, int64_t slabs, double elements) {
+  const int64_t full = items / 256, rounds = (items + 255) / 256;
+  const double part = (double)(items % 256) / 256;
+  const double t = c.start + rounds * (c.round + c.step * (double)steps) + c.full_step * ((double)full + part * part) * (double)steps;
+  return slabs > 1 ? t + c.sum + c.slab * 1e-6 * (double)slabs * elements : t;
 }
 int64_t tiles_of(int rows, int64_t M, int64_t Nout) { return ((M + rows - 1) / rows) * ((Nout + nmid_cols(rows) - 1) / nmid_cols(rows)); }
 }  // namespace
@@ -667,27 +667,34 @@ int64_t tiles_of(int rows, int64_t M, int64_t Nout) { return ((M + rows - 1) / r
 // Wide forwards (a gate or up projection: outputs twice the contraction and more) whose pair fills half the chip with whole
 // contractions stay whole: slices gain one of them 10 % (8192 x 3072 at 333 tokens 41 -> 37 us) and cost the pair's one launch, whose
 // members keep their own slices, 35 % (59 -> 80).
+//
+// The query and the call plan anew, and a pass of small layers waits for the host: the search ends where the slabs alone cost more
+// than the best plan so far (0.05 - 0.2 us; all 48 plans took 0.2 - 0.4).
 NMidPlan nmid_plan(int64_t M, int64_t Nout, int64_t Kc, bool may_slice, bool by_128, bool forward, double* cost) {
   const int chains = nmid_min_chains(M, Nout, Kc);
-  const bool whole = forward && Nout >= 2 * Kc && tiles_of(128, M, Nout) > 64;
+  const bool sliceable = may_slice && !(chains == 1 && forward && Nout >= 2 * Kc && tiles_of(128, M, Nout) > 64);
+  const double elements = (double)M * (double)Nout;
+  const int most = sliceable ? (int)(Kc / 256 < 16 ? Kc / 256 : 16) : 1;
   NMidPlan p = {};
   *cost = 0;
   for (const auto& c : kTerms) {
     const int groups = c.rows == 64 ? 4 : 2, step = 32 * groups;
     if (c.rows == 64 && (!by_128 || Kc < 128)) continue;
     const int64_t nk = (Kc + step - 1) / step, tiles = tiles_of(c.rows, M, Nout);
-    for (int64_t n = 1; n <= 16 && (n == 1 || (may_slice && Kc / n >= 256)); ++n) {
-      const int64_t steps = (nk + n - 1) / n;
-      if ((nk + steps - 1) / steps != n || (n > 1 && whole && chains == 1)) continue;
+    const double least = c.start + c.round + c.step * (double)tiles * (double)nk / 256 + c.sum;  // of slices, but for the slabs
+    for (int n = 1; n == 1 || n <= most; ++n) {
+      if (n > 1 && p.rows != 0 && least + c.slab * 1e-6 * (double)n * elements > *cost) break;
       // the wave groups' sums are chains of their own; whole contractions on the smallest tiles can end theirs early (no slower
       // beyond 1 - 2 %), the others have no registers for it
       const bool fold = n * groups < chains;
       if (fold && may_slice && (c.rows != 64 || n > 1)) continue;
-      const double t = launch_cost(c, tiles * n, steps, n, M, Nout);
+      const int64_t steps = (nk + n - 1) / n;
+      if (n > 1 && (nk + steps - 1) / steps != n) continue;
+      const double t = launch_cost(c, tiles * n, steps, n, elements);
       if (p.rows == 0 || t < *cost) {
         *cost = t;
         p.rows = c.rows;
-        p.slices = (int)n;
+        p.slices = n;
         p.steps = (int)steps;
         p.chain = fold && c.rows == 64 ? 2 * (int)((Kc / 64 + chains - 1) / chains) : 0;
       }
@@ -705,11 +712,11 @@ int nmid_group_rows(int64_t M, const int64_t* Nout, const NMidPlan* p, int n) {
     int64_t items = 0;
     double steps = 0;  // of a workgroup, on average
     for (int i = 0; i < n; ++i) {
-      const int64_t k = tiles_of(c.rows, M, Nout[i]) * p[i].slices;
+      const int64_t k = tiles_of(c.rows, M, Nout[i]) * (int64_t)p[i].slices;
       items += k;
-      steps += (double)(k * p[i].steps);
+      steps += (double)k * (double)p[i].steps;
     }
-    const double t = launch_cost(c, items, (int64_t)(steps / (double)items), 1, M, 0);
+    const double t = launch_cost(c, items, (int64_t)(steps / (double)items), 1, 0);
     if (best == 0 || t < least) {
       least = t;
       best = c.rows;

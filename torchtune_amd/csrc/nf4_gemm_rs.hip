@@ -972,12 +972,7 @@ int launch_segments(RsArgs& g, const RsSegs& sg, hipStream_t s) {
   return check_launch("nf4_gemm_rs");
 }
 
-// What a caller is asked to bring for slices: the slabs of the plan, and at least as many as the contraction has chains (some
-// products of several chains keep them in registers; few-token products need a caller's memory to leave their own kernel).
-size_t slabs_bytes(const NMidPlan& p, int64_t M, int64_t Nout, int64_t Kc) {
-  const int chains = nmid_min_chains(M, Nout, Kc), slabs = p.slices > chains ? p.slices : chains;
-  return slabs > 1 ? (size_t)slabs * (size_t)M * (size_t)Nout * sizeof(float) : 0;
-}
+size_t slabs_bytes(int slabs, int64_t M, int64_t Nout) { return slabs > 1 ? (size_t)slabs * (size_t)M * (size_t)Nout * sizeof(float) : 0; }
 
 // Whether a product of one chain of sums per output (nmid_min_chains) takes 256-row tiles: where they cost less than 1 / 0.95 of
 // nf4_gemm_mid_kernel's way.  Time in us by rounds of the 256 CUs and 64-wide steps, fitted to products of 600 - 2047 rows: 14336 x
@@ -995,43 +990,52 @@ bool wide_tiles_pay(int64_t M, int64_t Nout, int64_t Kc, double mid_cost) {
   return mid_cost > 0.95 * wide;
 }
 
-// How a product runs that is neither a few tokens' nor on the expanded weight, with `scratch` bytes at hand for slices: on 256-row
-// tiles, or as mid says.
-struct FusedPlan {
-  bool wide;
-  NMidPlan mid;
-};
-FusedPlan fused_plan(int64_t M, int64_t Nout, int64_t Kc, size_t scratch, bool forward) {
-  FusedPlan f = {};
+// A product that is neither a few tokens' nor on the expanded weight
+GemmPlan fused_plan(int64_t M, int64_t Nout, int64_t Kc, size_t scratch, bool forward) {
+  GemmPlan f = {};
   for (bool may_slice = true;; may_slice = false) {  // an unsliced plan of the first needs no memory
     double cost;
     f.mid = nmid_plan(M, Nout, Kc, may_slice, true, forward, &cost);
     f.wide = wide_tiles_pay(M, Nout, Kc, cost);
     if (f.wide) f.mid.slices = 1;
-    if (f.mid.slices == 1 || scratch >= (size_t)f.mid.slices * (size_t)M * (size_t)Nout * sizeof(float)) return f;
+    f.bytes = slabs_bytes(f.mid.slices, M, Nout);
+    if (f.bytes <= scratch) return f;
   }
 }
 
 }  // namespace
 
-// Bytes of workspace run_gemm_rs can use: slices of the contraction for a small launch, or the expanded copy of the
-// weight for a launch of many tokens (nf4_gemm_dense.hip); the two cases exclude each other.  0: it would use none.
+GemmPlan plan_gemm_rs(int64_t M, int64_t Nout, int64_t Kc, size_t scratch, bool forward) {
+  GemmPlan p = {};
+  p.bytes = dense_workspace_bytes(M, Nout, Kc);
+  p.dense = p.bytes > 0 && scratch >= p.bytes;
+  return p.dense ? p : fused_plan(M, Nout, Kc, scratch, forward);
+}
+
+// The expanded weight, or the slabs of the plan with the most of them, and at least as many as the contraction has chains of sums,
+// also where the plan keeps those in registers.
 size_t gemm_rs_workspace_bytes(int64_t M, int64_t Nout, int64_t Kc) {
-  if (dense_path_applies(M, Nout, Kc)) return dense_workspace_bytes(M, Nout, Kc);
-  size_t most = 0;
+  if (const size_t dense = dense_workspace_bytes(M, Nout, Kc)) return dense;
+  int slabs = nmid_min_chains(M, Nout, Kc);
   for (const bool forward : {false, true}) {
-    const size_t b = slabs_bytes(fused_plan(M, Nout, Kc, SIZE_MAX, forward).mid, M, Nout, Kc);
-    most = b > most ? b : most;
+    if (forward && Nout < 2 * Kc) break;  // the same plan
+    const int n = fused_plan(M, Nout, Kc, kAnyScratch, forward).mid.slices;
+    slabs = n > slabs ? n : slabs;
   }
-  return most;
+  return slabs_bytes(slabs, M, Nout);
+}
+
+// Up to 16 tokens, and up to 64 where that kernel is the faster or the tiles would not cut the contraction
+bool few_tokens(int64_t M, int64_t Nout, int64_t Kc) {
+  return small_m_applies(M, Nout, Kc, true) || (M <= small_m_limit() && gemm_rs_workspace_bytes(M, Nout, Kc) == 0);
 }
 
 extern "C" int ttamd_nf4_gemm_plan(int64_t M, int64_t n_out, int64_t k_contract, int may_slice, int by_128, int forward, int* tile_rows, int* slices, int* chain) {
   TT_REQUIRE(M > 0 && n_out > 0 && k_contract > 0 && n_out % 64 == 0 && k_contract % 64 == 0 && tile_rows && slices && chain, "nf4_gemm_plan: bad argument");
   if (dense_path_applies(M, n_out, k_contract)) return fail(TTAMD_EUNSUPPORTED, "nf4_gemm_plan: a product on the expanded weight");
-  FusedPlan f = {};
+  GemmPlan f = {};
   double cost;
-  if (by_128) f = fused_plan(M, n_out, k_contract, may_slice ? SIZE_MAX : 0, forward != 0);
+  if (by_128) f = fused_plan(M, n_out, k_contract, may_slice ? kAnyScratch : 0, forward != 0);
   else f.mid = nmid_plan(M, n_out, k_contract, may_slice != 0, false, forward != 0, &cost);
   const NMidPlan& p = f.mid;
   *tile_rows = f.wide ? 256 : p.rows;
@@ -1040,11 +1044,10 @@ extern "C" int ttamd_nf4_gemm_plan(int64_t M, int64_t n_out, int64_t k_contract,
   return TTAMD_OK;
 }
 
-// Entry used by the C-ABI wrappers.  `workspace` may be null: then small launches are not sliced.  The rows of the
-// adapter activation lX are ldlx elements apart (a group keeps its members' activations side by side).
+// The rows of the adapter activation lX are ldlx elements apart (a group keeps its members' activations side by side).
 int run_gemm_rs(const void* X, const uint8_t* codes, const void* scal, int mode, const void* lX, int ldlx, const void* lW,
                 bool lw_row_major, int R, float lscale, const void* bias, const void* cscale, void* C, int64_t M, int64_t Nout,
-                int64_t Kc, void* workspace, size_t workspace_bytes, hipStream_t s) {
+                int64_t Kc, const GemmPlan& p, void* workspace, hipStream_t s) {
   // per-lane byte offsets inside the kernel are 32-bit: the weight must fit them, and a token dimension too long for
   // them is cut into row ranges (multiples of the 256-row tile) that are launched one after the other
   TT_REQUIRE(Nout * Kc / 2 < (int64_t(1) << 32) && Nout * (Kc / 64) * 4 < (int64_t(1) << 32) && Kc * 2 * 256 < (int64_t(1) << 32),
@@ -1055,13 +1058,14 @@ int run_gemm_rs(const void* X, const uint8_t* codes, const void* scal, int mode,
       const int64_t rows = M - r0 < max_rows ? M - r0 : max_rows;
       const int rc = run_gemm_rs(reinterpret_cast<const uint16_t*>(X) + r0 * Kc, codes, scal, mode,
                                  lX ? reinterpret_cast<const uint16_t*>(lX) + r0 * ldlx : nullptr, ldlx, lW, lw_row_major, R, lscale, bias,
-                                 cscale, reinterpret_cast<uint16_t*>(C) + r0 * Nout, rows, Nout, Kc, nullptr, 0, s);
+                                 cscale, reinterpret_cast<uint16_t*>(C) + r0 * Nout, rows, Nout, Kc,
+                                 plan_gemm_rs(rows, Nout, Kc, 0, mode != 1), nullptr, s);
       if (rc != TTAMD_OK) return rc;
     }
     return TTAMD_OK;
   }
   // many tokens and room for the expanded weight: expand once, then the plain bf16 GEMM
-  if (workspace != nullptr && dense_path_applies(M, Nout, Kc) && workspace_bytes >= dense_workspace_bytes(M, Nout, Kc))
+  if (p.dense)
     return run_gemm_dense(X, codes, scal, mode, lX, ldlx, lW, lw_row_major, R, lscale, bias, cscale, C, M, Nout, Kc, workspace, s);
   RsArgs g = {};
   g.X = reinterpret_cast<const uint16_t*>(X);
@@ -1076,72 +1080,63 @@ int run_gemm_rs(const void* X, const uint8_t* codes, const void* scal, int mode,
   g.lw_row_major = lw_row_major ? 1 : 0;
   g.ldlx = ldlx;
   g.lscale = lscale;
-  const FusedPlan f = fused_plan(M, Nout, Kc, workspace ? workspace_bytes : 0, mode != 1);
-  if (f.wide) return mode == 1 ? launch_rs16<1>(g, s) : mode == 2 ? launch_rs16<2>(g, s) : launch_rs16<0>(g, s);
-  const int slices = f.mid.slices;
+  if (p.wide) return mode == 1 ? launch_rs16<1>(g, s) : mode == 2 ? launch_rs16<2>(g, s) : launch_rs16<0>(g, s);
+  const int slices = p.mid.slices;
   TT_REQUIRE(slices == 1 || aligned16(workspace), "nf4_gemm: workspace must be 16-byte aligned");
   g.part = slices > 1 ? reinterpret_cast<float*>(workspace) : nullptr;
-  const int rc = run_nf4_gemm_mid(mode, g, f.mid, nullptr, nullptr, s);
+  const int rc = run_nf4_gemm_mid(mode, g, p.mid, nullptr, nullptr, s);
   return rc != TTAMD_OK || slices == 1 ? rc : launch_reduce(g, slices, s);
 }
 
-namespace {
 // The grouped grad-input's plan: one contraction over the members' columns (steps of 128 only where each is whole steps).
-NMidPlan group_dx_plan(const GroupDx& d, bool may_slice) {
+GemmPlan plan_gemm_rs_group_dx(const GroupDx& d, size_t scratch) {
   int64_t n_total = 0;
   bool by_128 = true;
   for (int i = 0; i < d.n; ++i) {
     n_total += d.N[i];
     by_128 = by_128 && d.N[i] % 128 == 0;
   }
-  double cost;
-  return nmid_plan(d.M, d.K, n_total, may_slice, by_128, false, &cost);
-}
-}  // namespace
-
-size_t group_dx_slices_bytes(const GroupDx& d) {
-  for (int i = 0; i < d.n; ++i)
-    if (!d.codes_t[i] || !d.scal_t[i]) return 0;
-  int64_t n_total = 0;
-  for (int i = 0; i < d.n; ++i) n_total += d.N[i];
-  return slabs_bytes(group_dx_plan(d, true), d.M, d.K, n_total);
-}
-
-namespace {
-// Whether nf4_gemm_mid_kernel serves the members' forwards: then those on 64-row tiles share a launch and the others one, each
-// member with the slices and chains of a launch of its own (the same bits).  Launches of their own leave CUs idle and end in a
-// sum each: 4096 + 1024 + 1024 rows of 4096 at 333 tokens 63 us apart, 44 here.
-bool group_plan(const GroupGemm& d, bool may_slice, NMidPlan (&p)[kGroupMax]) {
-  if (d.n < 2 || d.M * d.K * 2 >= (int64_t(1) << 32) || d.K * 2 * 256 >= (int64_t(1) << 32)) return false;
-  for (int i = 0; i < d.n; ++i) {
-    if (!d.bscal_t[i] || d.N[i] * d.K / 2 >= (int64_t(1) << 32) || dense_path_applies(d.M, d.N[i], d.K)) return false;
-    const FusedPlan f = fused_plan(d.M, d.N[i], d.K, may_slice ? SIZE_MAX : 0, true);
-    if (f.wide) return false;
-    p[i] = f.mid;
+  GemmPlan p = {};
+  for (bool may_slice = true;; may_slice = false) {
+    double cost;
+    p.mid = nmid_plan(d.M, d.K, n_total, may_slice, by_128, false, &cost);
+    p.wide = p.mid.slices == 1 && ((d.M + kBM - 1) / kBM) * ((d.K + kBN - 1) / kBN) >= 256;
+    p.bytes = slabs_bytes(p.mid.slices, d.M, d.K);
+    if (p.bytes <= scratch) return p;
   }
-  return true;
-}
-size_t group_slabs_bytes(const GroupGemm& d, const NMidPlan (&p)[kGroupMax]) {
-  size_t bytes = 0;
-  for (int i = 0; i < d.n; ++i)
-    if (p[i].slices > 1) bytes += (size_t)p[i].slices * (size_t)d.M * (size_t)d.N[i] * sizeof(float);
-  return bytes;
-}
-}  // namespace
-
-size_t group_fwd_slices_bytes(const GroupGemm& d) {
-  NMidPlan p[kGroupMax];
-  return group_plan(d, true, p) ? group_slabs_bytes(d, p) : 0;
 }
 
-// The members' forwards in one launch or two (and, where some are sliced, one sum); *done = false where the rule above refuses it.
-// Without memory for the slices every member runs as a call of its own without a workspace does.
-int run_gemm_rs_group_fwd(const void* x, const GroupGemm& d, const void* h_cat, void* workspace, size_t workspace_bytes, bool* done, hipStream_t s) {
-  NMidPlan p[kGroupMax];
-  *done = group_plan(d, workspace != nullptr, p);
-  if (*done && workspace_bytes < group_slabs_bytes(d, p)) *done = group_plan(d, false, p);
-  if (!*done) return TTAMD_OK;
+// Where nf4_gemm_mid_kernel serves the members' forwards, those on 64-row tiles share a launch and the others one, each
+// member with the slices and chains of a launch of its own (the same bits).  Launches of their own leave CUs idle and end in a
+// sum each: 4096 + 1024 + 1024 rows of 4096 at 333 tokens 63 us apart, 44 here.  Without memory for the slices every member is
+// planned as a call of its own without a workspace.
+GroupFwdPlan plan_gemm_rs_group_fwd(const GroupGemm& d, bool room) {
+  GroupFwdPlan g = {};
+  g.one_launch = d.n >= 2 && d.M * d.K * 2 < (int64_t(1) << 32) && d.K * 2 * 256 < (int64_t(1) << 32);
+  size_t sum = 0, most = 0;
+  for (int i = 0; i < d.n; ++i) {
+    const GemmPlan& p = g.member[i] = plan_gemm_rs(d.M, d.N[i], d.K, room ? kAnyScratch : 0, true);
+    g.one_launch = g.one_launch && d.bscal_t[i] && d.N[i] * d.K / 2 < (int64_t(1) << 32) && !p.wide && !dense_path_applies(d.M, d.N[i], d.K);
+    sum += p.bytes;
+    most = p.bytes > most ? p.bytes : most;
+  }
+  g.bytes = g.one_launch ? sum : most;
+  return g;
+}
+
+int run_gemm_rs_group_fwd(const void* x, const GroupGemm& d, const void* h_cat, const GroupFwdPlan& gp, void* workspace, hipStream_t s) {
   TT_REQUIRE(aligned16(workspace), "nf4_lora_group_fwd: workspace must be 16-byte aligned");
+  if (!gp.one_launch) {
+    for (int i = 0; i < d.n; ++i) {
+      const void* sc = d.bscal_t[i] ? d.bscal_t[i] : d.bscal[i];
+      if (int rc = run_gemm_rs(x, d.codes[i], sc, d.bscal_t[i] ? 2 : 0, reinterpret_cast<const uint16_t*>(h_cat) + d.r_off[i], d.r_off[d.n],
+                               d.lora_b[i], true, d.rank[i], d.scale[i], d.bias[i], nullptr, d.y[i], d.M, d.N[i], d.K, gp.member[i], workspace, s))
+        return rc;
+    }
+    return TTAMD_OK;
+  }
+  NMidPlan p[kGroupMax];
+  for (int i = 0; i < d.n; ++i) p[i] = gp.member[i].mid;
   RsReduce r = {};
   int64_t part = 0;
   int sum_wgs = 0, sums = 0;
@@ -1211,11 +1206,11 @@ int run_gemm_rs_group_fwd(const void* x, const GroupGemm& d, const void* h_cat, 
 //   gx[M, K] = sum_i gy_i[M, N_i] . D(W_i)[N_i, K] + gh_i[M, R_i] . A_i[R_i, K]
 // with the members' transposed copies (codes [K, N_i / 2], per-element scalers [K / 64, N_i]); gh_i = columns
 // [r_off[i], r_off[i + 1]) of gh_cat.  The sum over members is taken in fp32, before the one rounding to bf16.
-// A launch of few tiles is sliced like a single layer's when the caller brought group_dx_slices_bytes(d) of memory: unsliced it
+// A launch of few tiles is sliced like a single layer's where there is memory for it: unsliced it
 // takes its 256 - 448 k-steps however few workgroups there are.  Unsliced -> sliced, us: 14336 + 14336 rows of 4096 at 100
 // tokens 287 -> 49, at 333 293 -> 111, at 1000 302 -> 246; 4096 + 1024 + 1024 at 333 67 -> 38, at 1000 75 -> 70; 8192 + 8192
 // rows of 2048 at 333 164 -> 45.
-int run_gemm_rs_group_dx(const GroupDx& d, const void* gh_cat, void* gx, hipStream_t s, void* workspace, size_t workspace_bytes) {
+int run_gemm_rs_group_dx(const GroupDx& d, const void* gh_cat, void* gx, const GemmPlan& p, void* workspace, hipStream_t s) {
   TT_REQUIRE(d.n >= 1 && d.n <= kGroupMax, "nf4_group_dx: %d members", d.n);
   RsSegs sg = {};
   sg.n = d.n;
@@ -1250,18 +1245,11 @@ int run_gemm_rs_group_dx(const GroupDx& d, const void* gh_cat, void* gx, hipStre
   g.lw_row_major = 0;
   g.ldlx = d.r_off[d.n];
   g.lscale = 1.0f;
-  NMidPlan p = group_dx_plan(d, true);
-  if (p.slices > 1) {
-    if (workspace != nullptr && workspace_bytes >= (size_t)p.slices * (size_t)d.M * (size_t)d.K * sizeof(float)) {
-      TT_REQUIRE(aligned16(workspace), "nf4_group_dx: workspace must be 16-byte aligned");
-      g.part = reinterpret_cast<float*>(workspace);
-    } else {
-      p = group_dx_plan(d, false);
-    }
-  }
-  if (p.slices == 1 && ((d.M + kBM - 1) / kBM) * ((d.K + kBN - 1) / kBN) >= 256) return launch_segments(g, sg, s);
-  const int rc = run_nf4_gemm_mid(1, g, p, &sg, nullptr, s);
-  return rc != TTAMD_OK || p.slices == 1 ? rc : launch_reduce(g, p.slices, s);
+  if (p.wide) return launch_segments(g, sg, s);
+  TT_REQUIRE(p.mid.slices == 1 || aligned16(workspace), "nf4_group_dx: workspace must be 16-byte aligned");
+  g.part = reinterpret_cast<float*>(workspace);
+  const int rc = run_nf4_gemm_mid(1, g, p.mid, &sg, nullptr, s);
+  return rc != TTAMD_OK || p.mid.slices == 1 ? rc : launch_reduce(g, p.mid.slices, s);
 }
 
 }  // namespace ttamd

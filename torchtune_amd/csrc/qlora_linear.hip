@@ -7,6 +7,7 @@
 // time).  The stages of a direction run one after the other on the caller's stream, so their scratch regions share
 // the workspace's bytes; only the backward's gh = scale . gy . B, which the second stage reads, has a region to itself.
 #include "common.h"
+#include "group.h"
 
 namespace ttamd {
 namespace {
@@ -20,6 +21,20 @@ int check_layer(const char* who, int64_t M, int64_t N, int64_t K, int rank) {
   TT_REQUIRE(rank >= 8 && rank <= 64 && rank % 8 == 0, "%s: the adapter rank (%d) must be a multiple of 8 in [8, 64]", who, rank);
   return TTAMD_OK;
 }
+
+// The forward's product with all the memory that it asks for; few: the few-token kernel instead
+struct FwdPlan {
+  bool few;
+  GemmPlan gemm;
+};
+FwdPlan fwd_plan(int64_t M, int64_t N, int64_t K) {
+  FwdPlan p = {};
+  p.few = few_tokens(M, N, K);
+  if (!p.few) p.gemm = plan_gemm_rs(M, N, K, kAnyScratch, true);
+  return p;
+}
+// The grad-input's: of as few tokens it is not sliced.  Without the transposed copies only the expanded weight takes memory.
+GemmPlan dx_plan(int64_t M, int64_t N, int64_t K) { return plan_gemm_rs(M, K, N, small_m_applies(M, K, N, true) ? 0 : kAnyScratch, false); }
 }  // namespace
 }  // namespace ttamd
 
@@ -27,7 +42,7 @@ using namespace ttamd;
 
 extern "C" size_t ttamd_qlora_linear_fwd_workspace_bytes(int64_t M, int64_t N, int64_t K, int rank) {
   if (M <= 0 || N <= 0 || K <= 0 || rank <= 0) return 0;
-  return align256(max2(ttamd_lora_fwd_workspace_bytes(M, K, rank), ttamd_nf4_gemm_workspace_bytes(M, N, K)));
+  return align256(max2(ttamd_lora_fwd_workspace_bytes(M, K, rank), fwd_plan(M, N, K).gemm.bytes));
 }
 
 extern "C" int ttamd_qlora_linear_fwd_bf16(const void* x, const uint8_t* quantized_data, const void* block_scalers,
@@ -36,22 +51,21 @@ extern "C" int ttamd_qlora_linear_fwd_bf16(const void* x, const uint8_t* quantiz
                                            size_t workspace_bytes, void* stream) {
   if (int rc = check_layer("qlora_linear_fwd", M, N, K, rank)) return rc;
   TT_REQUIRE(x && quantized_data && block_scalers && lora_a && lora_b && y && h, "qlora_linear_fwd: null pointer argument");
-  const size_t need = ttamd_qlora_linear_fwd_workspace_bytes(M, N, K, rank);
+  const FwdPlan plan = fwd_plan(M, N, K);
+  const size_t hid = ttamd_lora_fwd_workspace_bytes(M, K, rank), need = align256(max2(hid, plan.gemm.bytes));
   TT_REQUIRE(need == 0 || (workspace && aligned16(workspace)), "qlora_linear_fwd: workspace must be non-null and 16-byte aligned");
   if (workspace_bytes < need) return fail(TTAMD_EWORKSPACE, "qlora_linear_fwd: workspace has %zu bytes, needs %zu", workspace_bytes, need);
   // stage 1: h = bf16(x . A^T); its partial sums are consumed before stage 2 starts on the same stream
-  const size_t hid = ttamd_lora_fwd_workspace_bytes(M, K, rank);
   if (int rc = ttamd_lora_hidden_bf16(x, lora_a, h, M, K, rank, hid ? workspace : nullptr, hid, stream)) return rc;
   // stage 2: y = x . D(W)^T (+ bias) + scale . h . B^T
-  const size_t gemm = ttamd_nf4_gemm_workspace_bytes(M, N, K);
-  return ttamd_nf4_lora_linear_fwd_ws_bf16(x, quantized_data, block_scalers, block_scalers_t, h, lora_b, rank, scale, bias, nullptr, y, M,
-                                           N, K, gemm ? workspace : nullptr, gemm, stream);
+  return run_lora_linear_fwd("qlora_linear_fwd", x, quantized_data, block_scalers, block_scalers_t, h, lora_b, rank, scale, bias, nullptr, y,
+                             M, N, K, plan.few ? nullptr : &plan.gemm, workspace, reinterpret_cast<hipStream_t>(stream));
 }
 
 extern "C" size_t ttamd_qlora_linear_bwd_workspace_bytes(int64_t M, int64_t N, int64_t K, int rank) {
   if (M <= 0 || N <= 0 || K <= 0 || rank <= 0) return 0;
   return align256((size_t)M * (size_t)rank * 2) +
-         align256(max2(ttamd_lora_bwd_workspace_bytes(M, N, K, rank), ttamd_nf4_gemm_workspace_bytes(M, K, N)));
+         align256(max2(ttamd_lora_bwd_workspace_bytes(M, N, K, rank), small_m_applies(M, K, N, true) ? 0 : dx_plan(M, N, K).bytes));
 }
 
 extern "C" int ttamd_qlora_linear_bwd_bf16(const void* gy, const void* x, const void* h, const uint8_t* quantized_data,
@@ -64,22 +78,21 @@ extern "C" int ttamd_qlora_linear_bwd_bf16(const void* gy, const void* x, const 
              "qlora_linear_bwd: null pointer argument");
   TT_REQUIRE((quantized_data_t == nullptr) == (block_scalers_t == nullptr), "qlora_linear_bwd: pass both transposed copies or neither");
   // with the forward's tiles at hand (or no grad-input at all) the GEMM stage needs no scratch memory
-  const size_t need = (tiles_fwd || !gx) ? align256((size_t)M * (size_t)rank * 2) + align256(ttamd_lora_bwd_workspace_bytes(M, N, K, rank))
-                                         : ttamd_qlora_linear_bwd_workspace_bytes(M, N, K, rank);
+  GemmPlan plan = {};
+  if (gx && !tiles_fwd) plan = dx_plan(M, N, K);
+  const size_t skinny = ttamd_lora_bwd_workspace_bytes(M, N, K, rank);
+  const size_t need = align256((size_t)M * (size_t)rank * 2) + align256(max2(skinny, plan.bytes));
   TT_REQUIRE(workspace && aligned16(workspace), "qlora_linear_bwd: workspace must be non-null and 16-byte aligned");
   if (workspace_bytes < need) return fail(TTAMD_EWORKSPACE, "qlora_linear_bwd: workspace has %zu bytes, needs %zu", workspace_bytes, need);
   char* ws = reinterpret_cast<char*>(workspace);
   void* gh = ws;
   char* rest = ws + align256((size_t)M * (size_t)rank * 2);
   // stage 1: gh = scale . gy . B, gA = gh^T . x, gB = scale . gy^T . h
-  const size_t skinny = ttamd_lora_bwd_workspace_bytes(M, N, K, rank);
   if (int rc = ttamd_lora_bwd_bf16(gy, x, h, lora_b, scale, gh, grad_lora_a, grad_lora_b, M, N, K, rank, rest, skinny, stream)) return rc;
   if (gx == nullptr) return TTAMD_OK;  // the layer's input needs no gradient
   // the forward call's expanded weight is still at hand: the grad-input reads it (no expansion, no scratch memory)
   if (tiles_fwd) return ttamd_tiled_linear_dx_bf16(gy, tiles_fwd, gh, lora_a, rank, gx, M, N, K, stream);
-  // stage 2: gx = gy . D(W) + gh . A.  Without the transposed copies only the expanded-weight launch takes a workspace.
-  size_t gemm = ttamd_nf4_gemm_workspace_bytes(M, K, N);
-  if (!quantized_data_t && !ttamd_nf4_gemm_expands_weight(M, K, N)) gemm = 0;
-  return ttamd_nf4_linear_bwd_dx_ws_bf16(gy, quantized_data, block_scalers, quantized_data_t, block_scalers_t, gh, lora_a, rank, gx, M, N,
-                                         K, gemm ? rest : nullptr, gemm, stream);
+  // stage 2: gx = gy . D(W) + gh . A
+  return run_linear_bwd_dx(gy, quantized_data, block_scalers, quantized_data_t, block_scalers_t, gh, lora_a, rank, gx, M, N, K, plan, rest,
+                           reinterpret_cast<hipStream_t>(stream));
 }
