@@ -768,6 +768,16 @@ def test_layer_calls_ask_for_the_slabs_that_their_plans_write(M):
                 assert lib.ttamd_nf4_group_bwd_dx_workspace_bytes(group, len(widths), M, K) == (count * M * K * 4 if count > 1 else 0)
 
 
+@pytest.mark.parametrize("N,K,rank", [(1024, 1024, 8), (4096, 4096, 16), (4096, 14336, 16), (1024, 4096, 64)])
+def test_adapter_gradients_of_one_launch_ask_for_no_partial_sums(N, K, rank):
+    """Up to 2048 rows gA and gB leave finished, and what is asked for are gh's partial sums; the row splits of more rows need
+    rank * (N + K) floats each."""
+    q = _lib.load().ttamd_lora_bwd_workspace_bytes
+    assert q(2049, N, K, rank) >= 2 * rank * (N + K) * 4
+    for M in (48, 333, 700, 2048):
+        assert 0 < 4 * q(M, N, K, rank) <= q(2049, N, K, rank)
+
+
 def test_planning_a_group_costs_the_host_little():
     """The time of the query beside that of one which plans nothing (many tokens), the least of twenty: 0.2 - 0.3 us for three members
     of 4096 x 4096; a search over every slicing, twice for each member and again for the group, took 3."""

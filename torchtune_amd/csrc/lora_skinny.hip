@@ -13,6 +13,7 @@
 // put enough loads in flight and combine the fp32 partial sums in a second, fixed-order pass, so results
 // are deterministic (up to 2048 rows gA and gB are finished in one launch: skinny_tn_whole_kernel).  For wide layers of rank <= 16 the two products that read gy (gh and gB) come from one pass over
 // it (skinny_tn_gh_kernel).
+#include <algorithm>
 #include <atomic>
 #include "common.h"
 #include "group.h"
@@ -1539,8 +1540,8 @@ size_t group_lora_bwd_ws_bytes(const GroupSkinny& g) {
     widths[1 + i] = g.N[i];
     ranks[1 + i] = g.rank[i];
   }
-  const size_t tn = tn_part_bytes(g.M, 1 + g.n, widths, ranks);
-  return align256(nt > tn ? nt : tn);
+  const size_t tn = tn_whole_pays(g) ? 0 : tn_part_bytes(g.M, 1 + g.n, widths, ranks);
+  return align256(std::max({nt, tn, size_t(1)}));  // the calls want a workspace, however little of it they use
 }
 
 int run_group_lora_bwd(const uint16_t* x, const uint16_t* h_cat, const GroupSkinny& g, uint16_t* gh_cat, float* ws, hipStream_t s,
