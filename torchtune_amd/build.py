@@ -35,7 +35,6 @@ HIPCC_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wall",
     "-Wno-unused-function",
-    "-Wno-inline-asm",
 ]
 
 
@@ -62,8 +61,7 @@ def _compile_host(obj_dir: Path) -> Path:
 
     obj = obj_dir / "host_binding.o"
     cmd = [
-        shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
-    "-Wno-inline-asm", "-D__HIP_PLATFORM_AMD__=1",
+        shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function", "-D__HIP_PLATFORM_AMD__=1",
         "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-DTORCH_EXTENSION_NAME={HOST_MODULE}",
         *[f"-isystem{p}" for p in include_paths()], "-isystem/opt/rocm/include", f"-isystem{sysconfig.get_paths()['include']}",
         "-c", str(CSRC / "host_binding.cpp"), "-o", str(obj),
