@@ -73,7 +73,8 @@ def test_forward(M, N, K, rows, sliced, r):
 
 @pytest.mark.parametrize("M,K,N,rows,sliced", SIZES)
 def test_grad_input(M, K, N, rows, sliced):
-    assert _plan(M, K, N, forward=False)[0] == rows
+    got = _plan(M, K, N, forward=False)
+    assert got[0] == rows and (got[1] > 1) == sliced, got
     t = _Weight(N, K, M + N + K)
     D, g = t.dense, t.g
     gy = torch.randn(M, N, device=DEV, generator=g).to(BF)

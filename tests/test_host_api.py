@@ -474,8 +474,8 @@ def test_disable_adapter_and_adapter_state_dict():
 def test_gemm_workspace_query_is_a_host_function():
     """``ttamd_nf4_gemm_workspace_bytes`` needs no GPU: it is 0 where the launch uses no scratch memory (the few-token
     kernel: M <= 16, and M <= 32 on weights of at most 2^25 elements; launches with more than 128 tiles of 128 x 256 but
-    fewer than 256 of 256 x 256 or fewer than 2048 tokens; two-slice launches of a short contraction), slices * M * n_out * 4 bytes with 2 <= slices <= 16 and at least
-    four 64-wide k-steps per slice where the contraction is sliced, and 2 * n_out * k bytes (the weight expanded once)
+    fewer than 256 of 256 x 256 or fewer than 2048 tokens; two chains of a short contraction), a slab of M * n_out * 4 bytes for each of
+    2 - 16 chains of sums, of at least four 64-wide k-steps, where the contraction has several, and 2 * n_out * k bytes (the weight expanded once)
     from 2048 tokens and 256 tiles of 256 x 256 up, which ``ttamd_nf4_gemm_expands_weight`` tells apart."""
     from torchtune_amd import _lib
 
