@@ -1196,7 +1196,7 @@ int launch_dense(DenseArgs& g, hipStream_t s) {
 // kernel, whose tiles have 128 rows, on 8B / 70B shapes):
 //   * at least a full round of tiles and 2048 tokens: always;
 //   * at least a full round and 1280 - 2047 tokens: where its rounds and the expansion cost less than the rounds of the
-//     fused kernel (part_filled_rounds_pay; a group's members are fused launches of their own);
+//     fused kernels (part_filled_rounds_pay; the members of a group are priced as launches of their own);
 //   * between half a round and a full one, from 1280 tokens: the fused kernel needs a second round of its tiles there
 //     (+ 60 %), one partly filled round of this kernel is 15 - 30 % faster;
 //   * up to half a round the fused kernel fills the chip in one round of its own and wins.
@@ -1214,6 +1214,11 @@ int64_t rounds_of(int64_t M, int64_t rows, int64_t Nout) { return (((M + rows - 
 // The gate / up pair of 14336 x 4096 at 1500 tokens takes 3 rounds here and 2 x 3 of the smaller tiles (its layer forward +
 // backward 1743 -> 1668 us); alone at that size 2 rounds and the expansion are no faster than 3 small ones, from 1665
 // tokens (4 small ones or 2 full) they are: 1900 tokens 217 -> 196 us.
+// The prices of the smaller tiles are those of four-wave kernels; nf4_gemm_mid_kernel's eight waves cost the same a round at 4096 steps
+// (its terms: 5.2 + 64 x 0.915 = 63.8) and less where the contraction is short.  Both sides now, us, here / fused: pair of 14336 x 4096 at
+// 1500 329 / 386, at 2000 415 / 435, of 9728 x 3584 at 1500 208 / 194, at 2000 269 / 294, of 8192 x 2048 at 1500 114 / 109, of 6912 x
+// 2560 at 1500 139 / 122; 14336 x 4096 alone at 1900 214 / 222.  The line stays where it was drawn; moving it for short contractions is
+// worth 4 - 15 % of such pairs and changes the order of their sums.
 bool part_filled_rounds_pay(int64_t M, const int64_t* N, int n) {
   if (M < kDenseMinRowsPartRound || M >= kDenseMinRows) return false;
   int64_t n_total = 0;

@@ -665,8 +665,9 @@ int64_t tiles_of(int rows, int64_t M, int64_t Nout) { return ((M + rows - 1) / r
 }  // namespace
 
 // Wide forwards (a gate or up projection: outputs twice the contraction and more) whose pair fills half the chip with whole
-// contractions stay whole: slices gain one of them 10 % (8192 x 3072 at 333 tokens 41 -> 37 us) and cost the pair's one launch, whose
-// members keep their own slices, 35 % (59 -> 80).
+// contractions stay whole.  Slices gain one of them 4 % mostly and up to 17 (nine widths at 150 - 800 tokens, us: 8192 x 3072 at 260 36.6 ->
+// 32.6, 9728 x 3584 at 200 41.8 -> 34.8, at 384 44.7 -> 46.5) and cost the pair's one launch, whose members keep their own slices,
+// 14 - 60 % (42.1 -> 64.7, 47.1 -> 67.9, 6912 x 2560 at 384 40.0 -> 64.0).
 //
 // The query and the call plan anew, and a pass of small layers waits for the host: the search ends where the slabs alone cost more
 // than the best plan so far (0.05 - 0.2 us; all 48 plans took 0.2 - 0.4).

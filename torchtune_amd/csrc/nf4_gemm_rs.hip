@@ -979,7 +979,8 @@ size_t slabs_bytes(int slabs, int64_t M, int64_t Nout) { return slabs > 1 ? (siz
 // 4096 at 1000 tokens 108 against 124 on tiles of 128 rows, at 1500 (a second, part-filled round) 204 against 192; grad-input of
 // 4096 x 14336 at 900 112 and 127.
 // A 256-row tile adds the whole contraction in one chain, the other tiles' wave groups half of it each.  The longer chain is
-// admitted only where 256-row tiles take fewer than 5/9 of the rounds of 128-row ones (a round of theirs costs 1.8).
+// admitted only where 256-row tiles take fewer than 5/9 of the rounds of 128-row ones (a round of theirs costs 1.8): beyond, at more
+// than 16384 outputs, it gained 1 - 5 % (28672 x 8192 at 1200 tokens 609 -> 581 us) and had 1.5 times the rounding error.
 bool wide_tiles_pay(int64_t M, int64_t Nout, int64_t Kc, double mid_cost) {
   if (nmid_min_chains(M, Nout, Kc) > 1) return false;
   const int64_t tiles_n = (Nout + kBN - 1) / kBN, tiles = ((M + 255) / 256) * tiles_n;

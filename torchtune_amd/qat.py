@@ -635,9 +635,9 @@ def _int4_kernels_apply(x: torch.Tensor, weight: torch.Tensor, in_features: int,
     if bias is not None and (bias.dtype != torch.bfloat16 or not bias.is_cuda or (bias.requires_grad and torch.is_grad_enabled())):
         return False
     rows, N = x.numel() // in_features, weight.shape[0]
-    # Wide layers of more than 192 tokens keep the dense weight, whose product they have always had: the line was drawn where tiles
-    # of 16 tokens per product lost to the two passes (us at 200 tokens, uint4: 28672 x 8192 280 and 255).  The present ones are
-    # ahead beyond it as well (205 and 296; int8 242 and 262).
+    # Wide layers of more than 192 tokens keep the dense weight.  The line was drawn where tiles of 16 tokens per product lost to the
+    # two passes (us at 200 tokens, uint4: 28672 x 8192 280 and 255); the present kernels' tiles of 32 do not (205 and 296; int8 242 and
+    # 262).  A test holds the line: which products are the library's.
     if rows > 192 and N > 16384:
         return False
     return weight.is_contiguous() and ops.int4_linear_applies(rows, N, in_features, groupsize)
