@@ -729,6 +729,7 @@ def test_plans_of_fused_nf4_products_keep_their_chains_and_fit_the_workspace():
             assert not by_128 or M <= 32 or lib.ttamd_nf4_gemm_workspace_bytes(M, N, K) >= need
             whole = _nf4_gemm_plan(M, N, K, 0, by_128, forward)
             assert whole[1] == 1 and whole[2] <= _longest_chain(M, N, K, False), (M, N, K, whole)
+            assert slices > 1 or whole == plan  # what needs no memory runs without
 
 
 def _group_of(widths):

@@ -1036,8 +1036,12 @@ extern "C" int ttamd_nf4_gemm_plan(int64_t M, int64_t n_out, int64_t k_contract,
   if (dense_path_applies(M, n_out, k_contract)) return fail(TTAMD_EUNSUPPORTED, "nf4_gemm_plan: a product on the expanded weight");
   GemmPlan f = {};
   double cost;
-  if (by_128) f = fused_plan(M, n_out, k_contract, may_slice ? kAnyScratch : 0, forward != 0);
-  else f.mid = nmid_plan(M, n_out, k_contract, may_slice != 0, false, forward != 0, &cost);
+  if (by_128) {
+    f = fused_plan(M, n_out, k_contract, may_slice ? kAnyScratch : 0, forward != 0);
+  } else {  // as plan_gemm_rs_group_dx
+    f.mid = nmid_plan(M, n_out, k_contract, true, false, forward != 0, &cost);
+    if (!may_slice && f.mid.slices > 1) f.mid = nmid_plan(M, n_out, k_contract, false, false, forward != 0, &cost);
+  }
   const NMidPlan& p = f.mid;
   *tile_rows = f.wide ? 256 : p.rows;
   *slices = p.slices;
